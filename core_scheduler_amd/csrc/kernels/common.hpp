@@ -116,6 +116,20 @@ __device__ __forceinline__ void store16_stream(T *p, const Vec16<T> &v) {
   store_stream(reinterpret_cast<u32x4 *>(p), __builtin_bit_cast(u32x4, v));
 }
 
+// 16-byte accesses at any element boundary (gfx950 takes them at every byte address; a wave's
+// access then touches one cache line more).
+typedef uint32_t u32x4_at2 __attribute__((ext_vector_type(4), aligned(2)));
+template <typename T>
+__device__ __forceinline__ Vec16<T> load16_unaligned_stream(const T *p) {
+  const u32x4 raw = __builtin_nontemporal_load(reinterpret_cast<const u32x4_at2 *>(p));
+  return __builtin_bit_cast(Vec16<T>, raw);
+}
+template <typename T>
+__device__ __forceinline__ void store16_unaligned_stream(T *p, const Vec16<T> &v) {
+  const u32x4 raw = __builtin_bit_cast(u32x4, v);
+  __builtin_nontemporal_store(raw, reinterpret_cast<u32x4_at2 *>(p));
+}
+
 __host__ __device__ __forceinline__ bool is_aligned16(const void *p) {
   return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
 }

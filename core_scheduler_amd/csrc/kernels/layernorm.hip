@@ -19,9 +19,9 @@
 // per workgroup, and a second small kernel adds the partial rows in a fixed
 // order, so the result does not depend on scheduling and uses no atomics.
 //
-// Anything the fast path cannot take (C not a multiple of the vector width,
-// C beyond the register budget, unaligned pointers, fp64) goes through a
-// plain one-workgroup-per-row path.
+// Rows wider than one wave's registers, rows that are not whole vectors and unaligned pointers go
+// through the same scheme with several waves per row (ln_fwd_block_kernel, ln_bwd_block_kernel);
+// fp64 and rows beyond 16384 columns through a plain one-workgroup-per-row path.
 #include "common.hpp"
 
 #include <math.h>
@@ -379,14 +379,14 @@ struct LnPending {
 // latency), then row 0 adds the 16 sub-sums in order.  `sub` is 16 x 32 floats of LDS.
 constexpr int kLnFinCols = 32, kLnFinRows = 16, kLnFinInFlight = 16;
 
-template <typename TP, int THREADS = kLnFinCols * kLnFinRows>
+template <typename TP, int THREADS = kLnFinCols * kLnFinRows, typename A = float>
 __device__ __forceinline__ void ln_finalize_tile(const float *__restrict__ partial, int nparts, TP *__restrict__ out,
-                                                 int which, int tile, int C, int vn, int accumulate, float *sub,
+                                                 int which, int tile, int C, int vn, int accumulate, A *sub,
                                                  int tid) {
   static_assert(THREADS >= kLnFinCols * kLnFinRows, "a tile takes 512 threads; further ones only join the barrier");
   const int cx = tid % kLnFinCols, ry = tid / kLnFinCols;
   const int col = tile * kLnFinCols + cx;  // a position in the permuted row
-  float s = 0.f;
+  A s = 0;
   if (col < C && ry < kLnFinRows) {
     const float *src = partial + (int64_t)which * C + col;
     const int64_t stride = 2 * (int64_t)C;
@@ -398,28 +398,28 @@ __device__ __forceinline__ void ln_finalize_tile(const float *__restrict__ parti
         v[u] = src[(int64_t)(p < nparts ? p : nparts - 1) * stride];
       }
 #pragma unroll
-      for (int u = 0; u < kLnFinInFlight; ++u) s += p0 + u * kLnFinRows < nparts ? v[u] : 0.f;
+      for (int u = 0; u < kLnFinInFlight; ++u) s += (A)(p0 + u * kLnFinRows < nparts ? v[u] : 0.f);
     }
   }
   if (ry < kLnFinRows) sub[ry * kLnFinCols + cx] = s;
   __syncthreads();
   if (ry == 0 && col < C) {
-    float t = 0.f;
+    A t = 0;
 #pragma unroll
     for (int r = 0; r < kLnFinRows; ++r) t += sub[r * kLnFinCols + cx];
     const int nvec = C / vn;
     const int real = (col % nvec) * vn + col / nvec;  // the column this position stands for
-    if (accumulate) t += to_acc(out[real]);
-    out[real] = from_acc<TP>(t);
+    if (accumulate) t += (A)to_acc(out[real]);
+    out[real] = from_acc<TP>((float)t);
   }
 }
 // workgroup b of the 2 * ceil(C/32) that cover a pending call: even b dgamma, odd b dbeta
-template <typename TP, int THREADS = kLnFinCols * kLnFinRows>
-__device__ __forceinline__ void ln_finalize_pending(const LnPending &pend, int b, int C, int vn, float *sub, int tid) {
+template <typename TP, int THREADS = kLnFinCols * kLnFinRows, typename A = float>
+__device__ __forceinline__ void ln_finalize_pending(const LnPending &pend, int b, int C, int vn, A *sub, int tid) {
   const int which = b & 1;
   TP *out = (TP *)(which == 0 ? pend.dgamma : pend.dbeta);
   if (out == nullptr) return;  // block-uniform
-  ln_finalize_tile<TP, THREADS>(pend.partial, pend.nparts, out, which, b >> 1, C, vn, pend.accumulate, sub, tid);
+  ln_finalize_tile<TP, THREADS, A>(pend.partial, pend.nparts, out, which, b >> 1, C, vn, pend.accumulate, sub, tid);
 }
 
 // ----------------------------------------------------------- fast backward
@@ -433,9 +433,7 @@ __device__ __forceinline__ void ln_finalize_pending(const LnPending &pend, int b
 // variant of the kernel rounds alike): 17 VALU operations per element instead of 27, which
 // matters because at 16-bit storage this kernel is as close to its VALU limit as to HBM's.
 // HAS_DRES: dx_out = dx + dresidual, the gradient add that follows LayerNorm::backward on the
-// residual stream; dx is rounded to its type first, then the sum, as two kernels would.  Only
-// instantiated for the 2-vectors-per-lane plan: wider rows have no registers left for a third
-// input, and there the add runs as its own launch.
+// residual stream; dx is rounded to its type first, then the sum, as two kernels would.
 template <typename TDY, typename TX, typename TDX, typename TP, int VPL, int WPE, bool HAS_DX,
           bool HAS_DP, bool HAS_DRES>
 __global__ __launch_bounds__(kLnBwdThreads, WPE) void ln_bwd_rows_kernel(
@@ -770,88 +768,319 @@ __global__ __launch_bounds__(THREADS, WPE) void ln_bwd_kernel(
   }
 }
 
-// ------------------------------------------------- wide rows: two waves per row
-// Rows of 5 to 8 vectors per lane do not fit one wave's registers once the dgamma/dbeta
-// accumulators are there, so a pair of waves shares a row: wave h of the pair (h = 0, 1) owns
-// vectors lane + 64*(2j + h), j < VPLH.  The two halves of the row sums meet in the LDS (one
-// barrier per row; every pair makes the same number of steps so that all waves reach it).
-template <typename T, int VN, int VPLH>
-struct HalfRow {
-  Raw<T, VN> v[VPLH];
-};
-template <typename T, int VN, int VPLH>
-__device__ __forceinline__ void load_half_row(HalfRow<T, VN, VPLH> &dst, const T *__restrict__ src,
-                                              int64_t row, bool valid, int C, int nvec, int lane, int h) {
+// --------------------------------------------------- rows on several waves
+// Rows wider than the register plans above, and rows of any width that are not whole aligned
+// vectors.  A row belongs to a group of `gw` waves (1 to 16), lane i of the group's 64*gw lanes
+// owning vectors i, i + 64*gw, ... (VPT of them); a workgroup holds as many groups as fit and walks
+// rows.  UA: rows may start anywhere: vectors are accessed at element alignment, and the columns past
+// the last whole vector (fewer than one vector of them) are single elements of the group's first
+// lanes, which load them unconditionally (a load under a lane's condition would hold up the others).
+//
+// Bound by HBM; what it took to get near was the number of loads in flight.  A wave-sized row slice
+// per wave and 8 elements per lane leave registers for two rows (the next one requested as soon as
+// the one before the current is done), gamma, beta or the column sums.  [4096,5120] bf16 with the
+// residual: forward 31.9 us (5.3 TB/s; one workgroup per row behind a separate add 64 us), backward
+// 41.6 us (4.0 TB/s without the partial rows' 21 MB; 382 us with the plain kernels, whose column sums
+// ran on 80 workgroups).  [12000,1003] fp32: 38.9 + 40.1 us against 58.5 + 1121.
+template <typename T, int N, bool UA>
+__device__ __forceinline__ Raw<T, N> load_piece(const T *p) {
+  Raw<T, N> r;
 #pragma unroll
-  for (int j = 0; j < VPLH; ++j) {
-    const int idx = lane + kWave * (2 * j + h);
-    if (valid && idx < nvec) {
-      dst.v[j] = load_raw<T, VN>(src + row * C + (int64_t)idx * VN);
+  for (int q = 0; q < N / Vec16<T>::n; ++q) {
+    if constexpr (UA) {
+      r.v[q] = load16_unaligned_stream(p + q * Vec16<T>::n);
     } else {
-      dst.v[j] = zero_raw<T, VN>();
+      r.v[q] = load16_stream(p + q * Vec16<T>::n);
+    }
+  }
+  return r;
+}
+template <typename T, int N, bool UA>
+__device__ __forceinline__ void store_piece(T *p, const float (&in)[N]) {
+  constexpr int VN = Vec16<T>::n;
+#pragma unroll
+  for (int q = 0; q < N / VN; ++q) {
+    Vec16<T> v;
+#pragma unroll
+    for (int k = 0; k < VN; ++k) v.e[k] = from_acc<T>(in[q * VN + k]);
+    if constexpr (UA) {
+      store16_unaligned_stream(p + q * VN, v);
+    } else {
+      store16_stream(p + q * VN, v);
+    }
+  }
+}
+// One lane's share of a row: VPT vectors and, with UA, one single element.
+template <typename T, int VN, int VPT, bool UA>
+struct Share {
+  Raw<T, VN> v[VPT];
+  T e;
+};
+// Which columns a lane owns.
+template <int VN, int VPT, bool UA>
+struct Lanes {
+  int at[VPT];   // first column of each vector (a lane without a vector re-reads the row's last one)
+  bool has[VPT];
+  int ecol;      // the single element's column
+  bool ehas;
+  __device__ __forceinline__ Lanes(int C, int gw, int lane_in_group) {
+    const int nvec = C / VN;
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+      const int idx = lane_in_group + kWave * gw * j;
+      has[j] = idx < nvec;
+      at[j] = (has[j] ? idx : nvec - 1) * VN;
+      if (UA && nvec == 0) at[j] = 0;
+    }
+    const int tail = C - nvec * VN;
+    ehas = UA && lane_in_group < tail;
+    ecol = nvec * VN + (lane_in_group < tail ? lane_in_group : 0);
+    if (ecol >= C) ecol = C - 1;
+  }
+};
+template <typename T, int VN, int VPT, bool UA>
+__device__ __forceinline__ void load_share(Share<T, VN, VPT, UA> &s, const T *row, const Lanes<VN, VPT, UA> &l,
+                                           bool any_vec) {
+  if (!UA || any_vec) {  // grid-uniform: with fewer than VN columns there is no vector to read
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) s.v[j] = load_piece<T, VN, UA>(row + l.at[j]);
+  }
+  if constexpr (UA) s.e = row[l.ecol];
+}
+
+// Sums of A over the lanes of a group; `red` holds one A per wave of the workgroup.  Every wave of
+// the workgroup must call it.  The caller alternates between two arrays, so one barrier is enough.
+template <typename A>
+__device__ __forceinline__ A group_sum(A v, int gw, int wave, int first_wave, int lane, A *red) {
+  v = wave_reduce(v, SumOp{});
+  if (gw == 1) return v;  // workgroup-uniform
+  if (lane == 0) red[wave] = v;
+  lds_barrier();
+  const A r = red[first_wave + (lane < gw ? lane : 0)];
+  return wave_reduce(lane < gw ? r : (A)0, SumOp{});
+}
+
+constexpr int kLnBlockMaxWaves = 16;
+
+template <typename TX, typename TY, typename TP, int VPT, bool HAS_RES, bool UA>
+__global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
+    const TX *x /* sum_out may be x: not restrict */, const TP *__restrict__ gamma, const TP *__restrict__ beta,
+    TY *__restrict__ y, float *__restrict__ mean, float *__restrict__ rstd, int64_t rows, int C, float eps,
+    const TX *res, TX *sum_out, int gw, int groups) {
+  constexpr int VN = Vec16<TX>::n;
+  __shared__ float red[2][kLnBlockMaxWaves];
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+  const int group = wave / gw, lig = threadIdx.x - group * gw * kWave;
+  const bool any_vec = C >= VN;
+  const Lanes<VN, VPT, UA> own(C, gw, lig);
+  const float inv_c = 1.0f / (float)C;
+  const int64_t stride = (int64_t)gridDim.x * groups;
+  const int64_t steps = (rows + stride - 1) / stride;  // the same for every group: they share barriers
+  int64_t row = (int64_t)blockIdx.x * groups + group;
+
+  // Two rows' registers: a row is requested as soon as the registers of the one two steps before it
+  // are free, so that one row is on its way while another is worked on.
+  struct Row {
+    Share<TX, VN, VPT, UA> x, res;
+  };
+  auto fetch = [&](Row &d, int64_t r) {
+    const int64_t at = (r < rows ? r : rows - 1) * C;
+    load_share(d.x, x + at, own, any_vec);
+    if constexpr (HAS_RES) load_share(d.res, res + at, own, any_vec);
+  };
+  Row even, odd;
+  fetch(even, row);
+  if (steps > 1) fetch(odd, row + stride);
+  float g[VPT][VN], b[VPT][VN], ge = 0.f, be = 0.f;
+#pragma unroll
+  for (int j = 0; j < VPT; ++j) {
+#pragma unroll
+    for (int k = 0; k < VN; ++k) g[j][k] = b[j][k] = 0.f;
+    if (own.has[j]) {
+      if constexpr (UA) {
+#pragma unroll
+        for (int k = 0; k < VN; ++k) g[j][k] = to_acc(gamma[own.at[j] + k]);
+        if (beta)
+#pragma unroll
+          for (int k = 0; k < VN; ++k) b[j][k] = to_acc(beta[own.at[j] + k]);
+      } else {
+        load_n<TP, VN>(gamma + own.at[j], g[j]);
+        if (beta) load_n<TP, VN>(beta + own.at[j], b[j]);
+      }
+    }
+  }
+  if constexpr (UA) {
+    ge = to_acc(gamma[own.ecol]);
+    if (beta) be = to_acc(beta[own.ecol]);
+  }
+  auto work = [&](Row &in, int64_t row) {
+    Share<TX, VN, VPT, UA> &cur = in.x, &rcur = in.res;
+    const bool row_ok = row < rows;
+    const int64_t at = row * C;
+    if constexpr (HAS_RES) {
+      // cur = x + residual, one fp32 add and one rounding per element, as an add launch would give
+#pragma unroll
+      for (int j = 0; j < VPT; ++j) {
+        Vec16<TX> sum;
+#pragma unroll
+        for (int k = 0; k < VN; ++k)
+          sum.e[k] = from_acc<TX>(raw_get<TX, VN>(cur.v[j], k) + raw_get<TX, VN>(rcur.v[j], k));
+        cur.v[j].v[0] = sum;
+        if (own.has[j] && row_ok) {
+          if constexpr (UA) {
+            store16_unaligned_stream(sum_out + at + own.at[j], sum);
+          } else {
+            store16_stream(sum_out + at + own.at[j], sum);
+          }
+        }
+      }
+      if constexpr (UA) {
+        cur.e = from_acc<TX>(to_acc(cur.e) + to_acc(rcur.e));
+        if (own.ehas && row_ok) sum_out[at + own.ecol] = cur.e;
+      }
+    }
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+      float t = 0.f;
+#pragma unroll
+      for (int k = 0; k < VN; ++k) t += raw_get<TX, VN>(cur.v[j], k);
+      s += own.has[j] ? t : 0.f;
+    }
+    if constexpr (UA) s += own.ehas ? to_acc(cur.e) : 0.f;
+    const float mu = group_sum(s, gw, wave, group * gw, lane, red[0]) * inv_c;
+    float q = 0.f;
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+      float t = 0.f;
+#pragma unroll
+      for (int k = 0; k < VN; ++k) {
+        const float d = raw_get<TX, VN>(cur.v[j], k) - mu;
+        t += d * d;
+      }
+      q += own.has[j] ? t : 0.f;
+    }
+    if constexpr (UA) {
+      const float d = to_acc(cur.e) - mu;
+      q += own.ehas ? d * d : 0.f;
+    }
+    const float rs = 1.0f / sqrtf(group_sum(q, gw, wave, group * gw, lane, red[1]) * inv_c + eps);
+    if (row_ok) {
+      if (lig == 0) {
+        mean[row] = mu;
+        rstd[row] = rs;
+      }
+#pragma unroll
+      for (int j = 0; j < VPT; ++j) {
+        if (own.has[j]) {
+          float o[VN];
+#pragma unroll
+          for (int k = 0; k < VN; ++k) o[k] = (raw_get<TX, VN>(cur.v[j], k) - mu) * rs * g[j][k] + b[j][k];
+          store_piece<TY, VN, UA>(y + at + own.at[j], o);
+        }
+      }
+      if constexpr (UA) {
+        if (own.ehas) y[at + own.ecol] = from_acc<TY>((to_acc(cur.e) - mu) * rs * ge + be);
+      }
+    }
+  };
+  for (int64_t it = 0; it < steps; it += 2, row += 2 * stride) {
+    work(even, row);
+    if (it + 2 < steps) fetch(even, row + 2 * stride);
+    if (it + 1 < steps) {
+      work(odd, row + stride);
+      if (it + 3 < steps) fetch(odd, row + 3 * stride);
     }
   }
 }
 
-template <typename TDY, typename TX, typename TDX, typename TP, int VPLH, bool HAS_DX, bool HAS_DP>
-__global__ __launch_bounds__(kLnBwdThreads) void ln_bwd_split_rows_kernel(
+// Backward of the same rows.  The column sums of a lane's own columns stay in registers over all the
+// rows it visits, in double: they may span thousands of rows, and at full-rate fp64 the two adds per
+// element cost no time next to the row's traffic.  The groups of a workgroup meet in the LDS, one
+// fp32 partial row (columns in order) leaves per workgroup.
+// Whether a lane's next row fits the registers (128 at 16 waves a workgroup) next to its column sums,
+// gamma and the current row: requested a row ahead where it does.
+template <typename TDY, typename TX, typename TDX, int E, bool HAS_DP, bool HAS_DRES, bool UA>
+constexpr bool bwd_block_prefetches() {
+  const int row = E * (int)(sizeof(TDY) + sizeof(TX) + (HAS_DRES ? sizeof(TDX) : 0)) / 4;
+  return (HAS_DP ? 4 * E : 0) + E + 2 * row <= (UA ? 60 : 70);
+}
+template <typename TDY, typename TX, typename TDX, typename TP, int VPT, bool HAS_DX, bool HAS_DP, bool HAS_DRES,
+          bool UA>
+__global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_bwd_block_kernel(
     const TDY *__restrict__ dy, const TX *__restrict__ x, const float *__restrict__ mean,
-    const float *__restrict__ rstd, const TP *__restrict__ gamma, TDX *__restrict__ dx,
-    float *__restrict__ partial, int64_t rows, int C) {
+    const float *__restrict__ rstd, const TP *__restrict__ gamma, TDX *dx /* may be dres */,
+    float *__restrict__ partial, int64_t rows, int C, const TDX *dres, int gw, int groups) {
   constexpr int VN = Vec16<TX>::n;
-  constexpr int kWaves = kLnBwdThreads / kWave;
-  constexpr int kPairs = kWaves / 2;
-  constexpr int kRegion = VPLH * kWave * VN;  // floats one wave contributes to the fold
-  extern __shared__ float lds[];              // [kPairs][kRegion], one half of the row at a time
-  __shared__ float halves[2][kPairs][2][2];   // [parity][pair][half][s1, s2]
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x >> 6;
-  const int pair = wave >> 1, h = wave & 1;
-  const int64_t n_pairs = (int64_t)gridDim.x * kPairs;
-  const int64_t gp = (int64_t)blockIdx.x * kPairs + pair;
-  const int64_t steps = (rows + n_pairs - 1) / n_pairs;  // the same for every pair
-  const int nvec = C / VN;
+  constexpr bool PF = bwd_block_prefetches<TDY, TX, TDX, VPT * VN, HAS_DP, HAS_DRES, UA>();
+  extern __shared__ float lds[];  // [groups][C] for the fold
+  __shared__ float red[2][2][kLnBlockMaxWaves];
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+  const int group = wave / gw, lig = threadIdx.x - group * gw * kWave;
+  const bool any_vec = C >= VN;
+  const Lanes<VN, VPT, UA> own(C, gw, lig);
   const float inv_c = 1.0f / (float)C;
+  const int64_t stride = (int64_t)gridDim.x * groups;
+  const int64_t steps = (rows + stride - 1) / stride;
+  int64_t row = (int64_t)blockIdx.x * groups + group;
 
-  float acc_g[VPLH][VN], acc_b[VPLH][VN], g[VPLH][VN];
+  struct Row {
+    Share<TDY, VN, VPT, UA> dy;
+    Share<TX, VN, VPT, UA> x;
+    Share<TDX, VN, VPT, UA> res;
+    float mu, rs;
+  };
+  auto fetch = [&](Row &d, int64_t r) {
+    const int64_t rr = r < rows ? r : rows - 1;
+    load_share(d.dy, dy + rr * C, own, any_vec);
+    load_share(d.x, x + rr * C, own, any_vec);
+    if constexpr (HAS_DRES) load_share(d.res, dres + rr * C, own, any_vec);
+    d.mu = mean[rr];
+    d.rs = rstd[rr];
+  };
+  Row even, odd;  // as in the forward kernel, where both fit
+  fetch(even, row);
+  if (PF && steps > 1) fetch(odd, row + stride);
+  double acc_g[VPT][VN], acc_b[VPT][VN], eacc_g = 0., eacc_b = 0.;
+  float g[VPT][VN], ge = 0.f;
 #pragma unroll
-  for (int j = 0; j < VPLH; ++j) {
-    const int idx = lane + kWave * (2 * j + h);
+  for (int j = 0; j < VPT; ++j) {
 #pragma unroll
     for (int k = 0; k < VN; ++k) {
-      acc_g[j][k] = 0.f;
-      acc_b[j][k] = 0.f;
+      acc_g[j][k] = 0.;
+      acc_b[j][k] = 0.;
       g[j][k] = 0.f;
     }
-    if (HAS_DX && idx < nvec) load_n<TP, VN>(gamma + idx * VN, g[j]);
+    if (HAS_DX && own.has[j]) {
+      if constexpr (UA) {
+#pragma unroll
+        for (int k = 0; k < VN; ++k) g[j][k] = to_acc(gamma[own.at[j] + k]);
+      } else {
+        load_n<TP, VN>(gamma + own.at[j], g[j]);
+      }
+    }
   }
+  if constexpr (UA && HAS_DX) ge = to_acc(gamma[own.ecol]);
 
-  HalfRow<TDY, VN, VPLH> dcur;
-  HalfRow<TX, VN, VPLH> xcur;
-  int64_t row = gp;
-  load_half_row<TDY, VN, VPLH>(dcur, dy, row, row < rows, C, nvec, lane, h);
-  load_half_row<TX, VN, VPLH>(xcur, x, row, row < rows, C, nvec, lane, h);
-  float mu = row < rows ? mean[row] : 0.f, rs = row < rows ? rstd[row] : 0.f;
   int parity = 0;
-  for (int64_t it = 0; it < steps; ++it, row += n_pairs) {
-    const int64_t nrow = row + n_pairs;
-    HalfRow<TDY, VN, VPLH> dnxt;
-    HalfRow<TX, VN, VPLH> xnxt;
-    load_half_row<TDY, VN, VPLH>(dnxt, dy, nrow, nrow < rows, C, nvec, lane, h);
-    load_half_row<TX, VN, VPLH>(xnxt, x, nrow, nrow < rows, C, nvec, lane, h);
-    const float nmu = nrow < rows ? mean[nrow] : 0.f, nrs = nrow < rows ? rstd[nrow] : 0.f;
-
-    // a row past the end is all zeros here: it adds nothing and stores nothing
+  auto work = [&](Row &in, int64_t row) {
+    Share<TDY, VN, VPT, UA> &dcur = in.dy;
+    Share<TX, VN, VPT, UA> &xcur = in.x;
+    Share<TDX, VN, VPT, UA> &rcur = in.res;
+    const float mu = in.mu, rs = in.rs;
+    const bool row_ok = row < rows;
     float s1 = 0.f, s2 = 0.f;
 #pragma unroll
-    for (int j = 0; j < VPLH; ++j) {
+    for (int j = 0; j < VPT; ++j) {
+      const bool live = own.has[j] && row_ok;
 #pragma unroll
       for (int k = 0; k < VN; ++k) {
-        const float xh = (raw_get<TX, VN>(xcur.v[j], k) - mu) * rs;
-        const float dv = raw_get<TDY, VN>(dcur.v[j], k);
+        // both masked: 0 * inf would leave a NaN in the sums
+        const float xh = live ? (raw_get<TX, VN>(xcur.v[j], k) - mu) * rs : 0.f;
+        const float dv = live ? raw_get<TDY, VN>(dcur.v[j], k) : 0.f;
         if constexpr (HAS_DP) {
-          acc_g[j][k] = __builtin_fmaf(dv, xh, acc_g[j][k]);
-          acc_b[j][k] += dv;
+          acc_g[j][k] += (double)(dv * xh);
+          acc_b[j][k] += (double)dv;
         }
         if constexpr (HAS_DX) {
           const float gd = dv * g[j][k];
@@ -860,71 +1089,98 @@ __global__ __launch_bounds__(kLnBwdThreads) void ln_bwd_split_rows_kernel(
         }
       }
     }
+    float exh = 0.f, edv = 0.f;
+    if constexpr (UA) {
+      const bool live = own.ehas && row_ok;
+      exh = live ? (to_acc(xcur.e) - mu) * rs : 0.f;
+      edv = live ? to_acc(dcur.e) : 0.f;
+      if constexpr (HAS_DP) {
+        eacc_g += (double)(edv * exh);
+        eacc_b += (double)edv;
+      }
+      if constexpr (HAS_DX) {
+        const float gd = edv * ge;
+        s1 += gd;
+        s2 = __builtin_fmaf(gd, exh, s2);
+      }
+    }
     if constexpr (HAS_DX) {
       s1 = wave_reduce(s1, SumOp{});
       s2 = wave_reduce(s2, SumOp{});
-      if (lane == 0) {
-        halves[parity][pair][h][0] = s1;
-        halves[parity][pair][h][1] = s2;
+      if (gw > 1) {  // workgroup-uniform
+        if (lane == 0) {
+          red[parity][0][wave] = s1;
+          red[parity][1][wave] = s2;
+        }
+        lds_barrier();
+        const int from = group * gw + (lane < gw ? lane : 0);
+        const float a = red[parity][0][from], c = red[parity][1][from];
+        s1 = wave_reduce(lane < gw ? a : 0.f, SumOp{});
+        s2 = wave_reduce(lane < gw ? c : 0.f, SumOp{});
+        parity ^= 1;  // the other pair next time: one barrier per row is enough
       }
-      __syncthreads();
-      // both waves of the pair add the halves in the same order
-      s1 = (halves[parity][pair][0][0] + halves[parity][pair][1][0]) * inv_c;
-      s2 = (halves[parity][pair][0][1] + halves[parity][pair][1][1]) * inv_c;
-      parity ^= 1;  // the other buffer next step: one barrier per row is enough
-      if (row < rows) {
+      s1 *= inv_c;
+      s2 *= inv_c;
+      if (row_ok) {
 #pragma unroll
-        for (int j = 0; j < VPLH; ++j) {
-          forget_unpacked(xcur.v[j]);
-          forget_unpacked(dcur.v[j]);
-          const int idx = lane + kWave * (2 * j + h);
-          if (idx < nvec) {
+        for (int j = 0; j < VPT; ++j) {
+          if (own.has[j]) {
             float o[VN];
 #pragma unroll
             for (int k = 0; k < VN; ++k) {
               const float xh = (raw_get<TX, VN>(xcur.v[j], k) - mu) * rs;
               const float dv = raw_get<TDY, VN>(dcur.v[j], k);
               o[k] = rs * __builtin_fmaf(-xh, s2, __builtin_fmaf(dv, g[j][k], -s1));
+              if constexpr (HAS_DRES) o[k] = round_through<TDX>(o[k]) + raw_get<TDX, VN>(rcur.v[j], k);
             }
-            store_n<TDX, VN>(dx + row * C + (int64_t)idx * VN, o);
+            store_piece<TDX, VN, UA>(dx + row * C + own.at[j], o);
+          }
+        }
+        if constexpr (UA) {
+          if (own.ehas) {
+            float o = rs * __builtin_fmaf(-exh, s2, __builtin_fmaf(edv, ge, -s1));
+            if constexpr (HAS_DRES) o = round_through<TDX>(o) + to_acc(rcur.e);
+            dx[row * C + own.ecol] = from_acc<TDX>(o);
           }
         }
       }
     }
-    dcur = dnxt;
-    xcur = xnxt;
-    mu = nmu;
-    rs = nrs;
+  };
+  if constexpr (PF) {
+    for (int64_t it = 0; it < steps; it += 2, row += 2 * stride) {
+      work(even, row);
+      if (it + 2 < steps) fetch(even, row + 2 * stride);
+      if (it + 1 < steps) {
+        work(odd, row + stride);
+        if (it + 3 < steps) fetch(odd, row + 3 * stride);
+      }
+    }
+  } else {
+    for (int64_t it = 0; it < steps; ++it, row += stride) {
+      work(even, row);
+      if (it + 1 < steps) fetch(even, row + stride);
+    }
   }
 
   if constexpr (HAS_DP) {
-    // fold the four waves that own the same half, one half at a time; positions inside a wave's
-    // region are k*(64 VPLH) + lane + 64 j (conflict-free writes); the partial rows use the
-    // permuted layout of the narrow kernel, position k*nvec + idx for column idx*VN + k
 #pragma unroll
     for (int which = 0; which < 2; ++which) {
+      float *mine = lds + (size_t)group * C;
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        if (h == hh) {
+      for (int j = 0; j < VPT; ++j) {
+        if (own.has[j]) {
 #pragma unroll
-          for (int j = 0; j < VPLH; ++j)
-#pragma unroll
-            for (int k = 0; k < VN; ++k)
-              lds[pair * kRegion + k * (kWave * VPLH) + lane + kWave * j] = which == 0 ? acc_g[j][k] : acc_b[j][k];
+          for (int k = 0; k < VN; ++k) mine[own.at[j] + k] = (float)(which == 0 ? acc_g[j][k] : acc_b[j][k]);
         }
-        __syncthreads();
-        for (int local = threadIdx.x; local < kRegion; local += kLnBwdThreads) {
-          const int k = local / (kWave * VPLH), li = local % (kWave * VPLH);
-          const int idx = (li % kWave) + kWave * (2 * (li / kWave) + hh);
-          if (idx < nvec) {
-            float sum = 0.f;
-#pragma unroll
-            for (int pp = 0; pp < kPairs; ++pp) sum += lds[pp * kRegion + local];
-            partial[((int64_t)blockIdx.x * 2 + which) * C + k * nvec + idx] = sum;
-          }
-        }
-        __syncthreads();
       }
+      if (UA && own.ehas) mine[own.ecol] = (float)(which == 0 ? eacc_g : eacc_b);
+      lds_barrier();
+      for (int c = threadIdx.x; c < C; c += blockDim.x) {
+        float t = 0.f;
+        for (int w = 0; w < groups; ++w) t += lds[(size_t)w * C + c];
+        partial[((int64_t)blockIdx.x * 2 + which) * C + c] = t;
+      }
+      if (which == 0) lds_barrier();
     }
   }
 }
@@ -932,13 +1188,13 @@ __global__ __launch_bounds__(kLnBwdThreads) void ln_bwd_split_rows_kernel(
 // The column sums as a launch of their own: grid 2 * ceil(C/32) workgroups of 32 x 16 threads, even
 // ones dgamma, odd ones dbeta (the same tiles, in the same order of additions, as the pending
 // form inside the row kernel's launch).
-template <typename TP>
+template <typename TP, typename A>
 __global__ __launch_bounds__(kLnFinCols *kLnFinRows) void ln_bwd_finalize_kernel(
     const float *__restrict__ partial, int nparts, TP *__restrict__ dgamma, TP *__restrict__ dbeta,
     int C, int vn, int accumulate) {
-  __shared__ float sub[kLnFinRows * kLnFinCols];
+  __shared__ A sub[kLnFinRows * kLnFinCols];
   const LnPending pend{partial, dgamma, dbeta, nparts, accumulate, (int)gridDim.x};
-  ln_finalize_pending<TP>(pend, blockIdx.x, C, vn, sub, threadIdx.x);
+  ln_finalize_pending<TP, kLnFinCols * kLnFinRows, A>(pend, blockIdx.x, C, vn, sub, threadIdx.x);
 }
 
 // ------------------------------------------------------ elementwise add
@@ -1100,12 +1356,11 @@ struct FastPlan {
   int vpl = 0;       // 0: not eligible
   int fwd_rows = 1;  // rows a wave normalises per step, forward
 };
-// The widest plan whose backward kernel still has registers for a third input per row
-// (dresidual); wider rows get dx + dresidual from a second launch.
-constexpr int kMaxVplWithResidual = 4;
-
-// x vectors per lane needed for C columns of x_dtype; the fast kernels are
-// instantiated for 1, 2, 4 and 8.
+// x vectors per lane needed for C columns of x_dtype when a wave owns whole rows; those kernels are
+// instantiated for 1, 2 and 4 (a fifth to eighth vector per lane measured slower than several waves
+// per row: [4096,3072] bf16 with the residual 23.5 + 37.0 us forward and backward against 20.8 + 27.0,
+// [8192,2048] fp32 46.7 + 73.9 against 47.1 + 50.2, without it [4096,4096] bf16 15.9 + 28.3 against
+// 15.2 + 27.3).
 FastPlan fast_plan(int64_t C, int x_dtype) {
   FastPlan p;
   const int vn = 16 / (int)dtype_size(x_dtype);
@@ -1121,9 +1376,6 @@ FastPlan fast_plan(int64_t C, int x_dtype) {
   } else if (per_lane <= 4) {
     p.vpl = 4;
     p.fwd_rows = CS_LN_FWD_ROWS_VPL4;
-  } else if (per_lane <= 8) {
-    p.vpl = 8;
-    p.fwd_rows = 1;
   }
   return p;
 }
@@ -1142,6 +1394,43 @@ int ln_blocks(int64_t rows, int rows_per_wave, int cap, int threads = kLnThreads
   const int64_t rows_per_block = (int64_t)(threads / kWave) * rows_per_wave;
   const int64_t b = ceil_div(rows, rows_per_block);
   return (int)(b < cap ? b : cap);
+}
+
+// Rows on several waves (ln_fwd_block_kernel, ln_bwd_block_kernel): everything the row-per-wave plans
+// do not take, up to 16 elements per lane of 1024 lanes, at any width and alignment.
+struct BlockPlan {
+  int vpt = 0;                      // 16-byte vectors per lane; 0: not eligible
+  int gw = 0, groups = 0, blocks = 0;  // waves per row, rows side by side in a workgroup, workgroups
+};
+constexpr size_t kLnBlockFoldLds = (size_t)16 * kLnBlockMaxWaves * kWave * sizeof(float);  // the widest row
+BlockPlan block_plan(int64_t rows, int64_t C, int x_dtype, bool backward, bool residual) {
+  BlockPlan p;
+  if (x_dtype == CS_F64 || C <= 0) return p;
+  const int vn = 16 / (int)dtype_size(x_dtype);
+  const int64_t nvec = C >= vn ? C / vn : 1;
+  // One vector per lane: [4096,5120] bf16 backward 41.6 us against 58.2 with two (registers), forward
+  // with the residual 31.9 against 38.1.  A forward without residual has half the loads in flight
+  // per row, and two pay where the row then still has two waves or more: [4096,4096] 15.2 against
+  // 16.5, [4096,2304] 11.2 against 13.2, but [4096,5120] 23.1 against 20.5.
+  int vpt = !backward && !residual && nvec > 4 * kWave && nvec <= 8 * kWave ? 2 : 1;
+  while (ceil_div(nvec, (int64_t)kWave * vpt) > kLnBlockMaxWaves) vpt *= 2;
+  if (vpt * vn > 16) return p;
+  p.vpt = vpt;
+  p.gw = (int)ceil_div(nvec, (int64_t)kWave * vpt);
+  // Backward: as many rows side by side as 16 waves hold, so that one workgroup per CU, hence 256
+  // partial rows, keeps the CU busy ([12000,1003] fp32 40.3 us against 43.3 with 8 waves; 512
+  // workgroups 41.2, and [4096,5120] bf16 49.9 against 41.9).  Forward: 8 waves and two workgroups
+  // per CU ([4096,1001] bf16 9.7 us against 11.4 with 16 waves, [4096,5120] 32.3 against 37.5 with 1024
+  // workgroups).  Fewer where there are not rows enough for every CU.
+  int groups = (backward ? kLnBlockMaxWaves : kLnBlockMaxWaves / 2) / p.gw;
+  const int64_t per_cu = ceil_div(rows, (int64_t)256);
+  if (groups > per_cu) groups = (int)per_cu;
+  while (backward && groups > 1 && (size_t)groups * C * sizeof(float) > kLnBlockFoldLds) --groups;
+  p.groups = groups < 1 ? 1 : groups;
+  const int cap = backward ? 256 : 512;
+  const int64_t b = ceil_div(rows, (int64_t)p.groups);
+  p.blocks = (int)(b < cap ? b : cap);
+  return p;
 }
 
 template <typename TX, typename TY, typename TP>
@@ -1178,8 +1467,7 @@ int fwd_typed(const void *x, const void *gamma, const void *beta, void *y, void 
       // with the residual stream a wave holds two inputs per row: half the rows per step
       const int r_rows = res ? (p.vpl == 1   ? CS_LN_ADD_ROWS_VPL1
                                 : p.vpl == 2 ? CS_LN_ADD_ROWS_VPL2
-                                : p.vpl == 4 ? CS_LN_ADD_ROWS_VPL4
-                                             : 1)
+                                             : CS_LN_ADD_ROWS_VPL4)
                              : p.fwd_rows;
       const dim3 grid((unsigned)ln_blocks(rows, r_rows, kLnFwdMaxBlocks)), block(kLnThreads);
 #define CS_LN_FWD(VPL, R, HAS_RES)                                                          \
@@ -1191,21 +1479,50 @@ int fwd_typed(const void *x, const void *gamma, const void *beta, void *y, void 
           CS_LN_FWD(1, CS_LN_ADD_ROWS_VPL1, true);
         } else if (p.vpl == 2) {
           CS_LN_FWD(2, CS_LN_ADD_ROWS_VPL2, true);
-        } else if (p.vpl == 4) {
-          CS_LN_FWD(4, CS_LN_ADD_ROWS_VPL4, true);
         } else {
-          CS_LN_FWD(8, 1, true);
+          CS_LN_FWD(4, CS_LN_ADD_ROWS_VPL4, true);
         }
       } else if (p.vpl == 1) {
         CS_LN_FWD(1, CS_LN_FWD_ROWS_VPL1, false);
       } else if (p.vpl == 2) {
         CS_LN_FWD(2, CS_LN_FWD_ROWS_VPL2, false);
-      } else if (p.vpl == 4) {
-        CS_LN_FWD(4, CS_LN_FWD_ROWS_VPL4, false);
       } else {
-        CS_LN_FWD(8, 1, false);
+        CS_LN_FWD(4, CS_LN_FWD_ROWS_VPL4, false);
       }
 #undef CS_LN_FWD
+      return launch_status();
+    }
+  }
+  if constexpr (!std::is_same_v<TX, double>) {
+    const BlockPlan b = block_plan(rows, C, x_dtype, false, res != nullptr);
+    if (b.vpt != 0) {
+      const bool ua = !aligned || C % Vec16<TX>::n != 0;
+      const dim3 grid((unsigned)b.blocks), block((unsigned)(b.gw * b.groups * kWave));
+#define CS_LN_FWD_B(VPT, HAS_RES, UA)                                                                  \
+  ln_fwd_block_kernel<TX, TY, TP, VPT, HAS_RES, UA><<<grid, block, 0, s>>>(                             \
+      (const TX *)x, (const TP *)gamma, (const TP *)beta, (TY *)y, (float *)mean, (float *)rstd, rows, \
+      (int)C, (float)eps, (const TX *)res, (TX *)sum_out, b.gw, b.groups)
+#define CS_LN_FWD_B2(VPT)                             \
+  if (res && ua) {                                    \
+    CS_LN_FWD_B(VPT, true, true);                     \
+  } else if (res) {                                   \
+    CS_LN_FWD_B(VPT, true, false);                    \
+  } else if (ua) {                                    \
+    CS_LN_FWD_B(VPT, false, true);                    \
+  } else {                                            \
+    CS_LN_FWD_B(VPT, false, false);                   \
+  }
+      if (b.vpt == 1) {
+        CS_LN_FWD_B2(1)
+      } else if (b.vpt == 2) {
+        CS_LN_FWD_B2(2)
+      } else {
+        if constexpr (Vec16<TX>::n == 4) {
+          CS_LN_FWD_B2(4)
+        }
+      }
+#undef CS_LN_FWD_B2
+#undef CS_LN_FWD_B
       return launch_status();
     }
   }
@@ -1269,8 +1586,8 @@ enum BwdKind {
   kBwdHalf1,     // ln_bwd_kernel, two rows per wave, 1 vector per lane (rows of up to 32 vectors)
   kBwdHalf3,     // ln_bwd_kernel, two rows per wave, 3 vectors per lane (65 to 96 vectors: C = 768 at 16 bit)
   kBwdWave4,     // ln_bwd_kernel, a wave per row, 4 vectors per lane
-  kBwdRows,      // ln_bwd_rows_kernel, 1 / 2 / 4 / 8 (no parameter gradients) vectors per lane
-  kBwdSplit,     // ln_bwd_split_rows_kernel: 8 vectors per lane with parameter gradients
+  kBwdRows,      // ln_bwd_rows_kernel, 1 / 2 / 4 vectors per lane
+  kBwdBlock,     // ln_bwd_block_kernel, several waves per row
 };
 struct BwdPlan {
   BwdKind kind = kBwdNone;
@@ -1278,16 +1595,37 @@ struct BwdPlan {
   int threads = kLnBwdThreads;
   int blocks = 0;         // workgroups of row work = partial rows left behind when dgamma/dbeta are wanted
   size_t fold_lds = 0;    // LDS of the column-sum fold
+  bool two_calls = true;  // the partial rows may be added up by a later call (kBwdBlock: see block_two_calls)
+  BlockPlan block;
 };
 constexpr int kLnMaxPartialRows = 512;
 static_assert(kLnBwdMaxBlocksNarrow <= kLnMaxPartialRows && kLnBwdMaxBlocks <= kLnMaxPartialRows &&
                   CS_LN_PAIR_MAX_BLOCKS <= kLnMaxPartialRows,
               "every plan's grid cap fits the finalize step's row limit");
 
-BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool want_dp, bool want_dx = true) {
+// Widths of the several-waves kernel whose backward pass can be split into a row pass and a later
+// sum: whole vectors, up to 512 of them.  (Wider rows leave more partial rows than a caller that
+// holds on to them should have to keep, and ragged ones have no aligned form.)
+bool block_two_calls(int64_t C, int x_dtype) {
+  if (x_dtype == CS_F64 || C <= 0) return false;
+  const int vn = 16 / (int)dtype_size(x_dtype);
+  return C % vn == 0 && C / vn > 4 * kWave && C / vn <= 8 * kWave;
+}
+
+BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, bool want_dx = true) {
   BwdPlan b;
-  const FastPlan p = fast_plan(C, x_dtype);
-  if (p.vpl == 0) return b;
+  const FastPlan p = aligned ? fast_plan(C, x_dtype) : FastPlan{};
+  if (p.vpl == 0) {
+    b.block = block_plan(rows, C, x_dtype, true, false);
+    if (b.block.vpt == 0) return b;
+    b.kind = kBwdBlock;
+    b.vpl = b.block.vpt;
+    b.threads = b.block.gw * b.block.groups * kWave;
+    b.blocks = b.block.blocks;
+    b.fold_lds = (size_t)b.block.groups * C * sizeof(float);
+    b.two_calls = aligned && block_two_calls(C, x_dtype);
+    return b;
+  }
   const int vn = 16 / (int)dtype_size(x_dtype);
   const int64_t nvec = C / vn;
   b.vpl = p.vpl;
@@ -1302,12 +1640,6 @@ BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool want_dp, bool want_d
     b.threads = CS_LN_W4_THREADS;
     b.blocks = ln_blocks(rows, 1, kLnBwdMaxBlocks, b.threads);
     b.fold_lds = (size_t)(b.threads / kWave) * C * sizeof(float);
-  } else if (p.vpl == 8 && want_dp) {
-    // with the dgamma/dbeta accumulators a row no longer fits one wave's registers (a single-wave
-    // kernel spilled ~1 KB per lane), so two waves share each row
-    b.kind = kBwdSplit;
-    b.blocks = ln_blocks(rows, 1, kLnBwdMaxBlocks, kLnBwdThreads / 2);
-    b.fold_lds = (size_t)(kLnBwdThreads / kWave / 2) * 4 * kWave * vn * sizeof(float);
   } else {
     b.kind = kBwdRows;
     b.blocks = ln_blocks(rows, 1, p.vpl <= 2 ? kLnBwdMaxBlocksNarrow : kLnBwdMaxBlocks, kLnBwdThreads);
@@ -1316,9 +1648,11 @@ BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool want_dp, bool want_d
   return b;
 }
 
-// Column order inside a partial row, as the `vn` of ln_finalize_tile: every row kernel leaves
-// column idx*vn + k at position k*(C/vn) + idx.
-int partial_vn(int x_dtype) { return 16 / (int)dtype_size(x_dtype); }
+// Column order inside a partial row, as the `vn` of ln_finalize_tile: the row-per-wave kernels leave
+// column idx*vn + k at position k*(C/vn) + idx, the several-waves kernel keeps the columns in order.
+int partial_vn(int64_t C, int x_dtype) {
+  return fast_plan(C, x_dtype).vpl == 0 ? 1 : 16 / (int)dtype_size(x_dtype);
+}
 
 enum BwdPhase { kBwdWhole = 0, kBwdRowsOnly = 1 };
 
@@ -1331,12 +1665,20 @@ struct PendingSums {
   int accumulate = 0;
 };
 
+template <typename TP, typename A>
+int launch_finalize_in(const void *partial, int64_t nparts, void *dgamma, void *dbeta, int64_t C, int vn,
+                       int accumulate, hipStream_t s) {
+  ln_bwd_finalize_kernel<TP, A><<<dim3(2 * (unsigned)ceil_div(C, (int64_t)kLnFinCols)), dim3(kLnFinCols * kLnFinRows), 0, s>>>(
+      (const float *)partial, (int)nparts, (TP *)dgamma, (TP *)dbeta, (int)C, vn, accumulate);
+  return launch_status();
+}
+
 template <typename TP>
 int launch_finalize(const void *partial, int64_t nparts, void *dgamma, void *dbeta, int64_t C, int vn,
                     int accumulate, hipStream_t s) {
-  ln_bwd_finalize_kernel<TP><<<dim3(2 * (unsigned)ceil_div(C, (int64_t)kLnFinCols)), dim3(kLnFinCols * kLnFinRows), 0, s>>>(
-      (const float *)partial, (int)nparts, (TP *)dgamma, (TP *)dbeta, (int)C, vn, accumulate);
-  return launch_status();
+  // in double where the rows were summed in double
+  return vn == 1 ? launch_finalize_in<TP, double>(partial, nparts, dgamma, dbeta, C, vn, accumulate, s)
+                 : launch_finalize_in<TP, float>(partial, nparts, dgamma, dbeta, C, vn, accumulate, s);
 }
 
 // A launch may ask for more dynamic LDS than the 64 KB it gets by default once the kernel's limit
@@ -1372,6 +1714,23 @@ int launch_bwd_kernel(const void *dy, const void *x, const void *mean, const voi
   return launch_status();
 }
 
+template <typename TDY, typename TX, typename TDX, typename TP, int VPT, bool HAS_DX, bool HAS_DP, bool HAS_DRES>
+int launch_bwd_block(const void *dy, const void *x, const void *mean, const void *rstd, const void *gamma, void *dx,
+                     void *workspace, int64_t rows, int64_t C, const void *dres, const BwdPlan &plan, bool ua,
+                     size_t lds, hipStream_t s) {
+  const auto kernel = ua ? ln_bwd_block_kernel<TDY, TX, TDX, TP, VPT, HAS_DX, HAS_DP, HAS_DRES, true>
+                         : ln_bwd_block_kernel<TDY, TX, TDX, TP, VPT, HAS_DX, HAS_DP, HAS_DRES, false>;
+  if (!HAS_DP) lds = 0;
+  // the widest row alone takes 64 KB next to the kernel's own half kilobyte
+  static std::atomic<bool> lds_allowed[2][64];
+  const int st = allow_lds(kernel, lds + 512, kLnBlockFoldLds + 512, lds_allowed[ua]);
+  if (st != CS_OK) return st;
+  kernel<<<dim3((unsigned)plan.blocks), dim3((unsigned)plan.threads), lds, s>>>(
+      (const TDY *)dy, (const TX *)x, (const float *)mean, (const float *)rstd, (const TP *)gamma, (TDX *)dx,
+      (float *)workspace, rows, (int)C, (const TDX *)dres, plan.block.gw, plan.block.groups);
+  return launch_status();
+}
+
 template <typename TDY, typename TX, typename TDX, typename TP>
 int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
               const void *gamma, void *dx, void *dgamma, void *dbeta, void *workspace,
@@ -1381,25 +1740,23 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
   // rows only: the partial rows are the product, the parameter gradients come from a later
   // cs_layernorm_backward_finalize (or ride in a later call's launch)
   const bool want_dp = phase == kBwdRowsOnly || dgamma != nullptr || dbeta != nullptr;
-  const BwdPlan plan = aligned ? bwd_plan(rows, C, x_dtype, want_dp, dx != nullptr) : BwdPlan{};
-  if (phase == kBwdRowsOnly && (plan.kind == kBwdNone || std::is_same_v<TX, double>))
+  BwdPlan plan = bwd_plan(rows, C, x_dtype, aligned, dx != nullptr);
+  if (phase == kBwdRowsOnly && (plan.kind == kBwdNone || !plan.two_calls || std::is_same_v<TX, double>))
     return aligned ? CS_ERR_UNSUPPORTED : CS_ERR_MISALIGNED;
-  // dx + dresidual inside the kernel where it fits (rows of up to 4 vectors per lane), as a
-  // second, in-place launch elsewhere
-  const bool fuse_dres = dres != nullptr && plan.kind != kBwdNone && plan.vpl <= kMaxVplWithResidual && is_aligned16(dres);
-  const void *late_dres = fuse_dres ? nullptr : dres;
-  if (!fuse_dres) dres = nullptr;
+  const size_t need = want_dp ? (size_t)plan.blocks * 2 * C * sizeof(float) : 0;
+  const bool ws_ok = need == 0 || (workspace != nullptr && workspace_bytes >= need && aligned_to(workspace, 4));
+  // a caller may bring no workspace where no sum in two steps was promised: the general kernels
+  if (plan.kind == kBwdBlock && !plan.two_calls && !ws_ok) plan = BwdPlan{};
   if constexpr (!std::is_same_v<TX, double>) {
     if (plan.kind != kBwdNone) {
       const int blocks = plan.blocks;
-      const size_t need = want_dp ? (size_t)blocks * 2 * C * sizeof(float) : 0;
-      if (want_dp && (workspace == nullptr || workspace_bytes < need)) return CS_ERR_WORKSPACE;
-      // the split kernel carries no pending sums: those get their own launch first
+      if (!ws_ok) return CS_ERR_WORKSPACE;
+      // the several-waves kernel carries no pending sums: those get their own launch first
       LnPending pend{nullptr, nullptr, nullptr, 0, 0, 0};
       if (pending.partial != nullptr && (pending.dgamma != nullptr || pending.dbeta != nullptr)) {
-        if (plan.kind == kBwdSplit) {
+        if (plan.kind == kBwdBlock) {
           const int st = launch_finalize<TP>(pending.partial, pending.nparts, pending.dgamma, pending.dbeta, C,
-                                             partial_vn(x_dtype), pending.accumulate, s);
+                                             partial_vn(C, x_dtype), pending.accumulate, s);
           if (st != CS_OK) return st;
         } else {
           pend = LnPending{(const float *)pending.partial, pending.dgamma, pending.dbeta, (int)pending.nparts,
@@ -1409,7 +1766,7 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
       size_t lds = want_dp ? plan.fold_lds : 0;
       const size_t pend_lds = (size_t)kLnFinRows * kLnFinCols * sizeof(float);
       if (pend.blocks != 0 && lds < pend_lds) lds = pend_lds;
-      const dim3 grid((unsigned)(blocks + pend.blocks)), block(kLnBwdThreads);
+      const dim3 grid((unsigned)(blocks + pend.blocks)), block((unsigned)plan.threads);
       int st = CS_OK;
 #define CS_LN_BWD(VPL, WPE, HAS_DX, HAS_DP, HAS_DRES)                                       \
   ln_bwd_rows_kernel<TDY, TX, TDX, TP, VPL, WPE, HAS_DX, HAS_DP, HAS_DRES>                  \
@@ -1458,26 +1815,39 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
 #else
         CS_LN_K64(4, CS_LN_W4_WPE, false, true, false);
 #endif
-      } else if (plan.kind == kBwdSplit) {
-        if (dx) {
-          ln_bwd_split_rows_kernel<TDY, TX, TDX, TP, 4, true, true><<<dim3((unsigned)blocks), block, lds, s>>>(
-              (const TDY *)dy, (const TX *)x, (const float *)mean, (const float *)rstd, (const TP *)gamma,
-              (TDX *)dx, (float *)workspace, rows, (int)C);
+      } else if (plan.kind == kBwdBlock) {
+        const bool ua = !aligned || C % Vec16<TX>::n != 0;
+#define CS_LN_BWD_B(VPT, HAS_DX, HAS_DP, HAS_DRES)                                                                \
+  st = launch_bwd_block<TDY, TX, TDX, TP, VPT, HAS_DX, HAS_DP, HAS_DRES>(dy, x, mean, rstd, gamma, dx, workspace, \
+                                                                         rows, C, dres, plan, ua, lds, s)
+#define CS_LN_BWD_BLOCK(VPT, WPE, HAS_DX, HAS_DP, HAS_DRES)                      \
+  if constexpr (VPT * Vec16<TX>::n > 8 && HAS_DX && HAS_DP) {                    \
+    CS_LN_BWD_B(VPT, false, true, false);                                        \
+    if (st == CS_OK) CS_LN_BWD_B(VPT, true, false, HAS_DRES);                    \
+  } else {                                                                       \
+    CS_LN_BWD_B(VPT, HAS_DX, HAS_DP, HAS_DRES);                                  \
+  }
+        // with 16 elements per lane the column sums and dx do not fit the registers together: two
+        // passes over the rows ([1024,16000] bf16 with dresidual: 54 us against 136)
+        if (plan.vpl == 1) {
+          CS_LN_BWD_MASK(CS_LN_BWD_BLOCK, 1, 0)
+        } else if (plan.vpl == 2) {
+          CS_LN_BWD_MASK(CS_LN_BWD_BLOCK, 2, 0)
         } else {
-          ln_bwd_split_rows_kernel<TDY, TX, TDX, TP, 4, false, true><<<dim3((unsigned)blocks), block, lds, s>>>(
-              (const TDY *)dy, (const TX *)x, (const float *)mean, (const float *)rstd, (const TP *)gamma,
-              (TDX *)dx, (float *)workspace, rows, (int)C);
+          if constexpr (Vec16<TX>::n == 4) {
+            CS_LN_BWD_MASK(CS_LN_BWD_BLOCK, 4, 0)
+          }
         }
+#undef CS_LN_BWD_BLOCK
+#undef CS_LN_BWD_B
       } else if (plan.vpl == 1) {
         CS_LN_BWD_MASK(CS_LN_BWD, 1, 4)
       } else if (plan.vpl == 2 && dres && want_dp) {
         CS_LN_BWD(2, 3, true, true, true);  // four per SIMD would spill
       } else if (plan.vpl == 2) {
         CS_LN_BWD_MASK(CS_LN_BWD, 2, 4)
-      } else if (plan.vpl == 4) {
-        CS_LN_BWD_MASK(CS_LN_BWD, 4, 2)
       } else {
-        CS_LN_BWD(8, 2, true, false, false);
+        CS_LN_BWD_MASK(CS_LN_BWD, 4, 2)
       }
 #undef CS_LN_BWD_MASK
 #undef CS_LN_K32
@@ -1486,8 +1856,8 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
 #undef CS_LN_BWD
       if (st == CS_OK) st = launch_status();
       if (st == CS_OK && want_dp && phase == kBwdWhole)
-        st = launch_finalize<TP>(workspace, blocks, dgamma, dbeta, C, partial_vn(x_dtype), accumulate, s);
-      if (st == CS_OK && late_dres) st = launch_add<TDX>(dx, late_dres, dx, rows * C, s);
+        st = launch_finalize<TP>(workspace, blocks, dgamma, dbeta, C, plan.kind == kBwdBlock ? 1 : partial_vn(C, x_dtype),
+                                 accumulate, s);
       return st;
     }
   }
@@ -1496,7 +1866,7 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
   if (dx) {
     ln_bwd_dx_general_kernel<TDY, TX, TDX, TP><<<dim3((unsigned)rows), dim3(kLnThreads), 0, s>>>(
         (const TDY *)dy, (const TX *)x, (const U *)mean, (const U *)rstd, (const TP *)gamma,
-        (TDX *)dx, C, (const TDX *)late_dres);
+        (TDX *)dx, C, (const TDX *)dres);
     const int st = launch_status();
     if (st != CS_OK) return st;
   }
@@ -1583,8 +1953,10 @@ extern "C" size_t cs_layernorm_backward_workspace_bytes(int64_t rows, int64_t C)
   // the most partial rows any plan leaves for this many rows, whatever the storage type
   int most = 0;
   for (int dt : {CS_F32, CS_F16}) {
-    const BwdPlan b = bwd_plan(rows, C, dt, true);
-    if (b.blocks > most) most = b.blocks;
+    for (bool aligned : {true, false}) {
+      const BwdPlan b = bwd_plan(rows, C, dt, aligned);
+      if (b.blocks > most) most = b.blocks;
+    }
   }
   return (size_t)most * 2 * (size_t)C * sizeof(float);
 }
@@ -1673,7 +2045,8 @@ extern "C" int cs_layernorm_backward_add(const void *dy, const void *x, const vo
 
 extern "C" int64_t cs_layernorm_backward_partial_rows(int64_t rows, int64_t C, int x_dtype) {
   if (rows <= 0 || C <= 0 || dtype_size(x_dtype) == 0) return 0;
-  return bwd_plan(rows, C, x_dtype, true).blocks;
+  const BwdPlan b = bwd_plan(rows, C, x_dtype, true);
+  return b.two_calls ? b.blocks : 0;
 }
 
 extern "C" int cs_layernorm_backward_rows(const void *dy, const void *x, const void *mean,
@@ -1697,7 +2070,7 @@ extern "C" int cs_layernorm_backward_finalize(const void *partials, int64_t part
       !wide_ok(x_dtype, param_dtype))
     return CS_ERR_UNSUPPORTED;
   if (C % (16 / (int)dtype_size(x_dtype)) != 0 || partial_rows > kLnMaxPartialRows) return CS_ERR_INVALID_ARGUMENT;
-  const int vn = partial_vn(x_dtype);
+  const int vn = partial_vn(C, x_dtype);
   if (!dgamma && !dbeta) return CS_OK;
   if (!is_aligned16(partials) || (dgamma && !aligned_to(dgamma, dtype_size(param_dtype))) ||
       (dbeta && !aligned_to(dbeta, dtype_size(param_dtype))))

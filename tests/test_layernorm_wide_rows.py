@@ -1,0 +1,113 @@
+"""LayerNorm rows shared by several waves: widths beyond one wave's registers, ragged widths and
+unaligned tensors, at the edges of the kernels' tiles, against the CPU oracle."""
+import ctypes
+
+import pytest
+import torch
+
+from _util import assert_bit_exact, assert_close, assert_sum_close, randn, sum_tolerance
+
+pytestmark = pytest.mark.gpu
+BF16, F16, F32 = torch.bfloat16, torch.float16, torch.float32
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from core_scheduler_amd import ops as o
+    return o
+
+
+@pytest.fixture(scope="module")
+def co():
+    from oracle import c_oracle
+    return c_oracle
+
+
+def place(t, offset):
+    """t on the GPU, its first element `offset` elements past an aligned address."""
+    flat = torch.empty(t.numel() + offset, dtype=t.dtype, device="cuda:0")
+    flat[offset:].copy_(t.reshape(-1))
+    return flat[offset:].view(t.shape)
+
+
+@pytest.mark.parametrize("rows,C,x_dtype,p_dtype,wide_dy,offset", [
+    (700, 2056, BF16, F32, False, 0),    # just past a wave's 256 vectors: five waves, the last nearly empty
+    (515, 4096, F16, F16, False, 0),     # 512 vectors: two per lane in the plain forward
+    (260, 4104, BF16, F32, True, 0),     # 513: one per lane again; fp32 gradients of 16-bit rows
+    (300, 8192, BF16, BF16, False, 0),   # 16 full waves
+    (70, 8200, BF16, F32, False, 0),     # one vector more: two per lane, sums and dx in two passes
+    (33, 16384, F16, F32, False, 0),     # the widest row
+    (20, 16392, BF16, F32, False, 0),    # past it: the general kernels
+    (1100, 1028, F32, F32, False, 0),    # fp32: 257 vectors
+    (40, 16380, F32, F32, False, 0),     # four fp32 vectors per lane
+    (5000, 1, F32, F32, False, 0),       # no whole vector, one column
+    (3000, 7, BF16, F32, False, 0),      # no whole vector
+    (777, 71, F16, F16, False, 0),       # 8 vectors and 7 columns
+    (4099, 513, BF16, F32, False, 0),    # 64 vectors and a column; several rows per group, the last step ragged
+    (1, 1001, F32, F32, False, 0),       # a single row
+    (300, 4099, F32, F32, False, 0),     # 1024 vectors (16 waves) and 3 columns
+    (600, 768, BF16, F32, False, 1),     # an aligned width at an unaligned address
+    (600, 768, BF16, F32, True, 3),
+])
+def test_layernorm_rows_on_several_waves(ops, co, rows, C, x_dtype, p_dtype, wide_dy, offset):
+    g_dtype = F32 if wide_dy else x_dtype
+    x, res = randn((rows, C), 900, dtype=x_dtype), randn((rows, C), 901, dtype=x_dtype)
+    gamma, beta = randn(C, 902, std=0.02, mean=1.0, dtype=p_dtype), randn(C, 903, std=0.02, dtype=p_dtype)
+    dy, dres = randn((rows, C), 904, dtype=g_dtype), randn((rows, C), 905, dtype=g_dtype)
+    total_ref = (x.float() + res.float()).to(x_dtype)
+    gx, gres, gg, gb = place(x, offset), place(res, offset), place(gamma, 0), place(beta, 0)
+    y2, mean2, rstd2 = co.layernorm_forward(total_ref, gamma, beta, 1e-5)
+    # with one column the variance is 0 and rstd = 1/sqrt(eps) multiplies every rounding by 316
+    loose = 316 if C == 1 else 1
+    total, y, mean, rstd = ops.add_layernorm_forward(gx, gres, gg, gb, 1e-5)
+    assert_bit_exact(total, total_ref, "x + residual")
+    assert_close(y, y2, atol=2e-6 * loose, name="y")
+    assert_close(mean, mean2, atol=1e-7, name="mean")
+    assert_close(rstd, rstd2, atol=1e-6 * loose, name="rstd")
+    y_sep, mean_sep, _ = ops.layernorm_forward(place(total_ref, offset), gg, gb, 1e-5)
+    assert_close(y_sep, y2, atol=2e-6 * loose, name="y without residual")
+    assert_close(mean_sep, mean2, atol=1e-7, name="mean without residual")
+    ops.add_layernorm_forward(gx, gres, gg, gb, 1e-5, inplace=True)
+    assert_bit_exact(gx, total_ref, "in-place sum")
+
+    gdy, gt, gm, gr, gdr = place(dy, offset), place(total_ref, offset), place(mean2, 0), place(rstd2, 0), place(dres, offset)
+    dx, dg, db = ops.layernorm_backward(gdy, gt, gm, gr, gg, dx_dtype=g_dtype)
+    dx2, dg2, db2 = co.layernorm_backward(dy, total_ref, mean2, rstd2, gamma, **({"out_dtype": F32} if wide_dy else {}))
+    # dx = rstd * (three terms of size |dy gamma|): rstd scales their rounding
+    assert_close(dx, dx2, atol=5e-6 * max(1.0, float(rstd2.max())), name="dx")
+    xhat = (total_ref.double() - mean2.double().reshape(-1, 1)) * rstd2.double().reshape(-1, 1)
+    assert_sum_close(dg, dg2, sum_tolerance(dy.double() * xhat), name="dgamma")
+    assert_sum_close(db, db2, sum_tolerance(dy), name="dbeta")
+    # each output mask gives the bits of the full call; dresidual is added to the rounded dx
+    only_dx = ops.layernorm_backward(gdy, gt, gm, gr, gg, dx_dtype=g_dtype, need_dgamma=False, need_dbeta=False)[0]
+    assert_bit_exact(only_dx, dx, "dx alone")
+    _, dg1, db1 = ops.layernorm_backward(gdy, gt, gm, gr, gg, need_dx=False)
+    assert_bit_exact(dg1, dg, "dgamma alone")
+    assert_bit_exact(db1, db, "dbeta alone")
+    dxr, dgr, dbr = ops.layernorm_backward(gdy, gt, gm, gr, gg, dx_dtype=g_dtype, dresidual=gdr)
+    assert_bit_exact(dxr, (dx.cpu().float() + dres.float()).to(g_dtype), "dx + dresidual")
+    assert_bit_exact(dgr, dg, "dgamma with dresidual")
+    assert_bit_exact(dbr, db, "dbeta with dresidual")
+    # += into existing gradients
+    acc_g, acc_b = gg.clone(), gb.clone()
+    ops.layernorm_backward(gdy, gt, gm, gr, gg, dx_dtype=g_dtype, dgamma=acc_g, dbeta=acc_b)
+    want_g = (dg2.double() + gamma.double()).to(p_dtype) if p_dtype == F32 else None
+    if want_g is not None:
+        assert_sum_close(acc_g, want_g, sum_tolerance(dy.double() * xhat) + 1e-6, name="dgamma +=")
+
+
+def test_wide_rows_without_a_workspace(ops):
+    """A caller that brings no workspace for a ragged width still gets its gradients."""
+    from core_scheduler_amd import _capi
+    rows, C = 64, 50
+    x, dy = place(randn((rows, C), 910), 0), place(randn((rows, C), 911), 0)
+    gamma = place(randn(C, 912, std=0.02, mean=1.0), 0)
+    _, mean, rstd = ops.layernorm_forward(x, gamma)
+    want = ops.layernorm_backward(dy, x, mean, rstd, gamma)
+    dx, dg, db = torch.empty_like(x), torch.empty_like(gamma), torch.empty_like(gamma)
+    P = lambda t: ctypes.c_void_p(t.data_ptr())
+    code = _capi.load().cs_layernorm_backward(P(dy), P(x), P(mean), P(rstd), P(gamma), P(dx), P(dg), P(db), None, 0, rows,
+                                              C, 0, 0, 0, 0, 0, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert code == _capi.OK
+    for got, ref, name in zip((dx, dg, db), want, ("dx", "dgamma", "dbeta")):
+        assert_close(got, ref.cpu(), atol=1e-5, name=name)

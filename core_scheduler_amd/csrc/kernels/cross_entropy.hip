@@ -17,8 +17,8 @@
 //   up to 7168 (8192 at fp32)        ce_rows_stream_kernel: one persistent workgroup per
 //                                    CU that loads the next row while it works on the
 //                                    current one (50257 bf16 = 6283 vectors = 7 per lane)
-//   wider, or rows that do not       ce_rows_wide_kernel: two sweeps over the row, the
-//   start on 16-byte boundaries      second one served by the cache
+//   wider, or narrow rows that do    ce_rows_wide_kernel: two sweeps over the row, the
+//   not start on 16-byte boundaries  second one served by the cache
 //   fp64, unaligned base pointers    ce_rows_general_kernel
 // Probabilities are 2^(x*log2e - max*log2e) / sum with one fma and one hardware exp2 per
 // element; the row loss is ln(sum) - (x_t - max).
@@ -144,6 +144,14 @@ __device__ __forceinline__ void store_out(TD *p, const float (&o)[N_ELEMS]) {
   }
 }
 
+// The same for a vector that starts at column c0 of a row that does not own all of it.
+template <typename TD, int N_ELEMS>
+__device__ __forceinline__ void store_own(TD *p, const float (&o)[N_ELEMS], int c0, int stride) {
+#pragma unroll
+  for (int k = 0; k < N_ELEMS; ++k)
+    if (c0 + k >= 0 && c0 + k < stride) p[k] = from_acc<TD>(o[k]);
+}
+
 template <typename T, typename TD, int BLOCK, int VPT>
 __global__ __launch_bounds__(BLOCK) void ce_rows_kernel(
     const T *__restrict__ logits, TD *__restrict__ dlogits, const int64_t *__restrict__ targets,
@@ -254,6 +262,10 @@ __global__ __launch_bounds__(BLOCK) void ce_rows_kernel(
   }
 }
 
+// elements of T in a 128-byte line
+template <typename T>
+constexpr int kLineElems = 128 / (int)sizeof(T);
+
 // EPV elements of T in one 8- or 16-byte access.  The streaming kernel reads 16-bit logits 8
 // bytes per lane when it writes fp32 gradients, so that every store is a full 16 bytes per lane
 // and a wave's store covers one contiguous kilobyte (with 16-byte loads each lane would own 32
@@ -312,7 +324,14 @@ __device__ __forceinline__ float widen(const VecE<T, EPV> &v, int k) {
 //
 // HAS_W: per-class weights (nll_loss's `weight`): a row's gradient and loss carry w[target], and
 // the mean divides by the sum of those weights, which the count launch left next to the count.
-template <typename T, typename TD, int VPT, int EPV, bool HAS_W>
+//
+// RAGGED: the row stride is not a multiple of the access width (a vocabulary used unpadded), so rows
+// start anywhere.  The lanes still own whole aligned vectors of the [N, stride] array, counted from the
+// 128-byte line the row starts in; elements of the neighbouring rows count as padding, and a vector that
+// a row owns only part of is written element by element.  [8192,50257] unpadded bf16: 289 us against 366
+// in two sweeps (padded rows 287), with fp32 gradients [6000,50257] 341 against 442.  Counted from the
+// nearest 16-byte vector instead of the line, so that every access of a wave straddles lines: 312 and 373.
+template <typename T, typename TD, int VPT, int EPV, bool HAS_W, bool RAGGED>
 __global__ __launch_bounds__(1024) void ce_rows_stream_kernel(
     const T *logits, TD *dlogits, const int64_t *__restrict__ targets, float *__restrict__ row_loss,
     const int *__restrict__ ws_count, int64_t N, int64_t V, int64_t row_stride,
@@ -324,8 +343,16 @@ __global__ __launch_bounds__(1024) void ce_rows_stream_kernel(
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = tid >> 6;
-  const int nvec = (int)(row_stride / VN);
   const int iV = (int)V;
+  const int nvec_even = (int)(row_stride / VN);
+  // A ragged row: elements between the 128-byte line it starts in and its start, vectors from that line
+  // to its end, and how many of these lie whole inside the array (all but perhaps the last row's last
+  // one).  From the line, not only from the nearest vector, so that the waves' accesses cover whole lines.
+  auto off_of = [&](int64_t r) { return RAGGED ? (int)((r * row_stride) & (kLineElems<T> - 1)) : 0; };
+  auto vecs_of = [&](int off) { return RAGGED ? (int)((off + row_stride + VN - 1) / VN) : nvec_even; };
+  auto whole_of = [&](int64_t r, int off) {
+    return vecs_of(off) - (RAGGED && r == N - 1 && (off + (int)row_stride) % VN != 0 ? 1 : 0);
+  };
 
   float scale0 = dloss;
   if (reduction == CS_REDUCTION_MEAN)
@@ -346,13 +373,14 @@ __global__ __launch_bounds__(1024) void ce_rows_stream_kernel(
     live = target_counts(tgt, V, ignore_index);
     if (live) {
       if constexpr (HAS_W) wt = class_weight[tgt];
-      const T *x = logits + row * row_stride;
+      const int off = off_of(row), nload = whole_of(row, off);
+      const T *x = logits + row * row_stride - off;
 #pragma unroll
       for (int j = 0; j < VPT; ++j) {
         const int idx = tid + BLOCK * j;
-        if (idx < nvec) cur[j] = load_e_stream<T, EPV>(x + (int64_t)idx * VN);
+        if (idx < nload) cur[j] = load_e_stream<T, EPV>(x + (int64_t)idx * VN);
       }
-      if (tid == 0) x_t = to_acc(x[tgt]);
+      if (tid == 0) x_t = to_acc(x[off + tgt]);
     }
   }
   int parity = 0;
@@ -368,35 +396,57 @@ __global__ __launch_bounds__(1024) void ce_rows_stream_kernel(
       nlive = target_counts(ntgt, V, ignore_index);
       if (nlive) {
         if constexpr (HAS_W) nwt = class_weight[ntgt];
-        const T *x = logits + nrow * row_stride;
+        const int off = off_of(nrow), nload = whole_of(nrow, off);
+        const T *x = logits + nrow * row_stride - off;
 #pragma unroll
         for (int j = 0; j < VPT; ++j) {
           const int idx = tid + BLOCK * j;
           // (kept under the lane's condition here: the compiler issues these back to back as they
           // are, and the unconditional form spills 56 bytes per lane: 283 -> 305 us)
-          if (idx < nvec) nxt[j] = load_e_stream<T, EPV>(x + (int64_t)idx * VN);
+          if (idx < nload) nxt[j] = load_e_stream<T, EPV>(x + (int64_t)idx * VN);
         }
-        if (tid == 0) nx_t = to_acc(x[ntgt]);
+        if (tid == 0) nx_t = to_acc(x[off + ntgt]);
       }
     }
 
+    const int off = off_of(row), nvec = vecs_of(off);
     if (!live) {
       if (tid == 0 && row_loss) row_loss[row] = 0.f;
       if (dlogits) {
         float z[VN];
 #pragma unroll
         for (int k = 0; k < VN; ++k) z[k] = 0.f;
-        for (int idx = tid; idx < nvec; idx += BLOCK)
-          store_out<T, TD, VN>(dlogits + row * row_stride + (int64_t)idx * VN, z);
+        for (int idx = tid; idx < nvec; idx += BLOCK) {
+          const int c0 = idx * VN - off;
+          if (RAGGED && (c0 < 0 || c0 + VN > (int)row_stride)) {
+            store_own<TD, VN>(dlogits + row * row_stride + c0, z, c0, (int)row_stride);
+          } else {
+            store_out<T, TD, VN>(dlogits + row * row_stride - off + (int64_t)idx * VN, z);
+          }
+        }
       }
     } else {
+      if (RAGGED && row == N - 1 && whole_of(row, off) < nvec) {  // the array's last vector is not whole
+#pragma unroll
+        for (int j = 0; j < VPT; ++j) {
+          const int idx = tid + BLOCK * j;
+          if (idx == nvec - 1) {
+#pragma unroll
+            for (int k = 0; k < VN; ++k) {
+              const int c = idx * VN - off + k;
+              cur[j].e[k] = logits[row * row_stride + (c < (int)row_stride ? c : 0)];
+            }
+          }
+        }
+      }
       // ---- widen, mask what is not a class column to -inf, lane-local max
       float e[VPT][VN];
       float m = -INFINITY;
 #pragma unroll
       for (int j = 0; j < VPT; ++j) {
-        const int c0 = (tid + BLOCK * j) * VN;
-        if (c0 + VN <= iV) {
+        const int c0 = (tid + BLOCK * j) * VN - off;
+        const bool starts_before = RAGGED && j == 0 && c0 < 0;
+        if (c0 + VN <= iV && !starts_before) {
 #pragma unroll
           for (int k = 0; k < VN; ++k) {
             e[j][k] = widen(cur[j], k);
@@ -405,7 +455,8 @@ __global__ __launch_bounds__(1024) void ce_rows_stream_kernel(
         } else {
 #pragma unroll
           for (int k = 0; k < VN; ++k) {
-            e[j][k] = c0 + k < iV ? widen(cur[j], k) : -INFINITY;
+            const bool mine = c0 + k < iV && !(RAGGED && j == 0 && c0 + k < 0);
+            e[j][k] = mine ? widen(cur[j], k) : -INFINITY;
             m = fmaxf(m, e[j][k]);
           }
         }
@@ -453,8 +504,9 @@ __global__ __launch_bounds__(1024) void ce_rows_stream_kernel(
         // 0 * f cannot meet an overflowed factor
         float f = empty ? 0.f : __builtin_amdgcn_exp2f(ml2 - M2 - log2_S + log2_scale);
         f = negate ? -f : f;
-        const int t_vec = (int)(tgt / VN), t_sub = (int)(tgt % VN);
-        TD *d = dlogits + row * row_stride;
+        const int t_at = (int)tgt + off;
+        const int t_vec = t_at / VN, t_sub = t_at % VN;
+        TD *d = dlogits + row * row_stride - off;
 #pragma unroll
         for (int j = 0; j < VPT; ++j) {
           const int idx = tid + BLOCK * j;
@@ -471,7 +523,12 @@ __global__ __launch_bounds__(1024) void ce_rows_stream_kernel(
               for (int k = 0; k < VN; ++k)
                 if (k == t_sub) o[k] = e[j][k] * exact - scale;
             }
-            store_out<T, TD, VN>(d + (int64_t)idx * VN, o);
+            // (written out here: as a lambda the store cost 56 bytes of scratch per lane)
+            if (RAGGED && (idx * VN - off < 0 || idx * VN - off + VN > (int)row_stride)) {
+              store_own<TD, VN>(d + (int64_t)idx * VN, o, idx * VN - off, (int)row_stride);
+            } else {
+              store_out<T, TD, VN>(d + (int64_t)idx * VN, o);
+            }
           }
         }
       }
@@ -740,6 +797,50 @@ void launch_wide(const void *logits, void *dlogits, const int64_t *targets, floa
   }
 }
 
+// Accesses (of 16 bytes; 8 where 16-bit logits give fp32 gradients) a row may take for the streaming
+// kernel: 7 or 8 fp32, 7 16-bit or 13 half-width ones per lane.
+template <typename T, typename TD>
+struct StreamPlan {
+  static constexpr int kEpv = sizeof(T) == 2 && sizeof(TD) == 4 ? 4 : Vec16<T>::n;
+  static constexpr int kMostVecs = 1024 * (kEpv * sizeof(T) == 8 ? 13 : sizeof(T) == 4 ? 8 : 7);
+};
+
+// One persistent workgroup per CU, the row in registers.  The widest plans (8 vectors per lane at 16
+// bit, 16 half vectors with fp32 gradients) measured slower than the two-sweep kernel and are not
+// built.
+template <typename T, typename TD, bool RAGGED>
+void launch_stream(const void *logits, void *dlogits, const int64_t *targets, float *row_loss,
+                   const int *ws_count, int64_t N, int64_t V, int64_t row_stride, int64_t ignore_index,
+                   int reduction, float dloss, const float *class_weight, hipStream_t s) {
+  constexpr int EPV = StreamPlan<T, TD>::kEpv;
+  const int64_t cus = compute_units();
+  const dim3 grid((unsigned)(N < cus ? N : cus)), block(1024);
+  // a ragged row is counted from the line it starts in
+  const int64_t nvec = (row_stride + (RAGGED ? kLineElems<T> - 1 : 0) + EPV - 1) / EPV;
+#define CS_CE_STREAM(VPT)                                                                                \
+  if (class_weight != nullptr) {                                                                         \
+    ce_rows_stream_kernel<T, TD, VPT, EPV, true, RAGGED><<<grid, block, 0, s>>>(                          \
+        (const T *)logits, (TD *)dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index,   \
+        reduction, dloss, class_weight);                                                                 \
+  } else {                                                                                               \
+    ce_rows_stream_kernel<T, TD, VPT, EPV, false, RAGGED><<<grid, block, 0, s>>>(                         \
+        (const T *)logits, (TD *)dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index,   \
+        reduction, dloss, nullptr);                                                                      \
+  }
+  if constexpr (EPV * sizeof(T) == 8) {
+    CS_CE_STREAM(13);
+  } else if (nvec <= 1024 * 4) {
+    CS_CE_STREAM(4);
+  } else if (nvec <= 1024 * 7) {
+    CS_CE_STREAM(7);
+  } else {
+    if constexpr (sizeof(T) == 4) {
+      CS_CE_STREAM(8);
+    }
+  }
+#undef CS_CE_STREAM
+}
+
 template <typename T, typename TD>
 int launch_rows(const void *logits, void *dlogits, const int64_t *targets, float *row_loss,
                 const int *ws_count, int64_t N, int64_t V, int64_t row_stride,
@@ -755,7 +856,7 @@ int launch_rows(const void *logits, void *dlogits, const int64_t *targets, float
     // sets weights), so weighted calls on narrow rows go to the two-sweep kernel
     const int64_t nvec_all = row_stride / VN;
     const bool streams = nvec_all > 256 * 8 &&
-                         nvec_all <= (sizeof(T) == 4 ? 1024 * 8 : sizeof(TD) == 4 ? 512 * 13 : 1024 * 7);
+                         row_stride <= (int64_t)StreamPlan<T, TD>::kEpv * StreamPlan<T, TD>::kMostVecs;
     if (vec_ok && (class_weight == nullptr || streams)) {
       const int64_t nvec = row_stride / VN;
 #define CS_CE(BLOCK, VPT)                                                                   \
@@ -766,34 +867,9 @@ int launch_rows(const void *logits, void *dlogits, const int64_t *targets, float
         CS_CE(64, 8);
       } else if (nvec <= 256 * 8) {
         CS_CE(256, 8);
-      } else if (nvec <= (sizeof(T) == 4 ? 1024 * 8 : sizeof(TD) == 4 ? 512 * 13 : 1024 * 7)) {
-        // one persistent workgroup per CU, the row in registers.  The widest plans (8 vectors
-        // per lane at 16 bit, 16 half vectors with fp32 gradients) measured slower than the
-        // two-sweep kernel and are not built.
-        const int64_t cus = compute_units();
-        const dim3 pgrid((unsigned)(N < cus ? N : cus));
-#define CS_CE_STREAM(VPT, EPV)                                                                    \
-  if (class_weight != nullptr) {                                                                  \
-    ce_rows_stream_kernel<T, TD, VPT, EPV, true><<<pgrid, dim3(1024), 0, s>>>(                    \
-        (const T *)logits, (TD *)dlogits, targets, row_loss, ws_count, N, V, row_stride,          \
-        ignore_index, reduction, dloss, class_weight);                                            \
-  } else {                                                                                        \
-    ce_rows_stream_kernel<T, TD, VPT, EPV, false><<<pgrid, dim3(1024), 0, s>>>(                   \
-        (const T *)logits, (TD *)dlogits, targets, row_loss, ws_count, N, V, row_stride,          \
-        ignore_index, reduction, dloss, nullptr);                                                 \
-  }
-        if constexpr (sizeof(T) == 2 && sizeof(TD) == 4) {
-          CS_CE_STREAM(13, 4);  // 16-bit logits, fp32 gradients (autocast): 4 elements per lane per access
-        } else if (nvec <= 1024 * 4) {
-          CS_CE_STREAM(4, VN);
-        } else if (nvec <= 1024 * 7) {
-          CS_CE_STREAM(7, VN);
-        } else {
-          if constexpr (sizeof(T) == 4) {
-            CS_CE_STREAM(8, VN);
-          }
-        }
-#undef CS_CE_STREAM
+      } else if (row_stride <= (int64_t)StreamPlan<T, TD>::kEpv * StreamPlan<T, TD>::kMostVecs) {
+        launch_stream<T, TD, false>(logits, dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index,
+                                    reduction, dloss, class_weight, s);
       } else if (sizeof(T) == 4 && nvec <= 1024 * 16) {
         // fp32 rows up to 65536 columns still fit in registers (at 16 bit this plan spills)
         if constexpr (sizeof(T) == 4) CS_CE(1024, 16);
@@ -802,6 +878,12 @@ int launch_rows(const void *logits, void *dlogits, const int64_t *targets, float
                            reduction, dloss, class_weight, s);
       }
 #undef CS_CE
+      return launch_status();
+    }
+    if (base_ok && nvec_all > 256 * 8 &&
+        row_stride + kLineElems<T> <= (int64_t)StreamPlan<T, TD>::kEpv * StreamPlan<T, TD>::kMostVecs) {
+      launch_stream<T, TD, true>(logits, dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index,
+                                 reduction, dloss, class_weight, s);
       return launch_status();
     }
     if (base_ok && sizeof(TD) >= sizeof(T)) {

@@ -1,0 +1,69 @@
+"""Fused classifier rows that start anywhere (a vocabulary used unpadded) at the edges of the kernels'
+plans, against the CPU oracle."""
+import pytest
+import torch
+
+from _util import assert_bit_exact, assert_close, randint, randn
+
+pytestmark = pytest.mark.gpu
+BF16, F16, F32 = torch.bfloat16, torch.float16, torch.float32
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from core_scheduler_amd import ops as o
+    return o
+
+
+@pytest.fixture(scope="module")
+def co():
+    from oracle import c_oracle
+    return c_oracle
+
+
+@pytest.mark.parametrize("N,V,stride,dtype,gdt", [
+    (3, 16385, 16385, BF16, None),      # 2048 vectors and an element: the narrowest streamed row
+    (259, 16390, 16391, F16, None),     # more rows than workgroups, a padding column
+    (5, 32705, 32705, BF16, None),      # the four-vector plan with the line's 63 elements in front: its last width
+    (5, 32706, 32707, BF16, None),      # the next one
+    (3, 57279, 57279, F16, None),       # the widest streamed 16-bit row
+    (3, 57281, 57281, BF16, None),      # the next one: two sweeps
+    (2, 53183, 53183, BF16, F32),       # the widest with fp32 gradients
+    (2, 53185, 53185, F16, F32),
+    (260, 20011, 20011, BF16, F32),
+    (3, 8193, 8193, F32, None),         # fp32: 2048 vectors and an element
+    (2, 32735, 32735, F32, None),       # the widest streamed fp32 row
+    (2, 32737, 32737, F32, None),
+    (1, 50257, 50257, BF16, None),      # a single row, its last vector not whole
+    (7, 50255, 50257, F16, None),
+])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_unpadded_rows(ops, co, N, V, stride, dtype, gdt, weighted):
+    x = randn((N, stride), 950, std=2.0, dtype=dtype)
+    t = randint(0, V, (N,), 951)
+    t[0] = V - 1
+    if N > 1:
+        t[N - 1] = 0
+    if N > 2:
+        t[1] = -100
+    kw = dict(dlogits_dtype=gdt) if gdt else {}
+    w = randn(V, 952).abs() + 0.1 if weighted else None
+    gw = w.to("cuda:0") if weighted else None
+    gx, gt = x.to("cuda:0"), t.to("cuda:0")
+    loss, row, d, tw = ops.fused_classifier(gx, gt, V, class_weight=gw, **kw)
+    loss2, row2, d2, tw2 = co.cross_entropy(x, t, V, class_weight=w, **kw)
+    scale = 1.0 if w is None else float(w.max())
+    assert_close(tw, tw2.float(), atol=1e-5 * N, name="total weight")
+    assert_close(loss, loss2.float(), atol=1e-5 * scale, name="loss")
+    assert_close(row, row2.float(), atol=1e-5 * scale, name="row loss")
+    assert_close(d, d2, atol=1e-10 * scale, name="dlogits")
+    assert (d[:, V:] == 0).all()
+    if N > 2:
+        assert (d[1] == 0).all()
+    # the loss alone, and in place: nothing of a neighbouring row is touched
+    loss3, row3, none, _ = ops.fused_classifier(gx, gt, V, class_weight=gw, want_dlogits=False)
+    assert none is None
+    assert_close(row3, row2.float(), atol=1e-5 * scale, name="row loss alone")
+    if not gdt:
+        ops.fused_classifier(gx, gt, V, class_weight=gw, inplace=True)
+        assert_bit_exact(gx, d, "in place")

@@ -17,8 +17,10 @@
 //   up to 7168 (8192 at fp32)        ce_rows_stream_kernel: one persistent workgroup per
 //                                    CU that loads the next row while it works on the
 //                                    current one (50257 bf16 = 6283 vectors = 7 per lane)
-//   wider, or narrow rows that do    ce_rows_wide_kernel: two sweeps over the row, the
-//   not start on 16-byte boundaries  second one served by the cache
+//   up to 20480 with a gradient      ce_rows_hold_kernel: one persistent workgroup per CU keeps
+//                                    one row and loads the next into the registers it frees
+//   wider, the loss alone, or narrow ce_rows_wide_kernel: two sweeps over the row, the
+//   rows that start off 16 bytes     second one served by the cache
 //   fp64, unaligned base pointers    ce_rows_general_kernel
 // Probabilities are 2^(x*log2e - max*log2e) / sum with one fma and one hardware exp2 per
 // element; the row loss is ln(sum) - (x_t - max).
@@ -543,8 +545,258 @@ __global__ __launch_bounds__(1024) void ce_rows_stream_kernel(
   }
 }
 
-// Rows too wide for registers (more than 8192 16-byte vectors: vocabularies beyond 65536 at 16
-// bit, 32768 at fp32), and rows whose stride is not a multiple of the vector width (a
+// Rows too wide for two register sets (vocabularies of 57K to 160K at 16 bit, 32K to 80K at fp32): one
+// persistent 1024-lane workgroup per CU keeps ONE row, packed, in its registers.  The first pass takes the
+// running (max, sum) of the vectors as they arrive; the second forms each vector's gradient, stores it and
+// loads the same vector of the next row into the registers just freed, so loads and stores go out
+// side by side and the row is read from HBM once.  The two-sweep kernel below reads it again
+// out of the caches.  Two exponentials per element (13 us of VALU time a row) stay under the row's 20 us
+// of memory time because both passes run while memory does.
+//
+// Per call, against two sweeps: [4096,128256] bf16 457 -> 401 us (5.2 TB/s), [4096,152064] 536 -> 478,
+// [4096,100003] unpadded 374 -> 316, [2048,128256] with fp32 gradients 390 -> 308, [4096,60032] fp16
+// 210 -> 189, [2048,80000] fp32 288 -> 257.  What is left to the copy's 6.5 TB/s is the end of the
+// first pass and the exchange, during which a CU asks memory for nothing.
+//
+// A packed access as 32-bit words, and its element k as fp32.
+// Rows too wide for two register sets (vocabularies of 57K to 160K at 16 bit, 32K to 80K at fp32): one
+// persistent 1024-lane workgroup per CU keeps ONE row, packed, in its registers.  The first pass takes the
+// running (max, sum) of the vectors as they arrive; the second forms each vector's gradient, stores it and
+// loads the same vector of the next row into the registers just freed, so loads and stores go out
+// side by side and the row is read from HBM once.  The two-sweep kernel below reads it again
+// out of the caches.  Two exponentials per element (13 us of VALU time a row) stay under the row's 20 us
+// of memory time because both passes run while memory does.
+//
+// Per call, against two sweeps: [4096,128256] bf16 457 -> 401 us (5.2 TB/s), [4096,152064] 536 -> 478,
+// [4096,100003] unpadded 374 -> 316, [2048,128256] with fp32 gradients 390 -> 308, [4096,60032] fp16
+// 210 -> 189, [2048,80000] fp32 288 -> 257.  What is left to the copy's 6.5 TB/s is the end of the
+// first pass and the exchange, during which a CU asks memory for nothing.
+//
+template <typename T, int EPV>
+struct Words {
+  static constexpr int n = EPV * (int)sizeof(T) / 4;
+  typedef uint32_t type __attribute__((ext_vector_type(EPV * sizeof(T) / 4)));
+};
+template <typename T, int EPV>
+__device__ __forceinline__ float word_elem(const typename Words<T, EPV>::type &w, int k) {
+  if constexpr (std::is_same_v<T, float>) {
+    return __uint_as_float(w[k]);
+  } else if constexpr (std::is_same_v<T, bf16_t>) {
+    return __uint_as_float((k & 1) ? w[k >> 1] & 0xffff0000u : w[k >> 1] << 16);
+  } else {
+    return (float)__builtin_bit_cast(_Float16, (uint16_t)((k & 1) ? w[k >> 1] >> 16 : w[k >> 1]));
+  }
+}
+template <typename T, int EPV>
+__device__ __forceinline__ void set_word_elem(typename Words<T, EPV>::type &w, int k, T v) {
+  if constexpr (sizeof(T) == 4) {
+    w[k] = __builtin_bit_cast(uint32_t, v);
+  } else {
+    const uint32_t b = __builtin_bit_cast(uint16_t, v);
+    w[k >> 1] = (k & 1) ? (w[k >> 1] & 0xffffu) | b << 16 : (w[k >> 1] & 0xffff0000u) | b;
+  }
+}
+
+// The registers hold the row and little else (20 vectors of 16 bytes are 80 of 128), so the row is kept as
+// 32-bit words, and the empty asm statements keep the compiler from carrying widened elements
+// from the first pass into the second or a lane's VPT offsets from row to row (both spill).
+//
+// VPT accesses of EPV elements per lane; RAGGED as in the streaming kernel.  Lanes past the row's
+// end load its last vector again (one address per wave) instead of branching round the load.  Elements
+// that are no class column are overwritten with -inf in the packed registers, so that neither pass masks
+// element by element.
+template <typename T, typename TD, int VPT, int EPV, bool RAGGED>
+__global__ __launch_bounds__(1024) void ce_rows_hold_kernel(
+    const T *logits, TD *dlogits, const int64_t *__restrict__ targets, float *__restrict__ row_loss,
+    const int *__restrict__ ws_count, int64_t N, int64_t V, int64_t row_stride, int64_t ignore_index,
+    int reduction, float dloss, const float *__restrict__ class_weight) {
+  constexpr int BLOCK = 1024;
+  constexpr int VN = EPV;
+  constexpr int CH = 16 / VN;  // vectors per step of the first pass: 16 elements
+  static_assert(VPT % CH == 0, "whole steps");
+  constexpr int kWaves = BLOCK / kWave;
+  __shared__ float red_m[2][kWaves], red_s[2][kWaves];
+  using W = typename Words<T, EPV>::type;
+  int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = tid >> 6;
+  const int iV = (int)V, stride = (int)row_stride;
+  auto off_of = [&](int64_t r) { return RAGGED ? (int)((r * row_stride) & (kLineElems<T> - 1)) : 0; };
+  auto vecs_of = [&](int off) { return RAGGED ? (off + stride + VN - 1) / VN : stride / VN; };
+  auto whole_of = [&](int64_t r, int off) {
+    return vecs_of(off) - (RAGGED && r == N - 1 && (off + stride) % VN != 0 ? 1 : 0);
+  };
+  // vector j of this lane, of the row that starts at x; `last`: the last one to be loaded
+  auto load = [&](const T *x, int j, int last) {
+    const int idx = tid + BLOCK * j;
+    const uint32_t bytes = (uint32_t)(idx < last ? idx : last) * (uint32_t)(VN * sizeof(T));
+    return __builtin_nontemporal_load(reinterpret_cast<const W *>(reinterpret_cast<const char *>(x) + bytes));
+  };
+
+  float scale0 = dloss;
+  if (reduction == CS_REDUCTION_MEAN)
+    scale0 = class_weight ? dloss / reinterpret_cast<const float *>(ws_count)[1] : dloss / (float)(*ws_count);
+
+  // neighbouring rows on one XCD, as in the streaming kernel
+  int64_t row = (gridDim.x % 8 == 0) ? (int64_t)(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
+  if (row >= N) return;
+  W cur[VPT];
+  int64_t tgt = targets[row];
+  bool live = target_counts(tgt, V, ignore_index);
+  T x_t;
+  {
+    const int off = off_of(row), last = live ? whole_of(row, off) - 1 : 0;
+    const T *x = logits + row * row_stride - off;
+    x_t = x[off + (live ? tgt : 0)];
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) cur[j] = load(x, j, last);
+  }
+  int parity = 0;
+  for (;;) {
+    asm volatile("" : "+v"(tid));
+    // the next row; where there is none, or it is ignored, every load below is of one vector
+    const int64_t nrow = row + gridDim.x;
+    const bool more = nrow < N;
+    const int64_t ntgt = targets[more ? nrow : row];
+    const bool nlive = more && target_counts(ntgt, V, ignore_index);
+    const int noff = more ? off_of(nrow) : 0;
+    const T *nx = logits + (more ? nrow * row_stride - noff : 0);
+    const int nlast = nlive ? whole_of(nrow, noff) - 1 : 0;
+    const int off = off_of(row), nvec = vecs_of(off);
+    TD *d = dlogits + row * row_stride - off;
+    // An ignored row goes the same way as a row without class columns: no first pass, and zeros out.
+    // (A branch of its own, with the next row's loads in it, makes the compiler spill the row.)
+    const int vcols = live ? iV : 0, nsum = live ? nvec : 0;
+    const float wt = class_weight && live ? class_weight[tgt] : 1.f;
+    if (RAGGED && row == N - 1 && whole_of(row, off) < nvec) {  // the array's last vector is not whole
+#pragma unroll
+      for (int j = 0; j < VPT; ++j) {
+        const int idx = tid + BLOCK * j;
+        if (idx == nvec - 1) {
+#pragma unroll
+          for (int k = 0; k < VN; ++k) {
+            const int c = idx * VN - off + k;
+            set_word_elem<T, EPV>(cur[j], k, logits[row * row_stride + (c < stride ? c : 0)]);
+          }
+        }
+      }
+    }
+    // ---- running maximum (times log2 e) and the sum relative to it
+    float m2 = -INFINITY, s = 0.f;
+#pragma unroll
+    for (int q = 0; q < VPT / CH; ++q) {
+      if (q * CH * BLOCK < nsum) {  // block-uniform
+        float cm = -INFINITY;
+        float xs[CH][VN];
+#pragma unroll
+        for (int u = 0; u < CH; ++u) {
+          const int j = q * CH + u;
+          const int c0 = (tid + BLOCK * j) * VN - off;
+          if (c0 + VN > vcols || (RAGGED && j == 0 && c0 < 0)) {
+#pragma unroll
+            for (int k = 0; k < VN; ++k)
+              if (c0 + k >= vcols || (RAGGED && j == 0 && c0 + k < 0)) set_word_elem<T, EPV>(cur[j], k, from_acc<T>(-INFINITY));
+          }
+#pragma unroll
+          for (int k = 0; k < VN; ++k) {
+            xs[u][k] = word_elem<T, EPV>(cur[j], k);
+            cm = fmaxf(cm, xs[u][k]);
+          }
+        }
+        const float cm2 = cm * kLog2e;
+        if (cm2 > m2) {
+          s *= __builtin_amdgcn_exp2f(m2 - cm2);  // 0 the first time (m2 = -inf, s = 0)
+          m2 = cm2;
+        }
+        // nothing finite so far: every term is 2^-inf (or NaN) against any finite stand-in
+        const float ref = m2 == -INFINITY ? 0.f : m2;
+        // pairwise within the step and one add onto the running sum, as in the two-sweep kernel
+        float part[CH];
+#pragma unroll
+        for (int u = 0; u < CH; ++u) {
+          float e[VN];
+#pragma unroll
+          for (int k = 0; k < VN; ++k) e[k] = __builtin_amdgcn_exp2f(__builtin_fmaf(xs[u][k], kLog2e, -ref));
+#pragma unroll
+          for (int w = VN / 2; w > 0; w /= 2)
+#pragma unroll
+            for (int k = 0; k < w; ++k) e[k] += e[k + w];
+          part[u] = e[0];
+        }
+#pragma unroll
+        for (int w = CH / 2; w > 0; w /= 2)
+#pragma unroll
+          for (int u = 0; u < w; ++u) part[u] += part[u + w];
+        s += part[0];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // ---- (max, sum) across the wave, then across the waves.  A lane without a finite value
+    // brings its sum as it is: 0, or the NaN it met.
+    const float mw2 = wave_reduce(m2, MaxOp{});
+    const float sw = wave_reduce(m2 == -INFINITY ? s : s * __builtin_amdgcn_exp2f(m2 - mw2), SumOp{});
+    if (lane == 0) {
+      red_m[parity][wave] = mw2;
+      red_s[parity][wave] = sw;
+    }
+    lds_barrier();
+    const float pm = lane < kWaves ? red_m[parity][lane] : -INFINITY;
+    const float ps = lane < kWaves ? red_s[parity][lane] : 0.f;
+    const float M2 = wave_reduce(pm, MaxOp{});
+    const float S = wave_reduce(pm == -INFINITY ? ps : ps * __builtin_amdgcn_exp2f(pm - M2), SumOp{});
+    parity ^= 1;  // the other pair of arrays next time: one barrier per row is enough
+    const float scale = scale0 * wt;
+    if (tid == 0 && row_loss) {
+      const float l = (__builtin_amdgcn_logf(S) - __builtin_fmaf(to_acc(x_t), kLog2e, -M2)) * kLn2;
+      row_loss[row] = live ? l * wt : 0.f;
+    }
+    const T nx_t = nx[noff + (nlive ? ntgt : 0)];
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) asm volatile("" : "+v"(cur[j]));
+    asm volatile("" : "+v"(tid));
+    // ---- gradient (p - onehot) * scale with p = 2^(x log2e - M2) / S, and the next row's loads
+    const float factor = scale / S;
+    const int t_at = (int)tgt + off;
+    const int t_vec = live ? t_at / VN : -1, t_sub = t_at % VN;
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+      const int idx = tid + BLOCK * j, c0 = idx * VN - off;
+      if (j * BLOCK < nvec) {  // block-uniform
+        float o[VN];
+#pragma unroll
+        for (int k = 0; k < VN; ++k)
+          o[k] = __builtin_amdgcn_exp2f(__builtin_fmaf(word_elem<T, EPV>(cur[j], k), kLog2e, -M2)) * factor;
+        if (idx == t_vec) {
+#pragma unroll
+          for (int k = 0; k < VN; ++k)
+            if (k == t_sub) o[k] -= scale;
+        }
+        if (c0 + VN > vcols) {  // 0 also where the row's maximum or sum is not finite
+#pragma unroll
+          for (int k = 0; k < VN; ++k)
+            if (c0 + k >= vcols) o[k] = 0.f;
+        }
+        if (idx < nvec) {
+          if (RAGGED && (c0 < 0 || c0 + VN > stride)) {
+            store_own<TD, VN>(d + (int64_t)idx * VN, o, c0, stride);
+          } else {
+            store_out<T, TD, VN>(d + (int64_t)idx * VN, o);
+          }
+        }
+      }
+      cur[j] = load(nx, j, nlast);
+      __builtin_amdgcn_sched_barrier(0);  // a load hoisted above its vector's use would need registers of its own
+    }
+    if (!more) break;
+    row = nrow;
+    tgt = ntgt;
+    live = nlive;
+    x_t = nx_t;
+  }
+}
+
+// Rows too wide for registers, rows too wide for the streaming kernel where only the loss is wanted, and
+// narrow rows whose stride is not a multiple of the vector width (a
 // vocabulary used unpadded).  Persistent workgroups walk rows.  A row is split into a head of
 // single elements up to the first 16-byte boundary, a body of whole vectors and a tail; the
 // base pointers are 16-byte aligned, so gradient rows split at the same columns.  The body is
@@ -841,6 +1093,36 @@ void launch_stream(const void *logits, void *dlogits, const int64_t *targets, fl
 #undef CS_CE_STREAM
 }
 
+// Vectors per lane of the row-holding kernel: three, four or five units.
+template <typename T, typename TD>
+struct HoldPlan {
+  static constexpr int kEpv = StreamPlan<T, TD>::kEpv;
+  static constexpr int kUnit = kEpv * sizeof(T) == 8 ? 8 : 4;
+  static constexpr int kMostVecs = 1024 * 5 * kUnit;
+};
+
+template <typename T, typename TD, bool RAGGED>
+void launch_hold(const void *logits, void *dlogits, const int64_t *targets, float *row_loss,
+                 const int *ws_count, int64_t N, int64_t V, int64_t row_stride, int64_t ignore_index,
+                 int reduction, float dloss, const float *class_weight, hipStream_t s) {
+  constexpr int EPV = HoldPlan<T, TD>::kEpv, U = HoldPlan<T, TD>::kUnit;
+  const int64_t cus = compute_units();
+  const dim3 grid((unsigned)(N < cus ? N : cus)), block(1024);
+  const int64_t nvec = (row_stride + (RAGGED ? kLineElems<T> - 1 : 0) + EPV - 1) / EPV;
+#define CS_CE_HOLD(VPT)                                                                                  \
+  ce_rows_hold_kernel<T, TD, VPT, EPV, RAGGED><<<grid, block, 0, s>>>(                                    \
+      (const T *)logits, (TD *)dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index,     \
+      reduction, dloss, class_weight)
+  if (nvec <= 1024 * 3 * U) {
+    CS_CE_HOLD(3 * U);
+  } else if (nvec <= 1024 * 4 * U) {
+    CS_CE_HOLD(4 * U);
+  } else {
+    CS_CE_HOLD(5 * U);
+  }
+#undef CS_CE_HOLD
+}
+
 template <typename T, typename TD>
 int launch_rows(const void *logits, void *dlogits, const int64_t *targets, float *row_loss,
                 const int *ws_count, int64_t N, int64_t V, int64_t row_stride,
@@ -857,6 +1139,13 @@ int launch_rows(const void *logits, void *dlogits, const int64_t *targets, float
     const int64_t nvec_all = row_stride / VN;
     const bool streams = nvec_all > 256 * 8 &&
                          row_stride <= (int64_t)StreamPlan<T, TD>::kEpv * StreamPlan<T, TD>::kMostVecs;
+    // The loss alone needs no second pass: nothing to hold a row for.  A few rows more than there are
+    // CUs are a second round of whole rows for the row-holding kernel, while the two-sweep kernel runs two
+    // rows per CU: [300,128256] bf16 48.2 against 46.3 us, 257 rows 44.3 / 41.9, 384 rows 48.7 / 50.3, 256
+    // rows 29.6 / 35.4 (fp32 rows, where the alternative holds a row without streaming, gain there as well: [260,40000]
+    // 27.7 / 31.3).
+    const int64_t cus = compute_units();
+    const bool holds = dlogits != nullptr && nvec_all > 256 * 8 && (sizeof(T) == 4 || N <= cus || 4 * N > 5 * cus);
     if (vec_ok && (class_weight == nullptr || streams)) {
       const int64_t nvec = row_stride / VN;
 #define CS_CE(BLOCK, VPT)                                                                   \
@@ -870,6 +1159,9 @@ int launch_rows(const void *logits, void *dlogits, const int64_t *targets, float
       } else if (row_stride <= (int64_t)StreamPlan<T, TD>::kEpv * StreamPlan<T, TD>::kMostVecs) {
         launch_stream<T, TD, false>(logits, dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index,
                                     reduction, dloss, class_weight, s);
+      } else if (holds && row_stride <= (int64_t)HoldPlan<T, TD>::kEpv * HoldPlan<T, TD>::kMostVecs) {
+        launch_hold<T, TD, false>(logits, dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index,
+                                  reduction, dloss, class_weight, s);
       } else if (sizeof(T) == 4 && nvec <= 1024 * 16) {
         // fp32 rows up to 65536 columns still fit in registers (at 16 bit this plan spills)
         if constexpr (sizeof(T) == 4) CS_CE(1024, 16);
@@ -884,6 +1176,12 @@ int launch_rows(const void *logits, void *dlogits, const int64_t *targets, float
         row_stride + kLineElems<T> <= (int64_t)StreamPlan<T, TD>::kEpv * StreamPlan<T, TD>::kMostVecs) {
       launch_stream<T, TD, true>(logits, dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index,
                                  reduction, dloss, class_weight, s);
+      return launch_status();
+    }
+    if (base_ok && holds &&
+        row_stride + kLineElems<T> <= (int64_t)HoldPlan<T, TD>::kEpv * HoldPlan<T, TD>::kMostVecs) {
+      launch_hold<T, TD, true>(logits, dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index,
+                               reduction, dloss, class_weight, s);
       return launch_status();
     }
     if (base_ok && sizeof(TD) >= sizeof(T)) {

@@ -27,7 +27,7 @@ def co():
     (5, 32705, 32705, BF16, None),      # the four-vector plan with the line's 63 elements in front: its last width
     (5, 32706, 32707, BF16, None),      # the next one
     (3, 57279, 57279, F16, None),       # the widest streamed 16-bit row
-    (3, 57281, 57281, BF16, None),      # the next one: two sweeps
+    (3, 57281, 57281, BF16, None),      # the next one
     (2, 53183, 53183, BF16, F32),       # the widest with fp32 gradients
     (2, 53185, 53185, F16, F32),
     (260, 20011, 20011, BF16, F32),

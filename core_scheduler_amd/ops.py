@@ -38,18 +38,33 @@ def _dev(*tensors):
         if not t.is_contiguous():
             raise RuntimeError("core_scheduler_amd ops need contiguous tensors")
         if dev is None:
-            dev = t.device
-        elif t.device != dev:
+            dev, index = t.device, t.get_device()
+        elif t.get_device() != index:
             raise RuntimeError("tensors on different devices")
     return dev
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
-def _stream(dev):
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+def _call(name, dev, *args):
+    """The library call `name` on the current stream of `dev`, which every call takes last.
+
+    The small calls of a step cost more host time than device time, most of it around the call: the
+    device guard (1.3 us; entered only when another device is current), a stream object
+    for its handle (2.1 us, the handle itself 0.1) and a c_void_p object per pointer (the argument
+    types convert an int as well).
+    """
+    fn = getattr(_capi.load(), name)
+    index = dev.index
+    if index == torch._C._cuda_getDevice():
+        code = fn(*args, torch._C._cuda_getCurrentRawStream(index))
+    else:
+        with torch.cuda.device(dev):
+            code = fn(*args, torch._C._cuda_getCurrentRawStream(index))
+    if code != _capi.OK:
+        _capi.check(name, code)
 
 
 def _workspace(nbytes, dev):
@@ -77,10 +92,8 @@ def adamw_step(w, dw, m, v, *, lr, beta1, beta2, eps, weight_decay, t, v_max=Non
     _check_adamw_tensors(w, dw, m, v, v_max)
     dev = _dev(w, dw, m, v, v_max)
     lib = _capi.load()
-    with torch.cuda.device(dev):
-        code = lib.cs_adamw_step(_ptr(w), _ptr(dw), _ptr(m), _ptr(v), _ptr(v_max), w.numel(), _dt(w),
-                                 lr, beta1, beta2, eps, weight_decay, t, _stream(dev))
-    _capi.check("cs_adamw_step", code)
+    _call("cs_adamw_step", dev, _ptr(w), _ptr(dw), _ptr(m), _ptr(v), _ptr(v_max), w.numel(), _dt(w), lr, beta1, beta2,
+          eps, weight_decay, t)
 
 
 class MultiTensorAdamW:
@@ -145,21 +158,16 @@ class MultiTensorAdamW:
         taken first (two small launches) and the step applies the clipping coefficient to the
         gradients as it reads them; returns the norm as a 0-d device tensor then."""
         self.t += 1
-        lib = _capi.load()
         n = len(self.params)
-        with torch.cuda.device(self.dev):
-            if max_grad_norm is None:
-                code = lib.cs_adamw_multi_step(_ptr(self._table), n, self._slots, _DTYPES[self.dtype],
-                                               int(self.amsgrad), self.lr, self.beta1, self.beta2, self.eps,
-                                               self.weight_decay, self.t, _stream(self.dev))
-                _capi.check("cs_adamw_multi_step", code)
-                return None
-            norm = self.grad_norm(max_grad_norm, norm_type)
-            code = lib.cs_adamw_multi_step_clipped(_ptr(self._table), n, self._slots, _DTYPES[self.dtype],
-                                                   int(self.amsgrad), self.lr, self.beta1, self.beta2, self.eps,
-                                                   self.weight_decay, self.t, _ptr(self._clip), _stream(self.dev))
-            _capi.check("cs_adamw_multi_step_clipped", code)
-            return norm
+        if max_grad_norm is None:
+            _call("cs_adamw_multi_step", self.dev, _ptr(self._table), n, self._slots, _DTYPES[self.dtype],
+                  int(self.amsgrad), self.lr, self.beta1, self.beta2, self.eps, self.weight_decay, self.t)
+            return None
+        norm = self.grad_norm(max_grad_norm, norm_type)
+        _call("cs_adamw_multi_step_clipped", self.dev, _ptr(self._table), n, self._slots, _DTYPES[self.dtype],
+              int(self.amsgrad), self.lr, self.beta1, self.beta2, self.eps, self.weight_decay, self.t,
+              _ptr(self._clip))
+        return norm
 
     def grad_norm(self, max_norm, norm_type=2.0):
         """Global norm of all gradients; leaves the clipping coefficient in `self._clip`."""
@@ -169,20 +177,15 @@ class MultiTensorAdamW:
             self._norm_ws = torch.empty(nbytes, dtype=torch.uint8, device=self.dev)
             self._clip = torch.empty((), dtype=torch.float32, device=self.dev)
         norm = torch.empty((), dtype=torch.float32, device=self.dev)
-        with torch.cuda.device(self.dev):
-            code = lib.cs_grad_norm_multi(_ptr(self._table), len(self.params), self._slots, _DTYPES[self.dtype],
-                                          float(norm_type), float(max_norm), _ptr(self._norm_ws), nbytes,
-                                          _ptr(norm), _ptr(self._clip), _stream(self.dev))
-        _capi.check("cs_grad_norm_multi", code)
+        _call("cs_grad_norm_multi", self.dev, _ptr(self._table), len(self.params), self._slots, _DTYPES[self.dtype],
+              float(norm_type), float(max_norm), _ptr(self._norm_ws), nbytes, _ptr(norm), _ptr(self._clip))
         return norm
 
     def clip_grad_norm_(self, max_norm, norm_type=2.0):
         """The reference's Utils::clip_grad_norm_: scales the gradients in place, returns the norm."""
         norm = self.grad_norm(max_norm, norm_type)
-        with torch.cuda.device(self.dev):
-            code = _capi.load().cs_grad_scale_multi(_ptr(self._table), len(self.params), self._slots,
-                                                    _DTYPES[self.dtype], _ptr(self._clip), _stream(self.dev))
-        _capi.check("cs_grad_scale_multi", code)
+        _call("cs_grad_scale_multi", self.dev, _ptr(self._table), len(self.params), self._slots, _DTYPES[self.dtype],
+              _ptr(self._clip))
         return norm
 
 
@@ -190,10 +193,7 @@ class MultiTensorAdamW:
 def gelu_forward(x, approximate="none"):
     dev = _dev(x)
     y = torch.empty_like(x)
-    with torch.cuda.device(dev):
-        code = _capi.load().cs_gelu_forward(_ptr(x), _ptr(y), x.numel(), _dt(x), _GELU[approximate],
-                                            _stream(dev))
-    _capi.check("cs_gelu_forward", code)
+    _call("cs_gelu_forward", dev, _ptr(x), _ptr(y), x.numel(), _dt(x), _GELU[approximate])
     return y
 
 
@@ -202,10 +202,7 @@ def gelu_backward(dy, x, approximate="none"):
     if dy.dtype != x.dtype or dy.numel() != x.numel():
         raise ValueError("dy and x must match")
     dx = torch.empty_like(x)
-    with torch.cuda.device(dev):
-        code = _capi.load().cs_gelu_backward(_ptr(dy), _ptr(x), _ptr(dx), x.numel(), _dt(x),
-                                             _GELU[approximate], _stream(dev))
-    _capi.check("cs_gelu_backward", code)
+    _call("cs_gelu_backward", dev, _ptr(dy), _ptr(x), _ptr(dx), x.numel(), _dt(x), _GELU[approximate])
     return dx
 
 
@@ -224,11 +221,8 @@ def add_layernorm_forward(x, residual, gamma, beta=None, eps=1e-5, out_dtype=Non
     stat = torch.float64 if x.dtype == torch.float64 else torch.float32
     mean = torch.empty(rows, dtype=stat, device=dev)
     rstd = torch.empty(rows, dtype=stat, device=dev)
-    with torch.cuda.device(dev):
-        code = _capi.load().cs_add_layernorm_forward(_ptr(x), _ptr(residual), _ptr(total), _ptr(gamma), _ptr(beta),
-                                                     _ptr(y), _ptr(mean), _ptr(rstd), rows, C, eps, _dt(x),
-                                                     _dt(y), _dt(gamma), _stream(dev))
-    _capi.check("cs_add_layernorm_forward", code)
+    _call("cs_add_layernorm_forward", dev, _ptr(x), _ptr(residual), _ptr(total), _ptr(gamma), _ptr(beta), _ptr(y),
+          _ptr(mean), _ptr(rstd), rows, C, eps, _dt(x), _dt(y), _dt(gamma))
     return total, y, mean, rstd
 
 
@@ -243,11 +237,8 @@ def layernorm_forward(x, gamma, beta=None, eps=1e-5, out_dtype=None):
     stat = torch.float64 if x.dtype == torch.float64 else torch.float32
     mean = torch.empty(rows, dtype=stat, device=dev)
     rstd = torch.empty(rows, dtype=stat, device=dev)
-    with torch.cuda.device(dev):
-        code = _capi.load().cs_layernorm_forward(_ptr(x), _ptr(gamma), _ptr(beta), _ptr(y), _ptr(mean),
-                                                 _ptr(rstd), rows, C, eps, _dt(x), _dt(y), _dt(gamma),
-                                                 _stream(dev))
-    _capi.check("cs_layernorm_forward", code)
+    _call("cs_layernorm_forward", dev, _ptr(x), _ptr(gamma), _ptr(beta), _ptr(y), _ptr(mean), _ptr(rstd), rows, C, eps,
+          _dt(x), _dt(y), _dt(gamma))
     return y, mean, rstd
 
 
@@ -276,18 +267,14 @@ def layernorm_backward(dy, x, mean, rstd, gamma, *, need_dx=True, need_dgamma=Tr
     lib = _capi.load()
     ws_bytes = lib.cs_layernorm_backward_workspace_bytes(rows, C) if (need_dgamma or need_dbeta) else 0
     ws = _workspace(ws_bytes, dev) if ws_bytes else None
-    with torch.cuda.device(dev):
-        if dresidual is not None:
-            code = lib.cs_layernorm_backward_add(_ptr(dy), _ptr(x), _ptr(mean), _ptr(rstd), _ptr(gamma),
-                                                 _ptr(dresidual), _ptr(dx), _ptr(dgamma), _ptr(dbeta), _ptr(ws),
-                                                 ws_bytes, rows, C, _dt(dy), _dt(x), _dt(dx), _dt(gamma),
-                                                 int(accumulate), _stream(dev))
-        else:
-            code = lib.cs_layernorm_backward(_ptr(dy), _ptr(x), _ptr(mean), _ptr(rstd), _ptr(gamma), _ptr(dx),
-                                             _ptr(dgamma), _ptr(dbeta), _ptr(ws), ws_bytes, rows, C, _dt(dy),
-                                             _dt(x), _dt(dx) if dx is not None else _dt(dy), _dt(gamma),
-                                             int(accumulate), _stream(dev))
-    _capi.check("cs_layernorm_backward", code)
+    if dresidual is not None:
+        _call("cs_layernorm_backward_add", dev, _ptr(dy), _ptr(x), _ptr(mean), _ptr(rstd), _ptr(gamma),
+              _ptr(dresidual), _ptr(dx), _ptr(dgamma), _ptr(dbeta), _ptr(ws), ws_bytes, rows, C, _dt(dy), _dt(x),
+              _dt(dx), _dt(gamma), int(accumulate))
+    else:
+        _call("cs_layernorm_backward", dev, _ptr(dy), _ptr(x), _ptr(mean), _ptr(rstd), _ptr(gamma), _ptr(dx),
+              _ptr(dgamma), _ptr(dbeta), _ptr(ws), ws_bytes, rows, C, _dt(dy), _dt(x),
+              _dt(dx) if dx is not None else _dt(dy), _dt(gamma), int(accumulate))
     return dx, dgamma, dbeta
 
 
@@ -310,12 +297,9 @@ def layernorm_backward_rows(dy, x, mean, rstd, gamma, *, need_dx=True, dx_dtype=
         raise ValueError(f"no split form for rows of {C} {x.dtype} elements")
     dx = torch.empty(x.shape, dtype=dx_dtype or x.dtype, device=dev) if need_dx else None
     partials = torch.empty((n, 2, C), dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
-        code = lib.cs_layernorm_backward_rows(_ptr(dy), _ptr(x), _ptr(mean), _ptr(rstd), _ptr(gamma),
-                                              _ptr(dresidual), _ptr(dx), _ptr(partials), partials.numel() * 4,
-                                              rows, C, _dt(dy), _dt(x), _dt(dx) if dx is not None else _dt(dy),
-                                              _dt(gamma), _stream(dev))
-    _capi.check("cs_layernorm_backward_rows", code)
+    _call("cs_layernorm_backward_rows", dev, _ptr(dy), _ptr(x), _ptr(mean), _ptr(rstd), _ptr(gamma), _ptr(dresidual),
+          _ptr(dx), _ptr(partials), partials.numel() * 4, rows, C, _dt(dy), _dt(x), _dt(dx) if dx is not None else
+          _dt(dy), _dt(gamma))
     return dx, partials
 
 
@@ -341,11 +325,8 @@ def layernorm_backward_finalize(partials, x_dtype, param_dtype, *, need_dgamma=T
         dgamma = None
     if not need_dbeta:
         dbeta = None
-    with torch.cuda.device(dev):
-        code = _capi.load().cs_layernorm_backward_finalize(_ptr(partials), n, _ptr(dgamma), _ptr(dbeta), C,
-                                                           _DTYPES[x_dtype], _DTYPES[param_dtype], int(accumulate),
-                                                           _stream(dev))
-    _capi.check("cs_layernorm_backward_finalize", code)
+    _call("cs_layernorm_backward_finalize", dev, _ptr(partials), n, _ptr(dgamma), _ptr(dbeta), C, _DTYPES[x_dtype],
+          _DTYPES[param_dtype], int(accumulate))
     return dgamma, dbeta
 
 
@@ -389,13 +370,10 @@ class LayerNormBackwardChain:
             dgamma = torch.empty(C, dtype=gamma.dtype, device=dev)
             dbeta = torch.empty(C, dtype=gamma.dtype, device=dev)
         partials = torch.empty((n, 2, C), dtype=torch.float32, device=dev)
-        with torch.cuda.device(dev):
-            code = lib.cs_layernorm_backward_rows_pending(
-                _ptr(dy), _ptr(x), _ptr(mean), _ptr(rstd), _ptr(gamma), _ptr(dresidual), _ptr(dx), _ptr(partials),
-                partials.numel() * 4, _ptr(pend[0]) if pend else None, pend[0].shape[0] if pend else 0,
-                _ptr(pend[1]) if pend else None, _ptr(pend[2]) if pend else None, int(pend[3]) if pend else 0,
-                rows, C, _dt(dy), _dt(x), _dt(dx), _dt(gamma), _stream(dev))
-        _capi.check("cs_layernorm_backward_rows_pending", code)
+        _call("cs_layernorm_backward_rows_pending", dev, _ptr(dy), _ptr(x), _ptr(mean), _ptr(rstd), _ptr(gamma),
+              _ptr(dresidual), _ptr(dx), _ptr(partials), partials.numel() * 4, _ptr(pend[0]) if pend else None,
+              pend[0].shape[0] if pend else 0, _ptr(pend[1]) if pend else None, _ptr(pend[2]) if pend else None,
+              int(pend[3]) if pend else 0, rows, C, _dt(dy), _dt(x), _dt(dx), _dt(gamma))
         self._pending = (partials, dgamma, dbeta, accumulate, C, x.dtype, gamma.dtype)
         return dx, dgamma, dbeta
 
@@ -405,11 +383,8 @@ class LayerNormBackwardChain:
         if pend is None:
             return
         partials, dgamma, dbeta, accumulate, C, x_dtype, p_dtype = pend
-        with torch.cuda.device(partials.device):
-            code = _capi.load().cs_layernorm_backward_finalize(_ptr(partials), partials.shape[0], _ptr(dgamma),
-                                                               _ptr(dbeta), C, _DTYPES[x_dtype], _DTYPES[p_dtype],
-                                                               int(accumulate), _stream(partials.device))
-        _capi.check("cs_layernorm_backward_finalize", code)
+        _call("cs_layernorm_backward_finalize", partials.device, _ptr(partials), partials.shape[0], _ptr(dgamma),
+              _ptr(dbeta), C, _DTYPES[x_dtype], _DTYPES[p_dtype], int(accumulate))
 
 
 # -------------------------------------------------------------- Embedding
@@ -418,10 +393,8 @@ def embedding_forward(weight, indices):
     dev = _dev(weight, indices)
     V, C = weight.shape
     out = torch.empty(*indices.shape, C, dtype=weight.dtype, device=dev)
-    with torch.cuda.device(dev):
-        code = _capi.load().cs_embedding_forward(_ptr(weight), _ptr(indices), _ptr(out), indices.numel(), C,
-                                                 V, _dt(weight), _ITYPES[indices.dtype], _stream(dev))
-    _capi.check("cs_embedding_forward", code)
+    _call("cs_embedding_forward", dev, _ptr(weight), _ptr(indices), _ptr(out), indices.numel(), C, V, _dt(weight),
+          _ITYPES[indices.dtype])
     return out
 
 
@@ -433,10 +406,8 @@ def embedding_forward_add(wte, wpe, indices):
     if wpe.shape[0] < T or wpe.shape[1] != C or wpe.dtype != wte.dtype:
         raise ValueError("wpe must be [>=T, C] of wte's dtype")
     out = torch.empty(B, T, C, dtype=wte.dtype, device=dev)
-    with torch.cuda.device(dev):
-        code = _capi.load().cs_embedding_forward_add(_ptr(wte), _ptr(wpe), _ptr(indices), _ptr(out), B, T, C,
-                                                     V, _dt(wte), _ITYPES[indices.dtype], _stream(dev))
-    _capi.check("cs_embedding_forward_add", code)
+    _call("cs_embedding_forward_add", dev, _ptr(wte), _ptr(wpe), _ptr(indices), _ptr(out), B, T, C, V, _dt(wte),
+          _ITYPES[indices.dtype])
     return out
 
 
@@ -460,11 +431,9 @@ def embedding_backward(dout, indices, num_weights, padding_idx=-1, dweight=None,
     lib = _capi.load()
     ws_bytes = lib.cs_embedding_backward_workspace_bytes(n, C, num_weights)
     ws = _workspace(ws_bytes, dev)
-    with torch.cuda.device(dev):
-        call = lib.cs_embedding_backward_scaled if scale_grad_by_freq else lib.cs_embedding_backward
-        code = call(_ptr(dout), _ptr(indices), _ptr(dweight), _ptr(ws), ws_bytes, n, C, num_weights, padding_idx,
-                    _dt(dout), _ITYPES[indices.dtype], int(accumulate), _stream(dev))
-    _capi.check("cs_embedding_backward", code)
+    _call("cs_embedding_backward_scaled" if scale_grad_by_freq else "cs_embedding_backward", dev, _ptr(dout),
+          _ptr(indices), _ptr(dweight), _ptr(ws), ws_bytes, n, C, num_weights, padding_idx, _dt(dout),
+          _ITYPES[indices.dtype], int(accumulate))
     return dweight
 
 
@@ -484,11 +453,8 @@ def embedding_backward_fused(dout, indices, num_weights, dwte=None, dwpe=None):
     lib = _capi.load()
     ws_bytes = lib.cs_embedding_backward_workspace_bytes(B * T, C, num_weights)
     ws = _workspace(ws_bytes, dev)
-    with torch.cuda.device(dev):
-        code = lib.cs_embedding_backward_fused(_ptr(dout), _ptr(indices), _ptr(dwte), _ptr(dwpe), _ptr(ws),
-                                               ws_bytes, B, T, C, num_weights, _dt(dout),
-                                               _ITYPES[indices.dtype], int(accumulate), _stream(dev))
-    _capi.check("cs_embedding_backward_fused", code)
+    _call("cs_embedding_backward_fused", dev, _ptr(dout), _ptr(indices), _ptr(dwte), _ptr(dwpe), _ptr(ws), ws_bytes, B,
+          T, C, num_weights, _dt(dout), _ITYPES[indices.dtype], int(accumulate))
     return dwte, dwpe
 
 
@@ -500,10 +466,7 @@ def embedding_backward_positions(dout, dwpe=None):
     dev = _dev(dout, dwpe)
     if dwpe is None:
         dwpe = torch.empty(T, C, dtype=dout.dtype, device=dev)
-    with torch.cuda.device(dev):
-        code = _capi.load().cs_embedding_backward_positions(_ptr(dout), _ptr(dwpe), B, T, C, _dt(dout),
-                                                            int(accumulate), _stream(dev))
-    _capi.check("cs_embedding_backward_positions", code)
+    _call("cs_embedding_backward_positions", dev, _ptr(dout), _ptr(dwpe), B, T, C, _dt(dout), int(accumulate))
     return dwpe
 
 
@@ -538,13 +501,11 @@ def fused_classifier(logits, targets, num_classes=None, *, ignore_index=-100, re
     ws_bytes = lib.cs_fused_classifier_workspace_bytes(N)
     ws = _workspace(ws_bytes, dev)
     tail = (_ptr(ws), ws_bytes, N, V, stride, ignore_index, _REDUCTIONS[reduction], dloss, _dt(logits),
-            _dt(dlogits) if dlogits is not None else _dt(logits), _stream(dev))
-    with torch.cuda.device(dev):
-        if class_weight is None:
-            code = lib.cs_fused_classifier(_ptr(logits), _ptr(dlogits), _ptr(targets), _ptr(row_loss), _ptr(loss),
-                                           _ptr(total_weight), *tail)
-        else:
-            code = lib.cs_fused_classifier_weighted(_ptr(logits), _ptr(dlogits), _ptr(targets), _ptr(class_weight),
-                                                    _ptr(row_loss), _ptr(loss), _ptr(total_weight), *tail)
-    _capi.check("cs_fused_classifier", code)
+            _dt(dlogits) if dlogits is not None else _dt(logits))
+    if class_weight is None:
+        _call("cs_fused_classifier", dev, _ptr(logits), _ptr(dlogits), _ptr(targets), _ptr(row_loss), _ptr(loss),
+              _ptr(total_weight), *tail)
+    else:
+        _call("cs_fused_classifier_weighted", dev, _ptr(logits), _ptr(dlogits), _ptr(targets), _ptr(class_weight),
+              _ptr(row_loss), _ptr(loss), _ptr(total_weight), *tail)
     return (row_loss if reduction == "none" else loss), row_loss, dlogits, total_weight

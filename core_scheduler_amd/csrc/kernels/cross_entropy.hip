@@ -574,33 +574,7 @@ __global__ __launch_bounds__(1024) void ce_rows_stream_kernel(
   }
 }
 
-// Rows too wide for two register sets (vocabularies of 57K to 160K at 16 bit, 32K to 80K at fp32): one
-// persistent 1024-lane workgroup per CU keeps ONE row, packed, in its registers.  The first pass takes the
-// running (max, sum) of the vectors as they arrive; the second forms each vector's gradient, stores it and
-// loads the same vector of the next row into the registers just freed, so loads and stores go out
-// side by side and the row is read from HBM once.  The two-sweep kernel below reads it again
-// out of the caches.  Two exponentials per element (13 us of VALU time a row) stay under the row's 20 us
-// of memory time because both passes run while memory does.
-//
-// Per call, against two sweeps: [4096,128256] bf16 457 -> 401 us (5.2 TB/s), [4096,152064] 536 -> 478,
-// [4096,100003] unpadded 374 -> 316, [2048,128256] with fp32 gradients 390 -> 308, [4096,60032] fp16
-// 210 -> 189, [2048,80000] fp32 288 -> 257.  What is left to the copy's 6.5 TB/s is the end of the
-// first pass and the exchange, during which a CU asks memory for nothing.
-//
-// A packed access as 32-bit words, and its element k as fp32.
-// Rows too wide for two register sets (vocabularies of 57K to 160K at 16 bit, 32K to 80K at fp32): one
-// persistent 1024-lane workgroup per CU keeps ONE row, packed, in its registers.  The first pass takes the
-// running (max, sum) of the vectors as they arrive; the second forms each vector's gradient, stores it and
-// loads the same vector of the next row into the registers just freed, so loads and stores go out
-// side by side and the row is read from HBM once.  The two-sweep kernel below reads it again
-// out of the caches.  Two exponentials per element (13 us of VALU time a row) stay under the row's 20 us
-// of memory time because both passes run while memory does.
-//
-// Per call, against two sweeps: [4096,128256] bf16 457 -> 401 us (5.2 TB/s), [4096,152064] 536 -> 478,
-// [4096,100003] unpadded 374 -> 316, [2048,128256] with fp32 gradients 390 -> 308, [4096,60032] fp16
-// 210 -> 189, [2048,80000] fp32 288 -> 257.  What is left to the copy's 6.5 TB/s is the end of the
-// first pass and the exchange, during which a CU asks memory for nothing.
-//
+// A packed access as 32-bit words: element k as fp32, and element k replaced.
 template <typename T, int EPV>
 struct Words {
   static constexpr int n = EPV * (int)sizeof(T) / 4;
@@ -626,6 +600,20 @@ __device__ __forceinline__ void set_word_elem(typename Words<T, EPV>::type &w, i
   }
 }
 
+// Rows too wide for two register sets (vocabularies of 57K to 160K at 16 bit, 32K to 80K at fp32): one
+// persistent 1024-lane workgroup per CU keeps ONE row, packed, in its registers.  The first pass takes the
+// running (max, sum) of the vectors as they arrive; the second forms each vector's gradient, stores it and
+// loads the same vector of the next row into the registers just freed, so loads and stores go out
+// side by side and the row is read from HBM once.  The two-sweep kernel below reads it again
+// out of the caches.  Two exponentials per element (13 us of VALU time a row, by count) stay under the row's 20 us
+// of memory time because both passes run while memory does.
+//
+// Per call, against two sweeps: [4096,128256] bf16 457 -> 401 us (5.2 TB/s), [4096,152064] 536 -> 478,
+// [4096,100003] unpadded 374 -> 316, [2048,128256] with fp32 gradients 390 -> 308, [4096,60032] fp16
+// 210 -> 189, [2048,80000] fp32 288 -> 257.  Having a quarter of the next row under way before the
+// current one is finished (the registers allow it) did not matter, 400 us at [4096,128256] and 480 at 152064:
+// the exchange between the passes is not what keeps the kernel from the streaming kernel's 5.8 TB/s.
+//
 // The registers hold the row and little else (20 vectors of 16 bytes are 80 of 128), so the row is kept as
 // 32-bit words, and the empty asm statements keep the compiler from carrying widened elements
 // from the first pass into the second or a lane's VPT offsets from row to row (both spill).
@@ -1410,7 +1398,7 @@ extern "C" int cs_fused_classifier_static(const void *logits, void *dlogits, con
   void *ws = nullptr;
   const int st = static_scratch(&ws);
   if (st != CS_OK) return st;
-  // Nothing in the scratch has to start at zero: the counting launch overwrites the header and
+  // Nothing in the scratch has to start at zero: the launch that counts overwrites the header and
   // the row pass overwrites the N row losses that the reduction then reads.
   const CeArgs a{logits, dlogits, targets, row_loss, loss, total_weight, ws,
                  (size_t)CS_FUSED_CLASSIFIER_STATIC_SCRATCH_BYTES, N, V, row_stride, ignore_index,

@@ -19,6 +19,7 @@
 //                                    current one (50257 bf16 = 6283 vectors = 7 per lane)
 //   up to 20480 with a gradient      ce_rows_hold_kernel: one persistent workgroup per CU keeps
 //                                    one row and loads the next into the registers it frees
+//   the loss alone of many rows      ce_loss_rows_kernel: one workgroup per row, nothing kept
 //   wider, the loss alone, or narrow ce_rows_wide_kernel: two sweeps over the row, the
 //   rows that start off 16 bytes     second one served by the cache
 //   fp64, unaligned base pointers    ce_rows_general_kernel
@@ -812,6 +813,151 @@ __global__ __launch_bounds__(1024) void ce_rows_hold_kernel(
   }
 }
 
+// The loss alone (validation) of rows beyond the small register plans: one workgroup per row, the row read
+// once in chunks of four 16-byte vectors per lane, two chunks in registers (one on its way while the other
+// joins the lane's running (max, sum)).  No row is kept and no workgroup lives longer than its row, so six
+// workgroups of 256 share a CU and cover each other's waits and exchanges, where the streaming kernel
+// has one workgroup of 1024 per CU and one barrier per row between loads.  Bound by HBM reads.
+//
+// Per call, against the kernels for fewer rows: [8192,50257] bf16 152 -> 128 us (6.4 TB/s), [4096,50257] 81 -> 68,
+// [8192,17000] 92 -> 52, [8192,128256] 357 -> 312, [4096,50257] fp16 89 -> 69, fp32 [4096,10000] 42 -> 28,
+// [4096,50257] 141 -> 123, [4096,100000] 271 -> 240.  Six waves per SIMD: in the registers of eight
+// the 16-bit chunks spill 48 to 64 bytes a lane.
+//
+// Rows may start anywhere: vectors count from the 128-byte line a row starts in, as in the streaming
+// kernel, and what is no class column counts as -inf.  Lanes past the row's end load its last vector again.
+template <typename T, int BLOCK>
+__global__ __launch_bounds__(BLOCK, 6) void ce_loss_rows_kernel(
+    const T *__restrict__ logits, const int64_t *__restrict__ targets, float *__restrict__ row_loss, int64_t N,
+    int64_t V, int64_t row_stride, int64_t ignore_index, const float *__restrict__ class_weight) {
+  constexpr int VN = Vec16<T>::n;
+  constexpr int U = 4, CH = 8 / VN;  // vectors per chunk, and of these per step of 8 elements
+  constexpr int kWaves = BLOCK / kWave;
+  __shared__ float red_m[kWaves], red_s[kWaves];
+  using W = typename Words<T, VN>::type;
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int64_t row = blockIdx.x;
+  const int64_t tgt = targets[row];
+  if (!target_counts(tgt, V, ignore_index)) {
+    if (tid == 0) row_loss[row] = 0.f;
+    return;
+  }
+  const int stride = (int)row_stride;
+  const int off = (int)((row * row_stride) & (kLineElems<T> - 1));
+  const T *x = logits + row * row_stride - off;
+  // Vectors that hold class columns.  The array's last one may not lie whole inside it: its columns
+  // [iV, V) are then added one to a lane.
+  int nvec = (int)((off + V + VN - 1) / VN), iV = (int)V;
+  if (row == N - 1 && nvec * VN > off + stride) iV = --nvec * VN - off;
+  const int last = nvec - 1;
+  const int steps = (nvec + U * BLOCK - 1) / (U * BLOCK);
+
+  // (the empty asm statements keep the compiler from widening a vector before it is used and from carrying
+  // every vector's column from chunk to chunk: both spill)
+  auto load = [&](W (&c)[U], int q) {
+    int t = tid;
+    asm volatile("" : "+v"(t));
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int idx = t + BLOCK * (q * U + u);
+      const uint32_t bytes = (uint32_t)(idx < last ? idx : last) * 16u;
+      c[u] = __builtin_nontemporal_load(reinterpret_cast<const W *>(reinterpret_cast<const char *>(x) + bytes));
+    }
+  };
+  float m2 = -INFINITY, s = 0.f;  // maximum times log2 e, and the sum relative to it
+  auto step = [&](W (&c)[U], int q) {
+    int t = tid * VN - off;
+    asm volatile("" : "+v"(t));
+    // where a chunk may reach past the row's class columns (block-uniform)
+    const bool edge = q == 0 || (q + 1) * (U * BLOCK * VN) - off > iV;
+#pragma unroll
+    for (int h = 0; h < U; h += CH) {
+      float cm = -INFINITY;
+      float xs[CH][VN];
+#pragma unroll
+      for (int u = 0; u < CH; ++u) {
+        asm volatile("" : "+v"(c[h + u]));
+        const int c0 = t + VN * BLOCK * (q * U + h + u);
+#pragma unroll
+        for (int k = 0; k < VN; ++k) xs[u][k] = word_elem<T, VN>(c[h + u], k);
+        if (edge) {
+#pragma unroll
+          for (int k = 0; k < VN; ++k) xs[u][k] = (uint32_t)(c0 + k) < (uint32_t)iV ? xs[u][k] : -INFINITY;
+        }
+#pragma unroll
+        for (int k = 0; k < VN; ++k) cm = fmaxf(cm, xs[u][k]);
+      }
+      const float cm2 = cm * kLog2e;
+      if (cm2 > m2) {
+        s *= __builtin_amdgcn_exp2f(m2 - cm2);  // 0 the first time (m2 = -inf, s = 0)
+        m2 = cm2;
+      }
+      // nothing finite so far: every term is 2^-inf (or NaN) against any finite stand-in
+      const float ref = m2 == -INFINITY ? 0.f : m2;
+      float part[CH];
+#pragma unroll
+      for (int u = 0; u < CH; ++u) {
+        float e[VN];
+#pragma unroll
+        for (int k = 0; k < VN; ++k)
+          e[k] = __builtin_amdgcn_exp2f(__builtin_fmaf(xs[u][k], kLog2e, -ref));
+#pragma unroll
+        for (int w = VN / 2; w > 0; w /= 2)
+#pragma unroll
+          for (int k = 0; k < w; ++k) e[k] += e[k + w];
+        part[u] = e[0];
+      }
+#pragma unroll
+      for (int w = CH / 2; w > 0; w /= 2)
+#pragma unroll
+        for (int u = 0; u < w; ++u) part[u] += part[u + w];
+      s += part[0];
+      __builtin_amdgcn_sched_barrier(0);  // 8 elements widened at a time: 16 do not fit 64 registers at bf16
+    }
+  };
+
+  const T x_t = x[off + tgt];
+  W even[U], odd[U];
+  load(even, 0);
+  if (steps > 1) load(odd, 1);
+  for (int q = 0; q < steps; q += 2) {
+    step(even, q);
+    if (q + 2 < steps) load(even, q + 2);
+    if (q + 1 < steps) {
+      step(odd, q + 1);
+      if (q + 3 < steps) load(odd, q + 3);
+    }
+  }
+  if (tid < (int)V - iV) {
+    const float v = to_acc(x[off + iV + tid]), v2 = v * kLog2e;
+    if (v2 > m2) {
+      s *= __builtin_amdgcn_exp2f(m2 - v2);
+      m2 = v2;
+    }
+    s += __builtin_amdgcn_exp2f(__builtin_fmaf(v, kLog2e, m2 == -INFINITY ? 0.f : -m2));
+  }
+  // (max, sum) across the wave, then across the waves.  A lane without a finite value brings its
+  // sum as it is: 0, or the NaN it met.
+  const float mw2 = wave_reduce(m2, MaxOp{});
+  const float sw = wave_reduce(m2 == -INFINITY ? s : s * __builtin_amdgcn_exp2f(m2 - mw2), SumOp{});
+  if (lane == 0) {
+    red_m[tid >> 6] = mw2;
+    red_s[tid >> 6] = sw;
+  }
+  lds_barrier();
+  if (tid < kWave) {
+    const float pm = lane < kWaves ? red_m[lane] : -INFINITY;
+    const float ps = lane < kWaves ? red_s[lane] : 0.f;
+    const float M2 = wave_reduce(pm, MaxOp{});
+    const float S = wave_reduce(pm == -INFINITY ? ps : ps * __builtin_amdgcn_exp2f(pm - M2), SumOp{});
+    if (tid == 0) {
+      const float l = (__builtin_amdgcn_logf(S) - __builtin_fmaf(to_acc(x_t), kLog2e, -M2)) * kLn2;
+      row_loss[row] = class_weight ? l * class_weight[tgt] : l;
+    }
+  }
+}
+
 // Rows too wide for registers, rows too wide for the streaming kernel where only the loss is wanted, and
 // narrow rows whose stride is not a multiple of the vector width (a
 // vocabulary used unpadded).  Persistent workgroups walk rows.  A row is split into a head of
@@ -1162,6 +1308,20 @@ int launch_rows(const void *logits, void *dlogits, const int64_t *targets, float
     // rows 29.6 / 35.4 (fp32 rows, where the alternative holds a row without streaming, gain there as well: [260,40000]
     // 27.7 / 31.3).
     const int64_t cus = compute_units();
+    // The loss alone, of more than four rows per CU: a workgroup per row.  Of fewer rows each has too few loads
+    // under way, and what it saves is within the launches' time: [1024,50257] bf16 25.5 us against 27.3, but
+    // fp32 38.5 against 34.9 and [1024,128256] bf16 48.8 against 44.4; at 2048 rows 38.4 against 46.5 and 84.1
+    // against 97.8.  Rows of more than 8192 vectors: 512 lanes ([8192,128256] bf16 315 us; 318 with 256).
+    if (dlogits == nullptr && base_ok && nvec_all > 256 * 8 && N > 4 * cus && row_stride < (int64_t(1) << 29)) {
+      if (nvec_all <= 1024 * 8) {
+        ce_loss_rows_kernel<T, 256><<<grid, dim3(256), 0, s>>>((const T *)logits, targets, row_loss, N, V, row_stride,
+                                                               ignore_index, class_weight);
+      } else {
+        ce_loss_rows_kernel<T, 512><<<grid, dim3(512), 0, s>>>((const T *)logits, targets, row_loss, N, V,
+                                                                 row_stride, ignore_index, class_weight);
+      }
+      return launch_status();
+    }
     const bool holds = dlogits != nullptr && nvec_all > 256 * 8 && (sizeof(T) == 4 || N <= cus || 4 * N > 5 * cus);
     if (vec_ok && (class_weight == nullptr || streams)) {
       const int64_t nvec = row_stride / VN;

@@ -913,7 +913,7 @@ __global__ __launch_bounds__(BLOCK, 6) void ce_loss_rows_kernel(
 #pragma unroll
         for (int u = 0; u < w; ++u) part[u] += part[u + w];
       s += part[0];
-      __builtin_amdgcn_sched_barrier(0);  // 8 elements widened at a time: 16 do not fit 64 registers at bf16
+      __builtin_amdgcn_sched_barrier(0);  // 8 elements widened at a time
     }
   };
 

@@ -848,16 +848,25 @@ __device__ __forceinline__ void load_share(Share<T, VN, VPT, UA> &s, const T *ro
   if constexpr (UA) s.e = row[l.ecol];
 }
 
-// Sums of A over the lanes of a group; `red` holds one A per wave of the workgroup.  Every wave of
-// the workgroup must call it.  The caller alternates between two arrays, so one barrier is enough.
-template <typename A>
-__device__ __forceinline__ A group_sum(A v, int gw, int wave, int first_wave, int lane, A *red) {
-  v = wave_reduce(v, SumOp{});
-  if (gw == 1) return v;  // workgroup-uniform
-  if (lane == 0) red[wave] = v;
+// Sum over a group's row; v[j] belongs to the lane's vector j.  The 64 vectors that one wave holds under one j
+// are added first, then these slices in the order of their columns, whatever the number of waves they are
+// spread over: a plan with two vectors per lane gives the bits of one with a single vector.  `red` holds a
+// float per wave of the workgroup and vector of a lane.  Every wave of the workgroup must call it.  The caller
+// alternates between two arrays, so one barrier is enough.
+template <int VPT>
+__device__ __forceinline__ float row_sum(const float (&v)[VPT], int gw, int wave, int group, int lane, float *red) {
+  float slice[VPT];
+#pragma unroll
+  for (int j = 0; j < VPT; ++j) slice[j] = wave_reduce(v[j], SumOp{});
+  if (VPT == 1 && gw == 1) return slice[0];  // workgroup-uniform
+  float *mine = red + group * gw * VPT;
+  if (lane == 0) {
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) mine[wave - group * gw + gw * j] = slice[j];
+  }
   lds_barrier();
-  const A r = red[first_wave + (lane < gw ? lane : 0)];
-  return wave_reduce(lane < gw ? r : (A)0, SumOp{});
+  const float r = mine[lane < gw * VPT ? lane : 0];
+  return wave_reduce(lane < gw * VPT ? r : 0.f, SumOp{});
 }
 
 constexpr int kLnBlockMaxWaves = 16;
@@ -868,7 +877,8 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
     TY *__restrict__ y, float *__restrict__ mean, float *__restrict__ rstd, int64_t rows, int C, float eps,
     const TX *res, TX *sum_out, int gw, int groups) {
   constexpr int VN = Vec16<TX>::n;
-  __shared__ float red[2][kLnBlockMaxWaves];
+  static_assert(kLnBlockMaxWaves * VPT <= kWave, "a lane per slice");
+  __shared__ float red[2][kLnBlockMaxWaves * VPT];
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
   const int group = wave / gw, lig = threadIdx.x - group * gw * kWave;
   const bool any_vec = C >= VN;
@@ -939,17 +949,16 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
         if (own.ehas && row_ok) sum_out[at + own.ecol] = cur.e;
       }
     }
-    float s = 0.f;
+    float s[VPT], q[VPT];
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
       float t = 0.f;
 #pragma unroll
       for (int k = 0; k < VN; ++k) t += raw_get<TX, VN>(cur.v[j], k);
-      s += own.has[j] ? t : 0.f;
+      s[j] = own.has[j] ? t : 0.f;
     }
-    if constexpr (UA) s += own.ehas ? to_acc(cur.e) : 0.f;
-    const float mu = group_sum(s, gw, wave, group * gw, lane, red[0]) * inv_c;
-    float q = 0.f;
+    if constexpr (UA) s[0] += own.ehas ? to_acc(cur.e) : 0.f;
+    const float mu = row_sum(s, gw, wave, group, lane, red[0]) * inv_c;
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
       float t = 0.f;
@@ -958,13 +967,13 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
         const float d = raw_get<TX, VN>(cur.v[j], k) - mu;
         t += d * d;
       }
-      q += own.has[j] ? t : 0.f;
+      q[j] = own.has[j] ? t : 0.f;
     }
     if constexpr (UA) {
       const float d = to_acc(cur.e) - mu;
-      q += own.ehas ? d * d : 0.f;
+      q[0] += own.ehas ? d * d : 0.f;
     }
-    const float rs = 1.0f / sqrtf(group_sum(q, gw, wave, group * gw, lane, red[1]) * inv_c + eps);
+    const float rs = 1.0f / sqrtf(row_sum(q, gw, wave, group, lane, red[1]) * inv_c + eps);
     if (row_ok) {
       if (lig == 0) {
         mean[row] = mu;

@@ -376,14 +376,9 @@ def test_layernorm_with_residual_stream(ops, co, rows, C, x_dtype, p_dtype):
     total_ref = (x.to(wide) + res.to(wide)).to(x_dtype)   # one add, one rounding
     assert_bit_exact(total, total_ref, "x + residual")
     y_sep, mean_sep, rstd_sep = ops.layernorm_forward(dev(total_ref), gg, gb, 1e-5)
-    # rows of 5 to 8 vectors per lane run the register-resident kernel only without a residual,
-    # so there the two results come from different summation orders
-    vec_per_lane = -(-C * x.element_size() // 16 // 64)
-    same_kernel = not (4 < vec_per_lane <= 8 and C * x.element_size() % 16 == 0 and x_dtype != torch.float64)
-    same = assert_bit_exact if same_kernel else (lambda a, b, name: assert_close(a, b, atol=2e-6, name=name))
-    same(y, y_sep, "y: fused == separate kernels")
-    same(mean, mean_sep, "mean")
-    same(rstd, rstd_sep, "rstd")
+    assert_bit_exact(y, y_sep, "y: fused == separate kernels")
+    assert_bit_exact(mean, mean_sep, "mean")
+    assert_bit_exact(rstd, rstd_sep, "rstd")
     y2, mean2, rstd2 = co.layernorm_forward(total_ref, gamma, beta, 1e-5)
     assert_close(y, y2, atol=2e-6, name="y vs oracle")
     assert_close(rstd, rstd2, atol=1e-6, name="rstd vs oracle")
@@ -398,10 +393,9 @@ def test_layernorm_with_residual_stream(ops, co, rows, C, x_dtype, p_dtype):
     dx, dg, db = ops.layernorm_backward(gdy, dev(total_ref), gm, gr, gg, dresidual=gdres)
     dx_sep, dg_sep, db_sep = ops.layernorm_backward(gdy, dev(total_ref), gm, gr, gg)
     want = (dx_sep.to(wide) + gdres.to(wide)).to(x_dtype)
-    if same_kernel:
-        assert_bit_exact(dx, want, "dx: fused == separate kernels")
-        assert_bit_exact(dg, dg_sep, "dgamma")
-        assert_bit_exact(db, db_sep, "dbeta")
+    assert_bit_exact(dx, want, "dx: fused == separate kernels")
+    assert_bit_exact(dg, dg_sep, "dgamma")
+    assert_bit_exact(db, db_sep, "dbeta")
     # against the oracle: dx itself is held to one unit in the last place of dx, and that unit can
     # be several units of a smaller sum, so the bound is taken at the size of the terms
     dx2, _, _ = co.layernorm_backward(dy, total_ref, mean2, rstd2, gamma)

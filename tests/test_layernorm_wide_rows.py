@@ -64,9 +64,10 @@ def test_layernorm_rows_on_several_waves(ops, co, rows, C, x_dtype, p_dtype, wid
     assert_close(y, y2, atol=2e-6 * loose, name="y")
     assert_close(mean, mean2, atol=1e-7, name="mean")
     assert_close(rstd, rstd2, atol=1e-6 * loose, name="rstd")
-    y_sep, mean_sep, _ = ops.layernorm_forward(place(total_ref, offset), gg, gb, 1e-5)
-    assert_close(y_sep, y2, atol=2e-6 * loose, name="y without residual")
-    assert_close(mean_sep, mean2, atol=1e-7, name="mean without residual")
+    y_sep, mean_sep, rstd_sep = ops.layernorm_forward(place(total_ref, offset), gg, gb, 1e-5)
+    assert_bit_exact(y_sep, y, "y without residual")
+    assert_bit_exact(mean_sep, mean, "mean without residual")
+    assert_bit_exact(rstd_sep, rstd, "rstd without residual")
     ops.add_layernorm_forward(gx, gres, gg, gb, 1e-5, inplace=True)
     assert_bit_exact(gx, total_ref, "in-place sum")
 
@@ -94,6 +95,23 @@ def test_layernorm_rows_on_several_waves(ops, co, rows, C, x_dtype, p_dtype, wid
     want_g = (dg2.double() + gamma.double()).to(p_dtype) if p_dtype == F32 else None
     if want_g is not None:
         assert_sum_close(acc_g, want_g, sum_tolerance(dy.double() * xhat) + 1e-6, name="dgamma +=")
+
+
+@pytest.mark.parametrize("rows,C,dtype,offset", [
+    (300, 2056, BF16, 0), (300, 3072, F16, 0), (515, 4096, F16, 0), (300, 1028, F32, 0), (300, 2048, F32, 0),  # two
+    # vectors per lane without the residual, one with it
+    (300, 4099, BF16, 0), (300, 2051, F32, 0), (64, 4096, BF16, 3),  # the same at element alignment
+    (300, 5120, BF16, 0), (40, 8200, BF16, 0), (40, 16380, F32, 0), (40, 16383, BF16, 0),  # the same plan for both
+])
+def test_added_residual_gives_the_bits_of_two_calls(ops, rows, C, dtype, offset):
+    """x + residual inside the norm: y, mean and rstd are those of the norm of the rounded sum, bit for bit."""
+    x, res = place(randn((rows, C), 920, dtype=dtype), offset), place(randn((rows, C), 921, dtype=dtype), offset)
+    gamma, beta = place(randn(C, 922, std=0.02, mean=1.0), 0), place(randn(C, 923, std=0.02), 0)
+    total, y, mean, rstd = ops.add_layernorm_forward(x, res, gamma, beta, 1e-5)
+    y_sep, mean_sep, rstd_sep = ops.layernorm_forward(place(total, offset), gamma, beta, 1e-5)
+    assert_bit_exact(mean, mean_sep, "mean")
+    assert_bit_exact(rstd, rstd_sep, "rstd")
+    assert_bit_exact(y, y_sep, "y")
 
 
 def test_wide_rows_without_a_workspace(ops):

@@ -372,7 +372,7 @@ __global__ __launch_bounds__(1024) void ce_rows_stream_kernel(
   constexpr int VN = EPV;  // elements per lane per access
   constexpr int kWaves = BLOCK / kWave;
   __shared__ float red_m[2][kWaves], red_s[2][kWaves];
-  const int tid = threadIdx.x;
+  int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = tid >> 6;
   const int iV = (int)V;
@@ -417,6 +417,7 @@ __global__ __launch_bounds__(1024) void ce_rows_stream_kernel(
   }
   int parity = 0;
   while (row < N) {
+    if constexpr (RAGGED) asm volatile("" : "+v"(tid));  // a lane's column offsets, kept from row to row, would spill
     // ---- issue the next row's loads
     const int64_t nrow = row + gridDim.x;
     VecE<T, EPV> nxt[VPT];
@@ -504,11 +505,11 @@ __global__ __launch_bounds__(1024) void ce_rows_stream_kernel(
           s += e[j][k];
         }
       // ---- (max, sum) across the wave, then across the 16 waves.  A lane without a finite
-      // value takes no part: its stand-in maximum must not pass for a real one (the real ones
-      // may all lie far below it), and its empty sum must not meet an overflowed 2^(0 - max)
+      // value brings its sum as it is, 0 or the NaN it met: its stand-in maximum must not pass for a
+      // real one (the real ones may all lie far below it), and its sum must not meet an overflowed 2^(0 - max)
       const bool empty = m == -INFINITY;
       const float mw2 = wave_reduce(empty ? -INFINITY : ml2, MaxOp{});
-      const float sw = wave_reduce(empty ? 0.f : s * __builtin_amdgcn_exp2f(ml2 - mw2), SumOp{});
+      const float sw = wave_reduce(empty ? s : s * __builtin_amdgcn_exp2f(ml2 - mw2), SumOp{});
       if (lane == 0) {
         red_m[parity][wave] = mw2;
         red_s[parity][wave] = sw;
@@ -517,7 +518,7 @@ __global__ __launch_bounds__(1024) void ce_rows_stream_kernel(
       const float pm = lane < kWaves ? red_m[parity][lane] : -INFINITY;
       const float ps = lane < kWaves ? red_s[parity][lane] : 0.f;
       const float M2 = wave_reduce(pm, MaxOp{});
-      const float S = wave_reduce(pm == -INFINITY ? 0.f : ps * __builtin_amdgcn_exp2f(pm - M2), SumOp{});
+      const float S = wave_reduce(pm == -INFINITY ? ps : ps * __builtin_amdgcn_exp2f(pm - M2), SumOp{});
       parity ^= 1;  // the other pair of arrays next time: one barrier per row is enough
       const float log2_S = __builtin_amdgcn_logf(S);
       // loss = ln(sum exp(x - max)) - (x_t - max), the difference to the maximum formed with one
@@ -531,7 +532,13 @@ __global__ __launch_bounds__(1024) void ce_rows_stream_kernel(
       const float log2_scale = HAS_W ? log2_scale0 + __builtin_amdgcn_logf(fabsf(wt)) : log2_scale0;
       const bool negate = scale < 0.f;
 
-      if (dlogits) {
+      if (RAGGED && dlogits && !(S > 0.f)) {
+        // no finite logit, or a NaN or +inf among them: NaN for every class, 0 in the padding.  (Rows of whole
+        // vectors give 0 for all but the target where no logit is finite, and a NaN row's padding is NaN; the
+        // branch, in any form tried, costs them 1%: [8192,50257] bf16 285 -> 288 us.)
+        for (int c = tid; c < (int)row_stride; c += BLOCK)
+          dlogits[row * row_stride + c] = from_acc<TD>(c < iV ? __builtin_nanf("") : 0.f);
+      } else if (dlogits) {
         // a lane that holds no class column has e = 0 everywhere; give it f = 0 so that
         // 0 * f cannot meet an overflowed factor
         float f = empty ? 0.f : __builtin_amdgcn_exp2f(ml2 - M2 - log2_S + log2_scale);

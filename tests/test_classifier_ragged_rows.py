@@ -67,3 +67,35 @@ def test_unpadded_rows(ops, co, N, V, stride, dtype, gdt, weighted):
     if not gdt:
         ops.fused_classifier(gx, gt, V, class_weight=gw, inplace=True)
         assert_bit_exact(gx, d, "in place")
+
+
+@pytest.mark.parametrize("V,stride,dtype,gdt", [
+    (50257, 50257, BF16, None), (50255, 50257, F16, None), (40011, 40011, BF16, F32), (32001, 32003, F32, None),
+])
+def test_rows_that_are_not_finite(ops, V, stride, dtype, gdt):
+    """An unpadded row without a finite logit, or with a NaN or +inf, is NaN in every class and 0 in the padding, as a
+    softmax in 64 bits gives it; -inf elsewhere has no share."""
+    N, inf, nan = 10, float("inf"), float("nan")
+    x = randn((N, stride), 953, std=2.0, dtype=dtype)
+    t = randint(0, V, (N,), 954)
+    x[0, :V] = -inf
+    x[1, V // 2] = nan
+    x[2, 17] = inf
+    x[3, :V] = nan
+    x[4, :V - 1], t[4] = -inf, V - 1
+    x[5, 100:], t[5] = -inf, 7
+    x[6], t[6] = -inf, -100
+    x[7, 0], x[7, 5:V] = nan, -inf
+    x[8, 1000:], x[8, 30000], t[8] = -inf, nan, 50  # the NaN's lane holds no finite value
+    kw = dict(dlogits_dtype=gdt) if gdt else {}
+    loss, row, d, _ = ops.fused_classifier(x.to("cuda:0"), t.to("cuda:0"), V, reduction="sum", **kw)
+    want = x[:, :V].double().softmax(dim=1)
+    keep = t >= 0
+    want[keep, t[keep]] -= 1.0
+    want[~keep] = 0.0
+    # one rounding of the result, and 1e-6 for the target element that cancels
+    assert_close(d[:, :V], want.to(d.dtype), atol=1e-6, name="dlogits")
+    assert (d[:, V:] == 0).all()
+    want_row = torch.nn.functional.cross_entropy(x[:, :V].double(), t, reduction="none")
+    assert_close(row, want_row.float(), atol=1e-5, name="row loss")
+    assert torch.isnan(loss)

@@ -352,7 +352,7 @@ __device__ __forceinline__ float widen(const VecE<T, EPV> &v, int k) {
 // Each element costs one hardware exp2: lane-local max first, then
 // e = 2^((x - m_lane) log2e) is kept in registers, one exchange of (max, sum)
 // pairs across the 16 waves gives the row's max and sum, and the output is
-// e * f with one per-lane factor f = 2^(m_lane*log2e - log2(sum) - max*log2e) * scale.
+// e * f with one per-lane factor f = 2^(m_lane*log2e - max*log2e) * scale / sum.
 //
 // HAS_W: per-class weights (nll_loss's `weight`): a row's gradient and loss carry w[target], and
 // the mean divides by the sum of those weights, which the count launch left next to the count.
@@ -389,7 +389,7 @@ __global__ __launch_bounds__(1024) void ce_rows_stream_kernel(
   float scale0 = dloss;
   if (reduction == CS_REDUCTION_MEAN)
     scale0 = HAS_W ? dloss / reinterpret_cast<const float *>(ws_count)[1] : dloss / (float)(*ws_count);
-  const float log2_scale0 = __builtin_amdgcn_logf(fabsf(scale0));  // -inf for 0: every output 0
+  [[maybe_unused]] const float log2_scale0 = __builtin_amdgcn_logf(fabsf(scale0));  // -inf for 0: every output 0
 
   // Workgroups go round the eight XCDs in launch order.  The workgroups of one XCD take
   // neighbouring rows of each round of gridDim rows (XCD 0 the first eighth, and so on) rather
@@ -529,8 +529,6 @@ __global__ __launch_bounds__(1024) void ce_rows_stream_kernel(
       }
       // the row's scale: the call's, times the weight of the row's class
       const float scale = HAS_W ? scale0 * wt : scale0;
-      const float log2_scale = HAS_W ? log2_scale0 + __builtin_amdgcn_logf(fabsf(wt)) : log2_scale0;
-      const bool negate = scale < 0.f;
 
       if (RAGGED && dlogits && !(S > 0.f)) {
         // no finite logit, or a NaN or +inf among them: NaN for every class, 0 in the padding.  (Rows of whole
@@ -539,10 +537,19 @@ __global__ __launch_bounds__(1024) void ce_rows_stream_kernel(
         for (int c = tid; c < (int)row_stride; c += BLOCK)
           dlogits[row * row_stride + c] = from_acc<TD>(c < iV ? __builtin_nanf("") : 0.f);
       } else if (dlogits) {
-        // a lane that holds no class column has e = 0 everywhere; give it f = 0 so that
-        // 0 * f cannot meet an overflowed factor
-        float f = empty ? 0.f : __builtin_amdgcn_exp2f(ml2 - M2 - log2_S + log2_scale);
-        f = negate ? -f : f;
+        // e was taken relative to the lane's maximum.  A lane that holds no class column has e = 0 everywhere;
+        // give it f = 0 so that 0 * f cannot meet an overflowed factor
+        float f;
+        if constexpr (RAGGED) {
+          f = empty ? 0.f : __builtin_amdgcn_exp2f(ml2 - M2) * (scale / S);
+        } else {
+          // The logarithms of sum and scale folded into the exponent: one instruction a row, at 4.8e-7 rms
+          // of every element against 2.4e-7.  Rows of whole vectors have always been formed so, and have
+          // no registers for more (the product spills 4 a lane at 7 vectors of bf16).
+          const float log2_scale = HAS_W ? log2_scale0 + __builtin_amdgcn_logf(fabsf(wt)) : log2_scale0;
+          f = empty ? 0.f : __builtin_amdgcn_exp2f(ml2 - M2 - log2_S + log2_scale);
+          f = scale < 0.f ? -f : f;
+        }
         const int t_at = (int)tgt + off;
         const int t_vec = t_at / VN, t_sub = t_at % VN;
         TD *d = dlogits + row * row_stride - off;
@@ -554,10 +561,9 @@ __global__ __launch_bounds__(1024) void ce_rows_stream_kernel(
 #pragma unroll
             for (int k = 0; k < VN; ++k) o[k] = e[j][k] * f;
             if (idx == t_vec) {
-              // the exponent-folded factor f is good to ~1e-6 relative (its logarithms are),
-              // which subtracting `scale` amplifies when p is close to 1: the target element
-              // is formed as a product instead
-              const float exact = __builtin_amdgcn_exp2f(ml2 - M2) * (scale * __builtin_amdgcn_rcpf(S));
+              // the folded factor's error would be amplified by subtracting `scale` when p is close to 1: the
+              // target element is formed as a product
+              const float exact = RAGGED ? f : __builtin_amdgcn_exp2f(ml2 - M2) * (scale * __builtin_amdgcn_rcpf(S));
 #pragma unroll
               for (int k = 0; k < VN; ++k)
                 if (k == t_sub) o[k] = e[j][k] * exact - scale;

@@ -502,8 +502,35 @@ __global__ __launch_bounds__(1024) void ce_rows_stream_kernel(
 #pragma unroll
         for (int k = 0; k < VN; ++k) {
           e[j][k] = __builtin_amdgcn_exp2f(e[j][k] * kLog2e - ml2);
-          s += e[j][k];
+          if constexpr (!RAGGED) s += e[j][k];
         }
+      // Once a dominant term sits in s, every further add rounds at its size: unpadded rows, which the two-sweep
+      // kernel took before, are added pairwise within 16 elements and once onto the running sum, as there
+      // (1.3e-7 rms in the loss of confident rows; 2.5e-7 one element after the other)
+      if constexpr (RAGGED) {
+        constexpr int CH = 16 / VN;
+        float part[CH];
+#pragma unroll
+        for (int j = 0; j < VPT; ++j) {
+          float c[VN];
+#pragma unroll
+          for (int k = 0; k < VN; ++k) c[k] = e[j][k];
+#pragma unroll
+          for (int w = VN / 2; w > 0; w /= 2)
+#pragma unroll
+            for (int k = 0; k < w; ++k) c[k] += c[k + w];
+          part[j % CH] = c[0];
+          if (j % CH == CH - 1 || j == VPT - 1) {
+#pragma unroll
+            for (int u = j % CH + 1; u < CH; ++u) part[u] = 0.f;
+#pragma unroll
+            for (int w = CH / 2; w > 0; w /= 2)
+#pragma unroll
+              for (int u = 0; u < w; ++u) part[u] += part[u + w];
+            s += part[0];
+          }
+        }
+      }
       // ---- (max, sum) across the wave, then across the 16 waves.  A lane without a finite
       // value brings its sum as it is, 0 or the NaN it met: its stand-in maximum must not pass for a
       // real one (the real ones may all lie far below it), and its sum must not meet an overflowed 2^(0 - max)

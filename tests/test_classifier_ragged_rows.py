@@ -120,3 +120,23 @@ def test_every_gradient_element_keeps_its_digits(ops, V, stride, dtype):
     rel = (d - want) / want
     rel[torch.arange(N), t] = 0.0
     assert rel.square().mean().sqrt().item() < 2.8e-7
+
+
+@pytest.mark.parametrize("N,V,dtype,grad", [
+    (2000, 50257, BF16, "same"), (2000, 50257, F16, "fp32"), (2000, 32001, F32, "same"), (2000, 20001, BF16, "same"),
+    (1000, 50257, BF16, None), (1000, 57001, F16, None), (1000, 30001, F32, None),
+])
+def test_loss_of_confident_rows(ops, N, V, dtype, grad):
+    """Rows whose target holds nearly all of the sum: their loss, near 0, is the sum's distance from 1.
+
+    Every add onto a term of 1 rounds by 3.4e-8 rms (half a unit of 2^-23, uniform); a lane adds its columns in
+    groups of 16, at most four groups, then come ten levels of lanes and waves: 1.3e-7, here with a tenth more.
+    """
+    x = randn((N, V), 957, std=2.0, dtype=dtype).to("cuda:0")
+    t = randint(0, V, (N,), 958).to("cuda:0")
+    x[torch.arange(N, device="cuda:0"), t] = (18.0 + randn((N,), 959).abs()).to(dtype).to("cuda:0")
+    kw = dict(dlogits_dtype=F32) if grad == "fp32" else {}
+    row = ops.fused_classifier(x, t, V, want_dlogits=grad is not None, **kw)[1].double()
+    want = torch.cat([torch.nn.functional.cross_entropy(x[i:i + 100].double(), t[i:i + 100], reduction="none")
+                      for i in range(0, N, 100)])
+    assert (row - want).square().mean().sqrt().item() < 1.45e-7

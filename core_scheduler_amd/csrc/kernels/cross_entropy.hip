@@ -855,14 +855,13 @@ __global__ __launch_bounds__(1024) void ce_rows_hold_kernel(
 
 // The loss alone (validation) of rows beyond the small register plans: one workgroup per row, the row read
 // once in chunks of four 16-byte vectors per lane, two chunks in registers (one on its way while the other
-// joins the lane's running (max, sum)).  No row is kept and no workgroup lives longer than its row, so six
+// joins the lane's running (max, sum)).  No row is kept and no workgroup lives longer than its row, so eight
 // workgroups of 256 share a CU and cover each other's waits and exchanges, where the streaming kernel
 // has one workgroup of 1024 per CU and one barrier per row between loads.  Bound by HBM reads.
 //
 // Per call, against the kernels for fewer rows: [8192,50257] bf16 152 -> 128 us (6.4 TB/s), [4096,50257] 81 -> 68,
 // [8192,17000] 92 -> 52, [8192,128256] 357 -> 312, [4096,50257] fp16 89 -> 69, fp32 [4096,10000] 42 -> 28,
-// [4096,50257] 141 -> 123, [4096,100000] 271 -> 240.  Six waves per SIMD: in the registers of eight
-// the 16-bit chunks spill 48 to 64 bytes a lane.
+// [4096,50257] 141 -> 123, [4096,100000] 271 -> 240.
 //
 // Rows may start anywhere: vectors count from the 128-byte line a row starts in, as in the streaming
 // kernel, and what is no class column counts as -inf.  Lanes past the row's end load its last vector again.
@@ -905,7 +904,9 @@ __global__ __launch_bounds__(BLOCK, 6) void ce_loss_rows_kernel(
       c[u] = __builtin_nontemporal_load(reinterpret_cast<const W *>(reinterpret_cast<const char *>(x) + bytes));
     }
   };
-  float m2 = -INFINITY, s = 0.f;  // maximum times log2 e, and the sum relative to it
+  // Maximum times log2 e, the sum relative to it, the sum of the two chunks at hand, and what rounding took from
+  // the sum: once a dominant term sits in it, every further add rounds at its size
+  float m2 = -INFINITY, s = 0.f, pair = 0.f, lost = 0.f;
   auto step = [&](W (&c)[U], int q) {
     int t = tid * VN - off;
     asm volatile("" : "+v"(t));
@@ -930,7 +931,10 @@ __global__ __launch_bounds__(BLOCK, 6) void ce_loss_rows_kernel(
       }
       const float cm2 = cm * kLog2e;
       if (cm2 > m2) {
-        s *= __builtin_amdgcn_exp2f(m2 - cm2);  // 0 the first time (m2 = -inf, s = 0)
+        const float f = __builtin_amdgcn_exp2f(m2 - cm2);  // 0 the first time (m2 = -inf, s = 0)
+        s *= f;
+        pair *= f;
+        lost *= f;
         m2 = cm2;
       }
       // nothing finite so far: every term is 2^-inf (or NaN) against any finite stand-in
@@ -952,7 +956,7 @@ __global__ __launch_bounds__(BLOCK, 6) void ce_loss_rows_kernel(
       for (int w = CH / 2; w > 0; w /= 2)
 #pragma unroll
         for (int u = 0; u < w; ++u) part[u] += part[u + w];
-      s += part[0];
+      pair += part[0];
       __builtin_amdgcn_sched_barrier(0);  // 8 elements widened at a time
     }
   };
@@ -968,7 +972,12 @@ __global__ __launch_bounds__(BLOCK, 6) void ce_loss_rows_kernel(
       step(odd, q + 1);
       if (q + 3 < steps) load(odd, q + 3);
     }
+    const float sum = s + pair, added = sum - s;
+    lost += (s - (sum - added)) + (pair - added);
+    s = sum;
+    pair = 0.f;
   }
+  s += lost;
   if (tid < (int)V - iV) {
     const float v = to_acc(x[off + iV + tid]), v2 = v * kLog2e;
     if (v2 > m2) {

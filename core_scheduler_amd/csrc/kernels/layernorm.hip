@@ -367,20 +367,21 @@ __global__ __launch_bounds__(kLnThreads) void ln_fwd_rows_kernel(
 // rows (written by a launch that is complete when this one starts).  The first `blocks`
 // workgroups of the grid do that and leave; the row work starts at workgroup `blocks`.
 struct LnPending {
-  const float *partial;  // nullptr: nothing pending
+  const void *partial;   // nullptr: nothing pending
   void *dgamma, *dbeta;  // of the earlier call; either may be nullptr
   int nparts, accumulate, blocks;
 };
 
-// Adds `nparts` partial rows in a fixed order.  Partial rows are permuted: position
-// p = k*nvec + idx holds column idx*vn + k (nvec = C/vn).  One tile = 32 positions of dgamma or
+// Adds `nparts` partial rows of P in a fixed order.  Partial rows are permuted: position
+// p = k*nvec + idx holds column idx*vn + k (nvec = C/vn); columns past the last whole vector stay in
+// place.  One tile = 32 positions of dgamma or
 // dbeta: thread (cx, ry) of 32 x 16 sums partial rows ry, ry+16, ... for one position, sixteen
 // loads in flight and none of them under a condition (this work waits for a row kernel and is all
 // latency), then row 0 adds the 16 sub-sums in order.  `sub` is 16 x 32 floats of LDS.
 constexpr int kLnFinCols = 32, kLnFinRows = 16, kLnFinInFlight = 16;
 
-template <typename TP, int THREADS = kLnFinCols * kLnFinRows, typename A = float>
-__device__ __forceinline__ void ln_finalize_tile(const float *__restrict__ partial, int nparts, TP *__restrict__ out,
+template <typename TP, int THREADS = kLnFinCols * kLnFinRows, typename A = float, typename P = float>
+__device__ __forceinline__ void ln_finalize_tile(const P *__restrict__ partial, int nparts, TP *__restrict__ out,
                                                  int which, int tile, int C, int vn, int accumulate, A *sub,
                                                  int tid) {
   static_assert(THREADS >= kLnFinCols * kLnFinRows, "a tile takes 512 threads; further ones only join the barrier");
@@ -388,17 +389,17 @@ __device__ __forceinline__ void ln_finalize_tile(const float *__restrict__ parti
   const int col = tile * kLnFinCols + cx;  // a position in the permuted row
   A s = 0;
   if (col < C && ry < kLnFinRows) {
-    const float *src = partial + (int64_t)which * C + col;
+    const P *src = partial + (int64_t)which * C + col;
     const int64_t stride = 2 * (int64_t)C;
     for (int p0 = ry; p0 < nparts; p0 += kLnFinRows * kLnFinInFlight) {
-      float v[kLnFinInFlight];
+      P v[kLnFinInFlight];
 #pragma unroll
       for (int u = 0; u < kLnFinInFlight; ++u) {
         const int p = p0 + u * kLnFinRows;
         v[u] = src[(int64_t)(p < nparts ? p : nparts - 1) * stride];
       }
 #pragma unroll
-      for (int u = 0; u < kLnFinInFlight; ++u) s += (A)(p0 + u * kLnFinRows < nparts ? v[u] : 0.f);
+      for (int u = 0; u < kLnFinInFlight; ++u) s += (A)(p0 + u * kLnFinRows < nparts ? v[u] : (P)0);
     }
   }
   if (ry < kLnFinRows) sub[ry * kLnFinCols + cx] = s;
@@ -408,18 +409,20 @@ __device__ __forceinline__ void ln_finalize_tile(const float *__restrict__ parti
 #pragma unroll
     for (int r = 0; r < kLnFinRows; ++r) t += sub[r * kLnFinCols + cx];
     const int nvec = C / vn;
-    const int real = (col % nvec) * vn + col / nvec;  // the column this position stands for
+    // the column this position stands for
+    const int real = col < nvec * vn ? (col % nvec) * vn + col / nvec : col;
     if (accumulate) t += (A)to_acc(out[real]);
     out[real] = from_acc<TP>((float)t);
   }
 }
 // workgroup b of the 2 * ceil(C/32) that cover a pending call: even b dgamma, odd b dbeta
-template <typename TP, int THREADS = kLnFinCols * kLnFinRows, typename A = float>
+template <typename TP, int THREADS = kLnFinCols * kLnFinRows, typename A = float, typename P = float>
 __device__ __forceinline__ void ln_finalize_pending(const LnPending &pend, int b, int C, int vn, A *sub, int tid) {
   const int which = b & 1;
   TP *out = (TP *)(which == 0 ? pend.dgamma : pend.dbeta);
   if (out == nullptr) return;  // block-uniform
-  ln_finalize_tile<TP, THREADS, A>(pend.partial, pend.nparts, out, which, b >> 1, C, vn, pend.accumulate, sub, tid);
+  ln_finalize_tile<TP, THREADS, A, P>((const P *)pend.partial, pend.nparts, out, which, b >> 1, C, vn, pend.accumulate,
+                                      sub, tid);
 }
 
 // ----------------------------------------------------------- fast backward
@@ -1005,8 +1008,10 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
 
 // Backward of the same rows.  The column sums of a lane's own columns stay in registers over all the
 // rows it visits, in double: they may span thousands of rows, and at full-rate fp64 the two adds per
-// element cost no time next to the row's traffic.  The groups of a workgroup meet in the LDS, one
-// fp32 partial row (columns in order) leaves per workgroup.
+// element cost no time next to the row's traffic.  The groups of a workgroup meet in the LDS, and one
+// partial row leaves per workgroup, in the column order of ln_finalize_tile, in which a wave's LDS and global
+// accesses are contiguous.  It is in double too, so that a sum is rounded once (`wide`); in fp32 only where the
+// caller may keep partial rows for a later call (see block_two_calls).
 // Whether a lane's next row fits the registers (128 at 16 waves a workgroup) next to its column sums,
 // gamma and the current row: requested a row ahead where it does.
 template <typename TDY, typename TX, typename TDX, int E, bool HAS_DP, bool HAS_DRES, bool UA>
@@ -1019,10 +1024,10 @@ template <typename TDY, typename TX, typename TDX, typename TP, int VPT, bool HA
 __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_bwd_block_kernel(
     const TDY *__restrict__ dy, const TX *__restrict__ x, const float *__restrict__ mean,
     const float *__restrict__ rstd, const TP *__restrict__ gamma, TDX *dx /* may be dres */,
-    float *__restrict__ partial, int64_t rows, int C, const TDX *dres, int gw, int groups) {
+    void *__restrict__ partial, int wide, int64_t rows, int C, const TDX *dres, int gw, int groups) {
   constexpr int VN = Vec16<TX>::n;
   constexpr bool PF = bwd_block_prefetches<TDY, TX, TDX, VPT * VN, HAS_DP, HAS_DRES, UA>();
-  extern __shared__ float lds[];  // [groups][C] for the fold
+  extern __shared__ double group_sums[];  // [groups][C] for the fold
   __shared__ float red[2][2][kLnBlockMaxWaves];
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
   const int group = wave / gw, lig = threadIdx.x - group * gw * kWave;
@@ -1172,22 +1177,48 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_bwd_block_kernel(
   }
 
   if constexpr (HAS_DP) {
-#pragma unroll
-    for (int which = 0; which < 2; ++which) {
-      float *mine = lds + (size_t)group * C;
+    const int nvec = C / VN;
+    // one group: its registers are the partial row ([4096,5120] bf16 42.4 us against 44.1 through the LDS; where
+    // four vectors a lane spill anyway, [300,16384] fp32, 71 against 60)
+    if (VPT <= 2 && groups == 1 && wide) {
+      double *out = (double *)partial + (int64_t)blockIdx.x * 2 * C;
 #pragma unroll
       for (int j = 0; j < VPT; ++j) {
         if (own.has[j]) {
 #pragma unroll
-          for (int k = 0; k < VN; ++k) mine[own.at[j] + k] = (float)(which == 0 ? acc_g[j][k] : acc_b[j][k]);
+          for (int k = 0; k < VN; ++k) {
+            out[k * nvec + lig + kWave * gw * j] = acc_g[j][k];
+            out[C + k * nvec + lig + kWave * gw * j] = acc_b[j][k];
+          }
         }
       }
-      if (UA && own.ehas) mine[own.ecol] = (float)(which == 0 ? eacc_g : eacc_b);
+      if (UA && own.ehas) {
+        out[own.ecol] = eacc_g;
+        out[C + own.ecol] = eacc_b;
+      }
+      return;
+    }
+#pragma unroll
+    for (int which = 0; which < 2; ++which) {
+      double *mine = group_sums + (size_t)group * C;
+#pragma unroll
+      for (int j = 0; j < VPT; ++j) {
+        if (own.has[j]) {
+#pragma unroll
+          for (int k = 0; k < VN; ++k) mine[k * nvec + lig + kWave * gw * j] = which == 0 ? acc_g[j][k] : acc_b[j][k];
+        }
+      }
+      if (UA && own.ehas) mine[own.ecol] = which == 0 ? eacc_g : eacc_b;
       lds_barrier();
+      const int64_t at = ((int64_t)blockIdx.x * 2 + which) * C;
       for (int c = threadIdx.x; c < C; c += blockDim.x) {
-        float t = 0.f;
-        for (int w = 0; w < groups; ++w) t += lds[(size_t)w * C + c];
-        partial[((int64_t)blockIdx.x * 2 + which) * C + c] = t;
+        double t = 0.;
+        for (int w = 0; w < groups; ++w) t += group_sums[(size_t)w * C + c];
+        if (wide) {
+          ((double *)partial)[at + c] = t;
+        } else {
+          ((float *)partial)[at + c] = (float)t;
+        }
       }
       if (which == 0) lds_barrier();
     }
@@ -1197,13 +1228,13 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_bwd_block_kernel(
 // The column sums as a launch of their own: grid 2 * ceil(C/32) workgroups of 32 x 16 threads, even
 // ones dgamma, odd ones dbeta (the same tiles, in the same order of additions, as the pending
 // form inside the row kernel's launch).
-template <typename TP, typename A>
+template <typename TP, typename A, typename P>
 __global__ __launch_bounds__(kLnFinCols *kLnFinRows) void ln_bwd_finalize_kernel(
-    const float *__restrict__ partial, int nparts, TP *__restrict__ dgamma, TP *__restrict__ dbeta,
+    const P *__restrict__ partial, int nparts, TP *__restrict__ dgamma, TP *__restrict__ dbeta,
     int C, int vn, int accumulate) {
   __shared__ A sub[kLnFinRows * kLnFinCols];
   const LnPending pend{partial, dgamma, dbeta, nparts, accumulate, (int)gridDim.x};
-  ln_finalize_pending<TP, kLnFinCols * kLnFinRows, A>(pend, blockIdx.x, C, vn, sub, threadIdx.x);
+  ln_finalize_pending<TP, kLnFinCols * kLnFinRows, A, P>(pend, blockIdx.x, C, vn, sub, threadIdx.x);
 }
 
 // ------------------------------------------------------ elementwise add
@@ -1411,7 +1442,8 @@ struct BlockPlan {
   int vpt = 0;                      // 16-byte vectors per lane; 0: not eligible
   int gw = 0, groups = 0, blocks = 0;  // waves per row, rows side by side in a workgroup, workgroups
 };
-constexpr size_t kLnBlockFoldLds = (size_t)16 * kLnBlockMaxWaves * kWave * sizeof(float);  // the widest row
+// the fold of the widest row: 16 elements per lane and a tail of fewer than 8
+constexpr size_t kLnBlockFoldLds = ((size_t)16 * kLnBlockMaxWaves * kWave + 7) * sizeof(double);
 BlockPlan block_plan(int64_t rows, int64_t C, int x_dtype, bool backward, bool residual) {
   BlockPlan p;
   if (x_dtype == CS_F64 || C <= 0) return p;
@@ -1434,7 +1466,7 @@ BlockPlan block_plan(int64_t rows, int64_t C, int x_dtype, bool backward, bool r
   int groups = (backward ? kLnBlockMaxWaves : kLnBlockMaxWaves / 2) / p.gw;
   const int64_t per_cu = ceil_div(rows, (int64_t)256);
   if (groups > per_cu) groups = (int)per_cu;
-  while (backward && groups > 1 && (size_t)groups * C * sizeof(float) > kLnBlockFoldLds) --groups;
+  while (backward && groups > 1 && (size_t)groups * C * sizeof(double) > kLnBlockFoldLds) --groups;
   p.groups = groups < 1 ? 1 : groups;
   const int cap = backward ? 256 : 512;
   const int64_t b = ceil_div(rows, (int64_t)p.groups);
@@ -1604,6 +1636,7 @@ struct BwdPlan {
   int threads = kLnBwdThreads;
   int blocks = 0;         // workgroups of row work = partial rows left behind when dgamma/dbeta are wanted
   size_t fold_lds = 0;    // LDS of the column-sum fold
+  size_t partial_elem = sizeof(float);  // bytes of a partial row's element
   bool two_calls = true;  // the partial rows may be added up by a later call (kBwdBlock: see block_two_calls)
   BlockPlan block;
 };
@@ -1631,8 +1664,9 @@ BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, bool want_d
     b.vpl = b.block.vpt;
     b.threads = b.block.gw * b.block.groups * kWave;
     b.blocks = b.block.blocks;
-    b.fold_lds = (size_t)b.block.groups * C * sizeof(float);
+    b.fold_lds = (size_t)b.block.groups * C * sizeof(double);
     b.two_calls = aligned && block_two_calls(C, x_dtype);
+    b.partial_elem = b.two_calls ? sizeof(float) : sizeof(double);
     return b;
   }
   const int vn = 16 / (int)dtype_size(x_dtype);
@@ -1657,10 +1691,19 @@ BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, bool want_d
   return b;
 }
 
-// Column order inside a partial row, as the `vn` of ln_finalize_tile: the row-per-wave kernels leave
-// column idx*vn + k at position k*(C/vn) + idx, the several-waves kernel keeps the columns in order.
-int partial_vn(int64_t C, int x_dtype) {
-  return fast_plan(C, x_dtype).vpl == 0 ? 1 : 16 / (int)dtype_size(x_dtype);
+// Column order inside a partial row, as the `vn` of ln_finalize_tile: every row kernel leaves column
+// idx*vn + k at position k*(C/vn) + idx.
+int partial_vn(int x_dtype) { return 16 / (int)dtype_size(x_dtype); }
+
+// How partial rows are stored and added up.
+enum PartialRows {
+  kFloatRows,            // fp32, added in fp32: the row-per-wave kernels
+  kFloatRowsDoubleSums,  // fp32, added in double: the several-waves kernel where the sum may be a later call
+  kDoubleRows,           // double throughout: the several-waves kernel elsewhere
+};
+// partial rows that a caller holds on to
+PartialRows kept_rows(int64_t C, int x_dtype) {
+  return fast_plan(C, x_dtype).vpl == 0 ? kFloatRowsDoubleSums : kFloatRows;
 }
 
 enum BwdPhase { kBwdWhole = 0, kBwdRowsOnly = 1 };
@@ -1674,20 +1717,24 @@ struct PendingSums {
   int accumulate = 0;
 };
 
-template <typename TP, typename A>
+template <typename TP, typename A, typename P>
 int launch_finalize_in(const void *partial, int64_t nparts, void *dgamma, void *dbeta, int64_t C, int vn,
                        int accumulate, hipStream_t s) {
-  ln_bwd_finalize_kernel<TP, A><<<dim3(2 * (unsigned)ceil_div(C, (int64_t)kLnFinCols)), dim3(kLnFinCols * kLnFinRows), 0, s>>>(
-      (const float *)partial, (int)nparts, (TP *)dgamma, (TP *)dbeta, (int)C, vn, accumulate);
+  ln_bwd_finalize_kernel<TP, A, P><<<dim3(2 * (unsigned)ceil_div(C, (int64_t)kLnFinCols)), dim3(kLnFinCols * kLnFinRows), 0, s>>>(
+      (const P *)partial, (int)nparts, (TP *)dgamma, (TP *)dbeta, (int)C, vn, accumulate);
   return launch_status();
 }
 
 template <typename TP>
-int launch_finalize(const void *partial, int64_t nparts, void *dgamma, void *dbeta, int64_t C, int vn,
+int launch_finalize(PartialRows kind, const void *partial, int64_t nparts, void *dgamma, void *dbeta, int64_t C, int vn,
                     int accumulate, hipStream_t s) {
-  // in double where the rows were summed in double
-  return vn == 1 ? launch_finalize_in<TP, double>(partial, nparts, dgamma, dbeta, C, vn, accumulate, s)
-                 : launch_finalize_in<TP, float>(partial, nparts, dgamma, dbeta, C, vn, accumulate, s);
+  switch (kind) {
+    case kFloatRows: return launch_finalize_in<TP, float, float>(partial, nparts, dgamma, dbeta, C, vn, accumulate, s);
+    case kFloatRowsDoubleSums:
+      return launch_finalize_in<TP, double, float>(partial, nparts, dgamma, dbeta, C, vn, accumulate, s);
+    case kDoubleRows: return launch_finalize_in<TP, double, double>(partial, nparts, dgamma, dbeta, C, vn, accumulate, s);
+  }
+  return CS_ERR_UNSUPPORTED;
 }
 
 // A launch may ask for more dynamic LDS than the 64 KB it gets by default once the kernel's limit
@@ -1730,13 +1777,13 @@ int launch_bwd_block(const void *dy, const void *x, const void *mean, const void
   const auto kernel = ua ? ln_bwd_block_kernel<TDY, TX, TDX, TP, VPT, HAS_DX, HAS_DP, HAS_DRES, true>
                          : ln_bwd_block_kernel<TDY, TX, TDX, TP, VPT, HAS_DX, HAS_DP, HAS_DRES, false>;
   if (!HAS_DP) lds = 0;
-  // the widest row alone takes 64 KB next to the kernel's own half kilobyte
+  // the widest row alone takes 128 KB next to the kernel's own half kilobyte
   static std::atomic<bool> lds_allowed[2][64];
   const int st = allow_lds(kernel, lds + 512, kLnBlockFoldLds + 512, lds_allowed[ua]);
   if (st != CS_OK) return st;
   kernel<<<dim3((unsigned)plan.blocks), dim3((unsigned)plan.threads), lds, s>>>(
       (const TDY *)dy, (const TX *)x, (const float *)mean, (const float *)rstd, (const TP *)gamma, (TDX *)dx,
-      (float *)workspace, rows, (int)C, (const TDX *)dres, plan.block.gw, plan.block.groups);
+      workspace, plan.partial_elem == sizeof(double), rows, (int)C, (const TDX *)dres, plan.block.gw, plan.block.groups);
   return launch_status();
 }
 
@@ -1752,8 +1799,8 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
   BwdPlan plan = bwd_plan(rows, C, x_dtype, aligned, dx != nullptr);
   if (phase == kBwdRowsOnly && (plan.kind == kBwdNone || !plan.two_calls || std::is_same_v<TX, double>))
     return aligned ? CS_ERR_UNSUPPORTED : CS_ERR_MISALIGNED;
-  const size_t need = want_dp ? (size_t)plan.blocks * 2 * C * sizeof(float) : 0;
-  const bool ws_ok = need == 0 || (workspace != nullptr && workspace_bytes >= need && aligned_to(workspace, 4));
+  const size_t need = want_dp ? (size_t)plan.blocks * 2 * C * plan.partial_elem : 0;
+  const bool ws_ok = need == 0 || (workspace != nullptr && workspace_bytes >= need && aligned_to(workspace, plan.partial_elem));
   // a caller may bring no workspace where no sum in two steps was promised: the general kernels
   if (plan.kind == kBwdBlock && !plan.two_calls && !ws_ok) plan = BwdPlan{};
   if constexpr (!std::is_same_v<TX, double>) {
@@ -1764,11 +1811,11 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
       LnPending pend{nullptr, nullptr, nullptr, 0, 0, 0};
       if (pending.partial != nullptr && (pending.dgamma != nullptr || pending.dbeta != nullptr)) {
         if (plan.kind == kBwdBlock) {
-          const int st = launch_finalize<TP>(pending.partial, pending.nparts, pending.dgamma, pending.dbeta, C,
-                                             partial_vn(C, x_dtype), pending.accumulate, s);
+          const int st = launch_finalize<TP>(kept_rows(C, x_dtype), pending.partial, pending.nparts, pending.dgamma,
+                                             pending.dbeta, C, partial_vn(x_dtype), pending.accumulate, s);
           if (st != CS_OK) return st;
         } else {
-          pend = LnPending{(const float *)pending.partial, pending.dgamma, pending.dbeta, (int)pending.nparts,
+          pend = LnPending{pending.partial, pending.dgamma, pending.dbeta, (int)pending.nparts,
                            pending.accumulate, 2 * (int)ceil_div(C, (int64_t)kLnFinCols)};
         }
       }
@@ -1865,8 +1912,8 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
 #undef CS_LN_BWD
       if (st == CS_OK) st = launch_status();
       if (st == CS_OK && want_dp && phase == kBwdWhole)
-        st = launch_finalize<TP>(workspace, blocks, dgamma, dbeta, C, plan.kind == kBwdBlock ? 1 : partial_vn(C, x_dtype),
-                                 accumulate, s);
+        st = launch_finalize<TP>(plan.kind != kBwdBlock ? kFloatRows : plan.two_calls ? kFloatRowsDoubleSums : kDoubleRows,
+                                 workspace, blocks, dgamma, dbeta, C, partial_vn(x_dtype), accumulate, s);
       return st;
     }
   }
@@ -1960,14 +2007,14 @@ extern "C" int cs_add_layernorm_forward(const void *x, const void *residual, voi
 extern "C" size_t cs_layernorm_backward_workspace_bytes(int64_t rows, int64_t C) {
   if (rows <= 0 || C <= 0) return 0;
   // the most partial rows any plan leaves for this many rows, whatever the storage type
-  int most = 0;
+  size_t most = 0;
   for (int dt : {CS_F32, CS_F16}) {
     for (bool aligned : {true, false}) {
       const BwdPlan b = bwd_plan(rows, C, dt, aligned);
-      if (b.blocks > most) most = b.blocks;
+      if (b.blocks * b.partial_elem > most) most = b.blocks * b.partial_elem;
     }
   }
-  return (size_t)most * 2 * (size_t)C * sizeof(float);
+  return most * 2 * (size_t)C;
 }
 
 namespace {
@@ -2079,16 +2126,17 @@ extern "C" int cs_layernorm_backward_finalize(const void *partials, int64_t part
       !wide_ok(x_dtype, param_dtype))
     return CS_ERR_UNSUPPORTED;
   if (C % (16 / (int)dtype_size(x_dtype)) != 0 || partial_rows > kLnMaxPartialRows) return CS_ERR_INVALID_ARGUMENT;
-  const int vn = partial_vn(C, x_dtype);
+  const int vn = partial_vn(x_dtype);
+  const PartialRows kind = kept_rows(C, x_dtype);
   if (!dgamma && !dbeta) return CS_OK;
   if (!is_aligned16(partials) || (dgamma && !aligned_to(dgamma, dtype_size(param_dtype))) ||
       (dbeta && !aligned_to(dbeta, dtype_size(param_dtype))))
     return CS_ERR_MISALIGNED;
   hipStream_t s = as_stream(stream);
   switch (param_dtype) {
-    case CS_F32: return launch_finalize<float>(partials, partial_rows, dgamma, dbeta, C, vn, accumulate, s);
-    case CS_F16: return launch_finalize<f16_t>(partials, partial_rows, dgamma, dbeta, C, vn, accumulate, s);
-    case CS_BF16: return launch_finalize<bf16_t>(partials, partial_rows, dgamma, dbeta, C, vn, accumulate, s);
+    case CS_F32: return launch_finalize<float>(kind, partials, partial_rows, dgamma, dbeta, C, vn, accumulate, s);
+    case CS_F16: return launch_finalize<f16_t>(kind, partials, partial_rows, dgamma, dbeta, C, vn, accumulate, s);
+    case CS_BF16: return launch_finalize<bf16_t>(kind, partials, partial_rows, dgamma, dbeta, C, vn, accumulate, s);
   }
   return CS_ERR_UNSUPPORTED;
 }

@@ -114,6 +114,26 @@ def test_added_residual_gives_the_bits_of_two_calls(ops, rows, C, dtype, offset)
     assert_bit_exact(y, y_sep, "y")
 
 
+@pytest.mark.parametrize("rows,C,dtype,offset", [
+    (4096, 1003, F32, 0), (515, 4099, F32, 0), (5000, 71, F16, 0), (3000, 4, F32, 1), (2000, 5, BF16, 0),  # ragged
+    (600, 768, BF16, 1), (1000, 2056, BF16, 1),   # unaligned
+    (3000, 4104, BF16, 0), (300, 8200, BF16, 0), (100, 16380, F32, 0), (40, 16391, F32, 0),  # wide, and the widest
+])
+def test_column_sums_are_rounded_once(ops, rows, C, dtype, offset):
+    """dgamma and dbeta are the double sums of the fp32 terms, rounded once: half a unit in the last place, and
+    2^-53 of the terms for every add in double."""
+    x, dy = randn((rows, C), 930, mean=1.0, dtype=dtype), randn((rows, C), 931, dtype=dtype)
+    gamma = randn(C, 932, std=0.02, mean=1.0)
+    mean, rstd = randn(rows, 933, mean=1.0, std=0.1), randn(rows, 934).abs() + 0.5
+    _, dg, db = ops.layernorm_backward(place(dy, offset), place(x, offset), place(mean, 0), place(rstd, 0), place(gamma, 0))
+    terms = (dy.float() * ((x.float() - mean[:, None]) * rstd[:, None])).double()
+    for got, t, name in ((dg, terms, "dgamma"), (db, dy.double(), "dbeta")):
+        want = t.sum(0)
+        bound = 2.0 ** -24 * want.abs() + 2.0 ** -53 * rows * t.abs().sum(0)
+        err = (got.cpu().double() - want).abs()
+        assert (err <= bound).all(), f"{name}: {(err > bound).sum().item()} of {C} sums off"
+
+
 def test_wide_rows_without_a_workspace(ops):
     """A caller that brings no workspace for a ragged width still gets its gradients."""
     from core_scheduler_amd import _capi

@@ -872,6 +872,15 @@ __device__ __forceinline__ float row_sum(const float (&v)[VPT], int gw, int wave
   return wave_reduce(lane < gw * VPT ? r : 0.f, SumOp{});
 }
 
+// s / c as the general kernel divides: the product with 1/c alone would bring its rounding into the mean (rows of
+// one value 316 times, at rstd = 1/sqrt(eps)).  The remainder of the product corrects it (Markstein); a sum that is
+// not finite has none.
+__device__ __forceinline__ float over_columns(float s, float c, float inv_c) {
+  const float q = s * inv_c;
+  const float corrected = __builtin_fmaf(__builtin_fmaf(-q, c, s), inv_c, q);
+  return fabsf(s) < INFINITY ? corrected : q;
+}
+
 constexpr int kLnBlockMaxWaves = 16;
 
 template <typename TX, typename TY, typename TP, int VPT, bool HAS_RES, bool UA>
@@ -886,7 +895,7 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
   const int group = wave / gw, lig = threadIdx.x - group * gw * kWave;
   const bool any_vec = C >= VN;
   const Lanes<VN, VPT, UA> own(C, gw, lig);
-  const float inv_c = 1.0f / (float)C;
+  const float fc = (float)C, inv_c = 1.0f / fc;
   const int64_t stride = (int64_t)gridDim.x * groups;
   const int64_t steps = (rows + stride - 1) / stride;  // the same for every group: they share barriers
   int64_t row = (int64_t)blockIdx.x * groups + group;
@@ -961,7 +970,7 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
       s[j] = own.has[j] ? t : 0.f;
     }
     if constexpr (UA) s[0] += own.ehas ? to_acc(cur.e) : 0.f;
-    const float mu = row_sum(s, gw, wave, group, lane, red[0]) * inv_c;
+    const float mu = over_columns(row_sum(s, gw, wave, group, lane, red[0]), fc, inv_c);
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
       float t = 0.f;
@@ -976,7 +985,7 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
       const float d = to_acc(cur.e) - mu;
       q[0] += own.ehas ? d * d : 0.f;
     }
-    const float rs = 1.0f / sqrtf(row_sum(q, gw, wave, group, lane, red[1]) * inv_c + eps);
+    const float rs = 1.0f / sqrtf(over_columns(row_sum(q, gw, wave, group, lane, red[1]), fc, inv_c) + eps);
     if (row_ok) {
       if (lig == 0) {
         mean[row] = mu;

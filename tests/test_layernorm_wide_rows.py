@@ -114,6 +114,24 @@ def test_added_residual_gives_the_bits_of_two_calls(ops, rows, C, dtype, offset)
     assert_bit_exact(y, y_sep, "y")
 
 
+@pytest.mark.parametrize("C,dtype,offset", [(c, F32, 0) for c in (1, 3, 41, 47, 55, 61, 1003, 6145, 16380)] + [
+    (768, BF16, 1), (5120, BF16, 0), (4099, F16, 0), (12295, BF16, 0)])
+@pytest.mark.parametrize("residual", [False, True])
+def test_rows_of_one_value(ops, C, dtype, offset, residual):
+    """Sums of one small whole number are exact, so the mean is that number and y is beta."""
+    rows = 64
+    v = torch.arange(1, rows + 1, dtype=F32)
+    x = v[:, None].expand(rows, C).contiguous().to(dtype)
+    gamma, beta = place(randn(C, 940, std=0.02, mean=1.0), 0), randn(C, 941)
+    if residual:
+        zero = place(torch.zeros_like(x), offset)
+        y, mean, _ = ops.add_layernorm_forward(place(x, offset), zero, gamma, place(beta, 0), 1e-5, out_dtype=F32)[1:]
+    else:
+        y, mean, _ = ops.layernorm_forward(place(x, offset), gamma, place(beta, 0), 1e-5, out_dtype=F32)
+    assert_bit_exact(mean, v, "mean")
+    assert_bit_exact(y, beta.expand(rows, C), "y")
+
+
 @pytest.mark.parametrize("rows,C,dtype,offset", [
     (4096, 1003, F32, 0), (515, 4099, F32, 0), (5000, 71, F16, 0), (3000, 4, F32, 1), (2000, 5, BF16, 0),  # ragged
     (600, 768, BF16, 1), (1000, 2056, BF16, 1),   # unaligned

@@ -174,6 +174,15 @@ constexpr int kLnThreads = CS_LN_THREADS;  // 4 waves
 #endif
 constexpr int kLnBwdThreads = CS_LN_BWD_THREADS;
 
+// s / c as the general kernel divides: the product with 1/c alone would bring its rounding into the mean (rows of
+// one value 316 times, at rstd = 1/sqrt(eps)).  The remainder of the product corrects it (Markstein); a sum that is
+// not finite has none.
+__device__ __forceinline__ float over_columns(float s, float c, float inv_c) {
+  const float q = s * inv_c;
+  const float corrected = __builtin_fmaf(__builtin_fmaf(-q, c, s), inv_c, q);
+  return fabsf(s) < INFINITY ? corrected : q;
+}
+
 // ------------------------------------------------------------ fast forward
 // VPL: 16-byte x vectors per lane; R: rows a wave handles per step.  A wave
 // keeps gamma and beta for its columns in registers and walks rows
@@ -247,6 +256,7 @@ __global__ __launch_bounds__(kLnThreads) void ln_fwd_rows_kernel(
     float eps, const TX *res, TX *sum_out) {
   constexpr int VN = Vec16<TX>::n;
   constexpr int RPW = kWave / LPR;  // rows side by side in a wave: R * RPW rows per wave and step
+  constexpr bool BY_VECTOR = VPL > 4;  // sums formed as ln_fwd_block_kernel forms them, which takes these widths too
   const int lane = threadIdx.x & (kWave - 1);
   const int sub = lane / LPR, hl = lane % LPR;
   const bool upper = sub != 0;
@@ -310,30 +320,41 @@ __global__ __launch_bounds__(kLnThreads) void ln_fwd_rows_kernel(
     for (int r = 0; r < R; ++r) {
       float s = 0.f;
 #pragma unroll
-      for (int j = 0; j < VPL; ++j)
+      for (int j = 0; j < VPL; ++j) {
+        float t = BY_VECTOR ? 0.f : s;
 #pragma unroll
-        for (int k = 0; k < VN; ++k) s += raw_get<TX, VN>(cur.v[r][j], k);
+        for (int k = 0; k < VN; ++k) t += raw_get<TX, VN>(cur.v[r][j], k);
+        s = BY_VECTOR ? s + t : t;
+      }
       mu[r] = s;
     }
 #pragma unroll
-    for (int r = 0; r < R; ++r) mu[r] = row_lanes_sum<LPR>(mu[r], upper) * inv_c;
+    for (int r = 0; r < R; ++r) {
+      mu[r] = row_lanes_sum<LPR>(mu[r], upper);
+      mu[r] = BY_VECTOR ? over_columns(mu[r], (float)C, inv_c) : mu[r] * inv_c;
+    }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       float q = 0.f;
 #pragma unroll
       for (int j = 0; j < VPL; ++j) {
         if (hl + LPR * j < nvec) {
+          float t = BY_VECTOR ? 0.f : q;
 #pragma unroll
           for (int k = 0; k < VN; ++k) {
             const float d = raw_get<TX, VN>(cur.v[r][j], k) - mu[r];
-            q += d * d;
+            t += d * d;
           }
+          q = BY_VECTOR ? q + t : t;
         }
       }
       rs[r] = q;
     }
 #pragma unroll
-    for (int r = 0; r < R; ++r) rs[r] = 1.0f / sqrtf(row_lanes_sum<LPR>(rs[r], upper) * inv_c + eps);
+    for (int r = 0; r < R; ++r) {
+      rs[r] = row_lanes_sum<LPR>(rs[r], upper);
+      rs[r] = 1.0f / sqrtf((BY_VECTOR ? over_columns(rs[r], (float)C, inv_c) : rs[r] * inv_c) + eps);
+    }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       if (row0 + r * RPW >= rows) break;  // wave-uniform
@@ -851,37 +872,41 @@ __device__ __forceinline__ void load_share(Share<T, VN, VPT, UA> &s, const T *ro
   if constexpr (UA) s.e = row[l.ecol];
 }
 
-// Sum over a group's row; v[j] belongs to the lane's vector j.  The 64 vectors that one wave holds under one j
-// are added first, then these slices in the order of their columns, whatever the number of waves they are
-// spread over: a plan with two vectors per lane gives the bits of one with a single vector.  `red` holds a
-// float per wave of the workgroup and vector of a lane.  Every wave of the workgroup must call it.  The caller
-// alternates between two arrays, so one barrier is enough.
-template <int VPT>
-__device__ __forceinline__ float row_sum(const float (&v)[VPT], int gw, int wave, int group, int lane, float *red) {
-  float slice[VPT];
-#pragma unroll
-  for (int j = 0; j < VPT; ++j) slice[j] = wave_reduce(v[j], SumOp{});
-  if (VPT == 1 && gw == 1) return slice[0];  // workgroup-uniform
-  float *mine = red + group * gw * VPT;
-  if (lane == 0) {
-#pragma unroll
-    for (int j = 0; j < VPT; ++j) mine[wave - group * gw + gw * j] = slice[j];
-  }
-  lds_barrier();
-  const float r = mine[lane < gw * VPT ? lane : 0];
-  return wave_reduce(lane < gw * VPT ? r : 0.f, SumOp{});
-}
-
-// s / c as the general kernel divides: the product with 1/c alone would bring its rounding into the mean (rows of
-// one value 316 times, at rstd = 1/sqrt(eps)).  The remainder of the product corrects it (Markstein); a sum that is
-// not finite has none.
-__device__ __forceinline__ float over_columns(float s, float c, float inv_c) {
-  const float q = s * inv_c;
-  const float corrected = __builtin_fmaf(__builtin_fmaf(-q, c, s), inv_c, q);
-  return fabsf(s) < INFINITY ? corrected : q;
-}
-
 constexpr int kLnBlockMaxWaves = 16;
+
+// Sum over a group's row; v[j] belongs to the lane's vector j.  Rows of 257 to 512 vectors (`by_lane`) have three
+// plans, which all add in one order, so that they give the same bits: lane l's vectors l, l + 64, ... first, one after
+// the other, then the lanes.  Other widths have one plan each: a wave's lanes first, then the waves.  Every wave
+// of the workgroup must call it.  The caller alternates between two arrays, so one barrier is enough.
+// CAN: whether the plan takes such rows at all.
+template <bool CAN, int VPT>
+__device__ __forceinline__ float row_sum(const float (&v)[VPT], bool by_lane, int gw, int wave, int group, int lane,
+                                         float *red) {
+  if constexpr (CAN) {
+    if (by_lane) {  // grid-uniform
+      const int n = gw * VPT;  // at most 8
+      float *mine = red + group * n * kWave + lane;
+#pragma unroll
+      for (int j = 0; j < VPT; ++j) mine[(wave - group * gw + gw * j) * kWave] = v[j];
+      lds_barrier();
+      float part[8], t = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) part[i] = mine[(i < n ? i : 0) * kWave];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) t += i < n ? part[i] : 0.f;
+      return wave_reduce(t, SumOp{});
+    }
+  }
+  float t = v[0];
+#pragma unroll
+  for (int j = 1; j < VPT; ++j) t += v[j];
+  t = wave_reduce(t, SumOp{});
+  if (gw == 1) return t;  // workgroup-uniform
+  if (lane == 0) red[wave] = t;
+  lds_barrier();
+  const float r = red[group * gw + (lane < gw ? lane : 0)];
+  return wave_reduce(lane < gw ? r : 0.f, SumOp{});
+}
 
 template <typename TX, typename TY, typename TP, int VPT, bool HAS_RES, bool UA>
 __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
@@ -889,13 +914,14 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
     TY *__restrict__ y, float *__restrict__ mean, float *__restrict__ rstd, int64_t rows, int C, float eps,
     const TX *res, TX *sum_out, int gw, int groups) {
   constexpr int VN = Vec16<TX>::n;
-  static_assert(kLnBlockMaxWaves * VPT <= kWave, "a lane per slice");
-  __shared__ float red[2][kLnBlockMaxWaves * VPT];
+  constexpr bool CAN = VPT == 1 || (VPT == 2 && !HAS_RES);  // rows of 257 to 512 vectors, see block_plan
+  __shared__ float red[2][kLnBlockMaxWaves * (CAN ? VPT * kWave : 1)];
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
   const int group = wave / gw, lig = threadIdx.x - group * gw * kWave;
   const bool any_vec = C >= VN;
   const Lanes<VN, VPT, UA> own(C, gw, lig);
   const float fc = (float)C, inv_c = 1.0f / fc;
+  const bool by_lane = C / VN > 4 * kWave && C / VN <= 8 * kWave;
   const int64_t stride = (int64_t)gridDim.x * groups;
   const int64_t steps = (rows + stride - 1) / stride;  // the same for every group: they share barriers
   int64_t row = (int64_t)blockIdx.x * groups + group;
@@ -970,7 +996,7 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
       s[j] = own.has[j] ? t : 0.f;
     }
     if constexpr (UA) s[0] += own.ehas ? to_acc(cur.e) : 0.f;
-    const float mu = over_columns(row_sum(s, gw, wave, group, lane, red[0]), fc, inv_c);
+    const float mu = over_columns(row_sum<CAN>(s, by_lane, gw, wave, group, lane, red[0]), fc, inv_c);
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
       float t = 0.f;
@@ -985,7 +1011,7 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
       const float d = to_acc(cur.e) - mu;
       q[0] += own.ehas ? d * d : 0.f;
     }
-    const float rs = 1.0f / sqrtf(over_columns(row_sum(q, gw, wave, group, lane, red[1]), fc, inv_c) + eps);
+    const float rs = 1.0f / sqrtf(over_columns(row_sum<CAN>(q, by_lane, gw, wave, group, lane, red[1]), fc, inv_c) + eps);
     if (row_ok) {
       if (lig == 0) {
         mean[row] = mu;
@@ -1406,10 +1432,9 @@ struct FastPlan {
   int fwd_rows = 1;  // rows a wave normalises per step, forward
 };
 // x vectors per lane needed for C columns of x_dtype when a wave owns whole rows; those kernels are
-// instantiated for 1, 2 and 4 (a fifth to eighth vector per lane measured slower than several waves
-// per row: [4096,3072] bf16 with the residual 23.5 + 37.0 us forward and backward against 20.8 + 27.0,
-// [8192,2048] fp32 46.7 + 73.9 against 47.1 + 50.2, without it [4096,4096] bf16 15.9 + 28.3 against
-// 15.2 + 27.3).
+// instantiated for 1, 2 and 4.  A fifth to eighth vector per lane: the forward has both kinds of plan (see
+// wave_per_row8); in the backward several waves per row are faster ([4096,3072] bf16 with the residual 27.0 us
+// against 37.0, [8192,2048] fp32 50.2 / 73.9, without it [4096,4096] bf16 27.3 / 28.3).
 FastPlan fast_plan(int64_t C, int x_dtype) {
   FastPlan p;
   const int vn = 16 / (int)dtype_size(x_dtype);
@@ -1460,8 +1485,8 @@ BlockPlan block_plan(int64_t rows, int64_t C, int x_dtype, bool backward, bool r
   const int64_t nvec = C >= vn ? C / vn : 1;
   // One vector per lane: [4096,5120] bf16 backward 41.6 us against 58.2 with two (registers), forward
   // with the residual 31.9 against 38.1.  A forward without residual has half the loads in flight
-  // per row, and two pay where the row then still has two waves or more: [4096,4096] 15.2 against
-  // 16.5, [4096,2304] 11.2 against 13.2, but [4096,5120] 23.1 against 20.5.
+  // per row, and two pay where the row then still has two waves or more: [4096,4099] 13.9 against 15.6, but
+  // [4096,5120] 23.1 against 20.5.
   int vpt = !backward && !residual && nvec > 4 * kWave && nvec <= 8 * kWave ? 2 : 1;
   while (ceil_div(nvec, (int64_t)kWave * vpt) > kLnBlockMaxWaves) vpt *= 2;
   if (vpt * vn > 16) return p;
@@ -1481,6 +1506,21 @@ BlockPlan block_plan(int64_t rows, int64_t C, int x_dtype, bool backward, bool r
   const int64_t b = ceil_div(rows, (int64_t)p.groups);
   p.blocks = (int)(b < cap ? b : cap);
   return p;
+}
+
+// Forward of 257 to 512 whole vectors: a wave per row with eight vectors a lane, or several waves per row (the
+// same bits).  The several waves have more loads in flight where there are few rows, and where the residual
+// doubles a row's loads; in between their last step of 512 workgroups is nearly empty.  Wave per row / several
+// waves, us per call: bf16 [300,3072] 4.4 / 4.0, [600,3072] 4.6 / 5.1, [12000,2304] 24.7 / 28.4; with the residual
+// [300,3072] 5.4 / 4.7, [1024,3072] 6.4 / 7.8, [1500,3072] 10.8 / 10.5, [12000,2304] 51.5 / 44.5.  fp32, rows half as
+// long: [300,1280] 3.5 / 3.7, [3000,1280] 6.4 / 9.4; with the residual [300,1280] 4.2 / 3.9, [600,1280] 4.4 / 5.9,
+// [12000,1280] 45.5 / 46.4.
+bool wave_per_row8(int64_t rows, int64_t C, int x_dtype, bool residual) {
+  if (x_dtype == CS_F64 || C <= 0) return false;
+  const int vn = 16 / (int)dtype_size(x_dtype);
+  if (C % vn != 0 || C / vn <= 4 * kWave || C / vn > 8 * kWave) return false;
+  if (x_dtype == CS_F32) return !residual || rows > 512;
+  return rows > 512 && (!residual || rows <= 1024);
 }
 
 template <typename TX, typename TY, typename TP>
@@ -1544,6 +1584,19 @@ int fwd_typed(const void *x, const void *gamma, const void *beta, void *y, void 
     }
   }
   if constexpr (!std::is_same_v<TX, double>) {
+    if (aligned && wave_per_row8(rows, C, x_dtype, res != nullptr)) {
+      const dim3 grid((unsigned)ln_blocks(rows, 1, kLnFwdMaxBlocks)), block(kLnThreads);
+      if (res) {
+        ln_fwd_rows_kernel<TX, TY, TP, 8, 1, CS_LN_FWD_PF, true><<<grid, block, 0, s>>>(
+            (const TX *)x, (const TP *)gamma, (const TP *)beta, (TY *)y, (float *)mean, (float *)rstd, rows, (int)C,
+            (float)eps, (const TX *)res, (TX *)sum_out);
+      } else {
+        ln_fwd_rows_kernel<TX, TY, TP, 8, 1, CS_LN_FWD_PF, false><<<grid, block, 0, s>>>(
+            (const TX *)x, (const TP *)gamma, (const TP *)beta, (TY *)y, (float *)mean, (float *)rstd, rows, (int)C,
+            (float)eps, nullptr, nullptr);
+      }
+      return launch_status();
+    }
     const BlockPlan b = block_plan(rows, C, x_dtype, false, res != nullptr);
     if (b.vpt != 0) {
       const bool ua = !aligned || C % Vec16<TX>::n != 0;

@@ -98,8 +98,9 @@ def test_layernorm_rows_on_several_waves(ops, co, rows, C, x_dtype, p_dtype, wid
 
 
 @pytest.mark.parametrize("rows,C,dtype,offset", [
-    (300, 2056, BF16, 0), (300, 3072, F16, 0), (515, 4096, F16, 0), (300, 1028, F32, 0), (300, 2048, F32, 0),  # two
-    # vectors per lane without the residual, one with it
+    # 257 to 512 vectors: one or two per lane of several waves, or a wave per row, by rows and residual
+    (300, 2056, BF16, 0), (512, 4096, F16, 0), (513, 3072, BF16, 0), (1024, 2056, F16, 0), (1025, 4096, BF16, 0),
+    (300, 1028, F32, 0), (512, 2048, F32, 0), (513, 2044, F32, 0),
     (300, 4099, BF16, 0), (300, 2051, F32, 0), (64, 4096, BF16, 3),  # the same at element alignment
     (300, 5120, BF16, 0), (40, 8200, BF16, 0), (40, 16380, F32, 0), (40, 16383, BF16, 0),  # the same plan for both
 ])

@@ -98,6 +98,17 @@ def test_workspace_sizes():
     assert lib.cs_adamw_multi_table_bytes(148) >= 148 * 64 + 149 * 8
 
 
+def test_layernorm_sizes_grow_with_the_rows():
+    """A buffer sized for a long batch holds a short one's partial rows."""
+    lib = _capi.load()
+    for C in (50, 768, 1003, 1028, 2056, 2304, 3072, 4096, 4099, 5120, 8192, 16384):
+        sizes = [lib.cs_layernorm_backward_workspace_bytes(rows, C) for rows in range(1, 1600)]
+        assert sizes == sorted(sizes), C
+        for dtype in (_capi.F32, _capi.F16, _capi.BF16):
+            parts = [lib.cs_layernorm_backward_partial_rows(rows, C, dtype) for rows in range(1, 1600)]
+            assert parts == sorted(parts), (C, dtype)
+
+
 def test_multi_tensor_table_layout():
     # the table is built on the host, so its layout can be checked without a GPU
     lib = _capi.load()

@@ -874,28 +874,24 @@ __device__ __forceinline__ void load_share(Share<T, VN, VPT, UA> &s, const T *ro
 
 constexpr int kLnBlockMaxWaves = 16;
 
-// Sum over a group's row; v[j] belongs to the lane's vector j.  Rows of 257 to 512 vectors (`by_lane`) have three
+// Sum over a group's row; v[j] belongs to the lane's vector j.  Rows of 257 to 512 vectors (BY_LANE) have three
 // plans, which all add in one order, so that they give the same bits: lane l's vectors l, l + 64, ... first, one after
 // the other, then the lanes.  Other widths have one plan each: a wave's lanes first, then the waves.  Every wave
 // of the workgroup must call it.  The caller alternates between two arrays, so one barrier is enough.
-// CAN: whether the plan takes such rows at all.
-template <bool CAN, int VPT>
-__device__ __forceinline__ float row_sum(const float (&v)[VPT], bool by_lane, int gw, int wave, int group, int lane,
-                                         float *red) {
-  if constexpr (CAN) {
-    if (by_lane) {  // grid-uniform
-      const int n = gw * VPT;  // at most 8
-      float *mine = red + group * n * kWave + lane;
+template <bool BY_LANE, int VPT>
+__device__ __forceinline__ float row_sum(const float (&v)[VPT], int gw, int wave, int group, int lane, float *red) {
+  if constexpr (BY_LANE) {
+    const int n = gw * VPT;  // at most 8
+    float *mine = red + group * n * kWave + lane;
 #pragma unroll
-      for (int j = 0; j < VPT; ++j) mine[(wave - group * gw + gw * j) * kWave] = v[j];
-      lds_barrier();
-      float part[8], t = 0.f;
+    for (int j = 0; j < VPT; ++j) mine[(wave - group * gw + gw * j) * kWave] = v[j];
+    lds_barrier();
+    float part[8], t = 0.f;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) part[i] = mine[(i < n ? i : 0) * kWave];
+    for (int i = 0; i < 8; ++i) part[i] = mine[(i < n ? i : 0) * kWave];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) t += i < n ? part[i] : 0.f;
-      return wave_reduce(t, SumOp{});
-    }
+    for (int i = 0; i < 8; ++i) t += i < n ? part[i] : 0.f;
+    return wave_reduce(t, SumOp{});
   }
   float t = v[0];
 #pragma unroll
@@ -908,20 +904,18 @@ __device__ __forceinline__ float row_sum(const float (&v)[VPT], bool by_lane, in
   return wave_reduce(lane < gw ? r : 0.f, SumOp{});
 }
 
-template <typename TX, typename TY, typename TP, int VPT, bool HAS_RES, bool UA>
+template <typename TX, typename TY, typename TP, int VPT, bool HAS_RES, bool UA, bool BY_LANE>
 __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
     const TX *x /* sum_out may be x: not restrict */, const TP *__restrict__ gamma, const TP *__restrict__ beta,
     TY *__restrict__ y, float *__restrict__ mean, float *__restrict__ rstd, int64_t rows, int C, float eps,
     const TX *res, TX *sum_out, int gw, int groups) {
   constexpr int VN = Vec16<TX>::n;
-  constexpr bool CAN = VPT == 1 || (VPT == 2 && !HAS_RES);  // rows of 257 to 512 vectors, see block_plan
-  __shared__ float red[2][kLnBlockMaxWaves * (CAN ? VPT * kWave : 1)];
+  __shared__ float red[2][kLnBlockMaxWaves * (BY_LANE ? VPT * kWave : 1)];
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
   const int group = wave / gw, lig = threadIdx.x - group * gw * kWave;
   const bool any_vec = C >= VN;
   const Lanes<VN, VPT, UA> own(C, gw, lig);
   const float fc = (float)C, inv_c = 1.0f / fc;
-  const bool by_lane = C / VN > 4 * kWave && C / VN <= 8 * kWave;
   const int64_t stride = (int64_t)gridDim.x * groups;
   const int64_t steps = (rows + stride - 1) / stride;  // the same for every group: they share barriers
   int64_t row = (int64_t)blockIdx.x * groups + group;
@@ -996,7 +990,7 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
       s[j] = own.has[j] ? t : 0.f;
     }
     if constexpr (UA) s[0] += own.ehas ? to_acc(cur.e) : 0.f;
-    const float mu = over_columns(row_sum<CAN>(s, by_lane, gw, wave, group, lane, red[0]), fc, inv_c);
+    const float mu = over_columns(row_sum<BY_LANE>(s, gw, wave, group, lane, red[0]), fc, inv_c);
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
       float t = 0.f;
@@ -1011,7 +1005,7 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
       const float d = to_acc(cur.e) - mu;
       q[0] += own.ehas ? d * d : 0.f;
     }
-    const float rs = 1.0f / sqrtf(over_columns(row_sum<CAN>(q, by_lane, gw, wave, group, lane, red[1]), fc, inv_c) + eps);
+    const float rs = 1.0f / sqrtf(over_columns(row_sum<BY_LANE>(q, gw, wave, group, lane, red[1]), fc, inv_c) + eps);
     if (row_ok) {
       if (lig == 0) {
         mean[row] = mu;
@@ -1499,12 +1493,12 @@ BlockPlan block_plan(int64_t rows, int64_t C, int x_dtype, bool backward, bool r
   // workgroups).
   int groups = (backward ? kLnBlockMaxWaves : kLnBlockMaxWaves / 2) / p.gw;
   // Fewer side by side where there are not rows enough for every CU: [300,1003] bf16 backward 8.3 us against 8.5,
-  // [64,1003] 6.8 against 8.7; two side by side stay two ([300,4099] 16.2 against 17.6).  Rounded down in the backward,
-  // so that the number of partial rows grows with the rows: a buffer for a long batch holds a short one's.
+  // [64,1003] 6.8 against 8.7; up to three stay ([300,4099] 16.2 against 17.6, [300,2056] 9.9 / 11.8).  Rounded down in
+  // the backward, so that the number of partial rows grows with the rows: a buffer for a long batch holds a short one's.
   if (!backward) {
     const int64_t per_cu = ceil_div(rows, (int64_t)256);
     if (groups > per_cu) groups = (int)per_cu;
-  } else if (groups > 2 && groups > rows / 256) {
+  } else if (groups > 3 && groups > rows / 256) {
     groups = (int)(rows / 256);
   }
   if (groups < 1) groups = 1;
@@ -1609,27 +1603,37 @@ int fwd_typed(const void *x, const void *gamma, const void *beta, void *y, void 
     if (b.vpt != 0) {
       const bool ua = !aligned || C % Vec16<TX>::n != 0;
       const dim3 grid((unsigned)b.blocks), block((unsigned)(b.gw * b.groups * kWave));
-#define CS_LN_FWD_B(VPT, HAS_RES, UA)                                                                  \
-  ln_fwd_block_kernel<TX, TY, TP, VPT, HAS_RES, UA><<<grid, block, 0, s>>>(                             \
+      // rows of 257 to 512 vectors: see row_sum
+      const bool by_lane = C / Vec16<TX>::n > 4 * kWave && C / Vec16<TX>::n <= 8 * kWave;
+#define CS_LN_FWD_B(VPT, HAS_RES, UA, BY_LANE)                                                         \
+  ln_fwd_block_kernel<TX, TY, TP, VPT, HAS_RES, UA, BY_LANE><<<grid, block, 0, s>>>(                    \
       (const TX *)x, (const TP *)gamma, (const TP *)beta, (TY *)y, (float *)mean, (float *)rstd, rows, \
       (int)C, (float)eps, (const TX *)res, (TX *)sum_out, b.gw, b.groups)
-#define CS_LN_FWD_B2(VPT)                             \
+#define CS_LN_FWD_B2(VPT, BY_LANE)                    \
   if (res && ua) {                                    \
-    CS_LN_FWD_B(VPT, true, true);                     \
+    CS_LN_FWD_B(VPT, true, true, BY_LANE);            \
   } else if (res) {                                   \
-    CS_LN_FWD_B(VPT, true, false);                    \
+    CS_LN_FWD_B(VPT, true, false, BY_LANE);           \
   } else if (ua) {                                    \
-    CS_LN_FWD_B(VPT, false, true);                    \
+    CS_LN_FWD_B(VPT, false, true, BY_LANE);           \
   } else {                                            \
-    CS_LN_FWD_B(VPT, false, false);                   \
+    CS_LN_FWD_B(VPT, false, false, BY_LANE);          \
   }
-      if (b.vpt == 1) {
-        CS_LN_FWD_B2(1)
+      if (b.vpt == 1 && by_lane) {
+        CS_LN_FWD_B2(1, true)
+      } else if (b.vpt == 1) {
+        CS_LN_FWD_B2(1, false)
+      } else if (b.vpt == 2 && by_lane) {  // without the residual only
+        if (ua) {
+          CS_LN_FWD_B(2, false, true, true);
+        } else {
+          CS_LN_FWD_B(2, false, false, true);
+        }
       } else if (b.vpt == 2) {
-        CS_LN_FWD_B2(2)
+        CS_LN_FWD_B2(2, false)
       } else {
         if constexpr (Vec16<TX>::n == 4) {
-          CS_LN_FWD_B2(4)
+          CS_LN_FWD_B2(4, false)
         }
       }
 #undef CS_LN_FWD_B2
@@ -1728,6 +1732,7 @@ BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, bool want_d
   BwdPlan b;
   const FastPlan p = aligned ? fast_plan(C, x_dtype) : FastPlan{};
   if (p.vpl == 0) {
+    const bool two_calls = aligned && block_two_calls(C, x_dtype);
     b.block = block_plan(rows, C, x_dtype, true, false);
     if (b.block.vpt == 0) return b;
     b.kind = kBwdBlock;
@@ -1735,7 +1740,7 @@ BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, bool want_d
     b.threads = b.block.gw * b.block.groups * kWave;
     b.blocks = b.block.blocks;
     b.fold_lds = (size_t)b.block.groups * C * sizeof(double);
-    b.two_calls = aligned && block_two_calls(C, x_dtype);
+    b.two_calls = two_calls;
     b.partial_elem = b.two_calls ? sizeof(float) : sizeof(double);
     return b;
   }

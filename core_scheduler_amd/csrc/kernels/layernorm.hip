@@ -1732,7 +1732,11 @@ BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, bool want_d
   BwdPlan b;
   const FastPlan p = aligned ? fast_plan(C, x_dtype) : FastPlan{};
   if (p.vpl == 0) {
+    // A few rows of up to 512 vectors: the general kernels' two launches are the shorter ones ([16,257] bf16 4.6 us
+    // against 6.5, [64,65] 6.1 / 6.6, [64,1003] 7.0 / 6.9, [64,4099] 10.9 / 12.2; but [128,257] 9.1 / 7.5,
+    // [128,4099] 20.3 / 12.2).
     const bool two_calls = aligned && block_two_calls(C, x_dtype);
+    if (rows <= 64 && !two_calls && C / (16 / (int64_t)dtype_size(x_dtype)) <= 8 * kWave) return b;
     b.block = block_plan(rows, C, x_dtype, true, false);
     if (b.block.vpt == 0) return b;
     b.kind = kBwdBlock;

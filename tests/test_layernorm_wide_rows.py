@@ -40,6 +40,8 @@ def place(t, offset):
     (20, 16392, BF16, F32, False, 0),    # past it: the general kernels
     (1100, 1028, F32, F32, False, 0),    # fp32: 257 vectors
     (40, 16380, F32, F32, False, 0),     # four fp32 vectors per lane
+    (64, 4100, F16, F16, False, 0),      # as many rows as the general backward kernels take, up to 512 vectors
+    (65, 4100, BF16, F32, False, 0),     # one more
     (5000, 1, F32, F32, False, 0),       # no whole vector, one column
     (3000, 7, BF16, F32, False, 0),      # no whole vector
     (777, 71, F16, F16, False, 0),       # 8 vectors and 7 columns

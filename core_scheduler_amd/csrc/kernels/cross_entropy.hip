@@ -20,6 +20,8 @@
 //   up to 20480 with a gradient      ce_rows_hold_kernel: one persistent workgroup per CU keeps
 //                                    one row and loads the next into the registers it frees
 //   the loss alone of many rows      ce_loss_rows_kernel: one workgroup per row, nothing kept
+//   up to 16384 fp32 vectors of the  ce_rows_kernel with 1024 lanes (the loss alone, and the gradient
+//   few rows the last two leave      of a few rows more than there are CUs)
 //   wider, the loss alone, or narrow ce_rows_wide_kernel: two sweeps over the row, the
 //   rows that start off 16 bytes     second one served by the cache
 //   fp64, unaligned base pointers    ce_rows_general_kernel
@@ -1007,9 +1009,9 @@ __global__ __launch_bounds__(BLOCK, 6) void ce_loss_rows_kernel(
   }
 }
 
-// Rows too wide for registers, rows too wide for the streaming kernel where only the loss is wanted, and
-// narrow rows whose stride is not a multiple of the vector width (a
-// vocabulary used unpadded).  Persistent workgroups walk rows.  A row is split into a head of
+// Rows too wide for registers, rows too wide for the streaming kernel where only the loss is wanted or the
+// row-holding kernel would run a second round of few rows, and rows whose stride is not a multiple of the vector
+// width (a vocabulary used unpadded) where they are narrow.  Persistent workgroups walk rows.  A row is split into a head of
 // single elements up to the first 16-byte boundary, a body of whole vectors and a tail; the
 // base pointers are 16-byte aligned, so gradient rows split at the same columns.  The body is
 // read twice in chunks of kWideU vectors per lane: the first sweep keeps a running (max, sum)
@@ -1351,11 +1353,6 @@ int launch_rows(const void *logits, void *dlogits, const int64_t *targets, float
     const int64_t nvec_all = row_stride / VN;
     const bool streams = nvec_all > 256 * 8 &&
                          row_stride <= (int64_t)StreamPlan<T, TD>::kEpv * StreamPlan<T, TD>::kMostVecs;
-    // The loss alone needs no second pass: nothing to hold a row for.  A few rows more than there are
-    // CUs are a second round of whole rows for the row-holding kernel, while the two-sweep kernel runs two
-    // rows per CU: [300,128256] bf16 48.2 against 46.3 us, 257 rows 44.3 / 41.9, 384 rows 48.7 / 50.3, 256
-    // rows 29.6 / 35.4 (fp32 rows, where the alternative holds a row without streaming, gain there as well: [260,40000]
-    // 27.7 / 31.3).
     const int64_t cus = compute_units();
     // The loss alone, of more than four rows per CU: a workgroup per row.  Of fewer rows each has too few loads
     // under way, and what it saves is within the launches' time: [1024,50257] bf16 25.5 us against 27.3, but
@@ -1371,7 +1368,16 @@ int launch_rows(const void *logits, void *dlogits, const int64_t *targets, float
       }
       return launch_status();
     }
-    const bool holds = dlogits != nullptr && nvec_all > 256 * 8 && (sizeof(T) == 4 || N <= cus || 4 * N > 5 * cus);
+    // The loss alone needs no second pass: nothing to hold a row for.  A few rows more than there are
+    // CUs are a second round of whole rows for the row-holding kernel, while the others run two rows per CU or
+    // (fp32 rows of whole vectors) start the next row as soon as one ends.  Where the line lies, held row / the
+    // alternative in us: [340,57600] bf16 28.1 / 25.7, [384,57600] 28.3 / 26.4, [450,57600] 28.4 / 28.6; [340,100003]
+    // 42.3 / 43.3, [300,128256] 49.1 / 48.1, [384,128256] 48.0 / 53.5; with fp32 gradients [300,57601] 40.8 / 41.1,
+    // [384,57601] 39.7 / 42.8; fp32 [300,40000] 30.8 / 29.3, [340,40001] 32.4 / 30.8, [384,40001] 31.9 / 33.1.
+    const bool past_one_round = sizeof(T) == 4                                    ? 5 * N > 7 * cus
+                                : sizeof(TD) == sizeof(T) && row_stride < 80000 ? 2 * N > 3 * cus
+                                                                                : 4 * N > 5 * cus;
+    const bool holds = dlogits != nullptr && nvec_all > 256 * 8 && (N <= cus || past_one_round);
     if (vec_ok && (class_weight == nullptr || streams)) {
       const int64_t nvec = row_stride / VN;
 #define CS_CE(BLOCK, VPT)                                                                   \

@@ -24,7 +24,9 @@ def co():
 
 @pytest.mark.parametrize("N,V,stride,dtype,gdt", [
     (3, 57345, 57352, BF16, None),      # the narrowest 16-bit row of whole vectors
-    (330, 57347, 57352, F16, None),     # more rows than workgroups
+    (330, 57347, 57352, F16, None),     # more rows than workgroups, too few for a second round: two sweeps
+    (390, 57347, 57352, F16, None),     # enough
+    (300, 40000, 40000, F32, None),     # fp32: a row per workgroup in registers
     (3, 98304, 98304, BF16, None),      # the last width of the first plan, no padding
     (3, 98305, 98312, F16, None),
     (3, 131072, 131072, F16, None),

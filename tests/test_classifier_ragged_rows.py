@@ -30,7 +30,10 @@ def co():
     (3, 57281, 57281, BF16, None),      # the next one
     (2, 53183, 53183, BF16, F32),       # the widest with fp32 gradients
     (2, 53185, 53185, F16, F32),
-    (260, 20011, 20011, BF16, F32),
+    (260, 20011, 20011, BF16, F32),     # two sweeps up to 24576 columns with fp32 gradients
+    (3, 24575, 24575, BF16, F32),
+    (3, 24577, 24577, F16, F32),        # streamed
+    (520, 33001, 33001, BF16, None),    # the loss alone: two sweeps where rows are a few per CU
     (3, 8193, 8193, F32, None),         # fp32: 2048 vectors and an element
     (2, 32735, 32735, F32, None),       # the widest streamed fp32 row
     (2, 32737, 32737, F32, None),

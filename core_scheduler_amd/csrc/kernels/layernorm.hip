@@ -21,7 +21,7 @@
 //
 // Rows wider than one wave's registers, rows that are not whole vectors and unaligned pointers go
 // through the same scheme with several waves per row (ln_fwd_block_kernel, ln_bwd_block_kernel);
-// fp64 and rows beyond 16384 columns through a plain one-workgroup-per-row path.
+// fp64, rows beyond 16384 columns and a few ragged rows' backward through a plain one-workgroup-per-row path.
 #include "common.hpp"
 
 #include <math.h>
@@ -804,8 +804,8 @@ __global__ __launch_bounds__(THREADS, WPE) void ln_bwd_kernel(
 // per wave and 8 elements per lane leave registers for two rows (the next one requested as soon as
 // the one before the current is done), gamma, beta or the column sums.  [4096,5120] bf16 with the
 // residual: forward 31.9 us (5.3 TB/s; one workgroup per row behind a separate add 64 us), backward
-// 41.6 us (4.0 TB/s without the partial rows' 21 MB; 382 us with the plain kernels, whose column sums
-// ran on 80 workgroups).  [12000,1003] fp32: 38.9 + 40.1 us against 58.5 + 1121.
+// 43.9 us (3.8 TB/s without the partial rows' 42 MB; 41.6 with partial rows in fp32, 382 with the plain kernels,
+// whose column sums ran on 80 workgroups).  [12000,1003] fp32: 38.9 + 40.1 us against 58.5 + 1121.
 template <typename T, int N, bool UA>
 __device__ __forceinline__ Raw<T, N> load_piece(const T *p) {
   Raw<T, N> r;
@@ -1955,7 +1955,8 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
 #define CS_LN_BWD_B(VPT, HAS_DX, HAS_DP, HAS_DRES)                                                                \
   st = launch_bwd_block<TDY, TX, TDX, TP, VPT, HAS_DX, HAS_DP, HAS_DRES>(dy, x, mean, rstd, gamma, dx, workspace, \
                                                                          rows, C, dres, plan, ua, lds, s)
-#define CS_LN_BWD_BLOCK(VPT, WPE, HAS_DX, HAS_DP, HAS_DRES)                      \
+// (the second argument is CS_LN_BWD_MASK's and has no use here)
+#define CS_LN_BWD_BLOCK(VPT, UNUSED, HAS_DX, HAS_DP, HAS_DRES)                   \
   if constexpr (VPT * Vec16<TX>::n > 8 && HAS_DX && HAS_DP) {                    \
     CS_LN_BWD_B(VPT, false, true, false);                                        \
     if (st == CS_OK) CS_LN_BWD_B(VPT, true, false, HAS_DRES);                    \

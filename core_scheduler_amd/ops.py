@@ -91,7 +91,6 @@ def adamw_step(w, dw, m, v, *, lr, beta1, beta2, eps, weight_decay, t, v_max=Non
     """One AdamW step on one tensor, in place (cs::optimizer::AdamW::step).  `t` >= 1."""
     _check_adamw_tensors(w, dw, m, v, v_max)
     dev = _dev(w, dw, m, v, v_max)
-    lib = _capi.load()
     _call("cs_adamw_step", dev, _ptr(w), _ptr(dw), _ptr(m), _ptr(v), _ptr(v_max), w.numel(), _dt(w), lr, beta1, beta2,
           eps, weight_decay, t)
 

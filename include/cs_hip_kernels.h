@@ -219,7 +219,8 @@ size_t cs_layernorm_backward_workspace_bytes(int64_t rows, int64_t C);
  * {1,0,0}, {0,1,1}, {0,1,0}); dgamma/dbeta are stored in param_dtype and,
  * when accumulate != 0, added to what is already there.  dy is stored as
  * dy_dtype (x_dtype or CS_F32), dx as dx_dtype (same choice).  workspace
- * is needed whenever dgamma or dbeta is requested. */
+ * is needed whenever dgamma or dbeta is requested; its size never falls as
+ * rows grows, so one buffer sized for the most rows serves every batch. */
 int cs_layernorm_backward(const void *dy, const void *x, const void *mean,
                           const void *rstd, const void *gamma, void *dx,
                           void *dgamma, void *dbeta, void *workspace,
@@ -235,11 +236,11 @@ int cs_layernorm_backward(const void *dy, const void *x, const void *mean,
  *             replaces ln2->backward (:468) followed by Utils::add (:469)
  * Results are those of the two separate kernels, bit for bit: the sum is
  * rounded to x_dtype before it is normalised, and dx is rounded to dx_dtype
- * before dresidual is added.  Both adds run inside the LayerNorm kernel, which
- * saves a [rows, C] round trip and a launch: forward for every row width the
- * row-in-registers kernels take (up to 512 16-byte vectors: C <= 4096 for
- * 16-bit x), backward for rows of up to 256 vectors (C <= 2048 at 16 bit);
- * other shapes run an elementwise add launch next to the LayerNorm launch.
+ * before dresidual is added.  (A row that does not start on a 16-byte boundary
+ * is added up in another order: compare forms whose pointers are alike.)
+ * Both adds run inside the LayerNorm kernel, which saves a [rows, C] round trip
+ * and a launch, for rows of up to 16384 columns of any type but fp64; wider rows
+ * and fp64 run an elementwise add launch next to the LayerNorm launch.
  * residual and sum_out are [rows, C] of x_dtype (sum_out may be x or residual
  * itself); dresidual is [rows, C] of dx_dtype (dx may be dresidual itself).
  * All other arguments as in the plain calls. */
@@ -395,9 +396,10 @@ int cs_embedding_backward_positions(const void *dout, void *dwpe, int64_t B,
  * for MEAN and dloss otherwise; padding columns are written as zero.  The
  * reference has no upstream gradient (it passes ones_like(loss)):
  * dloss = 1 reproduces it.
- * Any row_stride >= V is accepted.  Rows that start on 16-byte boundaries
- * and have at most 57344 columns (16 bit) or 65536 (fp32) are read once;
- * other rows are read twice, the second time from cache.
+ * Any row_stride >= V is accepted.  Rows of up to 163840 columns (16 bit) or
+ * 81920 (fp32), from 16384 and 8192 on also where the row stride is no multiple
+ * of 16 bytes, are read once, with few exceptions; other rows are read twice,
+ * the second time from cache.
  * ---------------------------------------------------------------------- */
 size_t cs_fused_classifier_workspace_bytes(int64_t N);
 int cs_fused_classifier(const void *logits, void *dlogits,
@@ -413,8 +415,9 @@ int cs_fused_classifier(const void *logits, void *dlogits,
  * class_weight is [V] fp32; a row's loss and gradient are scaled by the weight
  * of its target, MEAN divides by the sum of those weights over the rows that
  * are not ignored, and total_weight returns that sum.  class_weight == NULL is
- * cs_fused_classifier.  No caller in the reference sets a weight, so this
- * form takes the two-sweep row kernel for every shape. */
+ * cs_fused_classifier.  Rows wider than 16384 columns (8192 at fp32) run as
+ * fast as without weights, narrower ones take the two-sweep row kernel (no
+ * caller in the reference sets a weight). */
 int cs_fused_classifier_weighted(const void *logits, void *dlogits,
                                  const int64_t *targets,
                                  const float *class_weight, float *row_loss,

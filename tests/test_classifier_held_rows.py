@@ -81,6 +81,22 @@ def test_wide_rows(ops, co, N, V, stride, dtype, gdt, weighted):
         assert_bit_exact(gx, d, "in place")
 
 
+@pytest.mark.parametrize("V,dtype", [(100003, BF16), (57281, F16), (32739, F32)])
+def test_unpadded_rows_in_place(ops, V, dtype):
+    """More rows than workgroups, each reading vectors that it shares with a neighbour whose gradient may be there."""
+    N = 400
+    x = (randn((N, V), 975, std=2.0)).to(dtype).to("cuda:0")
+    t = randint(0, V, (N,), 976)
+    t[::7] = -100
+    t = t.to("cuda:0")
+    loss, row, d, _ = ops.fused_classifier(x, t, V)
+    loss2, row2, d2, _ = ops.fused_classifier(x, t, V, inplace=True)
+    assert d2.data_ptr() == x.data_ptr()
+    assert_bit_exact(x, d, "in place")
+    assert_bit_exact(row2, row, "row loss")
+    assert_bit_exact(loss2, loss, "loss")
+
+
 @pytest.mark.parametrize("stride", [70016, 70001])
 def test_values_that_are_not_finite(ops, stride):
     """-inf logits have no share; a NaN or +inf makes its row NaN and no other; padding stays zero;

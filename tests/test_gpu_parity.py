@@ -481,7 +481,10 @@ def test_layernorm_masks_and_accumulate(ops, co):
     (700, 768, torch.bfloat16, torch.float32, True),      # the autocast combination: fp32 dy and dx
     (2048, 1600, torch.bfloat16, torch.float32, False),   # XL width
     (513, 768, torch.float16, torch.float16, False),
-    (77, 4096, torch.bfloat16, torch.float32, False),     # two waves per row
+    (77, 4096, torch.bfloat16, torch.float32, False),     # several waves per row
+    (600, 4096, torch.bfloat16, torch.float32, False),    # two rows side by side in a workgroup, two steps
+    (1100, 2056, torch.float16, torch.float16, False),    # three rows side by side
+    (300, 2048, torch.float32, torch.float32, False),
     (2051, 1600, torch.float32, torch.float32, False),
     (3, 768, torch.float32, torch.float32, False),
     (1500, 384, torch.bfloat16, torch.float32, True),     # one vector per lane
@@ -532,7 +535,8 @@ def test_layernorm_backward_as_two_calls(ops, rows, C, x_dtype, p_dtype, wide_dy
     (333, 256, torch.bfloat16, torch.bfloat16),    # two rows per wave, one vector per lane
     (515, 1600, torch.bfloat16, torch.float32),    # a wave per row, four vectors per lane
     (64, 1024, torch.float16, torch.float32),      # two vectors per lane
-    (77, 4096, torch.bfloat16, torch.float32),     # two waves per row: pending sums get a launch of their own
+    (77, 4096, torch.bfloat16, torch.float32),     # several waves per row: pending sums get a launch of their own
+    (700, 3072, torch.float16, torch.float32),     # the same with two rows side by side in a workgroup
 ])
 def test_layernorm_backward_chain(ops, rows, C, x_dtype, p_dtype):
     """Calls whose column sums ride in the next call's launch (cs_layernorm_backward_rows_pending):

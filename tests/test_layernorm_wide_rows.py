@@ -156,6 +156,36 @@ def test_column_sums_are_rounded_once(ops, rows, C, dtype, offset):
         assert (err <= bound).all(), f"{name}: {(err > bound).sum().item()} of {C} sums off"
 
 
+@pytest.mark.parametrize("rows,C,dtype,offset", [
+    (300, 2056, BF16, 0), (600, 3072, F16, 0), (600, 1003, F32, 0), (300, 4099, BF16, 1), (300, 5120, BF16, 0),
+    (70, 8200, F16, 0), (70, 16380, F32, 0)])
+@pytest.mark.parametrize("residual", [False, True])
+def test_values_that_are_not_finite_stay_in_their_rows(ops, rows, C, dtype, offset, residual):
+    """A row with a NaN or an infinity is NaN throughout, forward and backward; every other row has the bits it has
+    without them, although rows share a wave's registers in turn and workgroups share partial rows."""
+    x, dy, res = (randn((rows, C), s, dtype=dtype) for s in (980, 981, 982))
+    gamma, beta = place(randn(C, 983, std=0.02, mean=1.0), 0), place(randn(C, 984, std=0.02), 0)
+    bad = x.clone()
+    bad[1, 0], bad[rows // 2, C - 1], bad[rows - 1, C // 2] = float("nan"), float("inf"), float("-inf")
+    good_rows = torch.ones(rows, dtype=torch.bool)
+    good_rows[[1, rows // 2, rows - 1]] = False
+    out = []
+    for v in (x, bad):
+        gv, gdy, gres = place(v, offset), place(dy, offset), place(res, offset)
+        if residual:
+            total, y, mean, rstd = ops.add_layernorm_forward(gv, gres, gamma, beta)
+        else:
+            total, (y, mean, rstd) = gv, ops.layernorm_forward(gv, gamma, beta)
+        dx, dg, db = ops.layernorm_backward(gdy, place(total.cpu(), offset), mean, rstd, gamma)
+        out.append([t.cpu() for t in (y, mean, rstd, dx, dg, db)])
+    for clean, got, name in zip(out[0][:4], out[1][:4], ("y", "mean", "rstd", "dx")):
+        assert_bit_exact(got[good_rows], clean[good_rows], name)
+        if name in ("y", "dx"):
+            assert torch.isnan(got[~good_rows]).all(), name
+    assert torch.isnan(out[1][4]).all()              # every column of dgamma sums a NaN xhat
+    assert_bit_exact(out[1][5], out[0][5], "dbeta")  # dy is finite
+
+
 @pytest.mark.parametrize("C,dtype", [(4096, BF16), (1003, F32), (4099, F16), (5120, BF16)])
 def test_a_long_batchs_workspace_serves_a_short_one(ops, C, dtype):
     from core_scheduler_amd import _capi

@@ -1739,6 +1739,11 @@ BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, bool want_d
     if (rows <= 64 && !two_calls && C / (16 / (int64_t)dtype_size(x_dtype)) <= 8 * kWave) return b;
     b.block = block_plan(rows, C, x_dtype, true, false);
     if (b.block.vpt == 0) return b;
+    // Four fp32 vectors per lane spill up to 60 registers: worth it with rows enough (general / several waves, [16,8200]
+    // 14.0 / 18.7 us, [32,12288] 29.5 / 23.0, [4096,16384] 718 / 295; ragged, with the most spills, [300,16383] 75 / 97,
+    // [1024,16383] 165 / 140).
+    const bool whole = aligned && C % (16 / (int64_t)dtype_size(x_dtype)) == 0;
+    if (b.block.vpt == 4 && rows <= (whole ? 16 : 512)) return b;
     b.kind = kBwdBlock;
     b.vpl = b.block.vpt;
     b.threads = b.block.gw * b.block.groups * kWave;

@@ -40,6 +40,9 @@ def place(t, offset):
     (20, 16392, BF16, F32, False, 0),    # past it: the general kernels
     (1100, 1028, F32, F32, False, 0),    # fp32: 257 vectors
     (40, 16380, F32, F32, False, 0),     # four fp32 vectors per lane
+    (16, 8200, F32, F32, False, 0),      # too few rows for them in the backward
+    (17, 8200, F32, F32, False, 0),
+    (513, 8197, F32, F32, False, 0),     # enough at a ragged width
     (64, 4100, F16, F16, False, 0),      # as many rows as the general backward kernels take, up to 512 vectors
     (65, 4100, BF16, F32, False, 0),     # one more
     (5000, 1, F32, F32, False, 0),       # no whole vector, one column
@@ -139,7 +142,7 @@ def test_rows_of_one_value(ops, C, dtype, offset, residual):
 @pytest.mark.parametrize("rows,C,dtype,offset", [
     (4096, 1003, F32, 0), (515, 4099, F32, 0), (5000, 71, F16, 0), (3000, 4, F32, 1), (2000, 5, BF16, 0),  # ragged
     (600, 768, BF16, 1), (1000, 2056, BF16, 1),   # unaligned
-    (3000, 4104, BF16, 0), (300, 8200, BF16, 0), (100, 16380, F32, 0), (40, 16391, F32, 0),  # wide, and the widest
+    (3000, 4104, BF16, 0), (300, 8200, BF16, 0), (100, 16380, F32, 0), (40, 16391, F32, 0), (520, 16391, F32, 0),  # wide, and the widest
 ])
 def test_column_sums_are_rounded_once(ops, rows, C, dtype, offset):
     """dgamma and dbeta are the double sums of the fp32 terms, rounded once: half a unit in the last place, and

@@ -804,8 +804,8 @@ __global__ __launch_bounds__(THREADS, WPE) void ln_bwd_kernel(
 // per wave and 8 elements per lane leave registers for two rows (the next one requested as soon as
 // the one before the current is done), gamma, beta or the column sums.  [4096,5120] bf16 with the
 // residual: forward 31.9 us (5.3 TB/s; one workgroup per row behind a separate add 64 us), backward
-// 43.9 us (3.8 TB/s without the partial rows' 42 MB; 41.6 with partial rows in fp32, 382 with the plain kernels,
-// whose column sums ran on 80 workgroups).  [12000,1003] fp32: 38.9 + 40.1 us against 58.5 + 1121.
+// 42.1 us and 5.1 for the sums (4.0 TB/s without the partial rows' 42 MB; 40.7 and 4.6 with partial rows in fp32;
+// 382 with the plain kernels, whose column sums ran on 80 workgroups).  [12000,1003] fp32: 38.9 + 40.1 us against 58.5 + 1121.
 template <typename T, int N, bool UA>
 __device__ __forceinline__ Raw<T, N> load_piece(const T *p) {
   Raw<T, N> r;

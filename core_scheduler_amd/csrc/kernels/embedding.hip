@@ -13,8 +13,7 @@
 // independent of scheduling.  Four launches:
 //   1. tile sort  - each workgroup bitonic-sorts 1024 keys, one per lane:
 //                   exchanges below 64 lanes are wave shuffles, the rest go
-//                   through LDS.  Spare workgroups of the same launch sum the
-//                   position-table gradient, which needs no order.
+//                   through LDS.
 //   2. merge rank - every key finds its global rank by binary search in the
 //                   other tiles (staged in LDS) and is scattered to its place.
 //                   Launches 1 and 2 keep few CUs busy, so further workgroups
@@ -26,11 +25,14 @@
 //                   through LDS in wave order; a segment that crosses
 //                   workgroups leaves one fp32 partial row per workgroup, so
 //                   a hot row is read by as many CUs as it has windows.
-//   4. finish     - the workgroup of a crossing segment's first window adds
-//                   that segment's partial rows in window order.
+//   4. finish     - the workgroups of a crossing segment's first window add
+//                   that segment's partial rows in window order.  Further
+//                   workgroups of the same launch sum the position-table
+//                   gradient, which needs no order (of launch 3, where the
+//                   list is short).
 // A list of at most 8192 entries skips 1 and 2: one launch ranks every key by
 // comparing it with all others (see emb_bwd_rank_kernel), and does the zero
-// fill and the position-table sum next to that.
+// fill next to that.
 // The traffic that matters is the dense write of dweight (V*C elements), one
 // read of dout and a second write of the indexed rows.
 #include "common.hpp"
@@ -241,32 +243,32 @@ __device__ __forceinline__ void positions_vector(const T *__restrict__ dout, T *
   store16_stream(dwpe + f * VN, o);
 }
 
-// The same for a workgroup of kTile lanes, with the batch dimension split over S = 2^log2_s lanes
+// The same for a workgroup of THREADS lanes, with the batch dimension split over S = 2^log2_s lanes
 // per vector: a lane walks its rows with 8 loads in flight, so a long batch is a long chain of
 // round trips unless it is cut up.  Lane (v, q) adds the rows of slice q for vector v of the
-// workgroup's kTile / S; slices 1.. are left in LDS and slice 0 adds them in order, so the sum
-// is a fixed tree.  lds: (S - 1) * (kTile / S) * VN floats.  With S = 1 this is positions_vector.
+// workgroup's THREADS / S; slices 1.. are left in LDS and slice 0 adds them in order, so the sum
+// is a fixed tree.  lds: (S - 1) * (THREADS / S) * VN floats.  With S = 1 this is positions_vector.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kPosMaxLog2Slices = 4;
-constexpr size_t kPosLdsBytes = (size_t)kTile * 32;  // bound for every S and element type
+constexpr size_t kPosLdsBytesPerLane = 32;  // bound for every S and element type
 
-template <typename T>
+template <typename T, int THREADS>
 __device__ __forceinline__ void positions_block(const T *__restrict__ dout, T *__restrict__ dwpe,
                                                 int64_t blk, int64_t B, int64_t TC, int accumulate,
                                                 int log2_s, f32x4 *lds, int tid) {
   constexpr int VN = Vec16<T>::n;
   constexpr int kPieces = VN / 4;  // f32x4 pieces of one vector's sums
   if (log2_s == 0) {  // block-uniform
-    const int64_t f = blk * kTile + tid;
+    const int64_t f = blk * THREADS + tid;
     if (f < TC / VN) positions_vector<T>(dout, dwpe, f, B, TC, accumulate);
     return;
   }
   constexpr int kInFlight = 4;  // loads per lane: with the batch cut up there are lanes enough
   const int S = 1 << log2_s;
-  const int V = kTile >> log2_s;
+  const int V = THREADS >> log2_s;
+  static_assert((THREADS & (THREADS - 1)) == 0 && THREADS >> kPosMaxLog2Slices > 0, "a power of two above S");
   const int v = tid & (V - 1);
-  const int q = tid >> (10 - log2_s);
-  static_assert(kTile == 1024, "q is tid / V with V = 1024 >> log2_s");
+  const int q = tid / V;
   const int64_t f = blk * V + v;
   const bool ok = f < TC / VN;
   const int64_t per = (B + S - 1) / S;
@@ -359,26 +361,17 @@ __device__ __forceinline__ void zero_fill_block(u32x4 *__restrict__ dst, int64_t
 // Launch layout, in block order:
 //   [0, n_tiles)                sort one tile of 1024 keys
 //   + 1                         preset sorted_id to "no id"
-//   + pos_blocks                position-table gradient, 1024 vectors per block
 //   + the rest                  zero fill of fill_dst[0, fill_vecs)
-template <typename KeyT, typename IdxT, typename T>
+template <typename KeyT, typename IdxT>
 __global__ __launch_bounds__(kTile) void emb_bwd_tile_sort_kernel(
     const IdxT *__restrict__ ids, KeyT *__restrict__ tiles, uint32_t *__restrict__ sorted_id,
     int64_t n, int n_tiles, int shift, int64_t num_weights, int64_t padding_idx,
-    const T *__restrict__ dout, T *__restrict__ dwpe, int64_t B, int64_t TC, int accumulate,
-    int64_t pos_blocks, int pos_log2_slices, u32x4 *__restrict__ fill_dst, int64_t fill_vecs) {
-  // the sorting workgroups keep two key arrays here, the position workgroups their slice sums
-  static_assert(2 * kTile * sizeof(KeyT) <= kPosLdsBytes, "the key arrays fit the shared buffer");
-  __shared__ f32x4 shared_raw[kPosLdsBytes / sizeof(f32x4)];
-  KeyT(*keys)[kTile] = reinterpret_cast<KeyT(*)[kTile]>(shared_raw);
+    u32x4 *__restrict__ fill_dst, int64_t fill_vecs) {
+  __shared__ KeyT keys[2][kTile];
   const int tid = threadIdx.x;
   const int64_t blk = blockIdx.x;
-  if (blk > n_tiles + pos_blocks) {
-    zero_fill_block<kTile, kFillVecsSort>(fill_dst, fill_vecs, blk - n_tiles - pos_blocks - 1, tid);
-    return;
-  }
   if (blk > n_tiles) {
-    positions_block<T>(dout, dwpe, blk - n_tiles - 1, B, TC, accumulate, pos_log2_slices, shared_raw, tid);
+    zero_fill_block<kTile, kFillVecsSort>(fill_dst, fill_vecs, blk - n_tiles - 1, tid);
     return;
   }
   if (blk == n_tiles) {
@@ -505,7 +498,6 @@ __global__ __launch_bounds__(kThreads) void emb_bwd_merge_kernel(
 // address).  The 32 partial counts of a key are added through the LDS.
 // Launch layout, in block order (the ranking workgroups run longest, so they start first):
 //   [0, rank_blocks)            rank 32 keys each; also preset the unused tail of sorted_id
-//   + pos_blocks                position-table gradient, 1024 vectors per block
 //   + the rest                  zero fill of fill_dst[0, fill_vecs)
 constexpr int kRankThreads = 1024;
 constexpr int kRankOwn = 32;
@@ -516,25 +508,18 @@ constexpr int kRankGroups = kRankThreads / kRankOwn;
 constexpr size_t kRankMaxKeyBytes = CS_EMB_RANK_MAX_KEY_BYTES;  // longest key list that is ranked this way
 constexpr size_t kRankPartBytes = (size_t)kRankGroups * kRankOwn * sizeof(int);
 
-template <typename KeyT, typename IdxT, typename T>
+template <typename KeyT, typename IdxT>
 __global__ __launch_bounds__(kRankThreads) void emb_bwd_rank_kernel(
     const IdxT *__restrict__ ids, uint32_t *__restrict__ sorted_id,
     uint32_t *__restrict__ sorted_pos, int64_t n, int n_quads, int shift, int64_t num_weights,
-    int64_t padding_idx, const T *__restrict__ dout, T *__restrict__ dwpe, int64_t B, int64_t TC,
-    int accumulate, int rank_blocks, int64_t pos_blocks, int pos_log2_slices,
-    u32x4 *__restrict__ fill_dst, int64_t fill_vecs) {
+    int64_t padding_idx, int rank_blocks, u32x4 *__restrict__ fill_dst, int64_t fill_vecs) {
   typedef KeyT Quad __attribute__((ext_vector_type(4)));
-  extern __shared__ u32x4 rank_lds[];  // the key list and the partial counts; kPosLdsBytes at least when positions are sliced
+  extern __shared__ u32x4 rank_lds[];  // the key list and the partial counts
   __shared__ int valid_of_wave[kRankThreads / kWave];
   const int tid = threadIdx.x;
   const int64_t blk = blockIdx.x;
-  if (blk >= rank_blocks + pos_blocks) {
-    zero_fill_block<kRankThreads, kFillVecsRank>(fill_dst, fill_vecs, blk - rank_blocks - pos_blocks, tid);
-    return;
-  }
   if (blk >= rank_blocks) {
-    positions_block<T>(dout, dwpe, blk - rank_blocks, B, TC, accumulate, pos_log2_slices,
-                       reinterpret_cast<f32x4 *>(rank_lds), tid);
+    zero_fill_block<kRankThreads, kFillVecsRank>(fill_dst, fill_vecs, blk - rank_blocks, tid);
     return;
   }
   KeyT *keys = reinterpret_cast<KeyT *>(rank_lds);  // [4 n_quads], padded with sentinels
@@ -609,7 +594,7 @@ __global__ __launch_bounds__(kRankThreads) void emb_bwd_rank_kernel(
 constexpr int kOwn = 4;                         // sorted entries per wave
 constexpr int kRedWaves = kWindow / kOwn;       // 8
 constexpr int kRedThreads = kRedWaves * kWave;  // 512: two workgroups share a CU
-constexpr int kFinThreads = 1024;               // finish kernel
+constexpr int kFinThreads = 256;                // finish kernel: lanes, and columns of a workgroup
 constexpr int kFinWaves = kFinThreads / kWave;
 #ifndef CS_EMB_FIN_DIRECT_ROWS
 #define CS_EMB_FIN_DIRECT_ROWS 8
@@ -628,6 +613,12 @@ constexpr int kFinMaxGroups = CS_EMB_FIN_MAX_GROUPS;    // lane groups that shar
 #endif
 constexpr int kVpl = CS_EMB_VPL;                // 16-byte column vectors per lane per column chunk
 
+// Lists of up to this many windows (8192 entries, one reducing workgroup per CU) have the position-table sums in
+// the reduce launch, longer ones in the finish launch (see there): kernels of a call, us, reduce / finish /
+// before both, next to the zero fill: [1,123] x 768 24.3 / 25.3 / 24.1, [4,512] x 768 27.2 / 27.5 / 28.8,
+// [8,512] x 1600 49.7 / 50.1 / 53.2, [6,1024] x 768 30.3 / 30.7 / 31.8, [8,1024] x 1600 56.7 / 56.7 / 61.6.
+constexpr int64_t kPosEarlyWindows = 256;
+
 // Workgroup w reduces sorted entries [kWindow w, kWindow (w + 1)).  partial rows live at
 // partial[(w*2 + slot) * C]: slot 0 for a run that came in over the window's
 // left edge and ends inside, slot 1 for a run that leaves over its right edge.
@@ -635,7 +626,8 @@ template <typename T>
 __global__ __launch_bounds__(kRedThreads, 2048 / kRedThreads) void emb_bwd_reduce_kernel(
     const T *__restrict__ dout, const uint32_t *__restrict__ sorted_id,
     const uint32_t *__restrict__ sorted_pos, T *__restrict__ dweight, float *__restrict__ partial,
-    int64_t n, int64_t C, int accumulate, int by_freq) {
+    int64_t n, int64_t C, int accumulate, int by_freq, int64_t windows, T *__restrict__ dwpe, int64_t B, int64_t TC,
+    int pos_log2_slices) {
   constexpr int VN = Vec16<T>::n;
   constexpr int kChunkCols = kWave * kVpl * VN;
   extern __shared__ float lds[];  // [kRedWaves][2 slots][kChunkCols]
@@ -644,6 +636,11 @@ __global__ __launch_bounds__(kRedThreads, 2048 / kRedThreads) void emb_bwd_reduc
   const int wave = tid >> 6;
   const int nvec = (int)(C / VN);
   const int64_t w = blockIdx.x;
+  if (w >= windows) {
+    positions_block<T, kRedThreads>(dout, dwpe, w - windows, B, TC, accumulate, pos_log2_slices,
+                                    reinterpret_cast<f32x4 *>(lds), tid);
+    return;
+  }
   const int64_t p0 = w * kWindow;
 
   // ---- ids of the window (lane l <-> entry p0 + l), the entry before and the entry after
@@ -834,24 +831,40 @@ __global__ __launch_bounds__(kRedThreads, 2048 / kRedThreads) void emb_bwd_reduc
     }
     __syncthreads();
   }
-
 }
 
-// The last level of the segmented sum.  Workgroup w looks at window w: if the
-// run that leaves it over the right edge began in it (a true segment head),
-// this is that segment's first window, and the workgroup adds the segment's
-// partial rows in window order: slot 1 of every window the segment leaves,
-// slot 0 of the one it ends in.
+// The last level of the segmented sum.  A workgroup looks at window w for kFinThreads of the columns: if
+// the run that leaves the window over its right edge began in it (a true segment head), this is that
+// segment's first window, and the workgroup adds the segment's partial rows in window order: slot 1 of
+// every window the segment leaves, slot 0 of the one it ends in.
+//
+// Bound by a chain of trips to memory (ids, partial rows) that leaves HBM idle, so the position-table sums of
+// a long list, which read all of dout and wait for nothing, run next to it: the first workgroups of the grid,
+// because the others are short.  They ran next to the tile sort before, whose launch is bound by the bytes of its
+// zero fill.  Kernels of a call, us: 16384 tokens x 1600 Zipf ids 73.3 -> 69.2, uniform 85.9 -> 84.6,
+// 32768 x 768 fp32 93.5 -> 89.9; in the reduce launch of such a list they cost what they save.  256 columns per
+// workgroup, so that a hot row's sum is shared by several: 14.2 us with the positions at 16384 x 1600; 512
+// columns 14.4, 1024 15.2; positions last 17.3.  dout is read past the caches in both launches: kept there it
+// pushes out what the next call reads (this launch 14.2 -> 12.3 us, but the next gather 12.9 -> 20.1).
 template <typename T>
-__global__ __launch_bounds__(kFinThreads) void emb_bwd_finish_kernel(
+__global__ __launch_bounds__(kFinThreads, 5) void emb_bwd_finish_kernel(
     const uint32_t *__restrict__ sorted_id, const float *__restrict__ partial,
-    T *__restrict__ dweight, int64_t n, int64_t C, int accumulate, int by_freq) {
+    T *__restrict__ dweight, int64_t n, int64_t C, int accumulate, int by_freq, int64_t fin_blocks, int slices,
+    const T *__restrict__ dout, T *__restrict__ dwpe, int64_t B, int64_t TC, int pos_log2_slices) {
   __shared__ int first_other[kFinWaves];
   __shared__ int first_tail[kFinWaves];
+  __shared__ f32x4 lds[kFinThreads * kPosLdsBytesPerLane / sizeof(f32x4)];
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = tid >> 6;
-  const int64_t w = blockIdx.x;
+  const int64_t blk = (int64_t)blockIdx.x - (gridDim.x - fin_blocks);
+  if (blk < 0) {
+    positions_block<T, kFinThreads>(dout, dwpe, blockIdx.x, B, TC, accumulate, pos_log2_slices, lds, tid);
+    return;
+  }
+  const int64_t w = (unsigned)blk / (unsigned)slices;
+  const int c0 = (int)(blk - w * slices) * kFinThreads;  // the workgroup's first column
+  const int cols = (int)C - c0 < kFinThreads ? (int)C - c0 : kFinThreads;
   const int64_t last = w * kWindow + kWindow - 1;
   if (last + 1 >= n) return;  // nothing after this window
   // Everything the decisions below read, and the two partial rows of the usual case (a segment
@@ -867,16 +880,16 @@ __global__ __launch_bounds__(kFinThreads) void emb_bwd_finish_kernel(
   uint32_t raw_before = sorted_id[w > 0 ? w * kWindow - 1 : 0];
   uint32_t raw_q = sorted_id[pq < n ? pq : n - 1];
   uint32_t raw_f = sorted_id[pw * kWindow < n ? pw * kWindow : n - 1];
-  const int64_t col0 = tid < C ? tid : 0;
-  float pre_leave = partial[(w * 2 + 1) * C + col0];        // window w, left over its right edge
-  float pre_enter = partial[((w + 1) * 2 + 0) * C + col0];  // window w + 1, entered over its left edge
+  const int64_t col = c0 + (tid < cols ? tid : 0);
+  float pre_leave = partial[(w * 2 + 1) * C + col];        // window w, left over its right edge
+  float pre_enter = partial[((w + 1) * 2 + 0) * C + col];  // window w + 1, entered over its left edge
   asm volatile("" : "+v"(raw_last), "+v"(raw_next), "+v"(raw_first), "+v"(raw_before), "+v"(raw_q), "+v"(raw_f),
                     "+v"(pre_leave), "+v"(pre_enter));
   const uint32_t id = raw_last;
   if (id == kNoId || raw_next != id) return;  // no run leaves this window
   // its run began in this window unless the whole window (and the entry before it) has this id
   if (raw_first == id && w > 0 && raw_before == id) return;
-  // windows after w whose last entry still has this id are left by the segment too; 1024 windows
+  // windows after w whose last entry still has this id are left by the segment too; kFinThreads windows
   // per round.  w_hi: the first window whose last entry is not this id.  The segment ends inside
   // it when its first entry still has the id (`tail`), otherwise at the end of the window before.
   int64_t w_hi = -1;
@@ -925,9 +938,9 @@ __global__ __launch_bounds__(kFinThreads) void emb_bwd_finish_kernel(
   // group order.  Taken one column per lane instead, the hottest row of a Zipf batch was a chain of
   // 9-18 trips to memory in a single workgroup while all others had finished.
   const int64_t rows_in = w_end - w + 1;  // partial rows of the segment
-  const int vc = (int)(C >> 2);           // 16-byte pieces per row
-  if (rows_in > kFinDirectRows && (C & 3) == 0 && vc <= kFinThreads) {
-    __shared__ f32x4 group_sum[kFinThreads];
+  const int vc = cols >> 2;               // 16-byte pieces of a row (C is a multiple of four columns here)
+  if (rows_in > kFinDirectRows) {
+    f32x4 *group_sum = lds;
     int groups = kFinThreads / vc;
     if (groups > kFinMaxGroups) groups = kFinMaxGroups;
     const int g = tid / vc, v = tid - g * vc;
@@ -943,7 +956,7 @@ __global__ __launch_bounds__(kFinThreads) void emb_bwd_finish_kernel(
           const int64_t rr = r < rows_in ? r : rows_in - 1;
           // rows before the last were left over the right edge (slot 1), the last was entered (slot 0)
           const int64_t slot = rr < rows_in - 1 ? (w + rr) * 2 + 1 : w_end * 2;
-          x[u] = *reinterpret_cast<const f32x4 *>(partial + slot * C + 4 * v);
+          x[u] = *reinterpret_cast<const f32x4 *>(partial + slot * C + c0 + 4 * v);
         }
 #pragma unroll
         for (int u = 0; u < kFinInFlight; ++u) {
@@ -975,14 +988,13 @@ __global__ __launch_bounds__(kFinThreads) void emb_bwd_finish_kernel(
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         float o = out[k];
-        if (accumulate) o += to_acc(dst[4 * v + k]);
-        dst[4 * v + k] = from_acc<T>(o);
+        if (accumulate) o += to_acc(dst[c0 + 4 * v + k]);
+        dst[c0 + 4 * v + k] = from_acc<T>(o);
       }
     }
     return;
   }
-  for (int64_t col = tid; col < C; col += kFinThreads) {
-    const bool have = col == tid;  // the first column of the lane came in with the loads above
+  if (tid < cols) {
     // eight interleaved sums keep eight loads in flight; the order is fixed all the same
     float t[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     int64_t ww = w;
@@ -994,7 +1006,7 @@ __global__ __launch_bounds__(kFinThreads) void emb_bwd_finish_kernel(
 #pragma unroll
       for (int u = 0; u < 8; ++u) t[u] += v[u];
     }
-    if (usual && have) {
+    if (usual) {  // these came in with the loads above
       t[0] += pre_leave;
       t[7] += pre_enter;
     } else {
@@ -1012,14 +1024,14 @@ __global__ __launch_bounds__(kFinThreads) void emb_bwd_finish_kernel(
 }
 
 // Standalone position-table gradient.  The vector form is positions_block on its own (the
-// fused call runs it inside its first launch); the scalar form takes any C and any alignment.
+// fused call runs it inside its last launch); the scalar form takes any C and any alignment.
 template <typename T>
 __global__ __launch_bounds__(kTile) void emb_bwd_positions_vec_kernel(const T *__restrict__ dout,
                                                                       T *__restrict__ dwpe, int64_t B,
                                                                       int64_t TC, int accumulate,
                                                                       int log2_slices) {
-  __shared__ f32x4 slices[kPosLdsBytes / sizeof(f32x4)];
-  positions_block<T>(dout, dwpe, blockIdx.x, B, TC, accumulate, log2_slices, slices, threadIdx.x);
+  __shared__ f32x4 slices[kTile * kPosLdsBytesPerLane / sizeof(f32x4)];
+  positions_block<T, kTile>(dout, dwpe, blockIdx.x, B, TC, accumulate, log2_slices, slices, threadIdx.x);
 }
 
 template <typename T>
@@ -1179,11 +1191,11 @@ int allow_dynamic_lds_once(const void *kernel, size_t bytes, std::atomic<bool> *
   }
   return CS_OK;
 }
-template <typename KeyT, typename IdxT, typename T>
+template <typename KeyT, typename IdxT>
 int allow_rank_lds(size_t bytes) {
   static std::atomic<bool> done[64];
   return allow_dynamic_lds_once(
-      reinterpret_cast<const void *>(&emb_bwd_rank_kernel<KeyT, IdxT, T>), bytes, done);
+      reinterpret_cast<const void *>(&emb_bwd_rank_kernel<KeyT, IdxT>), bytes, done);
 }
 
 // lanes per vector of the position sum: enough that a lane walks at most ~16 rows of the batch
@@ -1193,34 +1205,26 @@ int position_slices(int64_t B) {
   return log2_slices;
 }
 
-// Sort + merge.  The sort launch also sums dwpe (`fused_positions`), and both launches clear
-// their share of fill_dst[0, fill_vecs), on the CUs the sorting leaves idle.
-template <typename KeyT, typename IdxT, typename T>
+// Sort + merge.  Both launches clear their share of fill_dst[0, fill_vecs), on the CUs the sorting leaves idle.
+template <typename KeyT, typename IdxT>
 int sort_launch(const void *ids, char *ws, const BwdLayout &L, int64_t n, int64_t num_weights,
-                int64_t padding_idx, const T *dout, T *dwpe, bool fused_positions, int64_t B,
-                int64_t TC, int accumulate, u32x4 *fill_dst, int64_t fill_vecs, hipStream_t s) {
+                int64_t padding_idx, u32x4 *fill_dst, int64_t fill_vecs, hipStream_t s) {
   KeyT *tiles = reinterpret_cast<KeyT *>(ws + L.off_tiles);
   uint32_t *sorted_id = reinterpret_cast<uint32_t *>(ws + L.off_sorted_id);
   uint32_t *sorted_pos = reinterpret_cast<uint32_t *>(ws + L.off_sorted_pos);
-  const int pos_log2_slices = position_slices(B);
-  const int64_t pos_blocks =
-      fused_positions ? ceil_div(TC / Vec16<T>::n, (int64_t)(kTile >> pos_log2_slices)) : 0;
   const int64_t n_quads = ceil_div(n, (int64_t)4);
   if ((size_t)n_quads * 4 * sizeof(KeyT) <= kRankMaxKeyBytes) {
     // a short list: one launch ranks every key against all others
-    static_assert(kRankThreads == kTile, "positions_block assumes kTile lanes");
     const int64_t rank_blocks = ceil_div(n_quads * 4, (int64_t)kRankOwn);
     const int64_t fill_blocks = ceil_div(fill_vecs, (int64_t)kFillVecsRank);
-    const int64_t blocks = rank_blocks + pos_blocks + fill_blocks;
+    const int64_t blocks = rank_blocks + fill_blocks;
     if (blocks == 0) return CS_OK;
-    size_t lds = (size_t)n_quads * 4 * sizeof(KeyT) + kRankPartBytes;
-    if (pos_blocks > 0 && pos_log2_slices > 0 && lds < kPosLdsBytes) lds = kPosLdsBytes;
-    static_assert(kPosLdsBytes <= kRankMaxKeyBytes + kRankPartBytes, "within the limit asked for");
-    const int st = allow_rank_lds<KeyT, IdxT, T>(kRankMaxKeyBytes + kRankPartBytes);
+    const size_t lds = (size_t)n_quads * 4 * sizeof(KeyT) + kRankPartBytes;
+    const int st = allow_rank_lds<KeyT, IdxT>(kRankMaxKeyBytes + kRankPartBytes);
     if (st != CS_OK) return st;
-    emb_bwd_rank_kernel<KeyT, IdxT, T><<<dim3((unsigned)blocks), dim3(kRankThreads), lds, s>>>(
+    emb_bwd_rank_kernel<KeyT, IdxT><<<dim3((unsigned)blocks), dim3(kRankThreads), lds, s>>>(
         (const IdxT *)ids, sorted_id, sorted_pos, n, (int)n_quads, L.shift, num_weights, padding_idx,
-        dout, dwpe, B, TC, accumulate, (int)rank_blocks, pos_blocks, pos_log2_slices, fill_dst, fill_vecs);
+        (int)rank_blocks, fill_dst, fill_vecs);
     return launch_status();
   }
   // whole fill workgroups to the sort launch, the remainder to the merge launch
@@ -1228,12 +1232,12 @@ int sort_launch(const void *ids, char *ws, const BwdLayout &L, int64_t n, int64_
   const int64_t sort_fill_vecs =
       sort_fill_blocks * kFillVecsSort < fill_vecs ? sort_fill_blocks * kFillVecsSort : fill_vecs;
   const int64_t merge_fill_blocks = ceil_div(fill_vecs - sort_fill_vecs, (int64_t)kFillVecsMerge);
-  const int64_t blocks = L.n_tiles + 1 + pos_blocks + sort_fill_blocks;
+  const int64_t blocks = L.n_tiles + 1 + sort_fill_blocks;
   const int64_t mblocks = L.n_tiles * kTile / kThreads + merge_fill_blocks;
   if (blocks > 0x7fffffffLL || mblocks > 0x7fffffffLL) return CS_ERR_TOO_LARGE;
-  emb_bwd_tile_sort_kernel<KeyT, IdxT, T><<<dim3((unsigned)blocks), dim3(kTile), 0, s>>>(
-      (const IdxT *)ids, tiles, sorted_id, n, (int)L.n_tiles, L.shift, num_weights, padding_idx,
-      dout, dwpe, B, TC, accumulate, pos_blocks, pos_log2_slices, fill_dst, sort_fill_vecs);
+  emb_bwd_tile_sort_kernel<KeyT, IdxT><<<dim3((unsigned)blocks), dim3(kTile), 0, s>>>(
+      (const IdxT *)ids, tiles, sorted_id, n, (int)L.n_tiles, L.shift, num_weights, padding_idx, fill_dst,
+      sort_fill_vecs);
   int st = launch_status();
   if (st != CS_OK) return st;
   emb_bwd_merge_kernel<KeyT><<<dim3((unsigned)mblocks), dim3(kThreads), 0, s>>>(
@@ -1255,15 +1259,13 @@ int bwd_typed(const void *dout, const void *ids, void *dweight, void *dwpe, char
   constexpr int VN = Vec16<T>::n;
   const bool vec_ok = !std::is_same_v<T, double> && C % VN == 0 && is_aligned16(dout) &&
                       is_aligned16(dweight) && (!dwpe || is_aligned16(dwpe));
-  const bool fused_positions = vec_ok && dwpe != nullptr;
   const int64_t TC = T_len * C;
   // `=` semantics on the fast path: the whole table is zeroed, then indexed rows are written
   u32x4 *fill_dst = vec_ok && !accumulate ? reinterpret_cast<u32x4 *>(dweight) : nullptr;
   const int64_t fill_vecs = fill_dst ? num_weights * (C / VN) : 0;
   int st;
-#define CS_SORT(KeyT, IdxT)                                                                      \
-  sort_launch<KeyT, IdxT, T>(ids, ws, L, n, num_weights, padding_idx, (const T *)dout, (T *)dwpe, \
-                             fused_positions, B, TC, accumulate, fill_dst, fill_vecs, s)
+#define CS_SORT(KeyT, IdxT) \
+  sort_launch<KeyT, IdxT>(ids, ws, L, n, num_weights, padding_idx, fill_dst, fill_vecs, s)
   if (L.key64) {
     st = idx_dtype == CS_I64 ? CS_SORT(uint64_t, int64_t) : CS_SORT(uint64_t, int32_t);
   } else {
@@ -1288,17 +1290,32 @@ int bwd_typed(const void *dout, const void *ids, void *dweight, void *dwpe, char
   if constexpr (!std::is_same_v<T, double>) {
     float *partial = reinterpret_cast<float *>(ws + L.off_partial);
     const int64_t windows = n > 0 ? L.n_windows : 0;
-    if (windows > 0x7fffffffLL) return CS_ERR_TOO_LARGE;
-    if (windows == 0) return CS_OK;
-    const size_t lds = (size_t)kRedWaves * 2 * kWave * kVpl * VN * sizeof(float);
-    st = allow_reduce_lds<T>(lds);
-    if (st != CS_OK) return st;
-    emb_bwd_reduce_kernel<T><<<dim3((unsigned)windows), dim3(kRedThreads), lds, s>>>(
-        (const T *)dout, sorted_id, sorted_pos, (T *)dweight, partial, n, C, accumulate, by_freq);
-    st = launch_status();
-    if (st != CS_OK) return st;
-    emb_bwd_finish_kernel<T><<<dim3((unsigned)windows), dim3(kFinThreads), 0, s>>>(
-        sorted_id, partial, (T *)dweight, n, C, accumulate, by_freq);
+    const int64_t slices = ceil_div(C, (int64_t)kFinThreads);
+    const int64_t fin_blocks = windows * slices;
+    // The position sums go where the chip is idle: next to the finish workgroups, or next to the reducing ones of a
+    // list too short to occupy the chip with those.
+    const int log2_s = position_slices(B);
+    const bool pos_early = windows > 0 && windows <= kPosEarlyWindows;
+    auto pos_blocks = [&](int threads) { return dwpe ? ceil_div(TC / VN, (int64_t)(threads >> log2_s)) : 0; };
+    const int64_t red_blocks = windows + (pos_early ? pos_blocks(kRedThreads) : 0);
+    const int64_t last_blocks = fin_blocks + (pos_early ? 0 : pos_blocks(kFinThreads));
+    if (red_blocks > 0x7fffffffLL || last_blocks > 0x7fffffffLL) return CS_ERR_TOO_LARGE;
+    if (windows > 0) {
+      const size_t lds = (size_t)kRedWaves * 2 * kWave * kVpl * VN * sizeof(float);
+      static_assert(kRedThreads * kPosLdsBytesPerLane <= (size_t)kRedWaves * 2 * kWave * kVpl * VN * sizeof(float),
+                    "the slice sums of the positions fit");
+      st = allow_reduce_lds<T>(lds);
+      if (st != CS_OK) return st;
+      emb_bwd_reduce_kernel<T><<<dim3((unsigned)red_blocks), dim3(kRedThreads), lds, s>>>(
+          (const T *)dout, sorted_id, sorted_pos, (T *)dweight, partial, n, C, accumulate, by_freq, windows, (T *)dwpe,
+          B, TC, log2_s);
+      st = launch_status();
+      if (st != CS_OK) return st;
+    }
+    if (last_blocks == 0) return CS_OK;
+    emb_bwd_finish_kernel<T><<<dim3((unsigned)last_blocks), dim3(kFinThreads), 0, s>>>(
+        sorted_id, partial, (T *)dweight, n, C, accumulate, by_freq, fin_blocks, (int)slices, (const T *)dout,
+        (T *)dwpe, B, TC, log2_s);
     return launch_status();
   }
   return CS_ERR_UNSUPPORTED;

@@ -491,28 +491,34 @@ __global__ __launch_bounds__(kThreads) void emb_bwd_merge_kernel(
 // n^2 comparisons, 2 VALU operations each and nothing else, spread evenly over the chip, next
 // to the zero fill that the same launch does.
 //
-// A workgroup of 1024 lanes ranks kRankOwn = 32 keys.  It first builds every key of the list
-// in its LDS.  Lane l then owns key (l mod 32) of the workgroup's 32 and belongs to one of
-// 32 groups; group g compares against the 16-byte key quads g, g + 32, g + 64, ...: the two
+// A workgroup of 1024 lanes ranks OWN = 32 or 16 keys.  It first builds every key of the list
+// in its LDS.  Lane l then owns key (l mod OWN) of the workgroup's and belongs to one of
+// 1024 / OWN groups; group g compares against the 16-byte key quads g, g + 1024 / OWN, ...: the
 // groups of a wave read adjacent quads (no bank conflict, every lane of a group the same
-// address).  The 32 partial counts of a key are added through the LDS.
+// address).  The partial counts of a key are added through the LDS.
+//
+// 16 keys where that is at most one workgroup per CU (4096 entries) and the fill takes less time than the
+// ranking (a table of up to 32 MB), 32 otherwise.  Launch, us, 32 / 16: 4000 entries and a table of 8 MB
+// 6.9 / 6.0, 30 MB 8.1 / 7.0, 46 MB 8.6 / 9.5, 77 MB 13.7 / 15.0; 8192 entries and 77 MB (a second round of ranking
+// workgroups) 14.8 / 20.4.  64 keys take 9.6 us at 4000 entries.
 // Launch layout, in block order (the ranking workgroups run longest, so they start first):
-//   [0, rank_blocks)            rank 32 keys each; also preset the unused tail of sorted_id
+//   [0, rank_blocks)            rank OWN keys each; also preset the unused tail of sorted_id
 //   + the rest                  zero fill of fill_dst[0, fill_vecs)
 constexpr int kRankThreads = 1024;
-constexpr int kRankOwn = 32;
-constexpr int kRankGroups = kRankThreads / kRankOwn;
+constexpr int64_t kRankFewKeys = 4096;          // 16 keys per workgroup up to here,
+constexpr int64_t kRankFewFill = (int64_t)1 << 21;  // and up to this many 16-byte vectors of fill
 #ifndef CS_EMB_RANK_MAX_KEY_BYTES
 #define CS_EMB_RANK_MAX_KEY_BYTES 32768
 #endif
 constexpr size_t kRankMaxKeyBytes = CS_EMB_RANK_MAX_KEY_BYTES;  // longest key list that is ranked this way
-constexpr size_t kRankPartBytes = (size_t)kRankGroups * kRankOwn * sizeof(int);
+constexpr size_t kRankPartBytes = (size_t)kRankThreads * sizeof(int);
 
-template <typename KeyT, typename IdxT>
+template <typename KeyT, typename IdxT, int kRankOwn>
 __global__ __launch_bounds__(kRankThreads) void emb_bwd_rank_kernel(
     const IdxT *__restrict__ ids, uint32_t *__restrict__ sorted_id,
     uint32_t *__restrict__ sorted_pos, int64_t n, int n_quads, int shift, int64_t num_weights,
     int64_t padding_idx, int rank_blocks, u32x4 *__restrict__ fill_dst, int64_t fill_vecs) {
+  constexpr int kRankGroups = kRankThreads / kRankOwn;
   typedef KeyT Quad __attribute__((ext_vector_type(4)));
   extern __shared__ u32x4 rank_lds[];  // the key list and the partial counts
   __shared__ int valid_of_wave[kRankThreads / kWave];
@@ -1191,11 +1197,21 @@ int allow_dynamic_lds_once(const void *kernel, size_t bytes, std::atomic<bool> *
   }
   return CS_OK;
 }
-template <typename KeyT, typename IdxT>
-int allow_rank_lds(size_t bytes) {
+template <typename KeyT, typename IdxT, int OWN>
+int rank_launch(const void *ids, uint32_t *sorted_id, uint32_t *sorted_pos, int64_t n, int64_t n_quads, int shift,
+                int64_t num_weights, int64_t padding_idx, u32x4 *fill_dst, int64_t fill_vecs, hipStream_t s) {
+  const int64_t rank_blocks = ceil_div(n_quads * 4, (int64_t)OWN);
+  const int64_t blocks = rank_blocks + ceil_div(fill_vecs, (int64_t)kFillVecsRank);
+  if (blocks == 0) return CS_OK;
+  const size_t lds = (size_t)n_quads * 4 * sizeof(KeyT) + kRankPartBytes;
   static std::atomic<bool> done[64];
-  return allow_dynamic_lds_once(
-      reinterpret_cast<const void *>(&emb_bwd_rank_kernel<KeyT, IdxT>), bytes, done);
+  const int st = allow_dynamic_lds_once(reinterpret_cast<const void *>(&emb_bwd_rank_kernel<KeyT, IdxT, OWN>),
+                                        kRankMaxKeyBytes + kRankPartBytes, done);
+  if (st != CS_OK) return st;
+  emb_bwd_rank_kernel<KeyT, IdxT, OWN><<<dim3((unsigned)blocks), dim3(kRankThreads), lds, s>>>(
+      (const IdxT *)ids, sorted_id, sorted_pos, n, (int)n_quads, shift, num_weights, padding_idx, (int)rank_blocks,
+      fill_dst, fill_vecs);
+  return launch_status();
 }
 
 // lanes per vector of the position sum: enough that a lane walks at most ~16 rows of the batch
@@ -1215,17 +1231,11 @@ int sort_launch(const void *ids, char *ws, const BwdLayout &L, int64_t n, int64_
   const int64_t n_quads = ceil_div(n, (int64_t)4);
   if ((size_t)n_quads * 4 * sizeof(KeyT) <= kRankMaxKeyBytes) {
     // a short list: one launch ranks every key against all others
-    const int64_t rank_blocks = ceil_div(n_quads * 4, (int64_t)kRankOwn);
-    const int64_t fill_blocks = ceil_div(fill_vecs, (int64_t)kFillVecsRank);
-    const int64_t blocks = rank_blocks + fill_blocks;
-    if (blocks == 0) return CS_OK;
-    const size_t lds = (size_t)n_quads * 4 * sizeof(KeyT) + kRankPartBytes;
-    const int st = allow_rank_lds<KeyT, IdxT>(kRankMaxKeyBytes + kRankPartBytes);
-    if (st != CS_OK) return st;
-    emb_bwd_rank_kernel<KeyT, IdxT><<<dim3((unsigned)blocks), dim3(kRankThreads), lds, s>>>(
-        (const IdxT *)ids, sorted_id, sorted_pos, n, (int)n_quads, L.shift, num_weights, padding_idx,
-        (int)rank_blocks, fill_dst, fill_vecs);
-    return launch_status();
+    return n_quads * 4 <= kRankFewKeys && fill_vecs <= kRankFewFill
+               ? rank_launch<KeyT, IdxT, 16>(ids, sorted_id, sorted_pos, n, n_quads, L.shift, num_weights, padding_idx,
+                                             fill_dst, fill_vecs, s)
+               : rank_launch<KeyT, IdxT, 32>(ids, sorted_id, sorted_pos, n, n_quads, L.shift, num_weights, padding_idx,
+                                             fill_dst, fill_vecs, s);
   }
   // whole fill workgroups to the sort launch, the remainder to the merge launch
   const int64_t sort_fill_blocks = ceil_div(fill_vecs, (int64_t)kFillVecsSort) * CS_EMB_FILL_SORT_PCT / 100;

@@ -1,6 +1,7 @@
 """Embedding backward with the position table, where its launches divide the work: the position sums move from the
 reduce launch to the finish launch beyond 256 windows of 32 entries, the finish launch deals columns to workgroups of
-256, and its probe for a segment's end takes 256 windows a round."""
+256, and its probe for a segment's end takes 256 windows a round.  And the ranking of short lists, which has 16 or
+32 keys to a workgroup by their number and by the size of the table."""
 import pytest
 import torch
 
@@ -50,3 +51,17 @@ def test_positions_and_table(B, T, C, hot, dtype):
             ok |= ulp_distance(got, want.to(dtype)) <= 1
         assert ok.all()
     assert torch.equal(ops.embedding_backward_positions(dout.cuda()), dwpe)
+
+
+@pytest.mark.parametrize("n", [15, 17, 4095, 4096, 4097])
+@pytest.mark.parametrize("V", [40, 60000])  # tables on either side of 32 MB at 192 columns fp32
+def test_short_lists(n, V):
+    from core_scheduler_amd import ops
+
+    C = 192
+    ids = torch.randint(-1, V + 1, (n,), generator=gen(6))  # some out of range
+    dout = torch.randint(-8, 9, (n, C), generator=gen(7)).float()  # whole numbers: every order gives the same sums
+    want = torch.zeros(V, C)
+    keep = (ids >= 0) & (ids < V) & (ids != 5)
+    want.index_add_(0, ids[keep], dout[keep])
+    assert torch.equal(ops.embedding_backward(dout.cuda(), ids.cuda(), V, padding_idx=5).cpu(), want)

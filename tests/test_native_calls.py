@@ -1,0 +1,98 @@
+"""The native forms of the calls of ops.py (csrc/host/src/calls.cpp): the same results as the Python bodies, and every
+call that is not the plain case is left to them."""
+import pytest
+import torch
+
+from core_scheduler_amd import ops
+
+NATIVE = [n for n in vars(ops) if n.startswith("_") and n[1:] in dir(ops._calls) and not n.startswith("__")]
+
+
+class Sub(torch.Tensor):
+    pass
+
+
+def test_every_native_form_is_built_and_used():
+    assert sorted(n[1:] for n in NATIVE) == sorted(n for n in dir(ops._calls) if not n.startswith("_"))
+
+
+def test_what_is_not_plain_is_left_alone():
+    x, ids = torch.zeros(4, 8), torch.zeros(4, dtype=torch.int64)  # on the CPU
+    c = ops._calls
+    for out in (c.gelu_forward(x, "none"), c.gelu_forward(None, "none"), c.gelu_forward(x), c.gelu_backward(x, x, 3),
+                c.layernorm_forward(x, x, None, 1e-5, None), c.embedding_forward(x, ids),
+                c.embedding_backward(x, ids, 10, -1, False), c.embedding_backward_fused(x, ids, 10),
+                c.fused_classifier(x, ids, None, -100, "mean", 1.0, True, None, None)):
+        assert out is NotImplemented
+
+
+def _calls(dt):
+    g = torch.Generator(device="cuda").manual_seed(3)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda").to(dt)
+    x, res, dy = r(2, 33, 72), r(2, 33, 72), r(2, 33, 72)
+    pt = dt if dt == torch.float64 else torch.float32
+    gamma, beta = r(72).to(pt) + 1, r(72).to(pt)
+    ids = torch.randint(0, 50, (2, 33), generator=g, device="cuda")
+    w, p = r(50, 72), r(40, 72)
+    logits, t = r(66, 72), torch.randint(0, 70, (66,), generator=g, device="cuda")
+    mean, rstd = ops.layernorm_forward(x, gamma, beta)[1:]
+    cw = torch.rand(70, generator=g, device="cuda")
+
+    def chain():
+        c = ops.LayerNormBackwardChain()
+        a = c.backward(dy, x, mean, rstd, gamma)
+        b = c.backward(res, x, mean, rstd, gamma, dresidual=a[0])
+        c.flush()
+        return a + b
+
+    return [lambda: ops.gelu_forward(x, "tanh"), lambda: ops.gelu_forward(x[:0]), lambda: ops.gelu_backward(dy, x),
+            lambda: ops.layernorm_forward(x, gamma), lambda: ops.layernorm_forward(x, gamma, beta, 1e-3, torch.float32),
+            lambda: ops.layernorm_forward(x, gamma, beta, 1), lambda: ops.add_layernorm_forward(x, res, gamma, beta),
+            lambda: ops.layernorm_backward(dy, x, mean, rstd, gamma),
+            lambda: ops.layernorm_backward(dy, x, mean, rstd, gamma, dresidual=res),
+            lambda: ops.layernorm_backward(dy, x, mean, rstd, gamma, need_dbeta=False), chain,
+            lambda: ops.embedding_forward(w, ids), lambda: ops.embedding_forward(w, ids.int()[0, 0]),
+            lambda: ops.embedding_forward_add(w, p, ids), lambda: ops.embedding_backward(dy, ids, 50, padding_idx=4),
+            lambda: ops.embedding_backward(dy, ids, 50, scale_grad_by_freq=True),
+            lambda: ops.embedding_backward_fused(dy, ids, 50), lambda: ops.fused_classifier(logits, t, 70, reduction="sum"),
+            lambda: ops.fused_classifier(logits, t, 70, class_weight=cw, dlogits_dtype=torch.float32),
+            lambda: ops.fused_classifier(logits, t, want_dlogits=False, reduction="none", dloss=2),
+            lambda: ops.gelu_forward(torch.nn.Parameter(x)), lambda: ops.gelu_forward(x.as_subclass(Sub))]
+
+
+def _raises(dt):
+    x, gamma = torch.zeros(4, 16, device="cuda", dtype=dt), torch.ones(16, device="cuda")
+    ids = torch.zeros(4, dtype=torch.int64, device="cuda")
+    return [lambda: ops.gelu_forward(x, "sigmoid"), lambda: ops.gelu_forward(x.t()), lambda: ops.gelu_forward(x.int()),
+            lambda: ops.gelu_backward(x, x[:2]), lambda: ops.layernorm_forward(x, gamma[:8]),
+            lambda: ops.layernorm_forward(x.cpu(), gamma), lambda: ops.add_layernorm_forward(x, x[:2], gamma),
+            lambda: ops.layernorm_backward(x, x, gamma, gamma, gamma, dresidual=x[:2]),
+            lambda: ops.embedding_forward(x, ids.float()), lambda: ops.embedding_forward_add(x, x[:, :8], ids[None]),
+            lambda: ops.embedding_backward(x, ids, 0), lambda: ops.fused_classifier(x, ids.int()),
+            lambda: ops.fused_classifier(x, ids, 17), lambda: ops.fused_classifier(x, ids, reduction="max")]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float64])
+def test_same_results_and_refusals(dt, monkeypatch):
+    def outcomes(calls):
+        out = []
+        for call in calls:
+            try:
+                r = call()
+                out.append([t if t is None else (type(t), t.dtype, t.stride(), t.cpu()) for t in
+                            (r if isinstance(r, tuple) else (r,))])
+            except Exception as e:
+                out.append((type(e), str(e)))
+        return out
+
+    native = outcomes(_calls(dt)), outcomes(_raises(dt))
+    with torch.inference_mode():
+        assert ops.gelu_forward(torch.ones(8, device="cuda")).is_inference()
+    for n in NATIVE:
+        monkeypatch.setattr(ops, n, lambda *args: NotImplemented)
+    plain = outcomes(_calls(dt)), outcomes(_raises(dt))
+    for a, b in zip(native[0], plain[0]):
+        assert len(a) == len(b) and all((p is None and q is None) or (p[:3] == q[:3] and torch.equal(p[3], q[3]))
+                                        if not isinstance(p, (type, str)) else p == q for p, q in zip(a, b)), (a, b)
+    assert native[1] == plain[1] and all(isinstance(r, tuple) for r in native[1]), native[1]

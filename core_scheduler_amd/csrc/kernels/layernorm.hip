@@ -446,6 +446,58 @@ __device__ __forceinline__ void ln_finalize_pending(const LnPending &pend, int b
                                       sub, tid);
 }
 
+// The column sums of few rows, straight from dy and x: they need the saved statistics but not the row sums of
+// the backward pass, so workgroups of the row kernel's own launch take them, and neither partial rows nor a
+// second launch (4 us behind the first, and 2.8 us of host time) are needed.  One tile = 32 columns of dgamma
+// and dbeta: thread (cx, ry) of 32 x 16 stands in for partial rows ry, ry+16, ... of RPP rows each, as the row
+// kernel and the finalize step would have left and added them, bit for bit.  All loads of a partial row are
+// requested before the first use.  sub: 2 x 16 x 32 floats of LDS.
+template <typename TDY, typename TX, typename TP, int RPP>
+__device__ __forceinline__ void ln_columns_direct(const TDY *__restrict__ dy, const TX *__restrict__ x,
+                                                  const float *__restrict__ mean, const float *__restrict__ rstd,
+                                                  const LnPending &side, int64_t rows, int tile, int C, float *sub,
+                                                  int tid) {
+  const int cx = tid % kLnFinCols, ry = tid / kLnFinCols;
+  const int col = tile * kLnFinCols + cx;
+  const int64_t at = col < C ? col : C - 1;
+  float sg = 0.f, sb = 0.f;
+  for (int p = ry; p < side.nparts; p += kLnFinRows) {
+    TDY d[RPP];
+    TX v[RPP];
+    float mu[RPP], rs[RPP];
+#pragma unroll
+    for (int w = 0; w < RPP; ++w) {
+      const int64_t row = (int64_t)p * RPP + w;
+      const int64_t rowc = row < rows ? row : rows - 1;
+      d[w] = dy[rowc * C + at];
+      v[w] = x[rowc * C + at];
+      mu[w] = mean[rowc];
+      rs[w] = rstd[rowc];
+    }
+    float pg = 0.f, pb = 0.f;
+#pragma unroll
+    for (int w = 0; w < RPP; ++w) {
+      const float dv = (int64_t)p * RPP + w < rows ? to_acc(d[w]) : 0.f;
+      const float xh = (to_acc(v[w]) - mu[w]) * rs[w];
+      pg += __builtin_fmaf(dv, xh, 0.f);
+      pb += dv;
+    }
+    sg += pg;
+    sb += pb;
+  }
+  sub[ry * kLnFinCols + cx] = sg;
+  sub[(kLnFinRows + ry) * kLnFinCols + cx] = sb;
+  __syncthreads();
+  TP *out = (TP *)(ry == 0 ? side.dgamma : side.dbeta);
+  if (ry < 2 && col < C && out != nullptr) {
+    float t = 0.f;
+#pragma unroll
+    for (int r = 0; r < kLnFinRows; ++r) t += sub[(ry * kLnFinRows + r) * kLnFinCols + cx];
+    if (side.accumulate) t += to_acc(out[col]);
+    out[col] = from_acc<TP>(t);
+  }
+}
+
 // ----------------------------------------------------------- fast backward
 // One wave per row, the row (dy and x) in registers, gamma and the per-column partial sums in
 // registers for all rows a wave visits (rows gw, gw + n_waves, ...).  No software prefetch:
@@ -458,8 +510,9 @@ __device__ __forceinline__ void ln_finalize_pending(const LnPending &pend, int b
 // matters because at 16-bit storage this kernel is as close to its VALU limit as to HBM's.
 // HAS_DRES: dx_out = dx + dresidual, the gradient add that follows LayerNorm::backward on the
 // residual stream; dx is rounded to its type first, then the sum, as two kernels would.
+// DIRECT: the launch's first workgroups take the column sums of this very call from its rows (ln_columns_direct).
 template <typename TDY, typename TX, typename TDX, typename TP, int VPL, int WPE, bool HAS_DX,
-          bool HAS_DP, bool HAS_DRES>
+          bool HAS_DP, bool HAS_DRES, bool DIRECT = false>
 __global__ __launch_bounds__(kLnBwdThreads, WPE) void ln_bwd_rows_kernel(
     const TDY *__restrict__ dy, const TX *__restrict__ x, const float *__restrict__ mean,
     const float *__restrict__ rstd, const TP *__restrict__ gamma, TDX *dx,
@@ -468,7 +521,11 @@ __global__ __launch_bounds__(kLnBwdThreads, WPE) void ln_bwd_rows_kernel(
   constexpr int VN = Vec16<TX>::n;
   extern __shared__ float lds[];  // [waves per block][C], at least 16 x 32 floats with pending sums
   if ((int)blockIdx.x < pend.blocks) {
-    ln_finalize_pending<TP>(pend, blockIdx.x, C, VN, lds, threadIdx.x);
+    if constexpr (DIRECT) {
+      ln_columns_direct<TDY, TX, TP, kLnBwdThreads / kWave>(dy, x, mean, rstd, pend, rows, blockIdx.x, C, lds, threadIdx.x);
+    } else {
+      ln_finalize_pending<TP>(pend, blockIdx.x, C, VN, lds, threadIdx.x);
+    }
     return;
   }
   const int bid = blockIdx.x - pend.blocks;
@@ -634,7 +691,7 @@ __device__ __forceinline__ void zero_strip_unless(Strip<T, VN, VPL> &r, bool row
 // limit as to the memory's); takes VPL * 2 * VN more registers.
 template <typename TDY, typename TX, typename TDX, typename TP, int THREADS, int LPR, int VPL, int WPE, bool PF,
           bool KEEP,
-          bool HAS_DX, bool HAS_DP, bool HAS_DRES>
+          bool HAS_DX, bool HAS_DP, bool HAS_DRES, bool DIRECT>
 __global__ __launch_bounds__(THREADS, WPE) void ln_bwd_kernel(
     const TDY *__restrict__ dy, const TX *__restrict__ x, const float *__restrict__ mean,
     const float *__restrict__ rstd, const TP *__restrict__ gamma, TDX *dx /* may be dres */,
@@ -643,7 +700,11 @@ __global__ __launch_bounds__(THREADS, WPE) void ln_bwd_kernel(
   constexpr int RPW = kWave / LPR;  // rows a wave works on side by side
   extern __shared__ float lds[];    // [RPW * waves per block][C], at least 16 x 32 floats
   if ((int)blockIdx.x < pend.blocks) {
-    ln_finalize_pending<TP, THREADS>(pend, blockIdx.x, C, VN, lds, threadIdx.x);
+    if constexpr (DIRECT) {
+      ln_columns_direct<TDY, TX, TP, RPW * THREADS / kWave>(dy, x, mean, rstd, pend, rows, blockIdx.x, C, lds, threadIdx.x);
+    } else {
+      ln_finalize_pending<TP, THREADS>(pend, blockIdx.x, C, VN, lds, threadIdx.x);
+    }
     return;
   }
   const int bid = blockIdx.x - pend.blocks, nblocks = gridDim.x - pend.blocks;
@@ -1775,6 +1836,16 @@ BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, bool want_d
   return b;
 }
 
+// Rows few enough that the column sums are taken straight from them (ln_columns_direct): up to 16 partial rows'
+// worth a thread makes one trip to memory, and up to 512 rows the one launch is the shorter way.  Kernels of a
+// backward call, us, two launches / one, with dresidual: bf16 [77,768] 9.0 / 4.2, [256,768] 9.5 / 4.6, [512,768]
+// 9.7 / 6.6, [1024,768] 10.0 / 10.3; [512,64] 7.0 / 5.7, [512,512] 7.3 / 7.0, [512,1024] 8.7 / 7.2, [512,1600]
+// 11.3 / 7.3, [1024,1024] 9.1 / 12.0; fp32 [512,384] 8.8 / 6.2, [1024,384] 9.0 / 9.8.
+constexpr int64_t kDirectRows = 512;
+bool direct_sums(const BwdPlan &p, int64_t rows) {
+  return (p.kind == kBwdHalf1 || p.kind == kBwdHalf3 || p.kind == kBwdRows) && rows <= kDirectRows;
+}
+
 // Column order inside a partial row, as the `vn` of ln_finalize_tile: every row kernel leaves column
 // idx*vn + k at position k*(C/vn) + idx.
 int partial_vn(int x_dtype) { return 16 / (int)dtype_size(x_dtype); }
@@ -1838,12 +1909,12 @@ int allow_lds(K kernel, size_t bytes, size_t most, std::atomic<bool> *done) {
 }
 
 template <typename TDY, typename TX, typename TDX, typename TP, int THREADS, int LPR, int VPL, int WPE, bool PF,
-          bool KEEP, bool HAS_DX, bool HAS_DP, bool HAS_DRES>
+          bool KEEP, bool HAS_DX, bool HAS_DP, bool HAS_DRES, bool DIRECT = false>
 int launch_bwd_kernel(const void *dy, const void *x, const void *mean, const void *rstd, const void *gamma,
                       void *dx, void *workspace, int64_t rows, int64_t C, const void *dres, const LnPending &pend,
                       int blocks, size_t lds, hipStream_t s) {
   static std::atomic<bool> lds_allowed[64];
-  auto kernel = ln_bwd_kernel<TDY, TX, TDX, TP, THREADS, LPR, VPL, WPE, PF, KEEP, HAS_DX, HAS_DP, HAS_DRES>;
+  auto kernel = ln_bwd_kernel<TDY, TX, TDX, TP, THREADS, LPR, VPL, WPE, PF, KEEP, HAS_DX, HAS_DP, HAS_DRES, DIRECT>;
   // the fold of the widest row this instantiation takes: [rows side by side x waves][C] floats
   constexpr size_t kMostLds = (size_t)THREADS * VPL * Vec16<TX>::n * sizeof(float);
   const int st = allow_lds(kernel, lds, kMostLds, lds_allowed);
@@ -1902,6 +1973,44 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
           pend = LnPending{pending.partial, pending.dgamma, pending.dbeta, (int)pending.nparts,
                            pending.accumulate, 2 * (int)ceil_div(C, (int64_t)kLnFinCols)};
         }
+      }
+      // Few rows: the sums straight from the rows, in this launch
+      if (direct_sums(plan, rows) && phase == kBwdWhole && want_dp && dx && pend.blocks == 0) {
+        const LnPending side{nullptr, dgamma, dbeta, blocks, accumulate, (int)ceil_div(C, (int64_t)kLnFinCols)};
+        const size_t lds = (size_t)2 * kLnFinRows * kLnFinCols * sizeof(float);
+        const dim3 grid((unsigned)(blocks + side.blocks)), block((unsigned)plan.threads);
+        int st = CS_OK;
+#define CS_LN_DIRECT(HALF_VPL, VPL, HAS_DRES)                                                                           \
+  if (HALF_VPL != 0) {                                                                                                  \
+    st = launch_bwd_kernel<TDY, TX, TDX, TP, kLnBwdThreads, 32, HALF_VPL ? HALF_VPL : 1, 2, false, CS_LN_PAIR_KEEP, true, \
+                           false, HAS_DRES, true>(dy, x, mean, rstd, gamma, dx, workspace, rows, C, dres, side, blocks, \
+                                                  lds, s);                                                              \
+  } else {                                                                                                              \
+    ln_bwd_rows_kernel<TDY, TX, TDX, TP, VPL, 2, true, false, HAS_DRES, true><<<grid, block, lds, s>>>(                 \
+        (const TDY *)dy, (const TX *)x, (const float *)mean, (const float *)rstd, (const TP *)gamma, (TDX *)dx,         \
+        (float *)workspace, rows, (int)C, (const TDX *)dres, side);                                                     \
+    st = launch_status();                                                                                               \
+  }
+#define CS_LN_DIRECT2(HALF_VPL, VPL)      \
+  if (dres) {                             \
+    CS_LN_DIRECT(HALF_VPL, VPL, true)     \
+  } else {                                \
+    CS_LN_DIRECT(HALF_VPL, VPL, false)    \
+  }
+        if (plan.kind == kBwdHalf1) {
+          CS_LN_DIRECT2(1, 1)
+        } else if (plan.kind == kBwdHalf3) {
+          CS_LN_DIRECT2(3, 1)
+        } else if (plan.vpl == 1) {
+          CS_LN_DIRECT2(0, 1)
+        } else if (plan.vpl == 2) {
+          CS_LN_DIRECT2(0, 2)
+        } else {
+          CS_LN_DIRECT2(0, 4)
+        }
+#undef CS_LN_DIRECT2
+#undef CS_LN_DIRECT
+        return st;
       }
       size_t lds = want_dp ? plan.fold_lds : 0;
       const size_t pend_lds = (size_t)kLnFinRows * kLnFinCols * sizeof(float);

@@ -82,6 +82,7 @@ SIGNATURES = {
     ),
     "cs_layernorm_backward_workspace_bytes": (c_size_t, [c_int64, c_int64]),
     "cs_layernorm_backward_partial_rows": (c_int64, [c_int64, c_int64, c_int]),
+    "cs_layernorm_backward_one_launch": (c_int, [c_int64, c_int64, c_int]),
     "cs_layernorm_backward_rows": (
         c_int,
         [c_void_p] * 8 + [c_size_t, c_int64, c_int64] + [c_int] * 4 + [c_void_p],

@@ -117,6 +117,8 @@ at::Tensor workspace(size_t bytes, const at::Tensor &like) {
 void *ptr(const at::Tensor &t) { return t.data_ptr(); }
 void *ptr(const at::Tensor *t) { return t ? t->data_ptr() : nullptr; }
 
+bool aligned16(const at::Tensor &t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+
 PyObject *wrap(const at::Tensor &t) {
   if (!t.defined()) Py_RETURN_NONE;
   return THPVariable_Wrap(t);
@@ -264,7 +266,8 @@ PyObject *layernorm_backward(Args a) {
 
 // One call of a LayerNormBackwardChain that adds up what the call before it left, if any, in its own launch.
 // dy, x, mean, rstd, gamma, dresidual, dx_dtype, pending partials, pending dgamma, pending dbeta, pending accumulate;
-// the pending sums are of x's width and type.  Returns (dx, dgamma, dbeta, partials).
+// the pending sums are of x's width and type.  Returns (dx, dgamma, dbeta, partials), partials None where the sums
+// were taken at once.
 PyObject *layernorm_backward_chained(Args a) {
   const at::Tensor &dy = a.tensor(0), &x = a.tensor(1), &mean = a.tensor(2), &rstd = a.tensor(3), &gamma = a.tensor(4);
   const at::Tensor *dres = a.optional(5);
@@ -277,18 +280,30 @@ PyObject *layernorm_backward_chained(Args a) {
   const int cg = dtype_code(gamma.scalar_type());
   const int64_t n = cs_layernorm_backward_partial_rows(ln.rows, ln.C, cx);
   need(n > 0);
+  const bool at_once = cs_layernorm_backward_one_launch(ln.rows, ln.C, cx) && aligned16(dy) && aligned16(x) &&
+                       aligned16(gamma) && (!dres || aligned16(*dres));
+  need(!at_once || !pend);  // the earlier sums first, in a launch of their own
   at::Tensor dx, dgamma, dbeta, partials;
   const int code = unlocked(a.device, [&](void *s) {
     dx = empty(x.sizes(), out, x);
     dgamma = empty({ln.C}, gamma.scalar_type(), x);
     dbeta = empty({ln.C}, gamma.scalar_type(), x);
+    if (at_once) {
+      const size_t bytes = cs_layernorm_backward_workspace_bytes(ln.rows, ln.C);
+      const at::Tensor ws = workspace(bytes, x);
+      if (dres)
+        return cs_layernorm_backward_add(ptr(dy), ptr(x), ptr(mean), ptr(rstd), ptr(gamma), ptr(dres), ptr(dx), ptr(dgamma),
+                                         ptr(dbeta), ptr(ws), bytes, ln.rows, ln.C, cdy, cx, cdx, cg, 0, s);
+      return cs_layernorm_backward(ptr(dy), ptr(x), ptr(mean), ptr(rstd), ptr(gamma), ptr(dx), ptr(dgamma), ptr(dbeta),
+                                   ptr(ws), bytes, ln.rows, ln.C, cdy, cx, cdx, cg, 0, s);
+    }
     partials = empty({n, 2, ln.C}, at::kFloat, x);
     return cs_layernorm_backward_rows_pending(
         ptr(dy), ptr(x), ptr(mean), ptr(rstd), ptr(gamma), ptr(dres), ptr(dx), (float *)ptr(partials),
         (size_t)partials.numel() * 4, (float *)ptr(pend), pend ? pend->size(0) : 0, ptr(pend_dgamma), ptr(pend_dbeta),
         pend_acc ? 1 : 0, ln.rows, ln.C, cdy, cx, cdx, cg, s);
   });
-  if (code != CS_OK) raise_for("cs_layernorm_backward_rows_pending", code);
+  if (code != CS_OK) raise_for(at_once ? "cs_layernorm_backward" : "cs_layernorm_backward_rows_pending", code);
   return tuple(dx, dgamma, dbeta, partials);
 }
 

@@ -661,13 +661,14 @@ struct LnBackwardBody final : Task::Impl {
   }
   // The row pass alone, with the column sums of the previous LayerNorm backward of this stream
   // added up in the same launch; this call's own sums stay partial rows until the next backward
-  // or until somebody needs the gradients.  False when the shape has no such form.
+  // or until somebody needs the gradients.  False when the shape has no such form, or few enough rows that the whole
+  // call is one launch anyway.
   bool chained(const at::Tensor &dy, const at::Tensor &x, const at::Tensor &mean, const at::Tensor &rstd,
                const at::Tensor &g, const at::Tensor &dres, const at::Tensor &dx, const at::Tensor &dg,
                const at::Tensor &db, const bool kernel_accumulates, const int64_t rows, const int64_t C) const {
     const int xt = dtype_of(x.scalar_type()), pt = dtype_of(g.scalar_type());
     const int64_t n = cs_layernorm_backward_partial_rows(rows, C, xt);
-    if (n <= 0) return false;
+    if (n <= 0 || cs_layernorm_backward_one_launch(rows, C, xt)) return false;
     for (const at::Tensor *t : {&dy, &x, &g, &dx, &dres})
       if (t->defined() && reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 != 0) return false;
     std::lock_guard<std::recursive_mutex> lock{LnSums::mutex()};

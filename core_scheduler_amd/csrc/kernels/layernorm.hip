@@ -1846,6 +1846,11 @@ bool direct_sums(const BwdPlan &p, int64_t rows) {
   return (p.kind == kBwdHalf1 || p.kind == kBwdHalf3 || p.kind == kBwdRows) && rows <= kDirectRows;
 }
 
+bool overlap(const void *a, size_t a_bytes, const void *b, size_t b_bytes) {
+  const char *p = (const char *)a, *q = (const char *)b;
+  return p < q + b_bytes && q < p + a_bytes;
+}
+
 // Column order inside a partial row, as the `vn` of ln_finalize_tile: every row kernel leaves column
 // idx*vn + k at position k*(C/vn) + idx.
 int partial_vn(int x_dtype) { return 16 / (int)dtype_size(x_dtype); }
@@ -1975,7 +1980,10 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
         }
       }
       // Few rows: the sums straight from the rows, in this launch
-      if (direct_sums(plan, rows) && phase == kBwdWhole && want_dp && dx && pend.blocks == 0) {
+      // (other workgroups write dx meanwhile: a caller that has it written over an input gets the two launches)
+      if (direct_sums(plan, rows) && phase == kBwdWhole && want_dp && dx && pend.blocks == 0 &&
+          !overlap(dx, (size_t)rows * C * sizeof(TDX), dy, (size_t)rows * C * sizeof(TDY)) &&
+          !overlap(dx, (size_t)rows * C * sizeof(TDX), x, (size_t)rows * C * sizeof(TX))) {
         const LnPending side{nullptr, dgamma, dbeta, blocks, accumulate, (int)ceil_div(C, (int64_t)kLnFinCols)};
         const size_t lds = (size_t)2 * kLnFinRows * kLnFinCols * sizeof(float);
         const dim3 grid((unsigned)(blocks + side.blocks)), block((unsigned)plan.threads);
@@ -2297,6 +2305,11 @@ extern "C" int64_t cs_layernorm_backward_partial_rows(int64_t rows, int64_t C, i
   if (rows <= 0 || C <= 0 || dtype_size(x_dtype) == 0) return 0;
   const BwdPlan b = bwd_plan(rows, C, x_dtype, true);
   return b.two_calls ? b.blocks : 0;
+}
+
+extern "C" int cs_layernorm_backward_one_launch(int64_t rows, int64_t C, int x_dtype) {
+  if (rows <= 0 || C <= 0 || dtype_size(x_dtype) == 0) return 0;
+  return direct_sums(bwd_plan(rows, C, x_dtype, true), rows) ? 1 : 0;
 }
 
 extern "C" int cs_layernorm_backward_rows(const void *dy, const void *x, const void *mean,

@@ -377,7 +377,8 @@ class LayerNormBackwardChain:
 
     `backward` returns (dx, dgamma, dbeta) at once; dgamma / dbeta hold their values once the next
     `backward` of the chain, or `flush`, has run.  The bits are those of `layernorm_backward`.
-    Shapes without partial rows (see `layernorm_backward_rows`) go through `layernorm_backward`.
+    Shapes without partial rows (see `layernorm_backward_rows`) go through `layernorm_backward`, and so do few
+    rows, whose sums that takes in the one launch: [123,768] bf16 with dresidual 6.8 -> 3.7 us per norm.
     """
 
     def __init__(self):
@@ -390,7 +391,8 @@ class LayerNormBackwardChain:
                                               *(pend[:4] if pend else (None, None, None, False)))
             if out is not NotImplemented:
                 dx, dgamma, dbeta, partials = out
-                self._pending = (partials, dgamma, dbeta, False, x.shape[-1], x.dtype, gamma.dtype)
+                if partials is not None:
+                    self._pending = (partials, dgamma, dbeta, False, x.shape[-1], x.dtype, gamma.dtype)
                 return dx, dgamma, dbeta
         dev = _dev(dy, x, mean, rstd, gamma, dgamma, dbeta, dresidual)
         C = x.shape[-1]
@@ -405,7 +407,9 @@ class LayerNormBackwardChain:
                 raise ValueError("dgamma / dbeta must be [C] of the parameter dtype")
         lib = _capi.load()
         n = lib.cs_layernorm_backward_partial_rows(rows, C, _dt(x))
-        if n == 0:
+        at_once = n and lib.cs_layernorm_backward_one_launch(rows, C, _dt(x)) and not any(
+            t.data_ptr() % 16 for t in (dy, x, gamma, dresidual) if t is not None)
+        if n == 0 or at_once:
             self.flush()
             return layernorm_backward(dy, x, mean, rstd, gamma, dgamma=dgamma, dbeta=dbeta, dx_dtype=dx_dtype,
                                       dresidual=dresidual)

@@ -288,6 +288,13 @@ int cs_layernorm_backward_finalize(const void *partials, int64_t partial_rows,
                                    int x_dtype, int param_dtype, int accumulate,
                                    void *stream);
 
+/* 1 where cs_layernorm_backward / _add, asked for dx and the parameter gradients
+ * with every pointer on a 16-byte boundary, is a single launch: few enough rows
+ * that the column sums are taken straight from them.  A sequence of such calls
+ * gains nothing from the split above or the combined form below: the launch of
+ * one with an earlier call's sums takes longer. */
+int cs_layernorm_backward_one_launch(int64_t rows, int64_t C, int x_dtype);
+
 /* cs_layernorm_backward_rows that also does an EARLIER call's
  * cs_layernorm_backward_finalize inside its own launch: a few workgroups ahead
  * of the row work add `pending_partials` (what that earlier rows call left,

@@ -1,5 +1,5 @@
 """LayerNorm backward of up to 512 rows takes its column sums straight from the rows, in one launch; the bits are those
-of the row pass followed by the sum of its partial rows (LayerNormBackwardChain), which more rows take."""
+of the row pass followed by the sum of its partial rows, which more rows take."""
 import pytest
 import torch
 
@@ -22,19 +22,67 @@ def test_bits_of_two_launches(rows, C, dtype):
         x[16, 0] = float("inf")  # the last row is also what missing rows read
     gamma = randn((C,), 4, 0.02, 1.0).cuda()
     _, mean, rstd = ops.layernorm_forward(x, gamma)
+
+    def two_launches(dresidual=None, **acc):
+        dx, partials = ops.layernorm_backward_rows(dy, x, mean, rstd, gamma, dresidual=dresidual)
+        return (dx, *ops.layernorm_backward_finalize(partials, x.dtype, gamma.dtype, **acc))
+
     for dresidual in (None, res):
+        want = two_launches(dresidual)
         chain = ops.LayerNormBackwardChain()
-        want = chain.backward(dy, x, mean, rstd, gamma, dresidual=dresidual)
+        chained = chain.backward(dy, x, mean, rstd, gamma, dresidual=dresidual)
+        assert (chain._pending is None) == (rows <= 512)
         chain.flush()
         got = ops.layernorm_backward(dy, x, mean, rstd, gamma, dresidual=dresidual)
-        for g, w in zip(got, want):
+        for g, w in zip(got + chained, want + want):
             assert torch.equal(torch.nan_to_num(g), torch.nan_to_num(w)) and torch.equal(g.isnan(), w.isnan())
     base = [randn((C,), s).cuda() for s in (5, 6)]
-    chain = ops.LayerNormBackwardChain()
-    want = chain.backward(dy, x, mean, rstd, gamma, dgamma=base[0].clone(), dbeta=base[1].clone())
-    chain.flush()
+    want = two_launches(dgamma=base[0].clone(), dbeta=base[1].clone())
     got = ops.layernorm_backward(dy, x, mean, rstd, gamma, dgamma=base[0].clone(), dbeta=base[1].clone())
     only = ops.layernorm_backward(dy, x, mean, rstd, gamma, need_dgamma=False)
     assert only[1] is None and torch.equal(torch.nan_to_num(only[0]), torch.nan_to_num(want[0]))
     for g, w in zip(got, want):
         assert torch.equal(torch.nan_to_num(g), torch.nan_to_num(w))
+
+
+def test_chain_of_many_and_few_rows():
+    """What many rows left is added up before a call of few rows that accumulates into the same gradients."""
+    from core_scheduler_amd import ops
+
+    gamma = randn((768,), 4, 0.02, 1.0).cuda()
+    calls = []
+    for rows in (600, 40, 1000, 33):
+        x, dy = (randn((rows, 768), s + rows, dtype=torch.bfloat16).cuda() for s in (1, 2))
+        calls.append((dy, x, *ops.layernorm_forward(x, gamma)[1:], gamma))
+    sums = [[torch.zeros(768, device="cuda") for _ in range(2)] for _ in range(2)]
+    chain = ops.LayerNormBackwardChain()
+    for c in calls:
+        chain.backward(*c, dgamma=sums[0][0], dbeta=sums[0][1])
+        ops.layernorm_backward(*c, dgamma=sums[1][0], dbeta=sums[1][1])
+    fresh = [chain.backward(*c) for c in calls]
+    chain.flush()
+    assert all(torch.equal(a, b) for a, b in zip(*sums))
+    for c, f in zip(calls, fresh):
+        assert all(torch.equal(a, b) for a, b in zip(f, ops.layernorm_backward(*c)))
+
+
+def test_dx_over_an_input():
+    """dx written over dy or x (a wave reads its row before it writes it): the bits of separate buffers."""
+    from core_scheduler_amd import _capi, ops
+
+    lib = _capi.load()
+    x, dy = (randn((300, 768), s, dtype=torch.bfloat16).cuda() for s in (1, 2))
+    gamma = randn((768,), 4, 0.02, 1.0).cuda()
+    _, mean, rstd = ops.layernorm_forward(x, gamma)
+    want = ops.layernorm_backward(dy, x, mean, rstd, gamma)
+    n = lib.cs_layernorm_backward_workspace_bytes(300, 768)
+    ws = torch.empty(n, dtype=torch.uint8, device="cuda")
+    for over in (0, 1):
+        ins = [dy.clone(), x.clone()]
+        dg, db = torch.empty_like(gamma), torch.empty_like(gamma)
+        code = lib.cs_layernorm_backward(ins[0].data_ptr(), ins[1].data_ptr(), mean.data_ptr(), rstd.data_ptr(),
+                                         gamma.data_ptr(), ins[over].data_ptr(), dg.data_ptr(), db.data_ptr(), ws.data_ptr(),
+                                         n, 300, 768, _capi.BF16, _capi.BF16, _capi.BF16, _capi.F32, 0,
+                                         torch.cuda.current_stream().cuda_stream)
+        assert code == _capi.OK
+        assert all(torch.equal(a, b) for a, b in zip((ins[over], dg, db), want))

@@ -383,6 +383,117 @@ __global__ __launch_bounds__(kLnThreads) void ln_fwd_rows_kernel(
   }
 }
 
+template <typename T, int VN, int VPL>
+struct Strip {
+  Raw<T, VN> v[VPL];
+};
+// every lane loads (from the last vector of the row again where it has none of its own)
+template <typename T, int VN, int VPL, int LPR>
+__device__ __forceinline__ void load_strip(Strip<T, VN, VPL> &dst, const T *src, int64_t row, int C, int nvec,
+                                           int hl) {
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) {
+    const int idx = hl + LPR * j;
+    dst.v[j] = load_raw<T, VN>(src + row * C + (int64_t)(idx < nvec ? idx : nvec - 1) * VN);
+  }
+}
+template <typename T, int VN, int VPL, int LPR>
+__device__ __forceinline__ void zero_strip_unless(Strip<T, VN, VPL> &r, bool row_ok, int nvec, int hl) {
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) {
+    const bool keep = row_ok && hl + LPR * j < nvec;
+#pragma unroll
+    for (int q = 0; q < VN / Vec16<T>::n; ++q) {
+      u32x4 w = __builtin_bit_cast(u32x4, r.v[j].v[q]);
+      w.x = keep ? w.x : 0u;
+      w.y = keep ? w.y : 0u;
+      w.z = keep ? w.z : 0u;
+      w.w = keep ? w.w : 0u;
+      r.v[j].v[q] = __builtin_bit_cast(Vec16<T>, w);
+    }
+  }
+}
+
+// One step of ln_fwd_rows_kernel per wave, one wave to a workgroup: few rows are spread over the chip, and every load
+// goes out at once (there the loads stand under the lane's condition, which makes each wait for the one before: hidden
+// where a CU has waves enough, a chain of trips to memory where it has one).  The same sums in the same order.
+template <typename TX, typename TY, typename TP, int VPL, bool HAS_RES, int LPR>
+__global__ __launch_bounds__(kWave) void ln_fwd_few_kernel(
+    const TX *x /* sum_out may be x: not restrict */, const TP *__restrict__ gamma, const TP *__restrict__ beta,
+    TY *__restrict__ y, float *__restrict__ mean, float *__restrict__ rstd, int64_t rows, int C,
+    float eps, const TX *res, TX *sum_out) {
+  constexpr int VN = Vec16<TX>::n;
+  static_assert(VPL <= 4, "the sums of longer rows are formed by vector");
+  const int lane = threadIdx.x;
+  const int sub = lane / LPR, hl = lane % LPR;
+  const bool upper = sub != 0;
+  const int64_t row = (int64_t)blockIdx.x * (kWave / LPR) + sub;
+  const bool row_ok = row < rows;
+  const int64_t rowc = row_ok ? row : rows - 1;
+  const int nvec = C / VN;
+  Strip<TX, VN, VPL> cur, rcur;
+  load_strip<TX, VN, VPL, LPR>(cur, x, rowc, C, nvec, hl);
+  if constexpr (HAS_RES) load_strip<TX, VN, VPL, LPR>(rcur, res, rowc, C, nvec, hl);
+  float g[VPL][VN], b[VPL][VN];
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) {
+    const int idx = hl + LPR * j < nvec ? hl + LPR * j : nvec - 1;
+    load_n<TP, VN>(gamma + idx * VN, g[j]);
+  }
+  const TP *bsrc = beta ? beta : gamma;
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) {
+    const int idx = hl + LPR * j < nvec ? hl + LPR * j : nvec - 1;
+    load_n<TP, VN>(bsrc + idx * VN, b[j]);
+  }
+  if constexpr (HAS_RES) {
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) {
+      Vec16<TX> sum;
+#pragma unroll
+      for (int k = 0; k < VN; ++k) sum.e[k] = from_acc<TX>(raw_get<TX, VN>(cur.v[j], k) + raw_get<TX, VN>(rcur.v[j], k));
+      cur.v[j].v[0] = sum;
+      const int idx = hl + LPR * j;
+      if (idx < nvec && row_ok) store16_stream(sum_out + row * C + (int64_t)idx * VN, sum);
+    }
+  }
+  zero_strip_unless<TX, VN, VPL, LPR>(cur, true, nvec, hl);
+  const float inv_c = 1.0f / (float)C;
+  float s = 0.f;
+#pragma unroll
+  for (int j = 0; j < VPL; ++j)
+#pragma unroll
+    for (int k = 0; k < VN; ++k) s += raw_get<TX, VN>(cur.v[j], k);
+  const float mu = row_lanes_sum<LPR>(s, upper) * inv_c;
+  float q = 0.f;
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) {
+    if (hl + LPR * j < nvec) {
+#pragma unroll
+      for (int k = 0; k < VN; ++k) {
+        const float d = raw_get<TX, VN>(cur.v[j], k) - mu;
+        q += d * d;
+      }
+    }
+  }
+  const float rs = 1.0f / sqrtf(row_lanes_sum<LPR>(q, upper) * inv_c + eps);
+  if (!row_ok) return;
+  if (hl == 0) {
+    mean[row] = mu;
+    rstd[row] = rs;
+  }
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) {
+    const int idx = hl + LPR * j;
+    if (idx < nvec) {
+      float o[VN];
+#pragma unroll
+      for (int k = 0; k < VN; ++k) o[k] = (raw_get<TX, VN>(cur.v[j], k) - mu) * rs * g[j][k] + (beta ? b[j][k] : 0.f);
+      store_n<TY, VN>(y + row * C + (int64_t)idx * VN, o);
+    }
+  }
+}
+
 // ------------------------------------------------- column sums of partial rows
 // What a launch of the row kernel may do on the side: the column sums of an EARLIER call's partial
 // rows (written by a launch that is complete when this one starts).  The first `blocks`
@@ -650,37 +761,6 @@ __global__ __launch_bounds__(kLnBwdThreads, WPE) void ln_bwd_rows_kernel(
 // vectors per lane and leaves a quarter of them empty), a wave finishes two rows per round trip to
 // memory, and the same number of waves leaves half as many rows behind them.  The two row sums
 // are reduced per half; the column sums of the halves meet in the LDS fold at the end.
-template <typename T, int VN, int VPL>
-struct Strip {
-  Raw<T, VN> v[VPL];
-};
-// every lane loads (from the last vector of the row again where it has none of its own)
-template <typename T, int VN, int VPL, int LPR>
-__device__ __forceinline__ void load_strip(Strip<T, VN, VPL> &dst, const T *src, int64_t row, int C, int nvec,
-                                           int hl) {
-#pragma unroll
-  for (int j = 0; j < VPL; ++j) {
-    const int idx = hl + LPR * j;
-    dst.v[j] = load_raw<T, VN>(src + row * C + (int64_t)(idx < nvec ? idx : nvec - 1) * VN);
-  }
-}
-template <typename T, int VN, int VPL, int LPR>
-__device__ __forceinline__ void zero_strip_unless(Strip<T, VN, VPL> &r, bool row_ok, int nvec, int hl) {
-#pragma unroll
-  for (int j = 0; j < VPL; ++j) {
-    const bool keep = row_ok && hl + LPR * j < nvec;
-#pragma unroll
-    for (int q = 0; q < VN / Vec16<T>::n; ++q) {
-      u32x4 w = __builtin_bit_cast(u32x4, r.v[j].v[q]);
-      w.x = keep ? w.x : 0u;
-      w.y = keep ? w.y : 0u;
-      w.z = keep ? w.z : 0u;
-      w.w = keep ? w.w : 0u;
-      r.v[j].v[q] = __builtin_bit_cast(Vec16<T>, w);
-    }
-  }
-}
-
 #ifndef CS_LN_PAIR_FOLD
 #define CS_LN_PAIR_FOLD 1
 #endif
@@ -1571,6 +1651,16 @@ BlockPlan block_plan(int64_t rows, int64_t C, int x_dtype, bool backward, bool r
   return p;
 }
 
+// Forward rows that ln_fwd_few_kernel takes: until its waves, one step each, are more than the chip holds at once,
+// which comes the earlier the more vectors a lane loads.  us per call, ln_fwd_rows_kernel / this one: bf16 [77,768] 3.6
+// / 2.9, with the residual 4.2 / 3.1, [1536,768] 5.2 / 4.2, [2048,768] 5.3 / 4.6, [3072,768] 5.6 / 6.3; [512,1024] 5.8 /
+// 3.4, [2048,1024] 6.2 / 4.7, [3072,1024] 6.7 / 6.7; [1024,1600] 5.8 / 4.9, [1536,1600] 6.2 / 6.9; [4096,64] 4.3 / 3.4,
+// without it [4096,512] 4.3 / 4.0, [8192,320] 5.0 / 5.2, [3072,768] 4.5 / 4.3, [4096,768] 4.7 / 4.8.
+bool few_forward_rows(int64_t rows, int vpl, bool halves, bool residual) {
+  const int64_t loads = rows * vpl * (residual ? 2 : 1);
+  return halves ? loads <= 9216 : loads <= 8192 && rows <= 4096;
+}
+
 // Forward of 257 to 512 whole vectors: a wave per row with eight vectors a lane, or several waves per row (the
 // same bits).  The several waves have more loads in flight where there are few rows, and where the residual
 // doubles a row's loads; in between their last step of 512 workgroups is nearly empty.  Wave per row / several
@@ -1597,6 +1687,33 @@ int fwd_typed(const void *x, const void *gamma, const void *beta, void *y, void 
       // slot stays empty
       const int64_t nvec = C / Vec16<TX>::n;
       const int half_vpl = !CS_LN_FWD_HALF ? 0 : nvec <= kHalf ? 1 : (nvec > kWave && nvec <= 3 * kHalf) ? 3 : 0;
+      if (few_forward_rows(rows, half_vpl != 0 ? half_vpl : p.vpl, half_vpl != 0, res != nullptr)) {
+#define CS_LN_FWD_FEW(VPL, HAS_RES, LPR)                                                                              \
+  ln_fwd_few_kernel<TX, TY, TP, VPL, HAS_RES, LPR>                                                                    \
+      <<<dim3((unsigned)ceil_div(rows, (int64_t)(kWave / LPR))), dim3(kWave), 0, s>>>(                                \
+          (const TX *)x, (const TP *)gamma, (const TP *)beta, (TY *)y, (float *)mean, (float *)rstd, rows, (int)C,    \
+          (float)eps, (const TX *)res, (TX *)sum_out)
+#define CS_LN_FWD_FEW2(VPL, LPR)      \
+  if (res) {                          \
+    CS_LN_FWD_FEW(VPL, true, LPR);    \
+  } else {                            \
+    CS_LN_FWD_FEW(VPL, false, LPR);   \
+  }
+        if (half_vpl == 1) {
+          CS_LN_FWD_FEW2(1, kHalf)
+        } else if (half_vpl == 3) {
+          CS_LN_FWD_FEW2(3, kHalf)
+        } else if (p.vpl == 1) {
+          CS_LN_FWD_FEW2(1, kWave)
+        } else if (p.vpl == 2) {
+          CS_LN_FWD_FEW2(2, kWave)
+        } else {
+          CS_LN_FWD_FEW2(4, kWave)
+        }
+#undef CS_LN_FWD_FEW2
+#undef CS_LN_FWD_FEW
+        return launch_status();
+      }
       if (half_vpl != 0) {
         const int groups = res ? (half_vpl == 1 ? CS_LN_ADD_ROWS_H1 : CS_LN_ADD_ROWS_H3)
                                : (half_vpl == 1 ? CS_LN_FWD_ROWS_H1 : CS_LN_FWD_ROWS_H3);

@@ -86,3 +86,30 @@ def test_dx_over_an_input():
                                          torch.cuda.current_stream().cuda_stream)
         assert code == _capi.OK
         assert all(torch.equal(a, b) for a, b in zip((ins[over], dg, db), want))
+
+
+# the plans of the row forward, with rows at the edges of their rule (few_forward_rows)
+@pytest.mark.parametrize("C,dtype,rows", [(8, torch.bfloat16, 9216), (256, torch.float16, 4608), (768, torch.bfloat16, 3072),
+                                          (776, torch.bfloat16, 4096), (512, torch.float16, 4096), (4, torch.float32, 9216),
+                                          (384, torch.float32, 1536), (1024, torch.float32, 2048), (1600, torch.bfloat16, 1024),
+                                          (2048, torch.bfloat16, 2048)])
+def test_forward_bits_of_many_rows(C, dtype, rows):
+    """A short batch is normalised by a wave per row or pair of rows: the bits that a long one's waves give."""
+    from core_scheduler_amd import ops
+
+    many = 9217 + 512
+    x, res = (randn((many, C), s, dtype=dtype).cuda() for s in (1, 2))
+    x[0, 0], x[2, C - 1] = float("inf"), float("nan")
+    gamma, beta = randn((C,), 4, 0.02, 1.0).cuda(), randn((C,), 5).cuda()
+    for b, out in ((beta, None), (None, torch.float32)):
+        want = ops.layernorm_forward(x, gamma, b, out_dtype=out), ops.add_layernorm_forward(x, res, gamma, b, out_dtype=out)
+        for n in (1, 2, 77, rows // 2 + 1, rows, rows + 1):
+            got = (ops.layernorm_forward(x[:n], gamma, b, out_dtype=out),
+                   ops.add_layernorm_forward(x[:n], res[:n], gamma, b, out_dtype=out))
+            for g, w in zip(sum(got, ()), sum(want, ())):
+                assert torch.equal(torch.nan_to_num(g), torch.nan_to_num(w[:n])) and torch.equal(g.isnan(), w[:n].isnan())
+    s = x[:77].clone()  # the sum over x itself
+    got = ops.add_layernorm_forward(s, res[:77], gamma, beta, inplace=True)
+    assert got[0].data_ptr() == s.data_ptr()
+    for g, w in zip(got, ops.add_layernorm_forward(x, res, gamma, beta)):
+        assert torch.equal(torch.nan_to_num(g), torch.nan_to_num(w[:77]))

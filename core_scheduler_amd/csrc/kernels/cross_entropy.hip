@@ -92,6 +92,26 @@ __device__ __forceinline__ void count_rows(const int64_t *__restrict__ targets, 
   }
 }
 
+// The same number for a row kernel of few rows, by every wave for itself: eight targets a lane, all requested at once,
+// and no launch ahead of the rows.  Only the gradient of a mean without class weights asks (see ce_run).
+constexpr int64_t kCountInRows = 8 * kWave;
+__device__ __forceinline__ int rows_that_count(const int *__restrict__ ws_count, const int64_t *__restrict__ targets,
+                                               int64_t N, int64_t V, int64_t ignore_index) {
+  if (ws_count != nullptr) return *ws_count;  // kernel-uniform: a launch ahead has counted
+  const int lane = threadIdx.x & (kWave - 1), n = (int)N;
+  int64_t t[kCountInRows / kWave];
+#pragma unroll
+  for (int u = 0; u < kCountInRows / kWave; ++u) {
+    const int i = u * kWave + lane;
+    t[u] = targets[i < n ? i : n - 1];
+  }
+  int c = 0;
+#pragma unroll
+  for (int u = 0; u < kCountInRows / kWave; ++u)
+    c += __popcll(__ballot(u * kWave + lane < n && target_counts(t[u], V, ignore_index)));
+  return c;
+}
+
 __global__ __launch_bounds__(1024) void ce_count_kernel(const int64_t *__restrict__ targets,
                                                         int64_t N, int64_t V,
                                                         int64_t ignore_index,
@@ -213,6 +233,8 @@ __global__ __launch_bounds__(BLOCK) void ce_rows_kernel(
     return;
   }
 
+  const int n_count =
+      reduction == CS_REDUCTION_MEAN ? rows_that_count(ws_count, targets, gridDim.x, V, ignore_index) : 0;
   Vec16<T> xr[VPT];
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
@@ -268,7 +290,7 @@ __global__ __launch_bounds__(BLOCK) void ce_rows_kernel(
   // accuracy; folding log2(s) and log2(scale) into the exponent instead costs ~1e-6 relative,
   // which the subtraction at the target column amplifies when p is close to 1.
   float scale = dloss;
-  if (reduction == CS_REDUCTION_MEAN) scale = dloss / (float)(*ws_count);
+  if (reduction == CS_REDUCTION_MEAN) scale = dloss / (float)n_count;
   const float factor = scale / s;  // s >= 1: the maximum contributes 2^0
   const int t_vec = (int)(target / VN), t_sub = (int)(target % VN);
   TD *d = dlogits + row * row_stride;
@@ -390,7 +412,8 @@ __global__ __launch_bounds__(1024) void ce_rows_stream_kernel(
 
   float scale0 = dloss;
   if (reduction == CS_REDUCTION_MEAN)
-    scale0 = HAS_W ? dloss / reinterpret_cast<const float *>(ws_count)[1] : dloss / (float)(*ws_count);
+    scale0 = dloss / (HAS_W ? reinterpret_cast<const float *>(ws_count)[1]
+                            : (float)rows_that_count(ws_count, targets, N, V, ignore_index));
   [[maybe_unused]] const float log2_scale0 = __builtin_amdgcn_logf(fabsf(scale0));  // -inf for 0: every output 0
 
   // Workgroups go round the eight XCDs in launch order.  The workgroups of one XCD take
@@ -695,7 +718,8 @@ __global__ __launch_bounds__(1024) void ce_rows_hold_kernel(
 
   float scale0 = dloss;
   if (reduction == CS_REDUCTION_MEAN)
-    scale0 = class_weight ? dloss / reinterpret_cast<const float *>(ws_count)[1] : dloss / (float)(*ws_count);
+    scale0 = dloss / (class_weight ? reinterpret_cast<const float *>(ws_count)[1]
+                                   : (float)rows_that_count(ws_count, targets, N, V, ignore_index));
 
   // neighbouring rows on one XCD, as in the streaming kernel
   int64_t row = (gridDim.x % 8 == 0) ? (int64_t)(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
@@ -1041,7 +1065,8 @@ __global__ __launch_bounds__(BLOCK, 8) void ce_rows_wide_kernel(
   // weight of its target, and the mean is over the sum of those weights
   float scale0 = dloss;
   if (reduction == CS_REDUCTION_MEAN)
-    scale0 = class_weight ? dloss / reinterpret_cast<const float *>(ws_count)[1] : dloss / (float)(*ws_count);
+    scale0 = dloss / (class_weight ? reinterpret_cast<const float *>(ws_count)[1]
+                                   : (float)rows_that_count(ws_count, targets, N, V, ignore_index));
 
   for (int64_t row = blockIdx.x; row < N; row += gridDim.x) {
     const int64_t tgt = targets[row];
@@ -1214,7 +1239,8 @@ __global__ __launch_bounds__(256) void ce_rows_general_kernel(
   if (!dlogits) return;
   U scale = (U)dloss;
   if (reduction == CS_REDUCTION_MEAN)
-    scale = class_weight ? (U)dloss / (U) reinterpret_cast<const float *>(ws_count)[1] : (U)dloss / (U)(*ws_count);
+    scale = (U)dloss / (class_weight ? (U) reinterpret_cast<const float *>(ws_count)[1]
+                                     : (U)rows_that_count(ws_count, targets, gridDim.x, V, ignore_index));
   scale *= wt;
   for (int64_t c = threadIdx.x; c < row_stride; c += 256) {
     U o = 0;
@@ -1503,7 +1529,9 @@ int ce_run(const CeArgs &a, int phases, void *stream) {
   float *rows = a.row_loss ? a.row_loss : reinterpret_cast<float *>(ws + kWsHeader);
   // Only the gradient of a mean needs the count before the rows; otherwise the last launch counts.
   const bool mean_gradient = a.dlogits != nullptr && a.reduction == CS_REDUCTION_MEAN;
-  const bool count_last = phases == (1 | 2 | 4) && !mean_gradient;
+  // Few rows are counted by the row kernel itself (rows_that_count).
+  const bool count_in_rows = mean_gradient && a.class_weight == nullptr && a.N <= kCountInRows;
+  const bool count_last = phases == (1 | 2 | 4) && (!mean_gradient || count_in_rows);
   if ((phases & 1) && !count_last) {
     ce_count_kernel<<<dim3(1), dim3(1024), 0, s>>>(a.targets, a.N, a.V, a.ignore_index, ws_count,
                                                    ws_weight, a.class_weight);
@@ -1512,7 +1540,7 @@ int ce_run(const CeArgs &a, int phases, void *stream) {
   }
   if ((phases & 2) && a.N > 0) {
 #define CS_CALL(T, TD)                                                                      \
-  st = launch_rows<T, TD>(a.logits, a.dlogits, a.targets, rows, ws_count, a.N, a.V,         \
+  st = launch_rows<T, TD>(a.logits, a.dlogits, a.targets, rows, count_last ? nullptr : ws_count, a.N, a.V, \
                           a.row_stride, a.ignore_index,                                     \
                           mean_gradient ? CS_REDUCTION_MEAN : CS_REDUCTION_SUM, a.dloss, a.class_weight, s)
     const bool wide = a.dlogits_dtype != a.dtype;

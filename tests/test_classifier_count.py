@@ -47,3 +47,33 @@ def test_no_row_counts():
     assert torch.isnan(loss) and tw.item() == 0 and (row == 0).all()
     loss, row, d, tw = ops.fused_classifier(x, t, reduction="sum")
     assert loss.item() == 0 and tw.item() == 0 and (d == 0).all()
+
+
+# one width of each row kernel: 64 and 256 lanes, streamed (padded, ragged, 16-bit to fp32), held, two sweeps, general
+@pytest.mark.parametrize("V,stride,dtype,out", [
+    (40, 40, torch.bfloat16, None), (5003, 5008, torch.bfloat16, None), (50257, 50304, torch.bfloat16, None),
+    (50257, 50257, torch.bfloat16, torch.float32), (60000, 60000, torch.float16, None), (60001, 60001, torch.float16, None),
+    (18001, 18001, torch.bfloat16, torch.float32), (1003, 1003, torch.float32, None), (40, 41, torch.float64, None)])
+def test_few_rows_count_themselves(V, stride, dtype, out):
+    """The gradient of a mean of up to 512 rows: the bits of the call whose count is a launch ahead of the rows."""
+    from core_scheduler_amd import _capi, ops
+
+    lib = _capi.load()
+    x = randn((513, stride), 983, std=2.0).to(dtype).cuda()
+    targets = randint(0, V, (513,), 984).cuda()
+    targets[1::5] = -100
+    for N in (1, 2, 63, 64, 65, 300, 512, 513):
+        got = ops.fused_classifier(x[:N], targets[:N], V, dlogits_dtype=out)
+        want = [torch.empty((), device="cuda"), torch.empty(N, device="cuda"),
+                torch.empty(N, stride, dtype=out or dtype, device="cuda"), torch.empty((), device="cuda")]
+        n = lib.cs_fused_classifier_workspace_bytes(N)
+        ws = torch.empty(n, dtype=torch.uint8, device="cuda")
+        for phase in (1, 2, 4):
+            code = lib.cs_fused_classifier_phases(
+                x.data_ptr(), want[2].data_ptr(), targets.data_ptr(), want[1].data_ptr(), want[0].data_ptr(),
+                want[3].data_ptr(), ws.data_ptr(), n, N, V, stride, -100, _capi.REDUCTION_MEAN, 1.0, ops._DTYPES[dtype],
+                ops._DTYPES[out or dtype], phase, torch.cuda.current_stream().cuda_stream)
+            assert code == _capi.OK
+        for g, w in zip(got, want):
+            assert torch.equal(g, w)
+        assert got[3].item() == (targets[:N] >= 0).sum().item()

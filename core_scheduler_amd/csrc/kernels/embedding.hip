@@ -57,11 +57,31 @@ constexpr int kThreads = 256;
 #endif
 constexpr int kFwdUnroll = CS_EMB_FWD_UNROLL;
 
-template <typename T, typename IdxT, bool ADD>
+//
+// UA: a row of any C >= VN columns, anywhere in memory.  Accesses are at element alignment and the last vector of
+// a row is moved back to end with it, so two lanes write its first elements, with the same values.
+// One element per thread and a 64-bit division each before: forward and backward together, see
+// emb_bwd_reduce_ragged_kernel.
+template <typename T, typename IdxT, bool ADD, bool UA>
 __global__ __launch_bounds__(kThreads) void emb_fwd_vec_kernel(
     const T *__restrict__ weight, const T *__restrict__ wpe, const IdxT *__restrict__ ids,
-    T *__restrict__ out, int64_t n_rows, uint32_t nvec, int64_t num_weights, uint32_t T_len) {
+    T *__restrict__ out, int64_t n_rows, int64_t C, uint32_t nvec, int64_t num_weights, uint32_t T_len) {
   constexpr int VN = Vec16<T>::n;
+  auto column = [&](uint32_t vec) {
+    const int64_t c = (int64_t)vec * VN;
+    return !UA || c + VN <= C ? c : C - VN;
+  };
+  auto load = [](const T *p) {
+    if constexpr (UA) return load16_unaligned_stream(p);
+    return load16(p);
+  };
+  auto store = [](T *p, const Vec16<T> &v) {
+    if constexpr (UA) {
+      store16_unaligned_stream(p, v);
+    } else {
+      store16_stream(p, v);
+    }
+  };
   constexpr uint32_t kChunk = kThreads * kFwdUnroll;
   const int64_t total = n_rows * nvec;
   // the workgroup's first row: 32-bit divisions where the whole output has fewer than 2^32
@@ -98,7 +118,7 @@ __global__ __launch_bounds__(kThreads) void emb_fwd_vec_kernel(
       ++drow;
     }
   }
-  const int64_t row_stride = (int64_t)nvec * VN;
+  const int64_t row_stride = UA ? C : (int64_t)nvec * VN;
   if (full) {
     IdxT raw_id[kFwdUnroll];
     Vec16<T> w[kFwdUnroll], p[kFwdUnroll];
@@ -109,7 +129,7 @@ __global__ __launch_bounds__(kThreads) void emb_fwd_vec_kernel(
       for (int u = 0; u < kFwdUnroll; ++u) {
         uint32_t t = t_base + drows[u];  // below 2 T_len + 256: the workgroup spans few rows
         t = t % T_len;
-        p[u] = load16(wpe + (int64_t)t * row_stride + (int64_t)vecs[u] * VN);
+        p[u] = load(wpe + (int64_t)t * row_stride + column(vecs[u]));
       }
     }
     bool ok[kFwdUnroll];
@@ -117,7 +137,7 @@ __global__ __launch_bounds__(kThreads) void emb_fwd_vec_kernel(
     for (int u = 0; u < kFwdUnroll; ++u) {
       const int64_t id = (int64_t)raw_id[u];
       ok[u] = id >= 0 && id < num_weights;
-      w[u] = load16(weight + (ok[u] ? id : 0) * row_stride + (int64_t)vecs[u] * VN);
+      w[u] = load(weight + (ok[u] ? id : 0) * row_stride + column(vecs[u]));
     }
 #pragma unroll
     for (int u = 0; u < kFwdUnroll; ++u) {
@@ -131,7 +151,7 @@ __global__ __launch_bounds__(kThreads) void emb_fwd_vec_kernel(
           r.e[k] = ok[u] ? w[u].e[k] : T{};
         }
       }
-      store16_stream(out + ((row_base + drows[u]) * nvec + vecs[u]) * VN, r);
+      store(out + (row_base + drows[u]) * row_stride + column(vecs[u]), r);
     }
     return;
   }
@@ -145,18 +165,18 @@ __global__ __launch_bounds__(kThreads) void emb_fwd_vec_kernel(
 #pragma unroll
     for (int k = 0; k < VN; ++k) r.e[k] = T{};
     if (ok) {
-      r = load16(weight + id * row_stride + (int64_t)vecs[u] * VN);
+      r = load(weight + id * row_stride + column(vecs[u]));
       if constexpr (ADD) {
-        const Vec16<T> pv = load16(wpe + (row % T_len) * row_stride + (int64_t)vecs[u] * VN);
+        const Vec16<T> pv = load(wpe + (row % T_len) * row_stride + column(vecs[u]));
 #pragma unroll
         for (int k = 0; k < VN; ++k) r.e[k] = from_acc<T>(to_acc(r.e[k]) + to_acc(pv.e[k]));
       }
     }
-    store16_stream(out + (row * nvec + vecs[u]) * VN, r);
+    store(out + row * row_stride + column(vecs[u]), r);
   }
 }
 
-// any C, any alignment
+// rows shorter than a vector
 template <typename T, typename IdxT, bool ADD>
 __global__ __launch_bounds__(kThreads) void emb_fwd_scalar_kernel(
     const T *__restrict__ weight, const T *__restrict__ wpe, const IdxT *__restrict__ ids,
@@ -358,6 +378,16 @@ __device__ __forceinline__ void zero_fill_block(u32x4 *__restrict__ dst, int64_t
   }
 }
 
+// The table's bytes ahead of its first whole vector and behind its last one (fewer than 16 each).
+struct FillEdges {
+  uint16_t *head, *tail;
+  int head_len, tail_len;  // in 2-byte units: every element type is a whole number of them
+};
+__device__ __forceinline__ void zero_edges(const FillEdges &e, int tid) {
+  if (tid < e.head_len) e.head[tid] = 0;
+  if (tid < e.tail_len) e.tail[tid] = 0;
+}
+
 // Launch layout, in block order:
 //   [0, n_tiles)                sort one tile of 1024 keys
 //   + 1                         preset sorted_id to "no id"
@@ -366,7 +396,7 @@ template <typename KeyT, typename IdxT>
 __global__ __launch_bounds__(kTile) void emb_bwd_tile_sort_kernel(
     const IdxT *__restrict__ ids, KeyT *__restrict__ tiles, uint32_t *__restrict__ sorted_id,
     int64_t n, int n_tiles, int shift, int64_t num_weights, int64_t padding_idx,
-    u32x4 *__restrict__ fill_dst, int64_t fill_vecs) {
+    u32x4 *__restrict__ fill_dst, int64_t fill_vecs, FillEdges edges) {
   __shared__ KeyT keys[2][kTile];
   const int tid = threadIdx.x;
   const int64_t blk = blockIdx.x;
@@ -375,6 +405,7 @@ __global__ __launch_bounds__(kTile) void emb_bwd_tile_sort_kernel(
     return;
   }
   if (blk == n_tiles) {
+    zero_edges(edges, tid);
     for (int64_t i = tid; i < n; i += kTile) sorted_id[i] = kNoId;
     return;
   }
@@ -517,13 +548,14 @@ template <typename KeyT, typename IdxT, int kRankOwn>
 __global__ __launch_bounds__(kRankThreads) void emb_bwd_rank_kernel(
     const IdxT *__restrict__ ids, uint32_t *__restrict__ sorted_id,
     uint32_t *__restrict__ sorted_pos, int64_t n, int n_quads, int shift, int64_t num_weights,
-    int64_t padding_idx, int rank_blocks, u32x4 *__restrict__ fill_dst, int64_t fill_vecs) {
+    int64_t padding_idx, int rank_blocks, u32x4 *__restrict__ fill_dst, int64_t fill_vecs, FillEdges edges) {
   constexpr int kRankGroups = kRankThreads / kRankOwn;
   typedef KeyT Quad __attribute__((ext_vector_type(4)));
   extern __shared__ u32x4 rank_lds[];  // the key list and the partial counts
   __shared__ int valid_of_wave[kRankThreads / kWave];
   const int tid = threadIdx.x;
   const int64_t blk = blockIdx.x;
+  if (blk == 0) zero_edges(edges, tid);
   if (blk >= rank_blocks) {
     zero_fill_block<kRankThreads, kFillVecsRank>(fill_dst, fill_vecs, blk - rank_blocks, tid);
     return;
@@ -1040,50 +1072,156 @@ __global__ __launch_bounds__(kTile) void emb_bwd_positions_vec_kernel(const T *_
   positions_block<T, kTile>(dout, dwpe, blockIdx.x, B, TC, accumulate, log2_slices, slices, threadIdx.x);
 }
 
+// Any C, any alignment: a column per lane, workgroup `blk` of `blocks`.
+template <typename T>
+__device__ __forceinline__ void positions_columns(const T *__restrict__ dout, T *__restrict__ dwpe, int64_t B,
+                                                  int64_t TC, int accumulate, int64_t blk, int64_t blocks) {
+  using U = typename Acc<T>::type;
+  for (int64_t f = blk * kThreads + threadIdx.x; f < TC; f += blocks * kThreads) {
+    double a = 0;  // sequential over the batch, so in double like the rows that are not whole vectors
+    for (int64_t b0 = 0; b0 < B; b0 += 8) {
+      T v[8];  // in flight together
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = dout[(b0 + u < B ? b0 + u : B - 1) * TC + f];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (b0 + u < B) a += (double)to_acc(v[u]);
+    }
+    if (accumulate) a += (double)to_acc(dwpe[f]);
+    dwpe[f] = from_acc<T>((U)a);
+  }
+}
 template <typename T>
 __global__ __launch_bounds__(kThreads) void emb_bwd_positions_kernel(const T *__restrict__ dout,
                                                                      T *__restrict__ dwpe,
                                                                      int64_t B, int64_t TC,
                                                                      int accumulate) {
+  positions_columns<T>(dout, dwpe, B, TC, accumulate, blockIdx.x, gridDim.x);
+}
+
+// ------------------------------------- backward: rows that are not whole vectors
+// fp64, and rows that are not whole aligned 16-byte vectors: the same two levels in double, a column per lane.  (The
+// wave-wide loads are contiguous, whatever the alignment; fp32 sums over vectors would round where these do not.)
+// A workgroup adds one window's 64 sorted entries, a wave's worth of ids, for 256 columns; 16 rows are in
+// flight.  Further workgroups of the launch sum the position table.  One workgroup per table row, which walked that row's entries one load at a time, was the path before: a
+// hot row was a chain of thousands of trips to memory.  us per gather + backward, before / now: bf16 8192 Zipf tokens x 301,
+// 50257 rows 650 / 40, uniform 122 / 39; 16384 x 1599 3213 / 86, uniform 245 / 95; 32768 x 769, 100000 rows 6834 / 106,
+// uniform 373 / 110; fp32 16384 x 1599 3489 / 124; 100 tokens x 301 19 / 20 (launches).
+constexpr int kRagWindow = kWave;
+constexpr int kRagThreads = 256;
+constexpr int kRagInFlight = 16;
+
+__device__ __forceinline__ uint32_t lane_value(uint32_t v, int lane) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, lane);
+}
+
+// partial rows as emb_bwd_reduce_kernel leaves them: slot 0 entered over the window's left edge, slot 1 left over the right
+template <typename T>
+__global__ __launch_bounds__(kRagThreads) void emb_bwd_reduce_ragged_kernel(
+    const T *__restrict__ dout, const uint32_t *__restrict__ sorted_id, const uint32_t *__restrict__ sorted_pos,
+    T *__restrict__ dweight, double *__restrict__ partial, int64_t n, int64_t C, int accumulate, int by_freq,
+    unsigned slices, unsigned row_blocks, T *__restrict__ dwpe, int64_t B, int64_t TC) {
   using U = typename Acc<T>::type;
-  for (int64_t f = (int64_t)blockIdx.x * kThreads + threadIdx.x; f < TC;
-       f += (int64_t)gridDim.x * kThreads) {
-    double a = 0;  // sequential over the batch, so in double like the general row kernel
-    for (int64_t b = 0; b < B; ++b) a += (double)to_acc(dout[b * TC + f]);
-    if (accumulate) a += (double)to_acc(dwpe[f]);
-    dwpe[f] = from_acc<T>((U)a);
+  static_assert(kRagThreads == kThreads, "the position sums' workgroups");
+  if (blockIdx.x >= row_blocks) {
+    positions_columns<T>(dout, dwpe, B, TC, accumulate, blockIdx.x - row_blocks, gridDim.x - row_blocks);
+    return;
+  }
+  const int lane = threadIdx.x & (kWave - 1);
+  const int64_t w = blockIdx.x / slices;
+  const int64_t c = (int64_t)(blockIdx.x % slices) * kRagThreads + threadIdx.x;
+  const int64_t cc = c < C ? c : C - 1;
+  const int64_t p0 = w * kRagWindow, p = p0 + lane, last = n - 1;
+  const uint32_t raw_pos = sorted_pos[p < last ? p : last];
+  const uint32_t raw_id = sorted_id[p < last ? p : last];
+  const uint32_t raw_prev = sorted_id[p > 0 ? (p - 1 < last ? p - 1 : last) : 0];
+  const uint32_t next_id = sorted_id[p0 + kRagWindow < last ? p0 + kRagWindow : last];
+  const uint32_t my_id = p < n ? raw_id : kNoId;
+  const uint64_t valid = __ballot(my_id != kNoId);
+  if (valid == 0) return;
+  const int n_valid = __popcll(valid);  // valid entries are a prefix
+  const uint64_t heads = __ballot(my_id != kNoId && (p == 0 || my_id != raw_prev));
+  const bool leaves = n_valid == kRagWindow && p0 + kRagWindow < n && next_id == lane_value(my_id, kWave - 1);
+  const uint32_t my_pos = my_id != kNoId ? raw_pos : 0u;  // an unused entry reads row 0 and is not added
+  double acc = 0;
+  int start = 0;
+  for (int e0 = 0; e0 < n_valid; e0 += kRagInFlight) {
+    T v[kRagInFlight];
+#pragma unroll
+    for (int u = 0; u < kRagInFlight; ++u) v[u] = dout[(int64_t)lane_value(my_pos, e0 + u) * C + cc];
+#pragma unroll
+    for (int u = 0; u < kRagInFlight; ++u) {
+      const int e = e0 + u;
+      if (e >= n_valid) break;  // wave-uniform, as every decision here
+      acc += (double)to_acc(v[u]);
+      const bool at_end = e + 1 == n_valid;
+      if (!at_end && !((heads >> (e + 1)) & 1)) continue;
+      const bool seg_ends = !(at_end && leaves);
+      if (((heads >> start) & 1) && seg_ends) {
+        if (by_freq) acc /= (double)(e + 1 - start);
+        T *dst = dweight + (int64_t)lane_value(my_id, e) * C + cc;
+        if (accumulate) acc += (double)to_acc(*dst);
+        if (c < C) *dst = from_acc<T>((U)acc);
+      } else if (c < C) {
+        partial[(w * 2 + (seg_ends ? 0 : 1)) * C + c] = acc;
+      }
+      acc = 0;
+      start = e + 1;
+    }
   }
 }
 
-// --------------------------------------------- backward: general (slow) path
-// For fp64 and for rows that are not whole aligned 16-byte vectors.  Same
-// sorted order, one workgroup per output row found by binary search.
+// The workgroup of a segment's first window adds its partial rows, as emb_bwd_finish_kernel does.
 template <typename T>
-__global__ __launch_bounds__(kThreads) void emb_bwd_rows_general_kernel(
-    const T *__restrict__ dout, const uint32_t *__restrict__ sorted_id,
-    const uint32_t *__restrict__ sorted_pos, T *__restrict__ dweight, int64_t n, int64_t C,
-    int accumulate, int by_freq) {
+__global__ __launch_bounds__(kRagThreads) void emb_bwd_finish_ragged_kernel(
+    const uint32_t *__restrict__ sorted_id, const double *__restrict__ partial, T *__restrict__ dweight, int64_t n,
+    int64_t C, int accumulate, int by_freq, unsigned slices) {
   using U = typename Acc<T>::type;
-  const uint32_t row = blockIdx.x;
-  // first sorted entry with id >= row (unused tail slots hold kNoId, the maximum)
-  int64_t lo = 0, len = n;
-  while (len > 0) {
-    const int64_t half = len >> 1;
-    const bool go = sorted_id[lo + half] < row;
-    lo = go ? lo + half + 1 : lo;
-    len = go ? len - half - 1 : half;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int64_t w = blockIdx.x / slices;
+  const int64_t c = (int64_t)(blockIdx.x % slices) * kRagThreads + threadIdx.x;
+  const int64_t p0 = w * kRagWindow, next = p0 + kRagWindow;
+  if (next >= n) return;  // nothing after this window
+  const uint32_t id = sorted_id[next - 1], after = sorted_id[next], first = sorted_id[p0];
+  const uint32_t before = sorted_id[p0 > 0 ? p0 - 1 : 0];
+  if (id == kNoId || after != id || (first == id && p0 > 0 && before == id)) return;
+  // lane l probes window base + l: does the segment leave it (its last entry), does it reach it (its first)?
+  int64_t w_end = -1;
+  for (int64_t base = w + 1; w_end < 0; base += kWave) {
+    const int64_t a = (base + lane) * kRagWindow, q = a + kRagWindow - 1;
+    const uint32_t id_a = sorted_id[a < n ? a : n - 1], id_q = sorted_id[q < n ? q : n - 1];
+    const uint64_t stays = __ballot(q >= n || id_q != id), reached = __ballot(a < n && id_a == id);
+    if (stays) {
+      const int at = __ffsll((long long)stays) - 1;
+      w_end = base + at - ((reached >> at) & 1 ? 0 : 1);
+    }
   }
-  // One thread adds a whole segment in order: thousands of sequential fp32 additions for a hot
-  // row drift by ~1e-4 of the terms' scale, so this path, which is not the fast one, adds in double.
-  for (int64_t c = threadIdx.x; c < C; c += kThreads) {
-    double a = 0;
-    int64_t count = 0;
-    for (int64_t p = lo; p < n && sorted_id[p] == row; ++p, ++count)
-      a += (double)to_acc(dout[(int64_t)sorted_pos[p] * C + c]);
-    if (by_freq && count > 0) a /= (double)count;  // scale_grad_by_freq
-    if (accumulate) a += (double)to_acc(dweight[(int64_t)row * C + c]);
-    dweight[(int64_t)row * C + c] = from_acc<T>((U)a);
+  double count = 1;
+  if (by_freq) {
+    const int64_t qa = p0 + lane, qb = w_end * kRagWindow + lane;
+    const uint64_t in_first = __ballot(sorted_id[qa] == id);
+    const uint64_t in_last = __ballot(qb < n && sorted_id[qb < n ? qb : n - 1] == id);
+    count = (double)(__popcll(in_first) + (w_end - w - 1) * kRagWindow + __popcll(in_last));
   }
+  if (c >= C) return;
+  const int64_t rows = w_end - w + 1;
+  double t[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  for (int64_t r0 = 0; r0 < rows; r0 += 8) {
+    double x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int64_t r = r0 + u < rows ? r0 + u : rows - 1;
+      x[u] = partial[((w + r) * 2 + (r < rows - 1 ? 1 : 0)) * C + c];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (r0 + u < rows) t[u] += x[u];
+  }
+  double total = ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+  if (by_freq) total /= count;
+  T *dst = dweight + (int64_t)id * C + c;
+  if (accumulate) total += (double)to_acc(*dst);
+  *dst = from_acc<T>((U)total);
 }
 
 // ---------------------------------------------------------------- workspace
@@ -1114,7 +1252,9 @@ BwdLayout bwd_layout(int64_t n, int64_t C, int64_t num_weights) {
   L.off_sorted_pos = o;
   o = align256(o + (size_t)n * 4);
   L.off_partial = o;
-  o = align256(o + (size_t)L.n_windows * 2 * (size_t)C * sizeof(float));
+  const size_t rows = (size_t)L.n_windows * 2 * sizeof(float);
+  const size_t ragged = (size_t)ceil_div(n, (int64_t)kRagWindow) * 2 * sizeof(double);
+  o = align256(o + (rows > ragged ? rows : ragged) * (size_t)C);
   L.bytes = o;
   return L;
 }
@@ -1123,15 +1263,19 @@ template <typename T, typename IdxT, bool ADD>
 int fwd_launch(const void *weight, const void *wpe, const void *ids, void *out, int64_t n_rows,
                int64_t C, int64_t num_weights, int64_t T_len, hipStream_t s) {
   constexpr int VN = Vec16<T>::n;
+  const int64_t nvec = ceil_div(C, (int64_t)VN);
+  const int64_t vec_blocks = ceil_div(n_rows * nvec, (int64_t)kThreads * kFwdUnroll);
   const bool vec_ok = C % VN == 0 && is_aligned16(weight) && is_aligned16(out) &&
-                      (!ADD || is_aligned16(wpe)) && C / VN <= 0x7fffffff;
+                      (!ADD || is_aligned16(wpe)) && nvec <= 0x7fffffff;
   if (vec_ok) {
-    const int64_t total = n_rows * (C / VN);
-    const int64_t blocks = ceil_div(total, (int64_t)kThreads * kFwdUnroll);
-    if (blocks > 0x7fffffffLL) return CS_ERR_TOO_LARGE;
-    emb_fwd_vec_kernel<T, IdxT, ADD><<<dim3((unsigned)blocks), dim3(kThreads), 0, s>>>(
-        (const T *)weight, (const T *)wpe, (const IdxT *)ids, (T *)out, n_rows, (uint32_t)(C / VN),
-        num_weights, (uint32_t)T_len);
+    if (vec_blocks > 0x7fffffffLL) return CS_ERR_TOO_LARGE;
+    emb_fwd_vec_kernel<T, IdxT, ADD, false><<<dim3((unsigned)vec_blocks), dim3(kThreads), 0, s>>>(
+        (const T *)weight, (const T *)wpe, (const IdxT *)ids, (T *)out, n_rows, C, (uint32_t)nvec, num_weights,
+        (uint32_t)T_len);
+  } else if (C >= VN && nvec <= 0x7fffffff && vec_blocks <= 0x7fffffffLL) {
+    emb_fwd_vec_kernel<T, IdxT, ADD, true><<<dim3((unsigned)vec_blocks), dim3(kThreads), 0, s>>>(
+        (const T *)weight, (const T *)wpe, (const IdxT *)ids, (T *)out, n_rows, C, (uint32_t)nvec, num_weights,
+        (uint32_t)T_len);
   } else {
     int64_t blocks = ceil_div(n_rows * C, (int64_t)kThreads);
     if (blocks > 65536) blocks = 65536;
@@ -1199,10 +1343,14 @@ int allow_dynamic_lds_once(const void *kernel, size_t bytes, std::atomic<bool> *
 }
 template <typename KeyT, typename IdxT, int OWN>
 int rank_launch(const void *ids, uint32_t *sorted_id, uint32_t *sorted_pos, int64_t n, int64_t n_quads, int shift,
-                int64_t num_weights, int64_t padding_idx, u32x4 *fill_dst, int64_t fill_vecs, hipStream_t s) {
+                int64_t num_weights, int64_t padding_idx, u32x4 *fill_dst, int64_t fill_vecs, const FillEdges &edges,
+                hipStream_t s) {
   const int64_t rank_blocks = ceil_div(n_quads * 4, (int64_t)OWN);
-  const int64_t blocks = rank_blocks + ceil_div(fill_vecs, (int64_t)kFillVecsRank);
-  if (blocks == 0) return CS_OK;
+  int64_t blocks = rank_blocks + ceil_div(fill_vecs, (int64_t)kFillVecsRank);
+  if (blocks == 0) {
+    if (edges.head_len + edges.tail_len == 0) return CS_OK;
+    blocks = 1;
+  }
   const size_t lds = (size_t)n_quads * 4 * sizeof(KeyT) + kRankPartBytes;
   static std::atomic<bool> done[64];
   const int st = allow_dynamic_lds_once(reinterpret_cast<const void *>(&emb_bwd_rank_kernel<KeyT, IdxT, OWN>),
@@ -1210,7 +1358,7 @@ int rank_launch(const void *ids, uint32_t *sorted_id, uint32_t *sorted_pos, int6
   if (st != CS_OK) return st;
   emb_bwd_rank_kernel<KeyT, IdxT, OWN><<<dim3((unsigned)blocks), dim3(kRankThreads), lds, s>>>(
       (const IdxT *)ids, sorted_id, sorted_pos, n, (int)n_quads, shift, num_weights, padding_idx, (int)rank_blocks,
-      fill_dst, fill_vecs);
+      fill_dst, fill_vecs, edges);
   return launch_status();
 }
 
@@ -1224,7 +1372,7 @@ int position_slices(int64_t B) {
 // Sort + merge.  Both launches clear their share of fill_dst[0, fill_vecs), on the CUs the sorting leaves idle.
 template <typename KeyT, typename IdxT>
 int sort_launch(const void *ids, char *ws, const BwdLayout &L, int64_t n, int64_t num_weights,
-                int64_t padding_idx, u32x4 *fill_dst, int64_t fill_vecs, hipStream_t s) {
+                int64_t padding_idx, u32x4 *fill_dst, int64_t fill_vecs, const FillEdges &edges, hipStream_t s) {
   KeyT *tiles = reinterpret_cast<KeyT *>(ws + L.off_tiles);
   uint32_t *sorted_id = reinterpret_cast<uint32_t *>(ws + L.off_sorted_id);
   uint32_t *sorted_pos = reinterpret_cast<uint32_t *>(ws + L.off_sorted_pos);
@@ -1233,9 +1381,9 @@ int sort_launch(const void *ids, char *ws, const BwdLayout &L, int64_t n, int64_
     // a short list: one launch ranks every key against all others
     return n_quads * 4 <= kRankFewKeys && fill_vecs <= kRankFewFill
                ? rank_launch<KeyT, IdxT, 16>(ids, sorted_id, sorted_pos, n, n_quads, L.shift, num_weights, padding_idx,
-                                             fill_dst, fill_vecs, s)
+                                             fill_dst, fill_vecs, edges, s)
                : rank_launch<KeyT, IdxT, 32>(ids, sorted_id, sorted_pos, n, n_quads, L.shift, num_weights, padding_idx,
-                                             fill_dst, fill_vecs, s);
+                                             fill_dst, fill_vecs, edges, s);
   }
   // whole fill workgroups to the sort launch, the remainder to the merge launch
   const int64_t sort_fill_blocks = ceil_div(fill_vecs, (int64_t)kFillVecsSort) * CS_EMB_FILL_SORT_PCT / 100;
@@ -1247,7 +1395,7 @@ int sort_launch(const void *ids, char *ws, const BwdLayout &L, int64_t n, int64_
   if (blocks > 0x7fffffffLL || mblocks > 0x7fffffffLL) return CS_ERR_TOO_LARGE;
   emb_bwd_tile_sort_kernel<KeyT, IdxT><<<dim3((unsigned)blocks), dim3(kTile), 0, s>>>(
       (const IdxT *)ids, tiles, sorted_id, n, (int)L.n_tiles, L.shift, num_weights, padding_idx, fill_dst,
-      sort_fill_vecs);
+      sort_fill_vecs, edges);
   int st = launch_status();
   if (st != CS_OK) return st;
   emb_bwd_merge_kernel<KeyT><<<dim3((unsigned)mblocks), dim3(kThreads), 0, s>>>(
@@ -1271,11 +1419,24 @@ int bwd_typed(const void *dout, const void *ids, void *dweight, void *dwpe, char
                       is_aligned16(dweight) && (!dwpe || is_aligned16(dwpe));
   const int64_t TC = T_len * C;
   // `=` semantics on the fast path: the whole table is zeroed, then indexed rows are written
-  u32x4 *fill_dst = vec_ok && !accumulate ? reinterpret_cast<u32x4 *>(dweight) : nullptr;
-  const int64_t fill_vecs = fill_dst ? num_weights * (C / VN) : 0;
+  u32x4 *fill_dst = nullptr;
+  int64_t fill_vecs = 0;
+  FillEdges edges{nullptr, nullptr, 0, 0};
+  if (!accumulate) {
+    char *table = static_cast<char *>(dweight);
+    const int64_t bytes = num_weights * C * (int64_t)sizeof(T);
+    int64_t head = (int64_t)((16 - reinterpret_cast<uintptr_t>(table) % 16) % 16);
+    if (head > bytes) head = bytes;
+    fill_dst = reinterpret_cast<u32x4 *>(table + head);
+    fill_vecs = (bytes - head) / 16;
+    char *tail = table + head + fill_vecs * 16;
+    edges = FillEdges{reinterpret_cast<uint16_t *>(table), reinterpret_cast<uint16_t *>(tail), (int)(head / 2),
+                      (int)((table + bytes - tail) / 2)};
+  }
+  if (!vec_ok && num_weights > 0x7fffffffLL) return CS_ERR_TOO_LARGE;
   int st;
 #define CS_SORT(KeyT, IdxT) \
-  sort_launch<KeyT, IdxT>(ids, ws, L, n, num_weights, padding_idx, fill_dst, fill_vecs, s)
+  sort_launch<KeyT, IdxT>(ids, ws, L, n, num_weights, padding_idx, fill_dst, fill_vecs, edges, s)
   if (L.key64) {
     st = idx_dtype == CS_I64 ? CS_SORT(uint64_t, int64_t) : CS_SORT(uint64_t, int32_t);
   } else {
@@ -1286,15 +1447,20 @@ int bwd_typed(const void *dout, const void *ids, void *dweight, void *dwpe, char
   const uint32_t *sorted_id = reinterpret_cast<const uint32_t *>(ws + L.off_sorted_id);
   const uint32_t *sorted_pos = reinterpret_cast<const uint32_t *>(ws + L.off_sorted_pos);
   if (!vec_ok) {
-    if (num_weights > 0x7fffffffLL) return CS_ERR_TOO_LARGE;
-    emb_bwd_rows_general_kernel<T><<<dim3((unsigned)num_weights), dim3(kThreads), 0, s>>>(
-        (const T *)dout, sorted_id, sorted_pos, (T *)dweight, n, C, accumulate, by_freq);
+    double *partial = reinterpret_cast<double *>(ws + L.off_partial);
+    const int64_t slices = ceil_div(C, (int64_t)kRagThreads);
+    const int64_t row_blocks = ceil_div(n, (int64_t)kRagWindow) * slices;
+    int64_t pos_blocks = dwpe ? ceil_div(TC, (int64_t)kThreads) : 0;
+    if (pos_blocks > 65536) pos_blocks = 65536;
+    if (row_blocks + pos_blocks > 0x7fffffffLL) return CS_ERR_TOO_LARGE;
+    if (row_blocks + pos_blocks == 0) return CS_OK;
+    emb_bwd_reduce_ragged_kernel<T><<<dim3((unsigned)(row_blocks + pos_blocks)), dim3(kRagThreads), 0, s>>>(
+        (const T *)dout, sorted_id, sorted_pos, (T *)dweight, partial, n, C, accumulate, by_freq, (unsigned)slices,
+        (unsigned)row_blocks, (T *)dwpe, B, TC);
     st = launch_status();
-    if (st != CS_OK || !dwpe) return st;
-    int64_t blocks = ceil_div(TC, (int64_t)kThreads);
-    if (blocks > 65536) blocks = 65536;
-    emb_bwd_positions_kernel<T><<<dim3((unsigned)blocks), dim3(kThreads), 0, s>>>(
-        (const T *)dout, (T *)dwpe, B, TC, accumulate);
+    if (st != CS_OK || n <= kRagWindow) return st;  // one window: no segment leaves it
+    emb_bwd_finish_ragged_kernel<T><<<dim3((unsigned)row_blocks), dim3(kRagThreads), 0, s>>>(
+        sorted_id, partial, (T *)dweight, n, C, accumulate, by_freq, (unsigned)slices);
     return launch_status();
   }
   if constexpr (!std::is_same_v<T, double>) {

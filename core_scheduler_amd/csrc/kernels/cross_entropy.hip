@@ -1253,6 +1253,133 @@ __global__ __launch_bounds__(256) void ce_rows_general_kernel(
   }
 }
 
+// The loss alone of few long rows: whole rows leave CUs idle (fewer rows than there are) or half of them to a second
+// round, so a row is split over several workgroups of 256 lanes, which leave a maximum and a sum each for the last
+// launch.  A workgroup's columns are in registers before the first is used, and its sum is a tree.  Rows may start
+// anywhere: vectors count from the 128-byte line a row starts in (counted from the row itself, at element alignment,
+// [1024,50257] bf16 took 30.0 us, [509,50257] 15.7).  Bound by HBM reads where the rows are many, by the two launches
+// otherwise.
+//
+// Per call, us, whole rows / split, bf16: [300,50257] 15.5 / 11.8, [509,50257] 17.3 / 14.6, [1024,50257] 28.1 / 23.0,
+// [600,16399] 15.3 / 11.8, [8,128256] 14.4 / 9.6, [128,128256] 18.1 / 12.3, [1024,128256] 52.5 / 46.4; fp32
+// [300,50257] 20.6 / 15.2, [1024,50257] 42.2 / 36.3.
+constexpr int kSplitThreads = 256;
+constexpr int kMostSplits = 32;
+constexpr int64_t kSplitRows = 1024;  // one row per lane of the last launch at most
+
+template <typename T, int VPT>
+__global__ __launch_bounds__(kSplitThreads) void ce_loss_split_kernel(
+    const T *__restrict__ logits, const int64_t *__restrict__ targets, float2 *__restrict__ parts,
+    float *__restrict__ target_logits, int64_t N, int64_t V, int64_t row_stride, int64_t ignore_index, int span,
+    unsigned splits) {
+  constexpr int VN = Vec16<T>::n;
+  constexpr int kWaves = kSplitThreads / kWave;
+  __shared__ float2 red[kWaves];
+  const int tid = threadIdx.x;
+  const int64_t row = blockIdx.x / splits;
+  const int sp = (int)(blockIdx.x % splits);
+  const int64_t tgt = targets[row];
+  if (!target_counts(tgt, V, ignore_index)) return;  // the last launch reads nothing of this row
+  const T *x = logits + row * row_stride;
+  // Columns [lo, hi), in vectors that count from the line the row starts in.  A lane's vectors past them are the last one
+  // again; the array's last one, which may not lie whole inside it, is moved back to end with the array.
+  const int iV = (int)V, off = (int)((row * row_stride) & (kLineElems<T> - 1));
+  const int lo = sp * span - off, hi = lo + span < iV ? lo + span : iV;
+  int last = hi > lo ? lo + (hi - lo - 1) / VN * VN : 0;
+  if (row == N - 1 && last > (int)row_stride - VN) last = (int)row_stride - VN;
+  Vec16<T> v[VPT];
+#pragma unroll
+  for (int j = 0; j < VPT; ++j) {
+    const int c = lo + (tid + kSplitThreads * j) * VN;
+    v[j] = load16_unaligned_stream(x + (c < last ? c : last));
+  }
+  if (sp == 0 && tid == 0) target_logits[row] = to_acc(x[tgt]);
+  float m = -INFINITY;
+#pragma unroll
+  for (int j = 0; j < VPT; ++j) {
+    const int c = lo + (tid + kSplitThreads * j) * VN;
+    if (c < 0 || c + VN > hi) {
+      const int at = c < last ? c : last, from = c > 0 ? c : 0;
+#pragma unroll
+      for (int k = 0; k < VN; ++k)
+        if (at + k < from || at + k >= hi) v[j].e[k] = from_acc<T>(-INFINITY);
+    }
+#pragma unroll
+    for (int k = 0; k < VN; ++k) m = fmaxf(m, to_acc(v[j].e[k]));
+  }
+  const float m2 = wave_reduce(m, MaxOp{}) * kLog2e;
+  const float ref = m2 == -INFINITY ? 0.f : m2;  // nothing finite: every term is 0, or the NaN that was met
+  float part[VPT];
+#pragma unroll
+  for (int j = 0; j < VPT; ++j) {
+    float e[VN];
+#pragma unroll
+    for (int k = 0; k < VN; ++k) e[k] = __builtin_amdgcn_exp2f(__builtin_fmaf(to_acc(v[j].e[k]), kLog2e, -ref));
+#pragma unroll
+    for (int w = VN / 2; w > 0; w /= 2)
+#pragma unroll
+      for (int k = 0; k < w; ++k) e[k] += e[k + w];
+    part[j] = e[0];
+  }
+#pragma unroll
+  for (int w = 1; w < VPT; w *= 2)
+#pragma unroll
+    for (int j = 0; j + w < VPT; j += 2 * w) part[j] += part[j + w];
+  const float sum = wave_reduce(part[0], SumOp{});
+  if ((tid & (kWave - 1)) == 0) red[tid >> 6] = float2{m2, sum};
+  lds_barrier();
+  if (tid == 0) {
+    float bm = red[0].x, bs = 0.f;
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) bm = fmaxf(bm, red[w].x);
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w)
+      bs += red[w].x == -INFINITY ? red[w].y : red[w].y * __builtin_amdgcn_exp2f(red[w].x - bm);
+    parts[(int64_t)row * splits + sp] = float2{bm, bs};
+  }
+}
+
+// Row losses from the splits, their sum in a fixed order and the count: a row per lane.
+__global__ __launch_bounds__(1024) void ce_loss_combine_kernel(
+    const float2 *__restrict__ parts, const float *__restrict__ target_logits, int splits,
+    float *__restrict__ row_loss, int64_t N, int *__restrict__ ws_count, int reduction, float *__restrict__ loss,
+    float *__restrict__ total_weight, const int64_t *__restrict__ targets, int64_t V, int64_t ignore_index,
+    const float *__restrict__ class_weight) {
+  __shared__ float scratch[16];
+  const int tid = threadIdx.x;
+  const int row = tid < (int)N ? tid : (int)N - 1;
+  const int64_t tgt = targets[row];
+  const float x_t = target_logits[row];
+  const bool counts = tid < (int)N && target_counts(tgt, V, ignore_index);
+  float m2 = -INFINITY, s = 0.f;
+  for (int q0 = 0; q0 < splits; q0 += 8) {
+    float2 p[8];  // in flight together
+#pragma unroll
+    for (int u = 0; u < 8; ++u) p[u] = parts[(int64_t)row * splits + (q0 + u < splits ? q0 + u : splits - 1)];
+    float pm = m2;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) pm = fmaxf(pm, p[u].x);
+    if (m2 != -INFINITY) s *= __builtin_amdgcn_exp2f(m2 - pm);
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (q0 + u < splits) s += p[u].x == -INFINITY ? p[u].y : p[u].y * __builtin_amdgcn_exp2f(p[u].x - pm);
+    m2 = pm;
+  }
+  const float wt = counts && class_weight != nullptr ? class_weight[tgt] : 1.f;
+  const float l = counts ? (__builtin_amdgcn_logf(s) - __builtin_fmaf(x_t, kLog2e, -m2)) * kLn2 * wt : 0.f;
+  if (tid < (int)N) row_loss[row] = l;
+  int c = 0;
+  float total;
+  count_rows(targets, N, V, ignore_index, class_weight, &c, &total);
+  const float sum = block_reduce(l, SumOp{}, 0.f, scratch);
+  if (tid == 0) {
+    *ws_count = c;
+    reinterpret_cast<float *>(ws_count)[1] = total;
+    if (loss) *loss = reduction == CS_REDUCTION_MEAN ? sum / total : sum;
+    if (total_weight) *total_weight = total;
+  }
+}
+
 // CUs of the current device, asked once per device (threads may race to fill a slot: they
 // store the same value).
 int64_t compute_units() {
@@ -1468,9 +1595,18 @@ int launch_rows(const void *logits, void *dlogits, const int64_t *targets, float
 
 using namespace cs_hip;
 
+namespace {
+// what every call takes: the header and a row loss each
+size_t ce_least_workspace(int64_t N) { return kWsHeader + ((size_t)N * sizeof(float) + 255) / 256 * 256; }
+// and behind it the splits of few rows: a target logit and kMostSplits pairs each
+size_t ce_split_workspace(int64_t N) {
+  return N <= kSplitRows ? (size_t)N * (sizeof(float) + kMostSplits * sizeof(float2)) + 256 : 0;
+}
+}  // namespace
+
 extern "C" size_t cs_fused_classifier_workspace_bytes(int64_t N) {
   if (N < 0) return 0;
-  return kWsHeader + ((size_t)N * sizeof(float) + 255) / 256 * 256;
+  return ce_least_workspace(N) + ce_split_workspace(N);
 }
 
 namespace {
@@ -1502,7 +1638,7 @@ int ce_validate(const CeArgs &a) {
     return CS_ERR_UNSUPPORTED;
   if (a.N > 0x7fffffffLL || a.V > 0x7fffffffLL || a.row_stride > 0x7fffffffLL)
     return CS_ERR_TOO_LARGE;
-  if (!a.workspace || a.workspace_bytes < cs_fused_classifier_workspace_bytes(a.N) ||
+  if (!a.workspace || a.workspace_bytes < ce_least_workspace(a.N) ||
       !aligned_to(a.workspace, 256))
     return CS_ERR_WORKSPACE;
   if (a.reduction == CS_REDUCTION_NONE && !a.row_loss) return CS_ERR_INVALID_ARGUMENT;
@@ -1517,6 +1653,60 @@ int ce_validate(const CeArgs &a) {
   return CS_OK;
 }
 
+// vectors of a row, the longest way it may lie to its first line
+int64_t split_vecs(const CeArgs &a) {
+  const int64_t es = (int64_t)dtype_size(a.dtype), line = a.row_stride % (128 / es) != 0 ? 128 / es - 1 : 0;
+  return ceil_div(a.V + line, 16 / es);
+}
+
+// Workgroups per row for the loss alone of few rows, each with at most eight vectors a lane: eight to a CU, four where
+// there are fewer rows than CUs.  0 where whole rows are taken: rows of up to 8192 vectors of which every CU has one
+// ([200,50257] bf16 10.6 us whole, 11.0 split) or more than four (ce_loss_rows_kernel).
+int loss_splits(const CeArgs &a) {
+  if (a.dlogits != nullptr || a.N <= 0 || a.N > kSplitRows || a.dtype == CS_F64) return 0;
+  if (a.workspace_bytes < cs_fused_classifier_workspace_bytes(a.N)) return 0;  // a caller who reckons it without this
+  const int64_t vn = 16 / (int64_t)dtype_size(a.dtype), cus = compute_units();
+  if (a.row_stride / vn <= (a.N <= cus ? 1024 * 8 : 256 * 8) || a.row_stride > (int64_t(1) << 30)) return 0;
+  const int64_t vecs = split_vecs(a), least = ceil_div(vecs, (int64_t)kSplitThreads * 8);
+  if (least > kMostSplits) return 0;
+  int64_t splits = ceil_div((a.N <= cus ? 4 : 8) * cus, a.N);
+  const int64_t most = ceil_div(vecs, (int64_t)kSplitThreads);
+  if (splits > most) splits = most;
+  if (splits > kMostSplits) splits = kMostSplits;
+  return (int)(splits > least ? splits : least);
+}
+
+template <typename T>
+int launch_loss_split(const CeArgs &a, int splits, float *rows, int *ws_count, hipStream_t s) {
+  constexpr int VN = Vec16<T>::n;
+  char *ws = static_cast<char *>(a.workspace) + ce_least_workspace(a.N);
+  float2 *parts = reinterpret_cast<float2 *>(ws);
+  float *target_logits = reinterpret_cast<float *>(parts + a.N * kMostSplits);
+  const int64_t span_vecs = ceil_div(split_vecs(a), (int64_t)splits);
+  const dim3 grid((unsigned)(a.N * splits)), block(kSplitThreads);
+#define CS_CE_SPLIT(VPT)                                                                                              \
+  ce_loss_split_kernel<T, VPT><<<grid, block, 0, s>>>((const T *)a.logits, a.targets, parts, target_logits, a.N, a.V, \
+                                                      a.row_stride, a.ignore_index, (int)(span_vecs * VN),          \
+                                                      (unsigned)splits)
+  switch (ceil_div(span_vecs, (int64_t)kSplitThreads)) {
+    case 1: CS_CE_SPLIT(1); break;
+    case 2: CS_CE_SPLIT(2); break;
+    case 3: CS_CE_SPLIT(3); break;
+    case 4: CS_CE_SPLIT(4); break;
+    case 5: CS_CE_SPLIT(5); break;
+    case 6: CS_CE_SPLIT(6); break;
+    case 7: CS_CE_SPLIT(7); break;
+    default: CS_CE_SPLIT(8); break;
+  }
+#undef CS_CE_SPLIT
+  const int st = launch_status();
+  if (st != CS_OK) return st;
+  ce_loss_combine_kernel<<<dim3(1), dim3(1024), 0, s>>>(
+      parts, target_logits, splits, rows, a.N, ws_count, a.reduction,
+      a.reduction == CS_REDUCTION_NONE ? nullptr : a.loss, a.total_weight, a.targets, a.V, a.ignore_index, a.class_weight);
+  return launch_status();
+}
+
 // phases: 1 = count the rows that are not ignored, 2 = the row pass,
 // 4 = reduce the row losses
 int ce_run(const CeArgs &a, int phases, void *stream) {
@@ -1527,6 +1717,16 @@ int ce_run(const CeArgs &a, int phases, void *stream) {
   int *ws_count = reinterpret_cast<int *>(ws);
   float *ws_weight = reinterpret_cast<float *>(ws) + 1;
   float *rows = a.row_loss ? a.row_loss : reinterpret_cast<float *>(ws + kWsHeader);
+  if (phases == (1 | 2 | 4)) {
+    const int splits = loss_splits(a);
+    if (splits > 0) {
+      switch (a.dtype) {
+        case CS_F32: return launch_loss_split<float>(a, splits, rows, ws_count, s);
+        case CS_F16: return launch_loss_split<f16_t>(a, splits, rows, ws_count, s);
+        case CS_BF16: return launch_loss_split<bf16_t>(a, splits, rows, ws_count, s);
+      }
+    }
+  }
   // Only the gradient of a mean needs the count before the rows; otherwise the last launch counts.
   const bool mean_gradient = a.dlogits != nullptr && a.reduction == CS_REDUCTION_MEAN;
   // Few rows are counted by the row kernel itself (rows_that_count).

@@ -406,7 +406,11 @@ int cs_embedding_backward_positions(const void *dout, void *dwpe, int64_t B,
  * Any row_stride >= V is accepted.  Rows of up to 163840 columns (16 bit) or
  * 81920 (fp32), from 16384 and 8192 on also where the row stride is no multiple
  * of 16 bytes, are read once, with few exceptions; other rows are read twice,
- * the second time from cache.
+ * the second time from cache.  The loss alone of up to 1024 long rows splits
+ * a row over several workgroups, with the workspace that
+ * cs_fused_classifier_workspace_bytes asks for; 256 bytes and a float per row
+ * (rounded up to 256 bytes) are enough for every other call, and for this one
+ * unsplit.
  * ---------------------------------------------------------------------- */
 size_t cs_fused_classifier_workspace_bytes(int64_t N);
 int cs_fused_classifier(const void *logits, void *dlogits,

@@ -609,6 +609,53 @@ __device__ __forceinline__ void ln_columns_direct(const TDY *__restrict__ dy, co
   }
 }
 
+// The same for rows on several waves (ln_bwd_block_kernel), any width and alignment: sums in double, terms as that
+// kernel forms them, so the two differ by roundings of a double.  A tile is 32 columns for 2 x `waves` row lanes, each
+// with 16 rows under way.  sub: 2 x 2 x waves x 32 doubles of LDS.
+constexpr int kLnWideTile = kHalf;
+template <typename TDY, typename TX, typename TP>
+__device__ __forceinline__ void ln_columns_wide(const TDY *__restrict__ dy, const TX *__restrict__ x,
+                                                const float *__restrict__ mean, const float *__restrict__ rstd,
+                                                const LnPending &side, int64_t rows, int tile, int C, double *sub) {
+  constexpr int kInFlight = 16;
+  const int cx = threadIdx.x % kLnWideTile, ry = threadIdx.x / kLnWideTile, lanes = blockDim.x / kLnWideTile;
+  const int col = tile * kLnWideTile + cx;
+  const int64_t at = col < C ? col : C - 1;
+  double sg = 0., sb = 0.;
+  for (int64_t r0 = ry; r0 < rows; r0 += (int64_t)lanes * kInFlight) {
+    TDY d[kInFlight];
+    TX v[kInFlight];
+    float mu[kInFlight], rs[kInFlight];
+#pragma unroll
+    for (int u = 0; u < kInFlight; ++u) {
+      const int64_t r = r0 + (int64_t)u * lanes, rr = r < rows ? r : rows - 1;
+      d[u] = dy[rr * C + at];
+      v[u] = x[rr * C + at];
+      mu[u] = mean[rr];
+      rs[u] = rstd[rr];
+    }
+#pragma unroll
+    for (int u = 0; u < kInFlight; ++u) {
+      const bool live = r0 + (int64_t)u * lanes < rows;
+      // both masked: 0 * inf would leave a NaN in the sums
+      const float xh = live ? (to_acc(v[u]) - mu[u]) * rs[u] : 0.f;
+      const float dv = live ? to_acc(d[u]) : 0.f;
+      sg += (double)(dv * xh);
+      sb += (double)dv;
+    }
+  }
+  sub[ry * kLnWideTile + cx] = sg;
+  sub[(lanes + ry) * kLnWideTile + cx] = sb;
+  __syncthreads();
+  TP *out = (TP *)(ry == 0 ? side.dgamma : side.dbeta);
+  if (ry < 2 && col < C && out != nullptr) {
+    double t = 0.;
+    for (int r = 0; r < lanes; ++r) t += sub[(ry * lanes + r) * kLnWideTile + cx];
+    if (side.accumulate) t += (double)to_acc(out[col]);
+    out[col] = from_acc<TP>((float)t);
+  }
+}
+
 // ----------------------------------------------------------- fast backward
 // One wave per row, the row (dy and x) in registers, gamma and the per-column partial sums in
 // registers for all rows a wave visits (rows gw, gw + n_waves, ...).  No software prefetch:
@@ -1190,23 +1237,33 @@ constexpr bool bwd_block_prefetches() {
   return (HAS_DP ? 4 * E : 0) + E + 2 * row <= (UA ? 60 : 70);
 }
 template <typename TDY, typename TX, typename TDX, typename TP, int VPT, bool HAS_DX, bool HAS_DP, bool HAS_DRES,
-          bool UA>
+          bool UA, bool DIRECT = false>
 __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_bwd_block_kernel(
     const TDY *__restrict__ dy, const TX *__restrict__ x, const float *__restrict__ mean,
     const float *__restrict__ rstd, const TP *__restrict__ gamma, TDX *dx /* may be dres */,
-    void *__restrict__ partial, int wide, int64_t rows, int C, const TDX *dres, int gw, int groups) {
+    void *__restrict__ partial, int wide, int64_t rows, int C, const TDX *dres, int gw, int groups,
+    const LnPending side) {
   constexpr int VN = Vec16<TX>::n;
+  static_assert(!DIRECT || !HAS_DP, "the launch's first workgroups take the column sums");
   constexpr bool PF = bwd_block_prefetches<TDY, TX, TDX, VPT * VN, HAS_DP, HAS_DRES, UA>();
   extern __shared__ double group_sums[];  // [groups][C] for the fold
   __shared__ float red[2][2][kLnBlockMaxWaves];
+  if constexpr (DIRECT) {
+    if ((int)blockIdx.x < side.blocks) {
+      ln_columns_wide<TDY, TX, TP>(dy, x, mean, rstd, side, rows, blockIdx.x, C, group_sums);
+      return;
+    }
+  }
+  const int bid = DIRECT ? (int)blockIdx.x - side.blocks : (int)blockIdx.x;
+  const int nblocks = DIRECT ? (int)gridDim.x - side.blocks : (int)gridDim.x;
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
   const int group = wave / gw, lig = threadIdx.x - group * gw * kWave;
   const bool any_vec = C >= VN;
   const Lanes<VN, VPT, UA> own(C, gw, lig);
   const float inv_c = 1.0f / (float)C;
-  const int64_t stride = (int64_t)gridDim.x * groups;
+  const int64_t stride = (int64_t)nblocks * groups;
   const int64_t steps = (rows + stride - 1) / stride;
-  int64_t row = (int64_t)blockIdx.x * groups + group;
+  int64_t row = (int64_t)bid * groups + group;
 
   struct Row {
     Share<TDY, VN, VPT, UA> dy;
@@ -1906,22 +1963,30 @@ bool block_two_calls(int64_t C, int x_dtype) {
   return C % vn == 0 && C / vn > 4 * kWave && C / vn <= 8 * kWave;
 }
 
+// Rows on several waves, few enough that the column sums are taken straight from them in the launch of dx
+// (ln_columns_wide); the split form's partial rows are fp32, so its widths keep the two launches.  Saved are a launch, and 16 bytes a column of partial row written and read again per workgroup, which was
+// more than the rows themselves.  As long as a row lane of ln_columns_wide has fewer than four rounds of 16 rows, up to
+// 512 rows, 1024 of 1536 columns and more.  us per call with dresidual, two launches / one: bf16 [16,1003] 6.1 / 3.8,
+// [64,4099] 16.7 / 6.2, [128,1909] 9.4 / 4.4, [300,5120] 21.0 / 10.4, [416,7424] 25 / 15, [1024,5120] 25.3 / 23.1,
+// [1536,5120] 29.0 / 31.1; [300,257] 7.9 / 13.8, [300,1003] 10.3 / 10.3; fp32 [512,1909] 14.9 / 9.8, [768,1003] 11.7 /
+// 12.1, [512,8192] 29.5 / 20.5, [1024,7424] 37.1 / 35.3.
+bool direct_wide_rows(const BlockPlan &b, int64_t rows, int64_t C) {
+  return rows <= (C < 1536 ? 512 : 1024) && rows < 64 * 2 * (int64_t)(b.gw * b.groups);
+}
+
 BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, bool want_dx = true) {
   BwdPlan b;
   const FastPlan p = aligned ? fast_plan(C, x_dtype) : FastPlan{};
   if (p.vpl == 0) {
-    // A few rows of up to 512 vectors: the general kernels' two launches are the shorter ones ([16,257] bf16 4.6 us
-    // against 6.5, [64,65] 6.1 / 6.6, [64,1003] 7.0 / 6.9, [64,4099] 10.9 / 12.2; but [128,257] 9.1 / 7.5,
-    // [128,4099] 20.3 / 12.2).
     const bool two_calls = aligned && block_two_calls(C, x_dtype);
-    if (rows <= 64 && !two_calls && C / (16 / (int64_t)dtype_size(x_dtype)) <= 8 * kWave) return b;
     b.block = block_plan(rows, C, x_dtype, true, false);
     if (b.block.vpt == 0) return b;
+    const bool direct = !two_calls && direct_wide_rows(b.block, rows, C);
     // Four fp32 vectors per lane spill up to 60 registers: worth it with rows enough (general / several waves, [16,8200]
     // 14.0 / 18.7 us, [32,12288] 29.5 / 23.0, [4096,16384] 718 / 295; ragged, with the most spills, [300,16383] 75 / 97,
     // [1024,16383] 165 / 140).
     const bool whole = aligned && C % (16 / (int64_t)dtype_size(x_dtype)) == 0;
-    if (b.block.vpt == 4 && rows <= (whole ? 16 : 512)) return b;
+    if (!direct && b.block.vpt == 4 && rows <= (whole ? 16 : 512)) return b;
     b.kind = kBwdBlock;
     b.vpl = b.block.vpt;
     b.threads = b.block.gw * b.block.groups * kWave;
@@ -1961,6 +2026,10 @@ BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, bool want_d
 constexpr int64_t kDirectRows = 512;
 bool direct_sums(const BwdPlan &p, int64_t rows) {
   return (p.kind == kBwdHalf1 || p.kind == kBwdHalf3 || p.kind == kBwdRows) && rows <= kDirectRows;
+}
+
+bool direct_wide_sums(const BwdPlan &p, int64_t rows, int64_t C) {
+  return p.kind == kBwdBlock && !p.two_calls && direct_wide_rows(p.block, rows, C);
 }
 
 bool overlap(const void *a, size_t a_bytes, const void *b, size_t b_bytes) {
@@ -2047,6 +2116,30 @@ int launch_bwd_kernel(const void *dy, const void *x, const void *mean, const voi
   return launch_status();
 }
 
+// dx and, by further workgroups of the launch, the column sums straight from the rows
+template <typename TDY, typename TX, typename TDX, typename TP, int VPT>
+int launch_bwd_block_direct(const void *dy, const void *x, const void *mean, const void *rstd, const void *gamma,
+                            void *dx, int64_t rows, int64_t C, const void *dres, const BlockPlan &b, bool ua,
+                            const LnPending &side, hipStream_t s) {
+  const dim3 grid((unsigned)(b.blocks + side.blocks)), block((unsigned)(b.gw * b.groups * kWave));
+  const size_t lds = (size_t)2 * block.x * sizeof(double);
+#define CS_LN_BLOCK_DIRECT(HAS_DRES, UA)                                                                            \
+  ln_bwd_block_kernel<TDY, TX, TDX, TP, VPT, true, false, HAS_DRES, UA, true><<<grid, block, lds, s>>>(              \
+      (const TDY *)dy, (const TX *)x, (const float *)mean, (const float *)rstd, (const TP *)gamma, (TDX *)dx,       \
+      nullptr, 0, rows, (int)C, (const TDX *)dres, b.gw, b.groups, side)
+  if (dres && ua) {
+    CS_LN_BLOCK_DIRECT(true, true);
+  } else if (dres) {
+    CS_LN_BLOCK_DIRECT(true, false);
+  } else if (ua) {
+    CS_LN_BLOCK_DIRECT(false, true);
+  } else {
+    CS_LN_BLOCK_DIRECT(false, false);
+  }
+#undef CS_LN_BLOCK_DIRECT
+  return launch_status();
+}
+
 template <typename TDY, typename TX, typename TDX, typename TP, int VPT, bool HAS_DX, bool HAS_DP, bool HAS_DRES>
 int launch_bwd_block(const void *dy, const void *x, const void *mean, const void *rstd, const void *gamma, void *dx,
                      void *workspace, int64_t rows, int64_t C, const void *dres, const BwdPlan &plan, bool ua,
@@ -2060,7 +2153,8 @@ int launch_bwd_block(const void *dy, const void *x, const void *mean, const void
   if (st != CS_OK) return st;
   kernel<<<dim3((unsigned)plan.blocks), dim3((unsigned)plan.threads), lds, s>>>(
       (const TDY *)dy, (const TX *)x, (const float *)mean, (const float *)rstd, (const TP *)gamma, (TDX *)dx,
-      workspace, plan.partial_elem == sizeof(double), rows, (int)C, (const TDX *)dres, plan.block.gw, plan.block.groups);
+      workspace, plan.partial_elem == sizeof(double), rows, (int)C, (const TDX *)dres, plan.block.gw, plan.block.groups,
+      LnPending{nullptr, nullptr, nullptr, 0, 0, 0});
   return launch_status();
 }
 
@@ -2076,6 +2170,23 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
   BwdPlan plan = bwd_plan(rows, C, x_dtype, aligned, dx != nullptr);
   if (phase == kBwdRowsOnly && (plan.kind == kBwdNone || !plan.two_calls || std::is_same_v<TX, double>))
     return aligned ? CS_ERR_UNSUPPORTED : CS_ERR_MISALIGNED;
+  const bool dx_apart = !dx || (!overlap(dx, (size_t)rows * C * sizeof(TDX), dy, (size_t)rows * C * sizeof(TDY)) &&
+                        !overlap(dx, (size_t)rows * C * sizeof(TDX), x, (size_t)rows * C * sizeof(TX)));
+  if constexpr (!std::is_same_v<TX, double>) {
+    // Few rows on several waves: the sums straight from the rows, in the launch of dx
+    if (phase == kBwdWhole && want_dp && dx_apart && direct_wide_sums(plan, rows, C)) {
+      BlockPlan b = plan.block;
+      if (!dx) b.blocks = 0;  // the sums alone
+      const bool ua = !aligned || C % Vec16<TX>::n != 0;
+      const LnPending side{nullptr, dgamma, dbeta, 0, accumulate, (int)ceil_div(C, (int64_t)kLnWideTile)};
+#define CS_LN_WIDE(VPT) \
+  return launch_bwd_block_direct<TDY, TX, TDX, TP, VPT>(dy, x, mean, rstd, gamma, dx, rows, C, dres, b, ua, side, s)
+      if (b.vpt == 1) CS_LN_WIDE(1);
+      if (b.vpt == 2) CS_LN_WIDE(2);
+      if constexpr (Vec16<TX>::n == 4) CS_LN_WIDE(4);
+#undef CS_LN_WIDE
+    }
+  }
   const size_t need = want_dp ? (size_t)plan.blocks * 2 * C * plan.partial_elem : 0;
   const bool ws_ok = need == 0 || (workspace != nullptr && workspace_bytes >= need && aligned_to(workspace, plan.partial_elem));
   // a caller may bring no workspace where no sum in two steps was promised: the general kernels
@@ -2098,9 +2209,7 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
       }
       // Few rows: the sums straight from the rows, in this launch
       // (other workgroups write dx meanwhile: a caller that has it written over an input gets the two launches)
-      if (direct_sums(plan, rows) && phase == kBwdWhole && want_dp && dx && pend.blocks == 0 &&
-          !overlap(dx, (size_t)rows * C * sizeof(TDX), dy, (size_t)rows * C * sizeof(TDY)) &&
-          !overlap(dx, (size_t)rows * C * sizeof(TDX), x, (size_t)rows * C * sizeof(TX))) {
+      if (direct_sums(plan, rows) && phase == kBwdWhole && want_dp && dx && dx_apart && pend.blocks == 0) {
         const LnPending side{nullptr, dgamma, dbeta, blocks, accumulate, (int)ceil_div(C, (int64_t)kLnFinCols)};
         const size_t lds = (size_t)2 * kLnFinRows * kLnFinCols * sizeof(float);
         const dim3 grid((unsigned)(blocks + side.blocks)), block((unsigned)plan.threads);

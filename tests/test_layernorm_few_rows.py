@@ -113,3 +113,42 @@ def test_forward_bits_of_many_rows(C, dtype, rows):
     assert got[0].data_ptr() == s.data_ptr()
     for g, w in zip(got, ops.add_layernorm_forward(x, res, gamma, beta)):
         assert torch.equal(torch.nan_to_num(g), torch.nan_to_num(w[:77]))
+
+
+# ragged, wide and unaligned rows: one, two and four vectors a lane, a tile of 32 columns that ends inside, the general kernels' range
+@pytest.mark.parametrize("C,dtype,shift", [(257, torch.bfloat16, 0), (1003, torch.float32, 0), (768, torch.bfloat16, 1),
+                                           (4099, torch.float16, 0), (5120, torch.bfloat16, 0), (9001, torch.float32, 0),
+                                           (3, torch.float32, 0), (2056, torch.float32, 1)])
+@pytest.mark.parametrize("rows", [1, 16, 17, 63, 300, 512, 513, 1024])
+def test_wide_rows_in_one_launch(rows, C, dtype, shift):
+    """dx has the bits it has in a long batch; each column sum is the double sum of its fp32 terms, rounded once."""
+    from core_scheduler_amd import ops
+
+    def put(t):
+        flat = torch.empty(t.numel() + shift, dtype=t.dtype, device="cuda")[shift:]
+        return flat.copy_(t.reshape(-1)).view(t.shape)
+
+    many = 1100
+    x, dy, res = (randn((many, C), s, dtype=dtype) for s in (1, 2, 3))
+    gamma = randn((C,), 4, 0.02, 1.0).cuda()
+    _, mean, rstd = ops.layernorm_forward(put(x), gamma)
+    want = ops.layernorm_backward(put(dy), put(x), mean, rstd, gamma, dresidual=put(res))[0][:rows]
+    m, r = mean[:rows].contiguous(), rstd[:rows].contiguous()
+    args = put(dy[:rows]), put(x[:rows]), m, r, gamma
+    dx, dgamma, dbeta = ops.layernorm_backward(*args, dresidual=put(res[:rows]))
+    assert torch.equal(dx, want)
+    terms_b = dy[:rows].float()
+    terms_g = terms_b * ((x[:rows].float() - m.cpu()[:, None]) * r.cpu()[:, None])
+    base = randn((C,), 5)
+    acc = ops.layernorm_backward(*args, dgamma=base.clone().cuda(), dbeta=base.clone().cuda())
+    for got, again, terms in ((dgamma, acc[1], terms_g), (dbeta, acc[2], terms_b)):
+        exact, size = terms.double().sum(0), terms.double().abs().sum(0)
+        assert ((got.cpu().double() - exact).abs() <= 2.0 ** -24 * exact.abs() + 2.0 ** -40 * size).all()
+        exact, size = exact + base.double(), size + base.double().abs()
+        assert ((again.cpu().double() - exact).abs() <= 2.0 ** -24 * exact.abs() + 2.0 ** -40 * size).all()
+    for mask in (dict(need_dx=False), dict(need_dgamma=False, need_dbeta=False)):  # the bits of the full call
+        part = ops.layernorm_backward(*args, **mask)
+        full = ops.layernorm_backward(*args)
+        assert all(p is None or torch.equal(p, f) for p, f in zip(part, full))
+    only = ops.layernorm_backward(*args, need_dgamma=False)
+    assert only[1] is None and torch.equal(only[2], dbeta)

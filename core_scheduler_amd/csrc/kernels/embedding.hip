@@ -1115,7 +1115,10 @@ __device__ __forceinline__ uint32_t lane_value(uint32_t v, int lane) {
   return (uint32_t)__builtin_amdgcn_readlane((int)v, lane);
 }
 
-// partial rows as emb_bwd_reduce_kernel leaves them: slot 0 entered over the window's left edge, slot 1 left over the right
+// Partial rows as emb_bwd_reduce_kernel leaves them: slot 0 entered over the window's left edge, slot 1 left over the
+// right.  The first window has no slot 0 and the last no slot 1, so they start one row earlier.
+__device__ __forceinline__ int64_t ragged_partial(int64_t w, int slot, int64_t C) { return (2 * w + slot - 1) * C; }
+
 template <typename T>
 __global__ __launch_bounds__(kRagThreads) void emb_bwd_reduce_ragged_kernel(
     const T *__restrict__ dout, const uint32_t *__restrict__ sorted_id, const uint32_t *__restrict__ sorted_pos,
@@ -1163,7 +1166,7 @@ __global__ __launch_bounds__(kRagThreads) void emb_bwd_reduce_ragged_kernel(
         if (accumulate) acc += (double)to_acc(*dst);
         if (c < C) *dst = from_acc<T>((U)acc);
       } else if (c < C) {
-        partial[(w * 2 + (seg_ends ? 0 : 1)) * C + c] = acc;
+        partial[ragged_partial(w, seg_ends ? 0 : 1, C) + c] = acc;
       }
       acc = 0;
       start = e + 1;
@@ -1211,7 +1214,7 @@ __global__ __launch_bounds__(kRagThreads) void emb_bwd_finish_ragged_kernel(
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const int64_t r = r0 + u < rows ? r0 + u : rows - 1;
-      x[u] = partial[((w + r) * 2 + (r < rows - 1 ? 1 : 0)) * C + c];
+      x[u] = partial[ragged_partial(w + r, r < rows - 1 ? 1 : 0, C) + c];
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u)
@@ -1252,9 +1255,9 @@ BwdLayout bwd_layout(int64_t n, int64_t C, int64_t num_weights) {
   L.off_sorted_pos = o;
   o = align256(o + (size_t)n * 4);
   L.off_partial = o;
-  const size_t rows = (size_t)L.n_windows * 2 * sizeof(float);
-  const size_t ragged = (size_t)ceil_div(n, (int64_t)kRagWindow) * 2 * sizeof(double);
-  o = align256(o + (rows > ragged ? rows : ragged) * (size_t)C);
+  // (the doubles of emb_bwd_reduce_ragged_kernel's windows, which are twice as long, fit as well)
+  static_assert(kRagWindow == 2 * kWindow, "2 ceil(n / 64) - 2 rows of doubles are no more than 2 ceil(n / 32) of floats");
+  o = align256(o + (size_t)L.n_windows * 2 * (size_t)C * sizeof(float));
   L.bytes = o;
   return L;
 }

@@ -100,3 +100,20 @@ def test_nothing_beside_the_table_is_written():
         want[lead:lead + V * C] = 0
         want[lead:lead + C] = 2
         assert torch.equal(buf, want)
+
+
+@pytest.mark.parametrize("n", [33, 64, 65, 97, 4129])
+def test_nothing_behind_the_workspace_is_written(n):
+    """The partial rows fit the workspace of a float row per slot of each 32 entries, whatever the remainder."""
+    from core_scheduler_amd import _capi
+
+    lib, V, C = _capi.load(), 3, 301
+    ids, dout = torch.ones(n, dtype=torch.int64, device="cuda"), randn((n, C), 1).cuda()
+    size = lib.cs_embedding_backward_workspace_bytes(n, C, V)
+    assert size <= 4 * 1024 * -(-n // 1024) + 8 * n + 8 * C * -(-n // 32) + 4 * 256
+    ws = torch.full((size + 65536,), 77, dtype=torch.uint8, device="cuda")
+    dw = torch.empty(V, C, device="cuda")
+    code = lib.cs_embedding_backward(dout.data_ptr(), ids.data_ptr(), dw.data_ptr(), ws.data_ptr(), size, n, C, V, -1, _capi.F32,
+                                     _capi.I64, 0, torch.cuda.current_stream().cuda_stream)
+    assert code == _capi.OK and (ws[size:] == 77).all()
+    assert rounded_once(dw[1].cpu(), dout.cpu().double().sum(0), dout.cpu().double().abs().sum(0))

@@ -1236,13 +1236,14 @@ constexpr bool bwd_block_prefetches() {
   const int row = E * (int)(sizeof(TDY) + sizeof(TX) + (HAS_DRES ? sizeof(TDX) : 0)) / 4;
   return (HAS_DP ? 4 * E : 0) + E + 2 * row <= (UA ? 60 : 70);
 }
+struct LnNoSide {};
 template <typename TDY, typename TX, typename TDX, typename TP, int VPT, bool HAS_DX, bool HAS_DP, bool HAS_DRES,
           bool UA, bool DIRECT = false>
 __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_bwd_block_kernel(
     const TDY *__restrict__ dy, const TX *__restrict__ x, const float *__restrict__ mean,
     const float *__restrict__ rstd, const TP *__restrict__ gamma, TDX *dx /* may be dres */,
     void *__restrict__ partial, int wide, int64_t rows, int C, const TDX *dres, int gw, int groups,
-    const LnPending side) {
+    const std::conditional_t<DIRECT, LnPending, LnNoSide> side) {
   constexpr int VN = Vec16<TX>::n;
   static_assert(!DIRECT || !HAS_DP, "the launch's first workgroups take the column sums");
   constexpr bool PF = bwd_block_prefetches<TDY, TX, TDX, VPT * VN, HAS_DP, HAS_DRES, UA>();
@@ -1254,8 +1255,11 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_bwd_block_kernel(
       return;
     }
   }
-  const int bid = DIRECT ? (int)blockIdx.x - side.blocks : (int)blockIdx.x;
-  const int nblocks = DIRECT ? (int)gridDim.x - side.blocks : (int)gridDim.x;
+  unsigned bid = blockIdx.x, nblocks = gridDim.x;
+  if constexpr (DIRECT) {
+    bid -= side.blocks;
+    nblocks -= side.blocks;
+  }
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
   const int group = wave / gw, lig = threadIdx.x - group * gw * kWave;
   const bool any_vec = C >= VN;
@@ -2154,7 +2158,7 @@ int launch_bwd_block(const void *dy, const void *x, const void *mean, const void
   kernel<<<dim3((unsigned)plan.blocks), dim3((unsigned)plan.threads), lds, s>>>(
       (const TDY *)dy, (const TX *)x, (const float *)mean, (const float *)rstd, (const TP *)gamma, (TDX *)dx,
       workspace, plan.partial_elem == sizeof(double), rows, (int)C, (const TDX *)dres, plan.block.gw, plan.block.groups,
-      LnPending{nullptr, nullptr, nullptr, 0, 0, 0});
+      LnNoSide{});
   return launch_status();
 }
 

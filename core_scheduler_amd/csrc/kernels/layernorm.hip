@@ -561,8 +561,8 @@ __device__ __forceinline__ void ln_finalize_pending(const LnPending &pend, int b
 // the backward pass, so workgroups of the row kernel's own launch take them, and neither partial rows nor a
 // second launch (4 us behind the first, and 2.8 us of host time) are needed.  One tile = 32 columns of dgamma
 // and dbeta: thread (cx, ry) of 32 x 16 stands in for partial rows ry, ry+16, ... of RPP rows each, as the row
-// kernel and the finalize step would have left and added them, bit for bit.  All loads of a partial row are
-// requested before the first use.  sub: 2 x 16 x 32 floats of LDS.
+// kernel and the finalize step would have left and added them, bit for bit where x-hat is finite.  All loads of a
+// partial row are requested before the first use.  sub: 2 x 16 x 32 floats of LDS.
 template <typename TDY, typename TX, typename TP, int RPP>
 __device__ __forceinline__ void ln_columns_direct(const TDY *__restrict__ dy, const TX *__restrict__ x,
                                                   const float *__restrict__ mean, const float *__restrict__ rstd,
@@ -588,8 +588,10 @@ __device__ __forceinline__ void ln_columns_direct(const TDY *__restrict__ dy, co
     float pg = 0.f, pb = 0.f;
 #pragma unroll
     for (int w = 0; w < RPP; ++w) {
-      const float dv = (int64_t)p * RPP + w < rows ? to_acc(d[w]) : 0.f;
-      const float xh = (to_acc(v[w]) - mu[w]) * rs[w];
+      const bool live = (int64_t)p * RPP + w < rows;
+      // both masked, as in ln_columns_wide
+      const float xh = live ? (to_acc(v[w]) - mu[w]) * rs[w] : 0.f;
+      const float dv = live ? to_acc(d[w]) : 0.f;
       pg += __builtin_fmaf(dv, xh, 0.f);
       pb += dv;
     }

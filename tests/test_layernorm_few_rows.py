@@ -45,6 +45,26 @@ def test_bits_of_two_launches(rows, C, dtype):
         assert torch.equal(torch.nan_to_num(g), torch.nan_to_num(w))
 
 
+# partial rows of 8 rows (a wave per row) and of 16 (two rows per wave) that are not full, and rows on several waves
+@pytest.mark.parametrize("rows,C,dtype", [(1, 768, torch.bfloat16), (2, 1600, torch.bfloat16), (17, 768, torch.float16),
+                                          (77, 1024, torch.float32), (130, 256, torch.bfloat16), (9, 257, torch.bfloat16)])
+def test_rows_that_do_not_exist_add_nothing(rows, C, dtype):
+    """An infinite x-hat in the last row, which stands in for missing rows: infinite in that column's dgamma, not NaN."""
+    from core_scheduler_amd import ops
+
+    x, dy = (randn((rows, C), s, dtype=dtype).cuda() for s in (1, 2))
+    x[rows - 1, 5] = float("inf")
+    dy[rows - 1, 5] = 2.0
+    mean, rstd = torch.zeros(rows, device="cuda"), torch.ones(rows, device="cuda")  # a caller's own statistics
+    _, dgamma, dbeta = ops.layernorm_backward(dy, x, mean, rstd, torch.ones(C, device="cuda"))
+    assert dgamma[5] == float("inf")
+    terms = dy.double() * x.double()
+    bound = 2.0 ** -24 * rows * terms.abs().sum(0) + 2.0 ** -149  # fp32 terms and sums of `rows` of them
+    others = torch.arange(C, device="cuda") != 5
+    assert ((dgamma.double() - terms.sum(0)).abs() <= bound)[others].all()
+    assert ((dbeta.double() - dy.double().sum(0)).abs() <= 2.0 ** -24 * rows * dy.double().abs().sum(0)).all()
+
+
 def test_chain_of_many_and_few_rows():
     """What many rows left is added up before a call of few rows that accumulates into the same gradients."""
     from core_scheduler_amd import ops

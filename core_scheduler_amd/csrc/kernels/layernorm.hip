@@ -2176,11 +2176,20 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
   BwdPlan plan = bwd_plan(rows, C, x_dtype, aligned, dx != nullptr);
   if (phase == kBwdRowsOnly && (plan.kind == kBwdNone || !plan.two_calls || std::is_same_v<TX, double>))
     return aligned ? CS_ERR_UNSUPPORTED : CS_ERR_MISALIGNED;
-  const bool dx_apart = !dx || (!overlap(dx, (size_t)rows * C * sizeof(TDX), dy, (size_t)rows * C * sizeof(TDY)) &&
-                        !overlap(dx, (size_t)rows * C * sizeof(TDX), x, (size_t)rows * C * sizeof(TX)));
+  // One launch reads the inputs for the sums, and for dx, while other workgroups of it write: a caller that has an
+  // output written over an input gets the two launches
+  const size_t n = (size_t)rows * C, stat = (size_t)rows * sizeof(float), params = (size_t)C * sizeof(TP);
+  const auto clear_of = [&](const void *out, size_t bytes, const void *in, size_t in_bytes) {
+    return out == nullptr || in == nullptr || !overlap(out, bytes, in, in_bytes);
+  };
+  bool apart = clear_of(dx, n * sizeof(TDX), dy, n * sizeof(TDY)) && clear_of(dx, n * sizeof(TDX), x, n * sizeof(TX));
+  for (const void *sum : {(const void *)dgamma, (const void *)dbeta})
+    apart = apart && clear_of(sum, params, dy, n * sizeof(TDY)) && clear_of(sum, params, x, n * sizeof(TX)) &&
+            clear_of(sum, params, mean, stat) && clear_of(sum, params, rstd, stat) && clear_of(sum, params, gamma, params) &&
+            clear_of(sum, params, dres, n * sizeof(TDX));
   if constexpr (!std::is_same_v<TX, double>) {
     // Few rows on several waves: the sums straight from the rows, in the launch of dx
-    if (phase == kBwdWhole && want_dp && dx_apart && direct_wide_sums(plan, rows, C)) {
+    if (phase == kBwdWhole && want_dp && apart && direct_wide_sums(plan, rows, C)) {
       BlockPlan b = plan.block;
       if (!dx) b.blocks = 0;  // the sums alone
       const bool ua = !aligned || C % Vec16<TX>::n != 0;
@@ -2214,8 +2223,7 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
         }
       }
       // Few rows: the sums straight from the rows, in this launch
-      // (other workgroups write dx meanwhile: a caller that has it written over an input gets the two launches)
-      if (direct_sums(plan, rows) && phase == kBwdWhole && want_dp && dx && dx_apart && pend.blocks == 0) {
+      if (direct_sums(plan, rows) && phase == kBwdWhole && want_dp && dx && apart && pend.blocks == 0) {
         const LnPending side{nullptr, dgamma, dbeta, blocks, accumulate, (int)ceil_div(C, (int64_t)kLnFinCols)};
         const size_t lds = (size_t)2 * kLnFinRows * kLnFinCols * sizeof(float);
         const dim3 grid((unsigned)(blocks + side.blocks)), block((unsigned)plan.threads);

@@ -108,6 +108,34 @@ def test_dx_over_an_input():
         assert all(torch.equal(a, b) for a, b in zip((ins[over], dg, db), want))
 
 
+@pytest.mark.parametrize("over,rows,C", [("gamma", 300, 768), ("gamma", 300, 1003), ("mean", 300, 300), ("mean", 301, 301),
+                                         ("rstd", 300, 300), ("rstd", 301, 301)])
+def test_sums_over_an_input(over, rows, C):
+    """A parameter gradient written over an input, which the rows' workgroups read: the bits of separate buffers."""
+    from core_scheduler_amd import _capi, ops
+
+    lib = _capi.load()
+    x, dy = (randn((rows, C), s, dtype=torch.float32).cuda() for s in (1, 2))
+    gamma = randn((C,), 4, 0.02, 1.0).cuda()
+    _, mean, rstd = ops.layernorm_forward(x, gamma)
+    want = ops.layernorm_backward(dy, x, mean, rstd, gamma)
+    n = lib.cs_layernorm_backward_workspace_bytes(rows, C)
+    ws = torch.empty(max(n, 256), dtype=torch.uint8, device="cuda")
+    for which in (0, 1):
+        ins = dict(gamma=gamma.clone(), mean=mean.clone(), rstd=rstd.clone())
+        dx, outs = torch.empty_like(x), [torch.empty_like(gamma) for _ in range(2)]
+        outs[which] = ins[over]
+        code = lib.cs_layernorm_backward(dy.data_ptr(), x.data_ptr(), ins["mean"].data_ptr(), ins["rstd"].data_ptr(),
+                                         ins["gamma"].data_ptr(), dx.data_ptr(), outs[0].data_ptr(), outs[1].data_ptr(),
+                                         ws.data_ptr(), n, rows, C, *[_capi.F32] * 4, 0,
+                                         torch.cuda.current_stream().cuda_stream)
+        assert code == _capi.OK
+        torch.testing.assert_close(dx, want[0], rtol=0, atol=0)
+        for got, w in zip(outs, want[1:]):
+            # the two forms of the several-waves sums differ by roundings of a double
+            assert ((got - w).abs() <= 2.0 ** -23 * w.abs() + 1e-12).all()
+
+
 # the plans of the row forward, with rows at the edges of their rule (few_forward_rows)
 @pytest.mark.parametrize("C,dtype,rows", [(8, torch.bfloat16, 9216), (256, torch.float16, 4608), (768, torch.bfloat16, 3072),
                                           (776, torch.bfloat16, 4096), (512, torch.float16, 4096), (4, torch.float32, 9216),

@@ -2182,7 +2182,8 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
   const auto clear_of = [&](const void *out, size_t bytes, const void *in, size_t in_bytes) {
     return out == nullptr || in == nullptr || !overlap(out, bytes, in, in_bytes);
   };
-  bool apart = clear_of(dx, n * sizeof(TDX), dy, n * sizeof(TDY)) && clear_of(dx, n * sizeof(TDX), x, n * sizeof(TX));
+  const bool dx_apart = clear_of(dx, n * sizeof(TDX), dy, n * sizeof(TDY)) && clear_of(dx, n * sizeof(TDX), x, n * sizeof(TX));
+  bool apart = dx_apart;
   for (const void *sum : {(const void *)dgamma, (const void *)dbeta})
     apart = apart && clear_of(sum, params, dy, n * sizeof(TDY)) && clear_of(sum, params, x, n * sizeof(TX)) &&
             clear_of(sum, params, mean, stat) && clear_of(sum, params, rstd, stat) && clear_of(sum, params, gamma, params) &&
@@ -2361,6 +2362,19 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
   }
   using U = typename Acc<TX>::type;
   if (rows > 0x7fffffffLL) return CS_ERR_TOO_LARGE;
+  const auto sums = [&] {
+    ln_bwd_param_general_kernel<TDY, TX, TP>
+        <<<dim3((unsigned)ceil_div(C, (int64_t)64)), dim3(64, 4), 0, s>>>(
+            (const TDY *)dy, (const TX *)x, (const U *)mean, (const U *)rstd, (TP *)dgamma,
+            (TP *)dbeta, rows, C, accumulate);
+    return launch_status();
+  };
+  // ahead of a dx that is written over what they read; otherwise behind it, as they may be written over gamma
+  const bool sums_first = want_dp && dx && !dx_apart;
+  if (sums_first) {
+    const int st = sums();
+    if (st != CS_OK) return st;
+  }
   if (dx) {
     ln_bwd_dx_general_kernel<TDY, TX, TDX, TP><<<dim3((unsigned)rows), dim3(kLnThreads), 0, s>>>(
         (const TDY *)dy, (const TX *)x, (const U *)mean, (const U *)rstd, (const TP *)gamma,
@@ -2368,14 +2382,7 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
     const int st = launch_status();
     if (st != CS_OK) return st;
   }
-  if (want_dp) {
-    ln_bwd_param_general_kernel<TDY, TX, TP>
-        <<<dim3((unsigned)ceil_div(C, (int64_t)64)), dim3(64, 4), 0, s>>>(
-            (const TDY *)dy, (const TX *)x, (const U *)mean, (const U *)rstd, (TP *)dgamma,
-            (TP *)dbeta, rows, C, accumulate);
-    return launch_status();
-  }
-  return CS_OK;
+  return want_dp && !sums_first ? sums() : CS_OK;
 }
 
 bool wide_ok(int narrow, int other) { return other == narrow || other == CS_F32; }

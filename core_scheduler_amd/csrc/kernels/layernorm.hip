@@ -1953,6 +1953,7 @@ struct BwdPlan {
   size_t fold_lds = 0;    // LDS of the column-sum fold
   size_t partial_elem = sizeof(float);  // bytes of a partial row's element
   bool two_calls = true;  // the partial rows may be added up by a later call (kBwdBlock: see block_two_calls)
+  bool direct = false;    // kBwdBlock: the launch of dx takes the column sums (direct_wide_rows)
   BlockPlan block;
 };
 constexpr int kLnMaxPartialRows = 512;
@@ -1970,29 +1971,53 @@ bool block_two_calls(int64_t C, int x_dtype) {
 }
 
 // Rows on several waves, few enough that the column sums are taken straight from them in the launch of dx
-// (ln_columns_wide); the split form's partial rows are fp32, so its widths keep the two launches.  Saved are a launch, and 16 bytes a column of partial row written and read again per workgroup, which was
-// more than the rows themselves.  As long as a row lane of ln_columns_wide has fewer than four rounds of 16 rows, up to
-// 512 rows, 1024 of 1536 columns and more.  us per call with dresidual, two launches / one: bf16 [16,1003] 6.1 / 3.8,
-// [64,4099] 16.7 / 6.2, [128,1909] 9.4 / 4.4, [300,5120] 21.0 / 10.4, [416,7424] 25 / 15, [1024,5120] 25.3 / 23.1,
-// [1536,5120] 29.0 / 31.1; [300,257] 7.9 / 13.8, [300,1003] 10.3 / 10.3; fp32 [512,1909] 14.9 / 9.8, [768,1003] 11.7 /
-// 12.1, [512,8192] 29.5 / 20.5, [1024,7424] 37.1 / 35.3.
+// (ln_columns_wide); the split form's partial rows are fp32, so its widths keep the two launches.  Saved are a launch,
+// and 16 bytes a column of partial row written and read again per workgroup, which was more than the rows themselves.
+// As long as a row lane of ln_columns_wide has fewer than four rounds of 16 rows, up to 512 rows, 1024 of 1536 columns
+// and more.  us per call with dresidual, two launches / one: bf16 [16,1003] 6.1 / 3.8, [64,4099] 16.7 / 6.2,
+// [128,1909] 9.4 / 4.4, [300,5120] 21.0 / 10.4, [416,7424] 25 / 15, [1024,5120] 25.3 / 23.1, [1536,5120] 29.0 / 31.1;
+// [300,257] 7.9 / 13.8, [300,1003] 10.3 / 10.3; fp32 [512,1909] 14.9 / 9.8, [768,1003] 11.7 / 12.1, [512,8192] 29.5 /
+// 20.5, [1024,7424] 37.1 / 35.3.  The sums alone take that form as well: [300,9001] fp32 25.0 / 12.8.
 bool direct_wide_rows(const BlockPlan &b, int64_t rows, int64_t C) {
   return rows <= (C < 1536 ? 512 : 1024) && rows < 64 * 2 * (int64_t)(b.gw * b.groups);
 }
 
-BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, bool want_dx = true) {
+// What a backward call asks for, as far as its plan depends on it.
+struct BwdWants {
+  bool dx = true, sums = true;
+  // no output lies over an input, and the sums are to be complete when the call is: they may be taken in the launch of dx
+  bool apart = false;
+};
+
+// Ragged, unaligned and wide rows that the general kernels are the shorter way for.  us, several waves per row /
+// general:
+// The sums alone are one launch there, a chain of rows / 4 steps at any width; better as long as a row lane of
+// ln_columns_wide has not 16 rows to load at once: bf16 [16,257] 3.6 / 3.0, [64,257] 4.5 / 4.5, [64,1003] 3.7 / 4.5,
+// [64,4099] 5.9 / 4.6, fp32 [64,1909] 5.6 / 4.4, [64,9001] 7.4 / 4.5, rows shorter than a vector [64,3] 4.3 / 4.1 (but
+// [65,257] 5.8 / 6.6 in two launches).
+// dx alone of a column per lane: bf16 [64,9] 3.8 / 3.1, [64,65] 3.5 / 3.1, [64,193] 3.4 / 3.2, [64,257] 3.5 / 3.4, fp32
+// [8,65] 3.2 / 3.0; rows shorter than a vector 3.2 / 3.1; wider ones [64,4099] bf16 4.6 / 7.8, [16,8200] fp32 4.5 / 12.6.
+// All three where an output lies over an input: bf16 [8,65] 6.5 / 5.1, [16,257] 7.3 / 6.2, [64,65] 7.3 / 8.6, [64,1003]
+// 7.6 / 10.3.  With four fp32 vectors per lane the kernel of several waves spills up to 60 registers: whole [16,8200]
+// 19.2 / 15.7, [16,12288] 21.5 / 20.2, [32,12288] 22.9 / 29.5, ragged [64,9001] 28.5 / 20.7, [300,9001] 51.4 / 46.4,
+// [512,9001] 51.1 / 67.5, [300,16383] 83.5 / 71.5, [512,16383] 81.3 / 90.6.
+bool general_rows(const BwdWants &w, const BlockPlan &b, int64_t rows, int64_t C, int x_dtype, bool aligned) {
+  const int64_t vn = 16 / (int64_t)dtype_size(x_dtype);
+  if (!w.dx) return rows <= 64 && (C < vn || rows < 16 * 2 * (int64_t)(b.gw * b.groups));
+  if (!w.sums) return rows <= 64 && C >= vn && C <= kLnThreads;
+  if (b.vpt == 4) return rows <= (aligned && C % vn == 0 ? 16 : 384);
+  return rows <= 16 && C / vn <= 8 * kWave;
+}
+
+BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, const BwdWants &w = BwdWants{}) {
   BwdPlan b;
   const FastPlan p = aligned ? fast_plan(C, x_dtype) : FastPlan{};
   if (p.vpl == 0) {
     const bool two_calls = aligned && block_two_calls(C, x_dtype);
     b.block = block_plan(rows, C, x_dtype, true, false);
     if (b.block.vpt == 0) return b;
-    const bool direct = !two_calls && direct_wide_rows(b.block, rows, C);
-    // Four fp32 vectors per lane spill up to 60 registers: worth it with rows enough (general / several waves, [16,8200]
-    // 14.0 / 18.7 us, [32,12288] 29.5 / 23.0, [4096,16384] 718 / 295; ragged, with the most spills, [300,16383] 75 / 97,
-    // [1024,16383] 165 / 140).
-    const bool whole = aligned && C % (16 / (int64_t)dtype_size(x_dtype)) == 0;
-    if (!direct && b.block.vpt == 4 && rows <= (whole ? 16 : 512)) return b;
+    const bool direct = w.sums && w.apart && !two_calls && direct_wide_rows(b.block, rows, C);
+    if (!two_calls && !(direct && w.dx) && general_rows(w, b.block, rows, C, x_dtype, aligned)) return b;
     b.kind = kBwdBlock;
     b.vpl = b.block.vpt;
     b.threads = b.block.gw * b.block.groups * kWave;
@@ -2000,6 +2025,7 @@ BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, bool want_d
     b.fold_lds = (size_t)b.block.groups * C * sizeof(double);
     b.two_calls = two_calls;
     b.partial_elem = b.two_calls ? sizeof(float) : sizeof(double);
+    b.direct = direct;
     return b;
   }
   const int vn = 16 / (int)dtype_size(x_dtype);
@@ -2011,7 +2037,7 @@ BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, bool want_d
     const int64_t n = ceil_div((rows + 1) / 2, (int64_t)(kLnBwdThreads / kWave));
     b.blocks = (int)(n < CS_LN_PAIR_MAX_BLOCKS ? n : CS_LN_PAIR_MAX_BLOCKS);
     b.fold_lds = (size_t)(kLnBwdThreads / kWave) * 2 * C * sizeof(float);
-  } else if (p.vpl == 4 && (CS_LN_W4_NEW == 2 || (CS_LN_W4_NEW == 1 && !want_dx))) {
+  } else if (p.vpl == 4 && (CS_LN_W4_NEW == 2 || (CS_LN_W4_NEW == 1 && !w.dx))) {
     b.kind = kBwdWave4;
     b.threads = CS_LN_W4_THREADS;
     b.blocks = ln_blocks(rows, 1, kLnBwdMaxBlocks, b.threads);
@@ -2032,10 +2058,6 @@ BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, bool want_d
 constexpr int64_t kDirectRows = 512;
 bool direct_sums(const BwdPlan &p, int64_t rows) {
   return (p.kind == kBwdHalf1 || p.kind == kBwdHalf3 || p.kind == kBwdRows) && rows <= kDirectRows;
-}
-
-bool direct_wide_sums(const BwdPlan &p, int64_t rows, int64_t C) {
-  return p.kind == kBwdBlock && !p.two_calls && direct_wide_rows(p.block, rows, C);
 }
 
 bool overlap(const void *a, size_t a_bytes, const void *b, size_t b_bytes) {
@@ -2173,9 +2195,6 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
   // rows only: the partial rows are the product, the parameter gradients come from a later
   // cs_layernorm_backward_finalize (or ride in a later call's launch)
   const bool want_dp = phase == kBwdRowsOnly || dgamma != nullptr || dbeta != nullptr;
-  BwdPlan plan = bwd_plan(rows, C, x_dtype, aligned, dx != nullptr);
-  if (phase == kBwdRowsOnly && (plan.kind == kBwdNone || !plan.two_calls || std::is_same_v<TX, double>))
-    return aligned ? CS_ERR_UNSUPPORTED : CS_ERR_MISALIGNED;
   // One launch reads the inputs for the sums, and for dx, while other workgroups of it write: a caller that has an
   // output written over an input gets the two launches
   const size_t n = (size_t)rows * C, stat = (size_t)rows * sizeof(float), params = (size_t)C * sizeof(TP);
@@ -2188,9 +2207,12 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
     apart = apart && clear_of(sum, params, dy, n * sizeof(TDY)) && clear_of(sum, params, x, n * sizeof(TX)) &&
             clear_of(sum, params, mean, stat) && clear_of(sum, params, rstd, stat) && clear_of(sum, params, gamma, params) &&
             clear_of(sum, params, dres, n * sizeof(TDX));
+  BwdPlan plan = bwd_plan(rows, C, x_dtype, aligned, {dx != nullptr, want_dp, apart && phase == kBwdWhole});
+  if (phase == kBwdRowsOnly && (plan.kind == kBwdNone || !plan.two_calls || std::is_same_v<TX, double>))
+    return aligned ? CS_ERR_UNSUPPORTED : CS_ERR_MISALIGNED;
   if constexpr (!std::is_same_v<TX, double>) {
     // Few rows on several waves: the sums straight from the rows, in the launch of dx
-    if (phase == kBwdWhole && want_dp && apart && direct_wide_sums(plan, rows, C)) {
+    if (plan.direct) {
       BlockPlan b = plan.block;
       if (!dx) b.blocks = 0;  // the sums alone
       const bool ua = !aligned || C % Vec16<TX>::n != 0;

@@ -5,8 +5,6 @@ import torch
 
 from _util import randn
 
-pytestmark = pytest.mark.gpu
-
 
 def kernels(call):
     """Names of the LayerNorm kernels of a call, in order."""
@@ -29,6 +27,7 @@ def operands(rows, C, dtype):
     return (dy, x, *ops.layernorm_forward(x, gamma)[1:], gamma)
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows,C,dtype", [
     (64, 257, torch.bfloat16), (64, 4099, torch.bfloat16), (16, 9001, torch.float32),
     (65, 257, torch.bfloat16), (384, 9001, torch.float32)])
@@ -39,6 +38,7 @@ def test_all_three_are_one_launch(rows, C, dtype):
     assert kernels(lambda: ops.layernorm_backward(*args)) == ["ln_bwd_block"]
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows,C,dtype,want", [
     (16, 257, torch.bfloat16, "param_general"), (64, 4099, torch.bfloat16, "param_general"),
     (64, 9001, torch.float32, "param_general"), (64, 1003, torch.bfloat16, "block"), (64, 3, torch.float32, "param_general"),
@@ -50,6 +50,7 @@ def test_sums_alone(rows, C, dtype, want):
     assert kernels(lambda: ops.layernorm_backward(*args, need_dx=False)) == ["ln_bwd_" + want]
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows,C,dtype,want", [
     (64, 9, torch.bfloat16, "dx_general"), (64, 65, torch.float32, "dx_general"), (65, 65, torch.float32, "block"),
     (64, 257, torch.bfloat16, "block"), (16, 8200, torch.float32, "block")])
@@ -61,8 +62,9 @@ def test_dx_alone(rows, C, dtype, want):
     assert kernels(call) == ["ln_bwd_" + want]
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows,C,dtype,general", [
-    (16, 257, torch.bfloat16, True), (17, 257, torch.bfloat16, False), (16, 8200, torch.float32, True),
+    (64, 257, torch.bfloat16, True), (65, 257, torch.bfloat16, False), (16, 8200, torch.float32, True),
     (17, 8200, torch.float32, False), (384, 9001, torch.float32, True), (385, 9001, torch.float32, False)])
 def test_dx_over_dy(rows, C, dtype, general):
     from core_scheduler_amd import _capi, ops
@@ -88,3 +90,14 @@ def test_dx_over_dy(rows, C, dtype, general):
     assert ((over.float() - want[0].float()).abs() <= eps * want[0].float().abs() + 2.0 ** -20).all()
     for got, w in zip((dg, db), want[1:]):  # double sums, rounded once
         assert ((got - w).abs() <= 2.0 ** -23 * w.abs() + 1e-12).all()
+
+
+def test_workspace_of_few_rows():
+    """Rows that every call takes in one launch or on the general kernels need none; its size never falls with the rows."""
+    from core_scheduler_amd import _capi
+
+    size = _capi.load().cs_layernorm_backward_workspace_bytes
+    assert size(64, 257) == size(64, 1003) == size(16, 65) == 0 < size(65, 257)
+    for C in (65, 257, 1003, 9001, 16383):
+        sizes = [size(rows, C) for rows in range(1, 1100)]
+        assert sizes == sorted(sizes)

@@ -169,6 +169,14 @@ void need_params(const at::Tensor &gamma, const at::Tensor *beta, int64_t C) {
   need(gamma.numel() == C && (!beta || (beta->numel() == C && beta->scalar_type() == gamma.scalar_type())));
 }
 
+// what a backward call reads: dy as x, the statistics by row, gamma by column
+void need_backward(const Ln &ln, const at::Tensor &dy, const at::Tensor &mean, const at::Tensor &rstd,
+                   const at::Tensor &gamma) {
+  need(dy.numel() == ln.x.numel() && gamma.numel() == ln.C);
+  need(mean.numel() == ln.rows && rstd.numel() == ln.rows && mean.scalar_type() == ln.stat() &&
+       rstd.scalar_type() == ln.stat());
+}
+
 // ---------------------------------------------------------------------- ops
 PyObject *gelu_forward(Args a) {  // x, approximate
   const at::Tensor &x = a.tensor(0);
@@ -244,6 +252,7 @@ PyObject *layernorm_backward(Args a) {
   const at::Tensor *dres = a.optional(6);
   need(!dres || (dres->sizes() == x.sizes() && dres->scalar_type() == out));
   const Ln ln(x);
+  need_backward(ln, dy, mean, rstd, gamma);
   const int cdy = dtype_code(dy.scalar_type()), cx = dtype_code(x.scalar_type()), cdx = dtype_code(out);
   const int cg = dtype_code(gamma.scalar_type());
   at::Tensor dx, dgamma, dbeta, ws;
@@ -276,6 +285,7 @@ PyObject *layernorm_backward_chained(Args a) {
   const bool pend_acc = a.flag(10);
   need(!dres || (dres->sizes() == x.sizes() && dres->scalar_type() == out));
   const Ln ln(x);
+  need_backward(ln, dy, mean, rstd, gamma);
   const int cdy = dtype_code(dy.scalar_type()), cx = dtype_code(x.scalar_type()), cdx = dtype_code(out);
   const int cg = dtype_code(gamma.scalar_type());
   const int64_t n = cs_layernorm_backward_partial_rows(ln.rows, ln.C, cx);
@@ -343,6 +353,7 @@ PyObject *embedding_backward(Args a) {  // dout, indices, num_weights, padding_i
   const bool by_freq = a.flag(4);
   need(dout.dim() > 0 && V >= 0);
   const int64_t n = ids.numel(), C = dout.size(-1);
+  need(dout.numel() == n * C);
   const int dt = dtype_code(dout.scalar_type()), it = index_code(ids.scalar_type());
   at::Tensor dw, ws;
   const int code = unlocked(a.device, [&](void *s) {
@@ -361,6 +372,7 @@ PyObject *embedding_backward_fused(Args a) {  // dout, indices, num_weights; new
   const int64_t V = a.integer(2);
   need(dout.dim() == 3 && V >= 0);
   const int64_t B = dout.size(0), T = dout.size(1), C = dout.size(2);
+  need(ids.numel() == B * T);
   const int dt = dtype_code(dout.scalar_type()), it = index_code(ids.scalar_type());
   at::Tensor dwte, dwpe, ws;
   const int code = unlocked(a.device, [&](void *s) {

@@ -278,6 +278,21 @@ def layernorm_forward(x, gamma, beta=None, eps=1e-5, out_dtype=None):
     return y, mean, rstd
 
 
+def _check_norm_operands(dy, x, mean, rstd, gamma, *sums):
+    """The kernels read dy as x, mean and rstd by row and gamma by column, and write the sums by column."""
+    C = x.shape[-1]
+    rows = x.numel() // C
+    stat = torch.float64 if x.dtype == torch.float64 else torch.float32
+    if mean.dtype != stat or rstd.dtype != stat or mean.numel() < rows or rstd.numel() < rows:
+        raise ValueError(f"mean and rstd must be [{rows}] of {stat}")
+    if dy.numel() < x.numel() or gamma.numel() < C:
+        raise ValueError("dy must match x, gamma must be [C]")
+    for g in sums:
+        if g is not None and (g.dtype != gamma.dtype or g.numel() < C):
+            raise ValueError("dgamma / dbeta must be [C] of the parameter dtype")
+    return rows, C
+
+
 def layernorm_backward(dy, x, mean, rstd, gamma, *, need_dx=True, need_dgamma=True, need_dbeta=True,
                        dgamma=None, dbeta=None, dx_dtype=None, dresidual=None):
     """Returns (dx, dgamma, dbeta).  Passing dgamma / dbeta accumulates into them; `dresidual`
@@ -286,12 +301,11 @@ def layernorm_backward(dy, x, mean, rstd, gamma, *, need_dx=True, need_dgamma=Tr
         out = _layernorm_backward(dy, x, mean, rstd, gamma, dx_dtype, dresidual)
         if out is not NotImplemented:
             return out
+    rows, C = _check_norm_operands(dy, x, mean, rstd, gamma, dgamma, dbeta)
     dev = _dev(dy, x, mean, rstd, gamma, dgamma, dbeta, dresidual)
     if dresidual is not None and (not need_dx or dresidual.shape != x.shape
                                   or dresidual.dtype != (dx_dtype or x.dtype)):
         raise ValueError("dresidual must match dx")
-    C = x.shape[-1]
-    rows = x.numel() // C
     accumulate = dgamma is not None or dbeta is not None
     if accumulate and ((need_dgamma and dgamma is None) or (need_dbeta and dbeta is None)):
         raise ValueError("accumulating needs every requested parameter gradient passed in")
@@ -325,12 +339,11 @@ def layernorm_backward_rows(dy, x, mean, rstd, gamma, *, need_dx=True, dx_dtype=
     may run on another stream once this call's work is done.  Raises ValueError for shapes that
     have no split form (use `layernorm_backward`).
     """
+    rows, C = _check_norm_operands(dy, x, mean, rstd, gamma)
     dev = _dev(dy, x, mean, rstd, gamma, dresidual)
     if dresidual is not None and (not need_dx or dresidual.shape != x.shape
                                   or dresidual.dtype != (dx_dtype or x.dtype)):
         raise ValueError("dresidual must match dx")
-    C = x.shape[-1]
-    rows = x.numel() // C
     lib = _capi.load()
     n = lib.cs_layernorm_backward_partial_rows(rows, C, _dt(x))
     if n == 0:
@@ -394,9 +407,8 @@ class LayerNormBackwardChain:
                 if partials is not None:
                     self._pending = (partials, dgamma, dbeta, False, x.shape[-1], x.dtype, gamma.dtype)
                 return dx, dgamma, dbeta
+        rows, C = _check_norm_operands(dy, x, mean, rstd, gamma)
         dev = _dev(dy, x, mean, rstd, gamma, dgamma, dbeta, dresidual)
-        C = x.shape[-1]
-        rows = x.numel() // C
         if dresidual is not None and (dresidual.shape != x.shape or dresidual.dtype != (dx_dtype or x.dtype)):
             raise ValueError("dresidual must match dx")
         accumulate = dgamma is not None or dbeta is not None
@@ -484,6 +496,8 @@ def embedding_backward(dout, indices, num_weights, padding_idx=-1, dweight=None,
             return out
     C = dout.shape[-1]
     n = indices.numel()
+    if dout.numel() < n * C:
+        raise ValueError("dout must have a row for every index")
     accumulate = dweight is not None
     if accumulate:
         _check_table_gradient(dweight, num_weights, C, dout.dtype, "dweight")
@@ -506,6 +520,8 @@ def embedding_backward_fused(dout, indices, num_weights, dwte=None, dwpe=None):
         if out is not NotImplemented:
             return out
     B, T, C = dout.shape
+    if indices.numel() < B * T:
+        raise ValueError("indices must be [B, T]")
     accumulate = dwte is not None
     if (dwte is None) != (dwpe is None):
         raise ValueError("pass both gradients to accumulate, or neither")

@@ -62,11 +62,17 @@ def _calls(dt):
 
 def _raises(dt):
     x, gamma = torch.zeros(4, 16, device="cuda", dtype=dt), torch.ones(16, device="cuda")
-    ids = torch.zeros(4, dtype=torch.int64, device="cuda")
+    ids, st = torch.zeros(4, dtype=torch.int64, device="cuda"), torch.float64 if dt == torch.float64 else torch.float32
     return [lambda: ops.gelu_forward(x, "sigmoid"), lambda: ops.gelu_forward(x.t()), lambda: ops.gelu_forward(x.int()),
             lambda: ops.gelu_backward(x, x[:2]), lambda: ops.layernorm_forward(x, gamma[:8]),
             lambda: ops.layernorm_forward(x.cpu(), gamma), lambda: ops.add_layernorm_forward(x, x[:2], gamma),
             lambda: ops.layernorm_backward(x, x, gamma, gamma, gamma, dresidual=x[:2]),
+            lambda: ops.layernorm_backward(x[:3], x, gamma.to(st)[:4], gamma.to(st)[:4], gamma),
+            lambda: ops.layernorm_backward(x, x, gamma.to(st)[:3], gamma.to(st)[:4], gamma),
+            lambda: ops.layernorm_backward(x, x, gamma.half()[:4], gamma.to(st)[:4], gamma),
+            lambda: ops.LayerNormBackwardChain().backward(x, x, gamma.to(st)[:4], gamma.to(st)[:3], gamma),
+            lambda: ops.LayerNormBackwardChain().backward(x, x, gamma.to(st)[:4], gamma.to(st)[:4], gamma[:8]),
+            lambda: ops.embedding_backward(x[:3], ids, 10), lambda: ops.embedding_backward_fused(x[None], ids[:3], 10),
             lambda: ops.embedding_forward(x, ids.float()), lambda: ops.embedding_forward_add(x, x[:, :8], ids[None]),
             lambda: ops.embedding_backward(x, ids, 0), lambda: ops.fused_classifier(x, ids.int()),
             lambda: ops.fused_classifier(x, ids, 17), lambda: ops.fused_classifier(x, ids, reduction="max")]

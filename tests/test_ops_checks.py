@@ -39,3 +39,30 @@ def test_embedding_backward_rejects_a_gradient_of_another_type_or_shape(bad):
 def test_ops_refuse_cpu_tensors():
     with pytest.raises(RuntimeError, match="no CPU path"):
         ops.gelu_forward(torch.zeros(8))
+
+
+@pytest.mark.parametrize("short", ["dy", "mean", "rstd", "gamma", "mean type", "rstd type"])
+@pytest.mark.parametrize("call", [ops.layernorm_backward, ops.layernorm_backward_rows,
+                                  lambda *t: ops.LayerNormBackwardChain().backward(*t)])
+def test_layernorm_backward_rejects_operands_it_would_read_past(call, short):
+    t = dict(dy=torch.zeros(4, 16), x=torch.zeros(4, 16), mean=torch.zeros(4), rstd=torch.ones(4), gamma=torch.ones(16))
+    name = short.split()[0]
+    t[name] = t[name].bfloat16() if short.endswith("type") else t[name][:3]
+    with pytest.raises(ValueError, match="must"):
+        call(*t.values())
+
+
+@pytest.mark.parametrize("bad", [torch.zeros(15), torch.zeros(16, dtype=torch.float64)])
+@pytest.mark.parametrize("which", ["dgamma", "dbeta"])
+def test_layernorm_backward_rejects_sums_it_would_write_past(which, bad):
+    sums = dict(dgamma=torch.zeros(16), dbeta=torch.zeros(16))
+    sums[which] = bad
+    with pytest.raises(ValueError, match="dgamma / dbeta"):
+        ops.layernorm_backward(torch.zeros(4, 16), torch.zeros(4, 16), torch.zeros(4), torch.ones(4), torch.ones(16), **sums)
+
+
+def test_embedding_backward_rejects_rows_or_indices_it_would_read_past():
+    with pytest.raises(ValueError, match="dout"):
+        ops.embedding_backward(torch.zeros(3, 8), torch.zeros(4, dtype=torch.int64), 10)
+    with pytest.raises(ValueError, match="indices"):
+        ops.embedding_backward_fused(torch.zeros(1, 4, 8), torch.zeros(1, 3, dtype=torch.int64), 10)

@@ -1995,8 +1995,8 @@ struct BwdWants {
 // ln_columns_wide has not 16 rows to load at once: bf16 [16,257] 3.6 / 3.0, [64,257] 4.5 / 4.5, [64,1003] 3.7 / 4.5,
 // [64,4099] 5.9 / 4.6, fp32 [64,1909] 5.6 / 4.4, [64,9001] 7.4 / 4.5, rows shorter than a vector [64,3] 4.3 / 4.1 (but
 // [65,257] 5.8 / 6.6 in two launches).
-// dx alone of a column per lane: bf16 [64,9] 3.8 / 3.1, [64,65] 3.5 / 3.1, [64,193] 3.4 / 3.2, [64,257] 3.5 / 3.4, fp32
-// [8,65] 3.2 / 3.0; rows shorter than a vector 3.2 / 3.1; wider ones [64,4099] bf16 4.6 / 7.8, [16,8200] fp32 4.5 / 12.6.
+// dx alone never: it has the bits it has with the sums (up to 256 columns are 0.2-0.5 us slower for that, [64,65] bf16 3.5
+// / 3.1; wider rows [64,4099] 4.6 / 7.8, [16,8200] fp32 4.5 / 12.6).
 // All three where an output lies over an input: up to 64 rows of up to 512 vectors, which then need no workspace whatever
 // the call (bf16 [8,65] 6.5 / 5.1, [16,257] 7.3 / 6.2; [64,65] 7.3 / 8.6, [64,1003] 7.6 / 10.3).  With four fp32 vectors
 // per lane the kernel of several waves spills up to 60 registers: whole [16,8200] 19.2 / 15.7, [16,12288] 21.5 / 20.2,
@@ -2005,7 +2005,7 @@ struct BwdWants {
 bool general_rows(const BwdWants &w, const BlockPlan &b, int64_t rows, int64_t C, int x_dtype, bool aligned) {
   const int64_t vn = 16 / (int64_t)dtype_size(x_dtype);
   if (!w.dx) return rows <= 64 && (C < vn || rows < 16 * 2 * (int64_t)(b.gw * b.groups));
-  if (!w.sums) return rows <= 64 && C >= vn && C <= kLnThreads;
+  if (!w.sums) return false;
   if (b.vpt == 4) return rows <= (aligned && C % vn == 0 ? 16 : 384);
   return rows <= 64 && C / vn <= 8 * kWave;
 }

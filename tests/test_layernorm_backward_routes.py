@@ -51,15 +51,13 @@ def test_sums_alone(rows, C, dtype, want):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows,C,dtype,want", [
-    (64, 9, torch.bfloat16, "dx_general"), (64, 65, torch.float32, "dx_general"), (65, 65, torch.float32, "block"),
-    (64, 257, torch.bfloat16, "block"), (16, 8200, torch.float32, "block")])
-def test_dx_alone(rows, C, dtype, want):
+@pytest.mark.parametrize("rows,C,dtype", [(64, 9, torch.bfloat16), (64, 65, torch.float32), (16, 8200, torch.float32)])
+def test_dx_alone(rows, C, dtype):
     from core_scheduler_amd import ops
 
     args = operands(rows, C, dtype)
     call = lambda: ops.layernorm_backward(*args, need_dgamma=False, need_dbeta=False)
-    assert kernels(call) == ["ln_bwd_" + want]
+    assert kernels(call) == ["ln_bwd_block"] and torch.equal(call()[0], ops.layernorm_backward(*args)[0])
 
 
 @pytest.mark.gpu

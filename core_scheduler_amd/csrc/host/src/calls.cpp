@@ -29,76 +29,77 @@
 namespace {
 
 // ---------------------------------------------------------------- arguments
-struct NotPlain {};  // thrown and caught inside one call: the general path in ops.py takes over
+// What is not plain is not refused by an exception: one costs 2.5 us and more, on top of the Python body's call.
+#define CS_PLAIN(condition) \
+  if (!(condition)) Py_RETURN_NOTIMPLEMENTED
 
-[[noreturn]] void not_plain() { throw NotPlain{}; }
-void need(bool ok) {
-  if (!ok) not_plain();
-}
-
+constexpr int kNoCode = -1;
 int dtype_code(at::ScalarType t) {
   switch (t) {
     case at::kFloat: return CS_F32;
     case at::kDouble: return CS_F64;
     case at::kHalf: return CS_F16;
     case at::kBFloat16: return CS_BF16;
-    default: not_plain();
+    default: return kNoCode;
   }
 }
-int index_code(at::ScalarType t) {
-  if (t == at::kInt) return CS_I32;
-  if (t == at::kLong) return CS_I64;
-  not_plain();
+int index_code(at::ScalarType t) { return t == at::kInt ? CS_I32 : t == at::kLong ? CS_I64 : kNoCode; }
+template <typename... Codes>
+bool supported(Codes... codes) {
+  return ((codes != kNoCode) && ...);
 }
 
-// The arguments of one call; `device` is that of its first tensor.
+// The arguments of one call; `device` is that of its first tensor, `plain` whether every one looked at is (what is
+// not reads as nothing, zero or an undefined tensor).
 struct Args {
   PyObject *const *items;
   Py_ssize_t n;
   int device = -1;
+  bool plain = true;
 
   PyObject *at(Py_ssize_t i) const { return items[i]; }
+  bool is(bool ok) {
+    plain = plain && ok;
+    return ok;
+  }
   const at::Tensor &tensor(Py_ssize_t i) {
+    static const at::Tensor none;
     PyObject *o = items[i];
-    need(THPVariable_CheckExact(o));
+    if (!is(THPVariable_CheckExact(o))) return none;
     const at::Tensor &t = THPVariable_Unpack(o);
-    need(t.defined() && t.is_cuda() && t.layout() == at::kStrided && t.has_storage() && t.is_contiguous());
+    if (!is(t.defined() && t.is_cuda() && t.layout() == at::kStrided && t.has_storage() && t.is_contiguous())) return none;
     if (device < 0) {
       device = t.get_device();
-      need(device == c10::hip::current_device());
-    } else {
-      need(t.get_device() == device);
+      is(device == c10::hip::current_device());
     }
+    is(t.get_device() == device);
     return t;
   }
   const at::Tensor *optional(Py_ssize_t i) { return items[i] == Py_None ? nullptr : &tensor(i); }
-  at::ScalarType dtype_or(Py_ssize_t i, at::ScalarType otherwise) const {
-    if (items[i] == Py_None) return otherwise;
-    need(THPDtype_Check(items[i]));
+  at::ScalarType dtype_or(Py_ssize_t i, at::ScalarType otherwise) {
+    if (items[i] == Py_None || !is(THPDtype_Check(items[i]))) return otherwise;
     return reinterpret_cast<THPDtype *>(items[i])->scalar_type;
   }
-  int64_t integer(Py_ssize_t i) const {
-    need(PyLong_CheckExact(items[i]));
+  int64_t integer(Py_ssize_t i) {
+    if (!is(PyLong_CheckExact(items[i]))) return 0;
     int overflow = 0;
     const long long v = PyLong_AsLongLongAndOverflow(items[i], &overflow);
-    need(overflow == 0);
+    is(overflow == 0);
     return v;
   }
-  double real(Py_ssize_t i) const {
-    need(PyFloat_CheckExact(items[i]));
-    return PyFloat_AS_DOUBLE(items[i]);
-  }
-  bool flag(Py_ssize_t i) const {
-    need(items[i] == Py_True || items[i] == Py_False);
+  double real(Py_ssize_t i) { return is(PyFloat_CheckExact(items[i])) ? PyFloat_AS_DOUBLE(items[i]) : 0.; }
+  bool flag(Py_ssize_t i) {
+    is(items[i] == Py_True || items[i] == Py_False);
     return items[i] == Py_True;
   }
   // the code of a text argument among `names`, in order from 0
   template <size_t N>
-  int choice(Py_ssize_t i, const std::array<const char *, N> &names) const {
-    need(PyUnicode_CheckExact(items[i]));
-    for (size_t k = 0; k < N; ++k)
-      if (PyUnicode_CompareWithASCIIString(items[i], names[k]) == 0) return (int)k;
-    not_plain();
+  int choice(Py_ssize_t i, const std::array<const char *, N> &names) {
+    if (is(PyUnicode_CheckExact(items[i])))
+      for (size_t k = 0; k < N; ++k)
+        if (PyUnicode_CompareWithASCIIString(items[i], names[k]) == 0) return (int)k;
+    is(false);
+    return 0;
   }
 };
 
@@ -152,35 +153,40 @@ int unlocked(int device, Body &&body) {
   return body(static_cast<void *>(c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream()));
 }
 
+// the rows of a norm; not plain without any
 struct Ln {
   const at::Tensor &x;
-  int64_t C, rows;
+  int64_t C = 0, rows = 0;
   explicit Ln(const at::Tensor &x_) : x(x_) {
-    need(x.dim() > 0 && x.numel() > 0);
+    if (x.dim() == 0 || x.numel() == 0) return;
     C = x.size(-1);
     rows = x.numel() / C;
   }
   at::ScalarType stat() const { return x.scalar_type() == at::kDouble ? at::kDouble : at::kFloat; }
+  bool params(const at::Tensor &gamma, const at::Tensor *beta) const {
+    return rows > 0 && gamma.numel() == C &&
+           (!beta || (beta->numel() == C && beta->scalar_type() == gamma.scalar_type()));
+  }
+  // what a backward call reads: dy as x, the statistics by row, gamma by column
+  bool backward(const at::Tensor &dy, const at::Tensor &mean, const at::Tensor &rstd, const at::Tensor &gamma) const {
+    return rows > 0 && dy.numel() == x.numel() && gamma.numel() == C && mean.numel() == rows && rstd.numel() == rows &&
+           mean.scalar_type() == stat() && rstd.scalar_type() == stat();
+  }
 };
 bool same(const at::Tensor &a, const at::Tensor &b) {
   return a.sizes() == b.sizes() && a.scalar_type() == b.scalar_type();
 }
-void need_params(const at::Tensor &gamma, const at::Tensor *beta, int64_t C) {
-  need(gamma.numel() == C && (!beta || (beta->numel() == C && beta->scalar_type() == gamma.scalar_type())));
-}
-
-// what a backward call reads: dy as x, the statistics by row, gamma by column
-void need_backward(const Ln &ln, const at::Tensor &dy, const at::Tensor &mean, const at::Tensor &rstd,
-                   const at::Tensor &gamma) {
-  need(dy.numel() == ln.x.numel() && gamma.numel() == ln.C);
-  need(mean.numel() == ln.rows && rstd.numel() == ln.rows && mean.scalar_type() == ln.stat() &&
-       rstd.scalar_type() == ln.stat());
+bool residual_of(const at::Tensor *dres, const at::Tensor &x, at::ScalarType t) {
+  return !dres || (dres->sizes() == x.sizes() && dres->scalar_type() == t);
 }
 
 // ---------------------------------------------------------------------- ops
 PyObject *gelu_forward(Args a) {  // x, approximate
   const at::Tensor &x = a.tensor(0);
-  const int mode = a.choice(1, kGelu), dt = dtype_code(x.scalar_type());
+  const int mode = a.choice(1, kGelu);
+  CS_PLAIN(a.plain);
+  const int dt = dtype_code(x.scalar_type());
+  CS_PLAIN(supported(dt));
   at::Tensor y;
   const int code = unlocked(a.device, [&](void *s) {
     y = at::empty_like(x);
@@ -192,8 +198,10 @@ PyObject *gelu_forward(Args a) {  // x, approximate
 
 PyObject *gelu_backward(Args a) {  // dy, x, approximate
   const at::Tensor &dy = a.tensor(0), &x = a.tensor(1);
-  need(dy.scalar_type() == x.scalar_type() && dy.numel() == x.numel());
-  const int mode = a.choice(2, kGelu), dt = dtype_code(x.scalar_type());
+  const int mode = a.choice(2, kGelu);
+  CS_PLAIN(a.plain && dy.scalar_type() == x.scalar_type() && dy.numel() == x.numel());
+  const int dt = dtype_code(x.scalar_type());
+  CS_PLAIN(supported(dt));
   at::Tensor dx;
   const int code = unlocked(a.device, [&](void *s) {
     dx = at::empty_like(x);
@@ -207,10 +215,11 @@ PyObject *layernorm_forward(Args a) {  // x, gamma, beta, eps, out_dtype
   const at::Tensor &x = a.tensor(0), &gamma = a.tensor(1);
   const at::Tensor *beta = a.optional(2);
   const double eps = a.real(3);
+  CS_PLAIN(a.plain);
   const at::ScalarType out = a.dtype_or(4, x.scalar_type());
   const Ln ln(x);
-  need_params(gamma, beta, ln.C);
   const int dx = dtype_code(x.scalar_type()), dy = dtype_code(out), dg = dtype_code(gamma.scalar_type());
+  CS_PLAIN(a.plain && ln.params(gamma, beta) && supported(dx, dy, dg));
   at::Tensor y, mean, rstd;
   const int code = unlocked(a.device, [&](void *s) {
     y = empty(x.sizes(), out, x);
@@ -223,15 +232,15 @@ PyObject *layernorm_forward(Args a) {  // x, gamma, beta, eps, out_dtype
   return tuple(y, mean, rstd);
 }
 
-PyObject *add_layernorm_forward(Args a) {  // x, residual, gamma, beta, eps, out_dtype, inplace
+PyObject *add_layernorm_forward(Args a) {  // x, residual, gamma, beta, eps, out_dtype; a new sum
   const at::Tensor &x = a.tensor(0), &residual = a.tensor(1), &gamma = a.tensor(2);
   const at::Tensor *beta = a.optional(3);
   const double eps = a.real(4);
+  CS_PLAIN(a.plain);
   const at::ScalarType out = a.dtype_or(5, x.scalar_type());
-  need(!a.flag(6) && same(x, residual));
   const Ln ln(x);
-  need_params(gamma, beta, ln.C);
   const int dx = dtype_code(x.scalar_type()), dy = dtype_code(out), dg = dtype_code(gamma.scalar_type());
+  CS_PLAIN(a.plain && same(x, residual) && ln.params(gamma, beta) && supported(dx, dy, dg));
   at::Tensor total, y, mean, rstd;
   const int code = unlocked(a.device, [&](void *s) {
     total = at::empty_like(x);
@@ -248,13 +257,13 @@ PyObject *add_layernorm_forward(Args a) {  // x, residual, gamma, beta, eps, out
 // dy, x, mean, rstd, gamma, dx_dtype, dresidual: every gradient, none added to
 PyObject *layernorm_backward(Args a) {
   const at::Tensor &dy = a.tensor(0), &x = a.tensor(1), &mean = a.tensor(2), &rstd = a.tensor(3), &gamma = a.tensor(4);
-  const at::ScalarType out = a.dtype_or(5, x.scalar_type());
   const at::Tensor *dres = a.optional(6);
-  need(!dres || (dres->sizes() == x.sizes() && dres->scalar_type() == out));
+  CS_PLAIN(a.plain);
+  const at::ScalarType out = a.dtype_or(5, x.scalar_type());
   const Ln ln(x);
-  need_backward(ln, dy, mean, rstd, gamma);
   const int cdy = dtype_code(dy.scalar_type()), cx = dtype_code(x.scalar_type()), cdx = dtype_code(out);
   const int cg = dtype_code(gamma.scalar_type());
+  CS_PLAIN(a.plain && residual_of(dres, x, out) && ln.backward(dy, mean, rstd, gamma) && supported(cdy, cx, cdx, cg));
   at::Tensor dx, dgamma, dbeta, ws;
   const int code = unlocked(a.device, [&](void *s) {
     dx = empty(x.sizes(), out, x);
@@ -280,19 +289,19 @@ PyObject *layernorm_backward(Args a) {
 PyObject *layernorm_backward_chained(Args a) {
   const at::Tensor &dy = a.tensor(0), &x = a.tensor(1), &mean = a.tensor(2), &rstd = a.tensor(3), &gamma = a.tensor(4);
   const at::Tensor *dres = a.optional(5);
-  const at::ScalarType out = a.dtype_or(6, x.scalar_type());
   const at::Tensor *pend = a.optional(7), *pend_dgamma = a.optional(8), *pend_dbeta = a.optional(9);
   const bool pend_acc = a.flag(10);
-  need(!dres || (dres->sizes() == x.sizes() && dres->scalar_type() == out));
+  CS_PLAIN(a.plain);
+  const at::ScalarType out = a.dtype_or(6, x.scalar_type());
   const Ln ln(x);
-  need_backward(ln, dy, mean, rstd, gamma);
   const int cdy = dtype_code(dy.scalar_type()), cx = dtype_code(x.scalar_type()), cdx = dtype_code(out);
   const int cg = dtype_code(gamma.scalar_type());
+  CS_PLAIN(a.plain && residual_of(dres, x, out) && ln.backward(dy, mean, rstd, gamma) && supported(cdy, cx, cdx, cg));
   const int64_t n = cs_layernorm_backward_partial_rows(ln.rows, ln.C, cx);
-  need(n > 0);
+  CS_PLAIN(n > 0);
   const bool at_once = cs_layernorm_backward_one_launch(ln.rows, ln.C, cx) && aligned16(dy) && aligned16(x) &&
                        aligned16(gamma) && (!dres || aligned16(*dres));
-  need(!at_once || !pend);  // the earlier sums first, in a launch of their own
+  CS_PLAIN(!at_once || !pend);  // the earlier sums first, in a launch of their own
   at::Tensor dx, dgamma, dbeta, partials;
   const int code = unlocked(a.device, [&](void *s) {
     dx = empty(x.sizes(), out, x);
@@ -319,8 +328,9 @@ PyObject *layernorm_backward_chained(Args a) {
 
 PyObject *embedding_forward(Args a) {  // weight, indices
   const at::Tensor &w = a.tensor(0), &ids = a.tensor(1);
-  need(w.dim() == 2);
+  CS_PLAIN(a.plain && w.dim() == 2);
   const int dt = dtype_code(w.scalar_type()), it = index_code(ids.scalar_type());
+  CS_PLAIN(supported(dt, it));
   std::vector<int64_t> shape(ids.sizes().begin(), ids.sizes().end());
   shape.push_back(w.size(1));
   at::Tensor out;
@@ -334,10 +344,10 @@ PyObject *embedding_forward(Args a) {  // weight, indices
 
 PyObject *embedding_forward_add(Args a) {  // wte, wpe, indices
   const at::Tensor &w = a.tensor(0), &p = a.tensor(1), &ids = a.tensor(2);
-  need(w.dim() == 2 && p.dim() == 2 && ids.dim() == 2);
+  CS_PLAIN(a.plain && w.dim() == 2 && p.dim() == 2 && ids.dim() == 2);
   const int64_t B = ids.size(0), T = ids.size(1), C = w.size(1);
-  need(p.size(0) >= T && p.size(1) == C && p.scalar_type() == w.scalar_type());
   const int dt = dtype_code(w.scalar_type()), it = index_code(ids.scalar_type());
+  CS_PLAIN(p.size(0) >= T && p.size(1) == C && p.scalar_type() == w.scalar_type() && supported(dt, it));
   at::Tensor out;
   const int code = unlocked(a.device, [&](void *s) {
     out = empty({B, T, C}, w.scalar_type(), w);
@@ -351,10 +361,10 @@ PyObject *embedding_backward(Args a) {  // dout, indices, num_weights, padding_i
   const at::Tensor &dout = a.tensor(0), &ids = a.tensor(1);
   const int64_t V = a.integer(2), pad = a.integer(3);
   const bool by_freq = a.flag(4);
-  need(dout.dim() > 0 && V >= 0);
+  CS_PLAIN(a.plain && dout.dim() > 0 && V >= 0);
   const int64_t n = ids.numel(), C = dout.size(-1);
-  need(dout.numel() == n * C);
   const int dt = dtype_code(dout.scalar_type()), it = index_code(ids.scalar_type());
+  CS_PLAIN(dout.numel() == n * C && supported(dt, it));
   at::Tensor dw, ws;
   const int code = unlocked(a.device, [&](void *s) {
     dw = empty({V, C}, dout.scalar_type(), dout);
@@ -370,10 +380,10 @@ PyObject *embedding_backward(Args a) {  // dout, indices, num_weights, padding_i
 PyObject *embedding_backward_fused(Args a) {  // dout, indices, num_weights; new dwte and dwpe
   const at::Tensor &dout = a.tensor(0), &ids = a.tensor(1);
   const int64_t V = a.integer(2);
-  need(dout.dim() == 3 && V >= 0);
+  CS_PLAIN(a.plain && dout.dim() == 3 && V >= 0);
   const int64_t B = dout.size(0), T = dout.size(1), C = dout.size(2);
-  need(ids.numel() == B * T);
   const int dt = dtype_code(dout.scalar_type()), it = index_code(ids.scalar_type());
+  CS_PLAIN(ids.numel() == B * T && supported(dt, it));
   at::Tensor dwte, dwpe, ws;
   const int code = unlocked(a.device, [&](void *s) {
     dwte = empty({V, C}, dout.scalar_type(), dout);
@@ -390,17 +400,17 @@ PyObject *embedding_backward_fused(Args a) {  // dout, indices, num_weights; new
 // a new dlogits.  Returns (loss, row_loss, dlogits, total_weight).
 PyObject *fused_classifier(Args a) {
   const at::Tensor &logits = a.tensor(0), &targets = a.tensor(1);
-  need(logits.dim() == 2);
+  const at::Tensor *weight = a.optional(8);
+  CS_PLAIN(a.plain && logits.dim() == 2);
   const int64_t N = logits.size(0), stride = logits.size(1);
   const int64_t V = a.at(2) == Py_None ? stride : a.integer(2), ignore = a.integer(3);
   const int reduction = a.choice(4, kReductions);
   const float dloss = (float)a.real(5);
   const bool want = a.flag(6);
   const at::ScalarType out = want ? a.dtype_or(7, logits.scalar_type()) : logits.scalar_type();
-  const at::Tensor *weight = a.optional(8);
-  need(targets.scalar_type() == at::kLong && targets.numel() == N);
-  need(!weight || (weight->scalar_type() == at::kFloat && weight->numel() == V));
   const int dl = dtype_code(logits.scalar_type()), dd = dtype_code(out);
+  CS_PLAIN(a.plain && targets.scalar_type() == at::kLong && targets.numel() == N && supported(dl, dd));
+  CS_PLAIN(!weight || (weight->scalar_type() == at::kFloat && weight->numel() == V));
   at::Tensor row_loss, loss, total, d, ws;
   const int code = unlocked(a.device, [&](void *s) {
     row_loss = empty({N}, at::kFloat, logits);
@@ -430,8 +440,6 @@ PyObject *entry(PyObject *, PyObject *const *items, Py_ssize_t n) {
     Py_RETURN_NOTIMPLEMENTED;
   try {
     return FN(Args{items, n});
-  } catch (const NotPlain &) {
-    Py_RETURN_NOTIMPLEMENTED;
   } catch (py::error_already_set &e) {
     e.restore();
     return nullptr;
@@ -444,7 +452,7 @@ PyObject *entry(PyObject *, PyObject *const *items, Py_ssize_t n) {
 PyMethodDef methods[] = {CS_ENTRY(gelu_forward, 2),
                          CS_ENTRY(gelu_backward, 3),
                          CS_ENTRY(layernorm_forward, 5),
-                         CS_ENTRY(add_layernorm_forward, 7),
+                         CS_ENTRY(add_layernorm_forward, 6),
                          CS_ENTRY(layernorm_backward, 7),
                          CS_ENTRY(layernorm_backward_chained, 11),
                          CS_ENTRY(embedding_forward, 2),

@@ -239,9 +239,10 @@ def gelu_backward(dy, x, approximate="none"):
 # -------------------------------------------------------------- LayerNorm
 def add_layernorm_forward(x, residual, gamma, beta=None, eps=1e-5, out_dtype=None, inplace=False):
     """s = x + residual; returns (s, LayerNorm(s), mean, rstd) from one pass.  `inplace` writes s over x."""
-    out = _add_layernorm_forward(x, residual, gamma, beta, eps, out_dtype, inplace)
-    if out is not NotImplemented:
-        return out
+    if not inplace:
+        out = _add_layernorm_forward(x, residual, gamma, beta, eps, out_dtype)
+        if out is not NotImplemented:
+            return out
     dev = _dev(x, residual, gamma, beta)
     if residual.shape != x.shape or residual.dtype != x.dtype:
         raise ValueError("residual must match x")

@@ -1,5 +1,7 @@
 """The native forms of the calls of ops.py (csrc/host/src/calls.cpp): the same results as the Python bodies, and every
 call that is not the plain case is left to them."""
+import timeit
+
 import pytest
 import torch
 
@@ -24,6 +26,21 @@ def test_what_is_not_plain_is_left_alone():
                 c.embedding_backward(x, ids, 10, -1, False), c.embedding_backward_fused(x, ids, 10),
                 c.fused_classifier(x, ids, None, -100, "mean", 1.0, True, None, None)):
         assert out is NotImplemented
+
+
+def test_leaving_a_call_alone_is_cheap():
+    """The Python body's call comes on top: no exception may stand between (2.5 us and more; the whole body takes 7)."""
+    x, c = torch.zeros(4, 8), ops._calls
+
+    def best(fn, *args):
+        return min(timeit.repeat(lambda: fn(*args), number=2000, repeat=15)) / 2000
+
+    nothing = best(c.gelu_forward, x)  # a wrong number of arguments: the way there and back
+    for fn, args in ((c.gelu_forward, (x, "none")), (c.add_layernorm_forward, (x, x, x, None, 1, None)),
+                     (c.layernorm_backward_chained, (x, x, x, x, x, None, None, None, None, None, False)),
+                     (c.fused_classifier, (x, x, None, -100, "mean", 1, True, None, None))):
+        assert fn(*args) is NotImplemented
+        assert best(fn, *args) < 5 * nothing + 0.5e-6
 
 
 def _calls(dt):

@@ -5,15 +5,28 @@ call into libcs_hip_kernels.so.  Tensors must live on a ROCm device and be
 contiguous; there is no CPU path.
 """
 import ctypes
+import importlib
+import warnings
 
 import torch
 
 from . import _capi
 
-try:
-    from . import _cs_calls as _calls  # csrc/host/src/calls.cpp
-except ImportError:  # not built: the same library calls, made from here
-    _calls = None
+
+def _load_calls():
+    """The native forms of the small calls (csrc/host/src/calls.cpp).  Without them the same library calls are made from
+    here, at twice the host time: silently where they are not built, with a warning where they do not load."""
+    name = f"{__package__}._cs_calls"
+    try:
+        return importlib.import_module(name)
+    except ImportError as e:
+        if isinstance(e, ModuleNotFoundError) and e.name == name:
+            return None
+        warnings.warn(f"{name} does not load, its calls are made from Python: {e}", RuntimeWarning, stacklevel=2)
+        return None
+
+
+_calls = _load_calls()
 
 _DTYPES = {
     torch.float32: _capi.F32,

@@ -1,6 +1,8 @@
 """The native forms of the calls of ops.py (csrc/host/src/calls.cpp): the same results as the Python bodies, and every
 call that is not the plain case is left to them."""
+import importlib
 import timeit
+import warnings
 
 import pytest
 import torch
@@ -16,6 +18,20 @@ class Sub(torch.Tensor):
 
 def test_every_native_form_is_built_and_used():
     assert sorted(n[1:] for n in NATIVE) == sorted(n for n in dir(ops._calls) if not n.startswith("_"))
+
+
+def test_a_broken_extension_is_reported(monkeypatch):
+    def load(error):
+        def fail(name):
+            raise error
+        monkeypatch.setattr(importlib, "import_module", fail)
+        return ops._load_calls()
+
+    with pytest.warns(RuntimeWarning, match="undefined symbol"):
+        assert load(ImportError("_cs_calls.so: undefined symbol: cs_gelu_forward")) is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert load(ModuleNotFoundError("not built", name="core_scheduler_amd._cs_calls")) is None
 
 
 def test_what_is_not_plain_is_left_alone():

@@ -1599,14 +1599,15 @@ namespace {
 // what every call takes: the header and a row loss each
 size_t ce_least_workspace(int64_t N) { return kWsHeader + ((size_t)N * sizeof(float) + 255) / 256 * 256; }
 // and behind it the splits of few rows: a target logit and kMostSplits pairs each
-size_t ce_split_workspace(int64_t N) {
-  return N <= kSplitRows ? (size_t)N * (sizeof(float) + kMostSplits * sizeof(float2)) + 256 : 0;
-}
+size_t ce_split_workspace(int64_t N) { return (size_t)N * (sizeof(float) + kMostSplits * sizeof(float2)) + 256; }
 }  // namespace
 
 extern "C" size_t cs_fused_classifier_workspace_bytes(int64_t N) {
   if (N < 0) return 0;
-  return ce_least_workspace(N) + ce_split_workspace(N);
+  if (N <= kSplitRows) return ce_least_workspace(N) + ce_split_workspace(N);
+  // what the most rows that are split take, at least: the size never falls as the rows grow
+  const size_t most = ce_least_workspace(kSplitRows) + ce_split_workspace(kSplitRows), least = ce_least_workspace(N);
+  return least > most ? least : most;
 }
 
 namespace {

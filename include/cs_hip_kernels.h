@@ -408,9 +408,10 @@ int cs_embedding_backward_positions(const void *dout, void *dwpe, int64_t B,
  * of 16 bytes, are read once, with few exceptions; other rows are read twice,
  * the second time from cache.  The loss alone of up to 1024 long rows splits
  * a row over several workgroups, with the workspace that
- * cs_fused_classifier_workspace_bytes asks for; 256 bytes and a float per row
- * (rounded up to 256 bytes) are enough for every other call, and for this one
- * unsplit.
+ * cs_fused_classifier_workspace_bytes asks for (its size never falls as N
+ * grows, so one buffer sized for the most rows serves every batch); 256 bytes
+ * and a float per row (rounded up to 256 bytes) are enough for every other
+ * call, and for this one unsplit, in another order of additions.
  * ---------------------------------------------------------------------- */
 size_t cs_fused_classifier_workspace_bytes(int64_t N);
 int cs_fused_classifier(const void *logits, void *dlogits,

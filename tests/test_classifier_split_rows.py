@@ -7,10 +7,9 @@ import torch
 
 from _util import randint, randn
 
-pytestmark = pytest.mark.gpu
-
 
 # widths at the edges of the vectors a lane holds (2, 4, 8 of them) and of the rule (more than 2048 vectors; 32 splits)
+@pytest.mark.gpu
 @pytest.mark.parametrize("N,V,stride,dtype", [
     (1, 16392, 16392, torch.bfloat16), (3, 16385, 16400, torch.float16), (64, 50257, 50304, torch.bfloat16),
     (509, 50257, 50257, torch.bfloat16), (1024, 16399, 16399, torch.bfloat16), (1025, 16399, 16399, torch.bfloat16),
@@ -46,6 +45,7 @@ def test_split_loss(N, V, stride, dtype):
                 assert abs(loss.item() - want) <= 2e-5 * max(1.0, abs(want))
 
 
+@pytest.mark.gpu
 def test_split_rows_that_have_no_loss():
     from core_scheduler_amd import ops
 
@@ -60,6 +60,7 @@ def test_split_rows_that_have_no_loss():
     assert abs(row[4].item() - exact.item()) <= 1e-5
 
 
+@pytest.mark.gpu
 def test_workspace_without_the_splits():
     """A caller that brings the header and a row loss each is served by whole rows, as before."""
     from core_scheduler_amd import _capi, ops
@@ -74,3 +75,12 @@ def test_workspace_without_the_splits():
     assert code == _capi.OK
     row = ops.fused_classifier(x, t, want_dlogits=False)[1]
     assert (row - out[0]).abs().max().item() <= 1e-5
+
+
+def test_workspace_never_falls_with_the_rows():
+    """One buffer for the longest batch gives every shorter one the splits that a buffer of its own size gives it."""
+    from core_scheduler_amd import _capi
+
+    size = _capi.load().cs_fused_classifier_workspace_bytes
+    sizes = [size(n) for n in (*range(0, 3000), 8192, 100000, 1 << 20)]
+    assert sizes == sorted(sizes)

@@ -1106,7 +1106,7 @@ __global__ __launch_bounds__(kThreads) void emb_bwd_positions_kernel(const T *__
 // flight.  Further workgroups of the launch sum the position table.  One workgroup per table row, which walked that row's entries one load at a time, was the path before: a
 // hot row was a chain of thousands of trips to memory.  us per gather + backward, before / now: bf16 8192 Zipf tokens x 301,
 // 50257 rows 650 / 40, uniform 122 / 39; 16384 x 1599 3213 / 86, uniform 245 / 95; 32768 x 769, 100000 rows 6834 / 106,
-// uniform 373 / 110; fp32 16384 x 1599 3489 / 124; 100 tokens x 301 19 / 20 (launches).
+// uniform 373 / 110; fp32 16384 x 1599 3489 / 124.  (Short lists: see emb_bwd_runs_ragged_kernel.)
 constexpr int kRagWindow = kWave;
 constexpr int kRagThreads = 256;
 constexpr int kRagInFlight = 16;
@@ -1148,10 +1148,15 @@ __global__ __launch_bounds__(kRagThreads) void emb_bwd_reduce_ragged_kernel(
   const uint32_t my_pos = my_id != kNoId ? raw_pos : 0u;  // an unused entry reads row 0 and is not added
   double acc = 0;
   int start = 0;
+  const uint32_t my_row = my_id != kNoId ? my_id : 0u;
   for (int e0 = 0; e0 < n_valid; e0 += kRagInFlight) {
-    T v[kRagInFlight];
+    T v[kRagInFlight], old[kRagInFlight];
 #pragma unroll
     for (int u = 0; u < kRagInFlight; ++u) v[u] = dout[(int64_t)lane_value(my_pos, e0 + u) * C + cc];
+    if (accumulate) {  // requested with the rows, and not one by one where a segment ends
+#pragma unroll
+      for (int u = 0; u < kRagInFlight; ++u) old[u] = dweight[(int64_t)lane_value(my_row, e0 + u) * C + cc];
+    }
 #pragma unroll
     for (int u = 0; u < kRagInFlight; ++u) {
       const int e = e0 + u;
@@ -1162,9 +1167,8 @@ __global__ __launch_bounds__(kRagThreads) void emb_bwd_reduce_ragged_kernel(
       const bool seg_ends = !(at_end && leaves);
       if (((heads >> start) & 1) && seg_ends) {
         if (by_freq) acc /= (double)(e + 1 - start);
-        T *dst = dweight + (int64_t)lane_value(my_id, e) * C + cc;
-        if (accumulate) acc += (double)to_acc(*dst);
-        if (c < C) *dst = from_acc<T>((U)acc);
+        if (accumulate) acc += (double)to_acc(old[u]);
+        if (c < C) dweight[(int64_t)lane_value(my_id, e) * C + c] = from_acc<T>((U)acc);
       } else if (c < C) {
         partial[ragged_partial(w, seg_ends ? 0 : 1, C) + c] = acc;
       }
@@ -1172,6 +1176,76 @@ __global__ __launch_bounds__(kRagThreads) void emb_bwd_reduce_ragged_kernel(
       start = e + 1;
     }
   }
+}
+
+// The same of a short list: a workgroup per sorted entry and 256 columns, which adds the run of equal ids that starts
+// there and returns at once where none does.  A wave that walks a window visits 64 entries one after the other while
+// most of the chip is idle.  WINDOWS: a run is cut at the edges of the windows above and leaves their partial rows, so
+// its chain is at most four rounds of loads; otherwise it is added whole, and neither partial rows nor the launch
+// behind this one are needed.  The additions are in the order of the windows' either way.
+//
+// Whole up to 256 entries, where a list of one id is no slower than in windows (n = 256 x 301: 15.8 us against 15.4;
+// n = 512 26 / 16); with windows up to 3072, as long as the workgroups are few enough to run at once.  us, windows' walk / this, bf16
+// x 301, table of 1000 rows, uniform: n = 100 21.0 / 6.2, 256 21.2 / 6.5, 500 21.7 / 9.8, 1000 22.2 / 11.6, 3000 20.9 /
+// 15.8; of one id: n = 500 15.5 / 13.7, 1000 17.1 / 17.3, 3000 21.5 / 23.6; a table of 50257 rows, Zipf: n = 1000 26.2 /
+// 15.5, 3000 27.3 / 18.5; x 1603, uniform: n = 1000 23.2 / 16.6, 2000 21.8 / 21.4, 4000 23.5 / 30.8.
+constexpr int64_t kRagWholeEntries = 256;
+constexpr int64_t kRagFewEntries = 3072;
+constexpr int64_t kRagFewWorkgroups = 8192;
+
+template <typename T, bool WINDOWS>
+__global__ __launch_bounds__(kRagThreads) void emb_bwd_runs_ragged_kernel(
+    const T *__restrict__ dout, const uint32_t *__restrict__ sorted_id, const uint32_t *__restrict__ sorted_pos,
+    T *__restrict__ dweight, double *__restrict__ partial, int64_t n, int64_t C, int accumulate, int by_freq,
+    unsigned slices, unsigned row_blocks, T *__restrict__ dwpe, int64_t B, int64_t TC) {
+  using U = typename Acc<T>::type;
+  if (blockIdx.x >= row_blocks) {
+    positions_columns<T>(dout, dwpe, B, TC, accumulate, blockIdx.x - row_blocks, gridDim.x - row_blocks);
+    return;
+  }
+  const int lane = threadIdx.x & (kWave - 1);
+  const int64_t p = blockIdx.x / slices, w = p / kRagWindow, last = n - 1;
+  const int64_t c = (int64_t)(blockIdx.x % slices) * kRagThreads + threadIdx.x;
+  const int64_t cc = c < C ? c : C - 1;
+  const int64_t limit = WINDOWS && (w + 1) * kRagWindow < n ? (w + 1) * kRagWindow : n;
+  const uint32_t id = sorted_id[p], prev = sorted_id[p > 0 ? p - 1 : 0];
+  const uint32_t next = sorted_id[limit < last ? limit : last];
+  uint32_t ids = sorted_id[p + lane < last ? p + lane : last], pos = sorted_pos[p + lane < last ? p + lane : last];
+  const bool head = p == 0 || prev != id;
+  if (id == kNoId || !(head || (WINDOWS && p % kRagWindow == 0))) return;
+  T *dst = dweight + (int64_t)id * C + cc;
+  const T old = accumulate ? *dst : T{};
+  double acc = 0;
+  auto add = [&](auto in_flight, int e0, int run) {
+    constexpr int K = decltype(in_flight)::value;
+    T v[K];
+#pragma unroll
+    for (int u = 0; u < K; ++u) v[u] = dout[(int64_t)lane_value(pos, e0 + u < run ? e0 + u : run - 1) * C + cc];
+#pragma unroll
+    for (int u = 0; u < K; ++u)
+      if (e0 + u < run) acc += (double)to_acc(v[u]);  // workgroup-uniform, as every decision here
+  };
+  int64_t q = p;
+  for (;;) {
+    const uint64_t other = __ballot(q + lane >= limit || ids != id);
+    const int run = other ? __ffsll((long long)other) - 1 : kWave;
+    int e0 = 0;
+    for (; run - e0 > 4; e0 += kRagInFlight) add(std::integral_constant<int, kRagInFlight>{}, e0, run);
+    if (e0 < run) add(std::integral_constant<int, 4>{}, e0, run);
+    q += run;
+    if (run < kWave || q >= limit) break;
+    ids = sorted_id[q + lane < last ? q + lane : last];
+    pos = sorted_pos[q + lane < last ? q + lane : last];
+  }
+  if (c >= C) return;
+  const bool leaves = WINDOWS && q == limit && limit < n && next == id;
+  if (WINDOWS && (!head || leaves)) {
+    partial[ragged_partial(w, leaves ? 1 : 0, C) + c] = acc;
+    return;
+  }
+  if (by_freq) acc /= (double)(q - p);
+  if (accumulate) acc += (double)to_acc(old);
+  *dst = from_acc<T>((U)acc);
 }
 
 // The workgroup of a segment's first window adds its partial rows, as emb_bwd_finish_kernel does.
@@ -1452,17 +1526,22 @@ int bwd_typed(const void *dout, const void *ids, void *dweight, void *dwpe, char
   if (!vec_ok) {
     double *partial = reinterpret_cast<double *>(ws + L.off_partial);
     const int64_t slices = ceil_div(C, (int64_t)kRagThreads);
-    const int64_t row_blocks = ceil_div(n, (int64_t)kRagWindow) * slices;
+    const bool whole = n <= kRagWholeEntries, runs = whole || (n <= kRagFewEntries && n * slices <= kRagFewWorkgroups);
+    const int64_t window_blocks = ceil_div(n, (int64_t)kRagWindow) * slices;
+    const int64_t row_blocks = runs ? n * slices : window_blocks;
     int64_t pos_blocks = dwpe ? ceil_div(TC, (int64_t)kThreads) : 0;
     if (pos_blocks > 65536) pos_blocks = 65536;
     if (row_blocks + pos_blocks > 0x7fffffffLL) return CS_ERR_TOO_LARGE;
     if (row_blocks + pos_blocks == 0) return CS_OK;
-    emb_bwd_reduce_ragged_kernel<T><<<dim3((unsigned)(row_blocks + pos_blocks)), dim3(kRagThreads), 0, s>>>(
+    const auto kernel = whole  ? emb_bwd_runs_ragged_kernel<T, false>
+                        : runs ? emb_bwd_runs_ragged_kernel<T, true>
+                               : emb_bwd_reduce_ragged_kernel<T>;
+    kernel<<<dim3((unsigned)(row_blocks + pos_blocks)), dim3(kRagThreads), 0, s>>>(
         (const T *)dout, sorted_id, sorted_pos, (T *)dweight, partial, n, C, accumulate, by_freq, (unsigned)slices,
         (unsigned)row_blocks, (T *)dwpe, B, TC);
     st = launch_status();
-    if (st != CS_OK || n <= kRagWindow) return st;  // one window: no segment leaves it
-    emb_bwd_finish_ragged_kernel<T><<<dim3((unsigned)row_blocks), dim3(kRagThreads), 0, s>>>(
+    if (st != CS_OK || whole || n <= kRagWindow) return st;  // no segment leaves its workgroup
+    emb_bwd_finish_ragged_kernel<T><<<dim3((unsigned)window_blocks), dim3(kRagThreads), 0, s>>>(
         sorted_id, partial, (T *)dweight, n, C, accumulate, by_freq, (unsigned)slices);
     return launch_status();
   }

@@ -33,7 +33,8 @@ def rounded_once(got, exact, terms):
                                            (255, torch.float32, False), (257, torch.bfloat16, True), (301, torch.float16, False),
                                            (513, torch.float32, True), (64, torch.bfloat16, True), (3, torch.float64, False),
                                            (300, torch.float64, False)])
-@pytest.mark.parametrize("n,V", [(0, 5), (1, 3), (63, 1), (64, 7), (65, 2), (129, 40), (1000, 30), (4097, 3000), (9001, 90)])
+@pytest.mark.parametrize("n,V", [(0, 5), (1, 3), (63, 1), (64, 7), (65, 2), (129, 40), (256, 9), (257, 9), (1000, 30),
+                                 (2731, 500), (3072, 70), (3073, 70), (4097, 3000), (9001, 90)])
 def test_ragged_rows(C, dtype, shift, n, V):
     from core_scheduler_amd import ops
 
@@ -63,6 +64,21 @@ def test_ragged_rows(C, dtype, shift, n, V):
     count = torch.bincount(at, minlength=V).clamp(min=1).double()[:, None]
     mean = ops.embedding_backward(d_dout, d_ids, V, scale_grad_by_freq=True).cpu()
     assert rounded_once(mean, exact / count, terms)
+
+
+@pytest.mark.parametrize("n,C,want", [(256, 301, ["runs"]), (257, 301, ["runs", "finish"]), (3072, 301, ["runs", "finish"]),
+                                      (3073, 301, ["reduce", "finish"]), (2731, 513, ["reduce", "finish"])])
+def test_launches_of_a_list(n, C, want):
+    """A short list has a workgroup per entry, and no second launch where that adds whole runs."""
+    from core_scheduler_amd import ops
+
+    ids, dout = randint(0, 50, (n,), 1).cuda(), randn((n, C), 2).cuda()
+    ops.embedding_backward(dout, ids, 50)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        ops.embedding_backward(dout, ids, 50)
+        torch.cuda.synchronize()
+    names = [e.name.split("_ragged")[0].split("emb_bwd_")[1] for e in prof.events() if "_ragged_kernel" in e.name]
+    assert names == want
 
 
 @pytest.mark.parametrize("B,T,C,dtype,shift", [(1, 1, 9, torch.bfloat16, False), (3, 50, 301, torch.float32, False),

@@ -176,7 +176,7 @@ __global__ __launch_bounds__(kThreads) void emb_fwd_vec_kernel(
   }
 }
 
-// rows shorter than a vector
+// rows shorter than a vector, and few elements of ragged ones (kFewElements)
 template <typename T, typename IdxT, bool ADD>
 __global__ __launch_bounds__(kThreads) void emb_fwd_scalar_kernel(
     const T *__restrict__ weight, const T *__restrict__ wpe, const IdxT *__restrict__ ids,
@@ -1349,6 +1349,12 @@ BwdLayout bwd_layout(int64_t n, int64_t C, int64_t num_weights) {
   return L;
 }
 
+// Ragged or unaligned rows of up to so many elements in all are gathered element by element: every lane has one, where
+// vectors leave most of the chip idle.  us, elements / vectors, bf16: 300 x 301 2.9 / 3.3, 1500 x 301 3.3 / 3.5, 2000 x 301
+// 3.6 / 3.5, 4000 x 301 4.4 / 3.7; with positions 3.0 / 3.6, 3.6 / 3.8, 3.9 / 3.8; 8000 x 65 3.4 / 3.7, 16000 x 65 4.1 /
+// 3.9; fp32 1500 x 301 3.4 / 3.5, 600 x 1003 3.7 / 3.6.
+constexpr int64_t kFewElements = 1 << 19;
+
 template <typename T, typename IdxT, bool ADD>
 int fwd_launch(const void *weight, const void *wpe, const void *ids, void *out, int64_t n_rows,
                int64_t C, int64_t num_weights, int64_t T_len, hipStream_t s) {
@@ -1362,7 +1368,7 @@ int fwd_launch(const void *weight, const void *wpe, const void *ids, void *out, 
     emb_fwd_vec_kernel<T, IdxT, ADD, false><<<dim3((unsigned)vec_blocks), dim3(kThreads), 0, s>>>(
         (const T *)weight, (const T *)wpe, (const IdxT *)ids, (T *)out, n_rows, C, (uint32_t)nvec, num_weights,
         (uint32_t)T_len);
-  } else if (C >= VN && nvec <= 0x7fffffff && vec_blocks <= 0x7fffffffLL) {
+  } else if (n_rows * C > kFewElements && C >= VN && nvec <= 0x7fffffff && vec_blocks <= 0x7fffffffLL) {
     emb_fwd_vec_kernel<T, IdxT, ADD, true><<<dim3((unsigned)vec_blocks), dim3(kThreads), 0, s>>>(
         (const T *)weight, (const T *)wpe, (const IdxT *)ids, (T *)out, n_rows, C, (uint32_t)nvec, num_weights,
         (uint32_t)T_len);

@@ -66,6 +66,25 @@ def test_ragged_rows(C, dtype, shift, n, V):
     assert rounded_once(mean, exact / count, terms)
 
 
+@pytest.mark.parametrize("n,C,positions,want", [(300, 301, False, "scalar"), (1000, 65, True, "scalar"), (2000, 301, True, "vec"),
+                                                (2, 3, False, "scalar"), (300000, 7, False, "scalar")])
+def test_gather_by_elements_or_vectors(n, C, positions, want):
+    """Few elements are gathered one by one, rows shorter than a vector always: the same bits."""
+    from core_scheduler_amd import ops
+
+    ids, wte, wpe = randint(-1, 52, (1, n), 1).cuda(), randn((50, C), 2).bfloat16().cuda(), randn((n, C), 3).bfloat16().cuda()
+    call = (lambda: ops.embedding_forward_add(wte, wpe, ids)) if positions else (lambda: ops.embedding_forward(wte, ids))
+    call()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        got = call()
+        torch.cuda.synchronize()
+    assert [e.name.split("emb_fwd_")[1].split("_")[0] for e in prof.events() if "emb_fwd_" in e.name] == [want]
+    ok = ((ids >= 0) & (ids < 50))[..., None]
+    rows = wte[ids.clamp(0, 49)]
+    rows = (rows.float() + wpe.float()).bfloat16() if positions else rows
+    assert torch.equal(got, torch.where(ok, rows, torch.zeros((), dtype=rows.dtype, device="cuda")))
+
+
 @pytest.mark.parametrize("n,C,want", [(256, 301, ["runs"]), (257, 301, ["runs", "finish"]), (3072, 301, ["runs", "finish"]),
                                       (3073, 301, ["reduce", "finish"]), (2731, 513, ["reduce", "finish"])])
 def test_launches_of_a_list(n, C, want):
@@ -82,7 +101,8 @@ def test_launches_of_a_list(n, C, want):
 
 
 @pytest.mark.parametrize("B,T,C,dtype,shift", [(1, 1, 9, torch.bfloat16, False), (3, 50, 301, torch.float32, False),
-                                               (17, 65, 257, torch.float16, False), (9, 33, 64, torch.bfloat16, True)])
+                                               (17, 65, 257, torch.float16, False), (9, 33, 64, torch.bfloat16, True),
+                                               (40, 65, 301, torch.bfloat16, False), (10, 900, 64, torch.bfloat16, True)])
 def test_ragged_positions(B, T, C, dtype, shift):
     from core_scheduler_amd import ops
 

@@ -28,8 +28,8 @@
 //   4. finish     - the workgroups of a crossing segment's first window add
 //                   that segment's partial rows in window order.  Further
 //                   workgroups of the same launch sum the position-table
-//                   gradient, which needs no order (of launch 3, where the
-//                   list is short).
+//                   gradient, which needs no order (of launch 3 where the list
+//                   is short, of launch 1 where that has little to fill).
 // A list of at most 8192 entries skips 1 and 2: one launch ranks every key by
 // comparing it with all others (see emb_bwd_rank_kernel), and does the zero
 // fill next to that.
@@ -379,6 +379,16 @@ __device__ __forceinline__ void zero_fill_block(u32x4 *__restrict__ dst, int64_t
   }
 }
 
+// The position sums that ride in another kernel's launch, on `blocks` workgroups of it.
+template <typename T>
+struct Positions {
+  const T *dout;
+  T *dwpe;
+  int64_t B, TC;
+  int accumulate, log2_slices;
+  int64_t blocks;
+};
+
 // The table's bytes ahead of its first whole vector and behind its last one (fewer than 16 each).
 struct FillEdges {
   uint16_t *head, *tail;
@@ -392,17 +402,26 @@ __device__ __forceinline__ void zero_edges(const FillEdges &e, int tid) {
 // Launch layout, in block order:
 //   [0, n_tiles)                sort one tile of 1024 keys
 //   + 1                         preset sorted_id to "no id"
+//   + positions.blocks          position-table gradient, where kPosFewFill says so
 //   + the rest                  zero fill of fill_dst[0, fill_vecs)
-template <typename KeyT, typename IdxT>
+template <typename KeyT, typename IdxT, typename T>
 __global__ __launch_bounds__(kTile) void emb_bwd_tile_sort_kernel(
     const IdxT *__restrict__ ids, KeyT *__restrict__ tiles, uint32_t *__restrict__ sorted_id,
     int64_t n, int n_tiles, int shift, int64_t num_weights, int64_t padding_idx,
-    u32x4 *__restrict__ fill_dst, int64_t fill_vecs, FillEdges edges) {
-  __shared__ KeyT keys[2][kTile];
+    u32x4 *__restrict__ fill_dst, int64_t fill_vecs, FillEdges edges, Positions<T> positions) {
+  // the sorting workgroups keep two key arrays here, the position workgroups their slice sums
+  __shared__ f32x4 shared_raw[kTile * kPosLdsBytesPerLane / sizeof(f32x4)];
+  static_assert(2 * kTile * sizeof(KeyT) <= sizeof(shared_raw), "the key arrays fit the shared buffer");
+  KeyT(*keys)[kTile] = reinterpret_cast<KeyT(*)[kTile]>(shared_raw);
   const int tid = threadIdx.x;
   const int64_t blk = blockIdx.x;
+  if (blk > n_tiles + positions.blocks) {
+    zero_fill_block<kTile, kFillVecsSort>(fill_dst, fill_vecs, blk - n_tiles - positions.blocks - 1, tid);
+    return;
+  }
   if (blk > n_tiles) {
-    zero_fill_block<kTile, kFillVecsSort>(fill_dst, fill_vecs, blk - n_tiles - 1, tid);
+    positions_block<T, kTile>(positions.dout, positions.dwpe, blk - n_tiles - 1, positions.B, positions.TC,
+                              positions.accumulate, positions.log2_slices, shared_raw, tid);
     return;
   }
   if (blk == n_tiles) {
@@ -656,6 +675,11 @@ constexpr int kVpl = CS_EMB_VPL;                // 16-byte column vectors per la
 // the reduce launch, longer ones in the finish launch (see there): kernels of a call, us, reduce / finish /
 // before both, next to the zero fill: [1,123] x 768 24.3 / 25.3 / 24.1, [4,512] x 768 27.2 / 27.5 / 28.8,
 // [8,512] x 1600 49.7 / 50.1 / 53.2, [6,1024] x 768 30.3 / 30.7 / 31.8, [8,1024] x 1600 56.7 / 56.7 / 61.6.
+// A longer list with little to fill (16-byte vectors; none where the gradient is added to) has them in the sort launch,
+// which leaves most of the chip idle then: kernels of a call, us, finish / sort: 16384 x 1600 bf16 accumulating 56.8 /
+// 51.9 (Zipf) and 63.1 / 58.4 (uniform), tables of 3 MB 45.1 / 41.5, 32 MB 49.1 / 47.2, 64 MB 51.2 / 51.4, 161 MB 55.7 /
+// 57.4; 32768 x 768 46 MB 54.5 / 53.8, 77 MB 55.1 / 57.1; 16384 x 512 fp32 8 MB 34.7 / 30.9, 103 MB 37.0 / 39.6.
+constexpr int64_t kPosFewFill = (int64_t)3 << 20;
 constexpr int64_t kPosEarlyWindows = 256;
 
 // Workgroup w reduces sorted entries [kWindow w, kWindow (w + 1)).  partial rows live at
@@ -879,8 +903,8 @@ __global__ __launch_bounds__(kRedThreads, 2048 / kRedThreads) void emb_bwd_reduc
 //
 // Bound by a chain of trips to memory (ids, partial rows) that leaves HBM idle, so the position-table sums of
 // a long list, which read all of dout and wait for nothing, run next to it: the first workgroups of the grid,
-// because the others are short.  They ran next to the tile sort before, whose launch is bound by the bytes of its
-// zero fill.  Kernels of a call, us: 16384 tokens x 1600 Zipf ids 73.3 -> 69.2, uniform 85.9 -> 84.6,
+// because the others are short.  Next to the tile sort they would wait for the bytes of its zero fill (but see
+// kPosFewFill).  Kernels of a call, us: 16384 tokens x 1600 Zipf ids 73.3 -> 69.2, uniform 85.9 -> 84.6,
 // 32768 x 768 fp32 93.5 -> 89.9; in the reduce launch of such a list they cost what they save.  256 columns per
 // workgroup, so that a hot row's sum is shared by several: 14.2 us with the positions at 16384 x 1600; 512
 // columns 14.4, 1024 15.2; positions last 17.3.  dout is read past the caches in both launches: kept there it
@@ -1465,15 +1489,23 @@ int position_slices(int64_t B) {
   return log2_slices;
 }
 
+// a list short enough that its keys are ranked in one launch
+template <typename KeyT>
+bool ranked(int64_t n) {
+  return (size_t)ceil_div(n, (int64_t)4) * 4 * sizeof(KeyT) <= kRankMaxKeyBytes;
+}
+
 // Sort + merge.  Both launches clear their share of fill_dst[0, fill_vecs), on the CUs the sorting leaves idle.
-template <typename KeyT, typename IdxT>
+// `positions` ride in the sort launch (the caller plans none for a list that is ranked).
+template <typename KeyT, typename IdxT, typename T>
 int sort_launch(const void *ids, char *ws, const BwdLayout &L, int64_t n, int64_t num_weights,
-                int64_t padding_idx, u32x4 *fill_dst, int64_t fill_vecs, const FillEdges &edges, hipStream_t s) {
+                int64_t padding_idx, u32x4 *fill_dst, int64_t fill_vecs, const FillEdges &edges,
+                const Positions<T> &positions, hipStream_t s) {
   KeyT *tiles = reinterpret_cast<KeyT *>(ws + L.off_tiles);
   uint32_t *sorted_id = reinterpret_cast<uint32_t *>(ws + L.off_sorted_id);
   uint32_t *sorted_pos = reinterpret_cast<uint32_t *>(ws + L.off_sorted_pos);
   const int64_t n_quads = ceil_div(n, (int64_t)4);
-  if ((size_t)n_quads * 4 * sizeof(KeyT) <= kRankMaxKeyBytes) {
+  if (ranked<KeyT>(n)) {
     // a short list: one launch ranks every key against all others
     return n_quads * 4 <= kRankFewKeys && fill_vecs <= kRankFewFill
                ? rank_launch<KeyT, IdxT, 16>(ids, sorted_id, sorted_pos, n, n_quads, L.shift, num_weights, padding_idx,
@@ -1486,12 +1518,12 @@ int sort_launch(const void *ids, char *ws, const BwdLayout &L, int64_t n, int64_
   const int64_t sort_fill_vecs =
       sort_fill_blocks * kFillVecsSort < fill_vecs ? sort_fill_blocks * kFillVecsSort : fill_vecs;
   const int64_t merge_fill_blocks = ceil_div(fill_vecs - sort_fill_vecs, (int64_t)kFillVecsMerge);
-  const int64_t blocks = L.n_tiles + 1 + sort_fill_blocks;
+  const int64_t blocks = L.n_tiles + 1 + positions.blocks + sort_fill_blocks;
   const int64_t mblocks = L.n_tiles * kTile / kThreads + merge_fill_blocks;
   if (blocks > 0x7fffffffLL || mblocks > 0x7fffffffLL) return CS_ERR_TOO_LARGE;
-  emb_bwd_tile_sort_kernel<KeyT, IdxT><<<dim3((unsigned)blocks), dim3(kTile), 0, s>>>(
+  emb_bwd_tile_sort_kernel<KeyT, IdxT, T><<<dim3((unsigned)blocks), dim3(kTile), 0, s>>>(
       (const IdxT *)ids, tiles, sorted_id, n, (int)L.n_tiles, L.shift, num_weights, padding_idx, fill_dst,
-      sort_fill_vecs, edges);
+      sort_fill_vecs, edges, positions);
   int st = launch_status();
   if (st != CS_OK) return st;
   emb_bwd_merge_kernel<KeyT><<<dim3((unsigned)mblocks), dim3(kThreads), 0, s>>>(
@@ -1530,9 +1562,14 @@ int bwd_typed(const void *dout, const void *ids, void *dweight, void *dwpe, char
                       (int)((table + bytes - tail) / 2)};
   }
   if (!vec_ok && num_weights > 0x7fffffffLL) return CS_ERR_TOO_LARGE;
+  using P = std::conditional_t<std::is_same_v<T, double>, float, T>;  // (fp64 rows are summed by column)
+  const int log2_s = position_slices(B);
+  auto pos_blocks = [&](int threads) { return dwpe ? ceil_div(TC / VN, (int64_t)(threads >> log2_s)) : 0; };
+  const bool pos_first = vec_ok && fill_vecs <= kPosFewFill && !(L.key64 ? ranked<uint64_t>(n) : ranked<uint32_t>(n));
+  const Positions<P> positions{(const P *)dout, (P *)dwpe, B, TC, accumulate, log2_s, pos_first ? pos_blocks(kTile) : 0};
   int st;
 #define CS_SORT(KeyT, IdxT) \
-  sort_launch<KeyT, IdxT>(ids, ws, L, n, num_weights, padding_idx, fill_dst, fill_vecs, edges, s)
+  sort_launch<KeyT, IdxT, P>(ids, ws, L, n, num_weights, padding_idx, fill_dst, fill_vecs, edges, positions, s)
   if (L.key64) {
     st = idx_dtype == CS_I64 ? CS_SORT(uint64_t, int64_t) : CS_SORT(uint64_t, int32_t);
   } else {
@@ -1571,11 +1608,9 @@ int bwd_typed(const void *dout, const void *ids, void *dweight, void *dwpe, char
     const int64_t fin_blocks = windows * slices;
     // The position sums go where the chip is idle: next to the finish workgroups, or next to the reducing ones of a
     // list too short to occupy the chip with those.
-    const int log2_s = position_slices(B);
     const bool pos_early = windows > 0 && windows <= kPosEarlyWindows;
-    auto pos_blocks = [&](int threads) { return dwpe ? ceil_div(TC / VN, (int64_t)(threads >> log2_s)) : 0; };
-    const int64_t red_blocks = windows + (pos_early ? pos_blocks(kRedThreads) : 0);
-    const int64_t last_blocks = fin_blocks + (pos_early ? 0 : pos_blocks(kFinThreads));
+    const int64_t red_blocks = windows + (pos_early && !pos_first ? pos_blocks(kRedThreads) : 0);
+    const int64_t last_blocks = fin_blocks + (pos_early || pos_first ? 0 : pos_blocks(kFinThreads));
     if (red_blocks > 0x7fffffffLL || last_blocks > 0x7fffffffLL) return CS_ERR_TOO_LARGE;
     if (windows > 0) {
       const size_t lds = (size_t)kRedWaves * 2 * kWave * kVpl * VN * sizeof(float);

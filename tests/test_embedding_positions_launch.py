@@ -65,3 +65,19 @@ def test_short_lists(n, V):
     keep = (ids >= 0) & (ids < V) & (ids != 5)
     want.index_add_(0, ids[keep], dout[keep])
     assert torch.equal(ops.embedding_backward(dout.cuda(), ids.cuda(), V, padding_idx=5).cpu(), want)
+
+
+@pytest.mark.parametrize("V", [24576, 24577])  # 3 * 2^20 vectors of fill, with which the sort launch still has the sums
+@pytest.mark.parametrize("n_batch", [9, 20])   # one lane per vector of the position table, and a sliced batch
+def test_positions_of_a_long_list(V, n_batch):
+    from core_scheduler_amd import ops
+
+    T, C = 911, 512
+    ids = torch.randint(0, V, (n_batch, T), generator=gen(8))
+    dout = torch.randint(-8, 9, (n_batch, T, C), generator=gen(9)).float()  # whole numbers: every order gives the same sums
+    want_t = torch.zeros(V, C).index_add_(0, ids.reshape(-1), dout.reshape(-1, C))
+    want_p = dout.sum(0)
+    dwte, dwpe = ops.embedding_backward_fused(dout.cuda(), ids.cuda(), V)
+    assert torch.equal(dwte.cpu(), want_t) and torch.equal(dwpe.cpu(), want_p)
+    dwte, dwpe = ops.embedding_backward_fused(dout.cuda(), ids.cuda().int(), V, dwte, dwpe)  # nothing to fill
+    assert torch.equal(dwte.cpu(), 2 * want_t) and torch.equal(dwpe.cpu(), 2 * want_p)

@@ -652,8 +652,9 @@ __global__ __launch_bounds__(kRankThreads) void emb_bwd_rank_kernel(
 constexpr int kOwn = 4;                         // sorted entries per wave
 constexpr int kRedWaves = kWindow / kOwn;       // 8
 constexpr int kRedThreads = kRedWaves * kWave;  // 512: two workgroups share a CU
-constexpr int kFinThreads = 256;                // finish kernel: lanes, and columns of a workgroup
-constexpr int kFinWaves = kFinThreads / kWave;
+constexpr int kFinThreads = 256;                // finish kernel: lanes of a workgroup
+constexpr int64_t kFinWideRow = 1024;           // two columns to each beyond this row length,
+constexpr int64_t kFinMostAtOnce = 2048;        // and where there are more workgroups than this
 #ifndef CS_EMB_FIN_DIRECT_ROWS
 #define CS_EMB_FIN_DIRECT_ROWS 8
 #endif
@@ -896,7 +897,7 @@ __global__ __launch_bounds__(kRedThreads, 2048 / kRedThreads) void emb_bwd_reduc
   }
 }
 
-// The last level of the segmented sum.  A workgroup looks at window w for kFinThreads of the columns: if
+// The last level of the segmented sum.  A workgroup looks at window w for kFinThreads * PER of the columns: if
 // the run that leaves the window over its right edge began in it (a true segment head), this is that
 // segment's first window, and the workgroup adds the segment's partial rows in window order: slot 1 of
 // every window the segment leaves, slot 0 of the one it ends in.
@@ -907,13 +908,17 @@ __global__ __launch_bounds__(kRedThreads, 2048 / kRedThreads) void emb_bwd_reduc
 // kPosFewFill).  Kernels of a call, us: 16384 tokens x 1600 Zipf ids 73.3 -> 69.2, uniform 85.9 -> 84.6,
 // 32768 x 768 fp32 93.5 -> 89.9; in the reduce launch of such a list they cost what they save.  256 columns per
 // workgroup, so that a hot row's sum is shared by several: 14.2 us with the positions at 16384 x 1600; 512
-// columns 14.4, 1024 15.2; positions last 17.3.  dout is read past the caches in both launches: kept there it
+// columns 14.4, 1024 15.2; positions last 17.3.  PER: columns a lane; two for many windows of more than 1024 columns,
+// whose workgroups are more than the chip holds at once if most windows are left by a run (backward, one / two: 16384 x
+// 1600 bf16 into 1000 rows 37.6 / 36.2, x 2048 fp32 59.5 / 54.4; Zipf ids of 50257 rows 48.5 / 48.5; but 32768 x 768 48.5 /
+// 50.0, and one id in every entry 42.4 / 51.2).  dout is read past the caches in both launches: kept there it
 // pushes out what the next call reads (this launch 14.2 -> 12.3 us, but the next gather 12.9 -> 20.1).
-template <typename T>
+template <typename T, int PER>
 __global__ __launch_bounds__(kFinThreads, 5) void emb_bwd_finish_kernel(
     const uint32_t *__restrict__ sorted_id, const float *__restrict__ partial,
     T *__restrict__ dweight, int64_t n, int64_t C, int accumulate, int by_freq, int64_t fin_blocks, int slices,
     const T *__restrict__ dout, T *__restrict__ dwpe, int64_t B, int64_t TC, int pos_log2_slices) {
+  constexpr int kFinWaves = kFinThreads / kWave;
   __shared__ int first_other[kFinWaves];
   __shared__ int first_tail[kFinWaves];
   __shared__ f32x4 lds[kFinThreads * kPosLdsBytesPerLane / sizeof(f32x4)];
@@ -926,8 +931,8 @@ __global__ __launch_bounds__(kFinThreads, 5) void emb_bwd_finish_kernel(
     return;
   }
   const int64_t w = (unsigned)blk / (unsigned)slices;
-  const int c0 = (int)(blk - w * slices) * kFinThreads;  // the workgroup's first column
-  const int cols = (int)C - c0 < kFinThreads ? (int)C - c0 : kFinThreads;
+  const int c0 = (int)(blk - w * slices) * kFinThreads * PER;  // the workgroup's first column
+  const int cols = (int)C - c0 < kFinThreads * PER ? (int)C - c0 : kFinThreads * PER;
   const int64_t last = w * kWindow + kWindow - 1;
   if (last + 1 >= n) return;  // nothing after this window
   // Everything the decisions below read, and the two partial rows of the usual case (a segment
@@ -943,11 +948,16 @@ __global__ __launch_bounds__(kFinThreads, 5) void emb_bwd_finish_kernel(
   uint32_t raw_before = sorted_id[w > 0 ? w * kWindow - 1 : 0];
   uint32_t raw_q = sorted_id[pq < n ? pq : n - 1];
   uint32_t raw_f = sorted_id[pw * kWindow < n ? pw * kWindow : n - 1];
-  const int64_t col = c0 + (tid < cols ? tid : 0);
-  float pre_leave = partial[(w * 2 + 1) * C + col];        // window w, left over its right edge
-  float pre_enter = partial[((w + 1) * 2 + 0) * C + col];  // window w + 1, entered over its left edge
-  asm volatile("" : "+v"(raw_last), "+v"(raw_next), "+v"(raw_first), "+v"(raw_before), "+v"(raw_q), "+v"(raw_f),
-                    "+v"(pre_leave), "+v"(pre_enter));
+  float pre_leave[PER], pre_enter[PER];
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int64_t col = c0 + (tid + kFinThreads * j < cols ? tid + kFinThreads * j : 0);
+    pre_leave[j] = partial[(w * 2 + 1) * C + col];        // window w, left over its right edge
+    pre_enter[j] = partial[((w + 1) * 2 + 0) * C + col];  // window w + 1, entered over its left edge
+  }
+  asm volatile("" : "+v"(raw_last), "+v"(raw_next), "+v"(raw_first), "+v"(raw_before), "+v"(raw_q), "+v"(raw_f));
+#pragma unroll
+  for (int j = 0; j < PER; ++j) asm volatile("" : "+v"(pre_leave[j]), "+v"(pre_enter[j]));
   const uint32_t id = raw_last;
   if (id == kNoId || raw_next != id) return;  // no run leaves this window
   // its run began in this window unless the whole window (and the entry before it) has this id
@@ -1057,7 +1067,10 @@ __global__ __launch_bounds__(kFinThreads, 5) void emb_bwd_finish_kernel(
     }
     return;
   }
-  if (tid < cols) {
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    if (tid + kFinThreads * j >= cols) break;
+    const int64_t col = c0 + tid + kFinThreads * j;
     // eight interleaved sums keep eight loads in flight; the order is fixed all the same
     float t[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     int64_t ww = w;
@@ -1070,8 +1083,8 @@ __global__ __launch_bounds__(kFinThreads, 5) void emb_bwd_finish_kernel(
       for (int u = 0; u < 8; ++u) t[u] += v[u];
     }
     if (usual) {  // these came in with the loads above
-      t[0] += pre_leave;
-      t[7] += pre_enter;
+      t[0] += pre_leave[j];
+      t[7] += pre_enter[j];
     } else {
       float v[8];
 #pragma unroll
@@ -1604,7 +1617,8 @@ int bwd_typed(const void *dout, const void *ids, void *dweight, void *dwpe, char
   if constexpr (!std::is_same_v<T, double>) {
     float *partial = reinterpret_cast<float *>(ws + L.off_partial);
     const int64_t windows = n > 0 ? L.n_windows : 0;
-    const int64_t slices = ceil_div(C, (int64_t)kFinThreads);
+    const bool wide = C > kFinWideRow && windows * ceil_div(C, (int64_t)kFinThreads) > kFinMostAtOnce;
+    const int64_t slices = ceil_div(C, (int64_t)kFinThreads * (wide ? 2 : 1));
     const int64_t fin_blocks = windows * slices;
     // The position sums go where the chip is idle: next to the finish workgroups, or next to the reducing ones of a
     // list too short to occupy the chip with those.
@@ -1625,7 +1639,8 @@ int bwd_typed(const void *dout, const void *ids, void *dweight, void *dwpe, char
       if (st != CS_OK) return st;
     }
     if (last_blocks == 0) return CS_OK;
-    emb_bwd_finish_kernel<T><<<dim3((unsigned)last_blocks), dim3(kFinThreads), 0, s>>>(
+    const auto finish = wide ? emb_bwd_finish_kernel<T, 2> : emb_bwd_finish_kernel<T, 1>;
+    finish<<<dim3((unsigned)last_blocks), dim3(kFinThreads), 0, s>>>(
         sorted_id, partial, (T *)dweight, n, C, accumulate, by_freq, fin_blocks, (int)slices, (const T *)dout,
         (T *)dwpe, B, TC, log2_s);
     return launch_status();

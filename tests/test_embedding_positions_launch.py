@@ -81,3 +81,21 @@ def test_positions_of_a_long_list(V, n_batch):
     assert torch.equal(dwte.cpu(), want_t) and torch.equal(dwpe.cpu(), want_p)
     dwte, dwpe = ops.embedding_backward_fused(dout.cuda(), ids.cuda().int(), V, dwte, dwpe)  # nothing to fill
     assert torch.equal(dwte.cpu(), 2 * want_t) and torch.equal(dwpe.cpu(), 2 * want_p)
+
+
+@pytest.mark.parametrize("C", [1020, 1024, 1028, 1100, 1600])  # one column a lane up to 1024, two beyond; a last slice that is not full
+@pytest.mark.parametrize("n,hot", [(1500, 0.5), (13200, 0.0), (13200, 0.5)])  # few workgroups (one column), and more than 2048
+def test_finish_of_wide_rows(C, n, hot):
+    from core_scheduler_amd import ops
+
+    V = 600  # nearly every window is left by a run; a hot id has partial rows of its own to add
+    ids = torch.randint(0, V, (n,), generator=gen(10))
+    ids[torch.rand(n, generator=gen(11)) < hot] = 7
+    dout = torch.randint(-8, 9, (n, C), generator=gen(12)).float()  # whole numbers: every order gives the same sums
+    want = torch.zeros(V, C).index_add_(0, ids, dout)
+    got = ops.embedding_backward(dout.cuda(), ids.cuda(), V)
+    assert torch.equal(got.cpu(), want)
+    assert torch.equal(ops.embedding_backward(dout.cuda(), ids.cuda(), V, dweight=got).cpu(), 2 * want)
+    mean = ops.embedding_backward(dout.cuda(), ids.cuda(), V, scale_grad_by_freq=True).cpu()
+    exact = want.double() / torch.bincount(ids, minlength=V).clamp(min=1).double()[:, None]
+    assert ((mean.double() - exact).abs() <= 2.0 ** -22 * exact.abs()).all()  # a reciprocal and a product, rounded each

@@ -572,14 +572,16 @@ __device__ __forceinline__ void ln_columns_direct(const TDY *__restrict__ dy, co
   const int col = tile * kLnFinCols + cx;
   const int64_t at = col < C ? col : C - 1;
   float sg = 0.f, sb = 0.f;
-  for (int p = ry; p < side.nparts; p += kLnFinRows) {
+  static_assert(kWave == 2 * kLnFinCols, "a wave has the columns of two partial rows");
+  auto add = [&](int p, auto all_rows) {
+    constexpr bool full = decltype(all_rows)::value;
     TDY d[RPP];
     TX v[RPP];
     float mu[RPP], rs[RPP];
 #pragma unroll
     for (int w = 0; w < RPP; ++w) {
       const int64_t row = (int64_t)p * RPP + w;
-      const int64_t rowc = row < rows ? row : rows - 1;
+      const int64_t rowc = full || row < rows ? row : rows - 1;
       d[w] = dy[rowc * C + at];
       v[w] = x[rowc * C + at];
       mu[w] = mean[rowc];
@@ -588,15 +590,29 @@ __device__ __forceinline__ void ln_columns_direct(const TDY *__restrict__ dy, co
     float pg = 0.f, pb = 0.f;
 #pragma unroll
     for (int w = 0; w < RPP; ++w) {
-      const bool live = (int64_t)p * RPP + w < rows;
-      // both masked, as in ln_columns_wide
-      const float xh = live ? (to_acc(v[w]) - mu[w]) * rs[w] : 0.f;
-      const float dv = live ? to_acc(d[w]) : 0.f;
+      float xh = (to_acc(v[w]) - mu[w]) * rs[w], dv = to_acc(d[w]);
+      if constexpr (!full) {
+        // both masked, as in ln_columns_wide, and only now: under the condition the loads would wait for one another
+        asm volatile("" : "+v"(xh), "+v"(dv));
+        const bool live = (int64_t)p * RPP + w < rows;
+        xh = live ? xh : 0.f;
+        dv = live ? dv : 0.f;
+      }
       pg += __builtin_fmaf(dv, xh, 0.f);
       pb += dv;
     }
     sg += pg;
     sb += pb;
+  };
+  // The last partial row may lack rows.  A wave stands in for two neighbouring ones and takes both the same way: apart
+  // they were two trips to memory ([123,768] bf16 4.5 us against 3.8).
+  const int whole = (int)(rows / RPP);
+  for (int p = ry; p < side.nparts; p += kLnFinRows) {
+    if ((p | 1) < whole) {
+      add(p, std::true_type{});
+    } else {
+      add(p, std::false_type{});
+    }
   }
   sub[ry * kLnFinCols + cx] = sg;
   sub[(kLnFinRows + ry) * kLnFinCols + cx] = sb;

@@ -9,7 +9,9 @@ import torch
 
 from core_scheduler_amd import ops
 
-NATIVE = [n for n in vars(ops) if n.startswith("_") and n[1:] in dir(ops._calls) and not n.startswith("__")]
+NATIVE = ["_" + n for n in ("add_layernorm_forward", "embedding_backward", "embedding_backward_fused", "embedding_forward",
+                            "embedding_forward_add", "fused_classifier", "gelu_backward", "gelu_forward", "layernorm_backward",
+                            "layernorm_backward_chained", "layernorm_forward")]
 
 
 class Sub(torch.Tensor):
@@ -17,7 +19,10 @@ class Sub(torch.Tensor):
 
 
 def test_every_native_form_is_built_and_used():
-    assert sorted(n[1:] for n in NATIVE) == sorted(n for n in dir(ops._calls) if not n.startswith("_"))
+    assert ops._calls is not None
+    assert NATIVE == sorted("_" + n for n in dir(ops._calls) if not n.startswith("_"))
+    for n in NATIVE:
+        assert getattr(ops, n) is getattr(ops._calls, n[1:])
 
 
 def test_a_broken_extension_is_reported(monkeypatch):
@@ -78,19 +83,30 @@ def _calls(dt):
         c.flush()
         return a + b
 
-    return [lambda: ops.gelu_forward(x, "tanh"), lambda: ops.gelu_forward(x[:0]), lambda: ops.gelu_backward(dy, x),
-            lambda: ops.layernorm_forward(x, gamma), lambda: ops.layernorm_forward(x, gamma, beta, 1e-3, torch.float32),
-            lambda: ops.layernorm_forward(x, gamma, beta, 1), lambda: ops.add_layernorm_forward(x, res, gamma, beta),
-            lambda: ops.layernorm_backward(dy, x, mean, rstd, gamma),
-            lambda: ops.layernorm_backward(dy, x, mean, rstd, gamma, dresidual=res),
-            lambda: ops.layernorm_backward(dy, x, mean, rstd, gamma, need_dbeta=False), chain,
-            lambda: ops.embedding_forward(w, ids), lambda: ops.embedding_forward(w, ids.int()[0, 0]),
-            lambda: ops.embedding_forward_add(w, p, ids), lambda: ops.embedding_backward(dy, ids, 50, padding_idx=4),
-            lambda: ops.embedding_backward(dy, ids, 50, scale_grad_by_freq=True),
-            lambda: ops.embedding_backward_fused(dy, ids, 50), lambda: ops.fused_classifier(logits, t, 70, reduction="sum"),
-            lambda: ops.fused_classifier(logits, t, 70, class_weight=cw, dlogits_dtype=torch.float32),
-            lambda: ops.fused_classifier(logits, t, want_dlogits=False, reduction="none", dloss=2),
-            lambda: ops.gelu_forward(torch.nn.Parameter(x)), lambda: ops.gelu_forward(x.as_subclass(Sub))]
+    # (call, the native forms that take it: a chain's calls are several)
+    return [(lambda: ops.gelu_forward(x, "tanh"), "gelu_forward"), (lambda: ops.gelu_forward(x[:0]), "gelu_forward"),
+            (lambda: ops.gelu_backward(dy, x), "gelu_backward"), (lambda: ops.layernorm_forward(x, gamma), "layernorm_forward"),
+            (lambda: ops.layernorm_forward(x, gamma, beta, 1e-3, torch.float32),
+             "layernorm_forward" if dt != torch.float64 else None),
+            (lambda: ops.layernorm_forward(x, gamma, beta, 1), None),
+            (lambda: ops.add_layernorm_forward(x, res, gamma, beta), "add_layernorm_forward"),
+            (lambda: ops.layernorm_backward(dy, x, mean, rstd, gamma), "layernorm_backward"),
+            (lambda: ops.layernorm_backward(dy, x, mean, rstd, gamma, dresidual=res), "layernorm_backward"),
+            (lambda: ops.layernorm_backward(dy, x, mean, rstd, gamma, need_dbeta=False), None),
+            # (fp64 rows have no split form: the chain's Python body asks for the whole call instead)
+            (chain, "layernorm_backward_chained" if dt != torch.float64 else "layernorm_backward"),
+            (lambda: ops.embedding_forward(w, ids), "embedding_forward"),
+            (lambda: ops.embedding_forward(w, ids.int()[0, 0]), "embedding_forward"),
+            (lambda: ops.embedding_forward_add(w, p, ids), "embedding_forward_add"),
+            (lambda: ops.embedding_backward(dy, ids, 50, padding_idx=4), "embedding_backward"),
+            (lambda: ops.embedding_backward(dy, ids, 50, scale_grad_by_freq=True), "embedding_backward"),
+            (lambda: ops.embedding_backward_fused(dy, ids, 50), "embedding_backward_fused"),
+            (lambda: ops.fused_classifier(logits, t, 70, reduction="sum"), "fused_classifier"),
+            (lambda: ops.fused_classifier(logits, t, 70, class_weight=cw, dlogits_dtype=torch.float32),
+             "fused_classifier" if dt != torch.float64 else None),
+            (lambda: ops.fused_classifier(logits, t, want_dlogits=False, reduction="none", dloss=2), None),
+            (lambda: ops.gelu_forward(torch.nn.Parameter(x)), "gelu_forward"),
+            (lambda: ops.gelu_forward(x.as_subclass(Sub)), None)]
 
 
 def _raises(dt):
@@ -114,6 +130,16 @@ def _raises(dt):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float64])
 def test_same_results_and_refusals(dt, monkeypatch):
+    taken = []  # the native forms that took a call
+
+    def noted(name, native):
+        def call(*args):
+            out = native(*args)
+            if out is not NotImplemented:
+                taken.append(name[1:])
+            return out
+        return call
+
     def outcomes(calls):
         out = []
         for call in calls:
@@ -125,13 +151,23 @@ def test_same_results_and_refusals(dt, monkeypatch):
                 out.append((type(e), str(e)))
         return out
 
-    native = outcomes(_calls(dt)), outcomes(_raises(dt))
+    calls, raises = _calls(dt), _raises(dt)
+    for n in NATIVE:
+        monkeypatch.setattr(ops, n, noted(n, getattr(ops, n)))
+    native = []
+    for call, form in calls:
+        taken.clear()
+        native += outcomes([call])
+        assert set(taken) == ({form} if form and not isinstance(native[-1], tuple) else set()), (form, taken, native[-1])
+    taken.clear()
+    refused = outcomes(raises)
+    assert not taken
     with torch.inference_mode():
         assert ops.gelu_forward(torch.ones(8, device="cuda")).is_inference()
     for n in NATIVE:
         monkeypatch.setattr(ops, n, lambda *args: NotImplemented)
-    plain = outcomes(_calls(dt)), outcomes(_raises(dt))
-    for a, b in zip(native[0], plain[0]):
+    plain = outcomes([call for call, _ in calls])
+    for a, b in zip(native, plain):
         assert len(a) == len(b) and all((p is None and q is None) or (p[:3] == q[:3] and torch.equal(p[3], q[3]))
                                         if not isinstance(p, (type, str)) else p == q for p, q in zip(a, b)), (a, b)
-    assert native[1] == plain[1] and all(isinstance(r, tuple) for r in native[1]), native[1]
+    assert refused == outcomes(raises) and all(isinstance(r, tuple) for r in refused), refused

@@ -1069,33 +1069,34 @@ __global__ __launch_bounds__(kFinThreads, 5) void emb_bwd_finish_kernel(
   }
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
-    if (tid + kFinThreads * j >= cols) break;
-    const int64_t col = c0 + tid + kFinThreads * j;
-    // eight interleaved sums keep eight loads in flight; the order is fixed all the same
-    float t[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    int64_t ww = w;
-    // every window before the last is left over its right edge (slot 1)
-    for (; ww + 8 <= w_end; ww += 8) {
-      float v[8];
+    if (tid + kFinThreads * j < cols) {
+      const int64_t col = c0 + tid + kFinThreads * j;
+      // eight interleaved sums keep eight loads in flight; the order is fixed all the same
+      float t[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      int64_t ww = w;
+      // every window before the last is left over its right edge (slot 1)
+      for (; ww + 8 <= w_end; ww += 8) {
+        float v[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = partial[((ww + u) * 2 + 1) * C + col];
+        for (int u = 0; u < 8; ++u) v[u] = partial[((ww + u) * 2 + 1) * C + col];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) t[u] += v[u];
+        for (int u = 0; u < 8; ++u) t[u] += v[u];
+      }
+      if (usual) {  // these came in with the loads above
+        t[0] += pre_leave[j];
+        t[7] += pre_enter[j];
+      } else {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = ww + u < w_end ? partial[((ww + u) * 2 + 1) * C + col] : 0.f;
+#pragma unroll
+        for (int u = 0; u < 7; ++u) t[u] += v[u];  // at most seven windows are left
+        t[7] += partial[(w_end * 2 + 0) * C + col];  // the run that ends there came in over the left edge
+      }
+      float total = (((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]))) * inv;
+      if (accumulate) total += to_acc(dst[col]);
+      dst[col] = from_acc<T>(total);
     }
-    if (usual) {  // these came in with the loads above
-      t[0] += pre_leave[j];
-      t[7] += pre_enter[j];
-    } else {
-      float v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = ww + u < w_end ? partial[((ww + u) * 2 + 1) * C + col] : 0.f;
-#pragma unroll
-      for (int u = 0; u < 7; ++u) t[u] += v[u];  // at most seven windows are left
-      t[7] += partial[(w_end * 2 + 0) * C + col];  // the run that ends there came in over the left edge
-    }
-    float total = (((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]))) * inv;
-    if (accumulate) total += to_acc(dst[col]);
-    dst[col] = from_acc<T>(total);
   }
 }
 

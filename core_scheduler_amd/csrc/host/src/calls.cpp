@@ -3,13 +3,13 @@
 //
 // A step's small ops cost more host than device time, and most of that was Python's: 1.3 us for an allocation,
 // 3-4 us of argument checks and ctypes conversions for a call, against 2.8 us for a launch, which stays.  One norm of
-// 77 rows, forward and backward: 30.7 -> 16.7 us; the 25 calls of two short blocks 232 -> 121-150; embedding forward
-// and backward of 4000 tokens 23 -> 17.6 (device time again).
+// 77 rows, forward and backward: 30.7 -> 16.7 us (12 since its backward is one launch); the 25 calls of two short blocks
+// 237 -> 115; embedding forward and backward of 4000 tokens 23 -> 17.7 (device time again).
 //
 // Every function takes the arguments of its counterpart in ops.py by position and returns NotImplemented for
-// anything but the plain case: exact torch tensors, contiguous, on the current device, of matching shapes and
-// supported types, exact ints and floats, no torch mode active.  ops.py then goes its own way, which checks,
-// raises or runs as ever; nothing is refused here.
+// anything but the plain case: exact torch tensors, contiguous, on the current device, of exactly matching shapes and
+// supported types, exact ints and floats, no torch mode active.  ops.py then goes its own way, which checks, raises
+// or runs as ever; nothing is refused here.
 #define PY_SSIZE_T_CLEAN
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/ops/empty.h>

@@ -1560,7 +1560,8 @@ int launch_rows(const void *logits, void *dlogits, const int64_t *targets, float
     // Unpadded rows that fill little of the streaming plan take two sweeps: with fp32 gradients of 16-bit logits rows
     // of up to six of its 13 accesses ([1030,18001] bf16 39.6 us streamed, 35.0 in two sweeps, [257,22001] 19.1 / 17.1,
     // [3100,22001] 100 / 103; [3100,26001] 108 / 116), and the loss alone of more than two rows per CU of four to six
-    // of its seven ([600,38001] 21.4 / 19.5, [860,46001] 27.8 / 27.0; but [600,50257] 22.3 / 23.5).
+    // of its seven ([600,38001] 21.4 / 19.5, [860,46001] 27.8 / 27.0; but [600,50257] 22.3 / 23.5).  So few rows come here
+    // for the loss alone only in separate phases, or with a workspace that has no room for their splits (loss_splits).
     const bool sparse = sizeof(TD) > sizeof(T) ? row_stride <= 24 * 1024
                                                : sizeof(T) == 2 && dlogits == nullptr && N > 2 * cus &&
                                                      row_stride > 32 * 1024 && row_stride <= 48 * 1024;

@@ -909,10 +909,12 @@ __global__ __launch_bounds__(kRedThreads, 2048 / kRedThreads) void emb_bwd_reduc
 // 32768 x 768 fp32 93.5 -> 89.9; in the reduce launch of such a list they cost what they save.  256 columns per
 // workgroup, so that a hot row's sum is shared by several: 14.2 us with the positions at 16384 x 1600; 512
 // columns 14.4, 1024 15.2; positions last 17.3.  PER: columns a lane; two for many windows of more than 1024 columns,
-// whose workgroups are more than the chip holds at once if most windows are left by a run (backward, one / two: 16384 x
-// 1600 bf16 into 1000 rows 37.6 / 36.2, x 2048 fp32 59.5 / 54.4; Zipf ids of 50257 rows 48.5 / 48.5; but 32768 x 768 48.5 /
-// 50.0, and one id in every entry 42.4 / 51.2).  dout is read past the caches in both launches: kept there it
-// pushes out what the next call reads (this launch 14.2 -> 12.3 us, but the next gather 12.9 -> 20.1).
+// whose workgroups are more than the chip holds at once if most windows are left by a run (backward, one / two:
+// 16384 x 1600 bf16 into 1000 rows 37.6 / 36.2, x 2048 fp32 59.5 / 54.4; Zipf ids of 50257 rows 48.5 / 48.5; but
+// 32768 x 768 48.5 / 50.0, and one id in every entry 42.4 / 51.2).  dout is read past the caches in both launches:
+// kept there it pushes out what a call right behind reads (this launch 14.2 -> 12.3 us, but a gather of the same
+// tokens next 12.9 -> 20.1).  That weighs calls back to back; where other work lies between them, the next gather
+// finds nothing in the caches either way.
 template <typename T, int PER>
 __global__ __launch_bounds__(kFinThreads, 5) void emb_bwd_finish_kernel(
     const uint32_t *__restrict__ sorted_id, const float *__restrict__ partial,
@@ -1100,8 +1102,8 @@ __global__ __launch_bounds__(kFinThreads, 5) void emb_bwd_finish_kernel(
   }
 }
 
-// Standalone position-table gradient.  The vector form is positions_block on its own (the
-// fused call runs it inside its last launch); the scalar form takes any C and any alignment.
+// Standalone position-table gradient.  The vector form is positions_block on its own (the fused call runs it inside
+// one of its launches: see kPosEarlyWindows and kPosFewFill); the scalar form takes any C and any alignment.
 template <typename T>
 __global__ __launch_bounds__(kTile) void emb_bwd_positions_vec_kernel(const T *__restrict__ dout,
                                                                       T *__restrict__ dwpe, int64_t B,
@@ -1153,11 +1155,12 @@ __global__ __launch_bounds__(kThreads) void emb_bwd_positions_kernel(const T *__
 // ------------------------------------- backward: rows that are not whole vectors
 // fp64, and rows that are not whole aligned 16-byte vectors: the same two levels in double, a column per lane.  (The
 // wave-wide loads are contiguous, whatever the alignment; fp32 sums over vectors would round where these do not.)
-// A workgroup adds one window's 64 sorted entries, a wave's worth of ids, for 256 columns; 16 rows are in
-// flight.  Further workgroups of the launch sum the position table.  One workgroup per table row, which walked that row's entries one load at a time, was the path before: a
-// hot row was a chain of thousands of trips to memory.  us per gather + backward, before / now: bf16 8192 Zipf tokens x 301,
-// 50257 rows 650 / 40, uniform 122 / 39; 16384 x 1599 3213 / 86, uniform 245 / 95; 32768 x 769, 100000 rows 6834 / 106,
-// uniform 373 / 110; fp32 16384 x 1599 3489 / 124.  (Short lists: see emb_bwd_runs_ragged_kernel.)
+// A workgroup adds one window's 64 sorted entries, a wave's worth of ids, for 256 columns; 16 rows are in flight.
+// Further workgroups of the launch sum the position table.  One workgroup per table row, which walked that row's
+// entries one load at a time, was the path before: a hot row was a chain of thousands of trips to memory.  us per
+// gather + backward, before / now: bf16 8192 Zipf tokens x 301, 50257 rows 650 / 40, uniform 122 / 39; 16384 x 1599
+// 3213 / 86, uniform 245 / 95; 32768 x 769, 100000 rows 6834 / 106, uniform 373 / 110; fp32 16384 x 1599 3489 / 124.
+// (Short lists: see emb_bwd_runs_ragged_kernel.)
 constexpr int kRagWindow = kWave;
 constexpr int kRagThreads = 256;
 constexpr int kRagInFlight = 16;
@@ -1236,10 +1239,10 @@ __global__ __launch_bounds__(kRagThreads) void emb_bwd_reduce_ragged_kernel(
 // behind this one are needed.  The additions are in the order of the windows' either way.
 //
 // Whole up to 256 entries, where a list of one id is no slower than in windows (n = 256 x 301: 15.8 us against 15.4;
-// n = 512 26 / 16); with windows up to 3072, as long as the workgroups are few enough to run at once.  us, windows' walk / this, bf16
-// x 301, table of 1000 rows, uniform: n = 100 21.0 / 6.2, 256 21.2 / 6.5, 500 21.7 / 9.8, 1000 22.2 / 11.6, 3000 20.9 /
-// 15.8; of one id: n = 500 15.5 / 13.7, 1000 17.1 / 17.3, 3000 21.5 / 23.6; a table of 50257 rows, Zipf: n = 1000 26.2 /
-// 15.5, 3000 27.3 / 18.5; x 1603, uniform: n = 1000 23.2 / 16.6, 2000 21.8 / 21.4, 4000 23.5 / 30.8.
+// n = 512 26 / 16); with windows up to 3072, as long as the workgroups are few enough to run at once.  us, windows'
+// walk / this, bf16 x 301, table of 1000 rows, uniform: n = 100 21.0 / 6.2, 256 21.2 / 6.5, 500 21.7 / 9.8, 1000 22.2 /
+// 11.6, 3000 20.9 / 15.8; of one id: n = 500 15.5 / 13.7, 1000 17.1 / 17.3, 3000 21.5 / 23.6; a table of 50257 rows,
+// Zipf: n = 1000 26.2 / 15.5, 3000 27.3 / 18.5; x 1603, uniform: n = 1000 23.2 / 16.6, 2000 21.8 / 21.4, 4000 23.5 / 30.8.
 constexpr int64_t kRagWholeEntries = 256;
 constexpr int64_t kRagFewEntries = 3072;
 constexpr int64_t kRagFewWorkgroups = 8192;
@@ -1388,9 +1391,9 @@ BwdLayout bwd_layout(int64_t n, int64_t C, int64_t num_weights) {
 }
 
 // Ragged or unaligned rows of up to so many elements in all are gathered element by element: every lane has one, where
-// vectors leave most of the chip idle.  us, elements / vectors, bf16: 300 x 301 2.9 / 3.3, 1500 x 301 3.3 / 3.5, 2000 x 301
-// 3.6 / 3.5, 4000 x 301 4.4 / 3.7; with positions 3.0 / 3.6, 3.6 / 3.8, 3.9 / 3.8; 8000 x 65 3.4 / 3.7, 16000 x 65 4.1 /
-// 3.9; fp32 1500 x 301 3.4 / 3.5, 600 x 1003 3.7 / 3.6.
+// vectors leave most of the chip idle.  us, elements / vectors, bf16: 300 x 301 2.9 / 3.3, 1500 x 301 3.3 / 3.5, 2000 x
+// 301 3.6 / 3.5, 4000 x 301 4.4 / 3.7; with positions 3.0 / 3.6, 3.6 / 3.8, 3.9 / 3.8; 8000 x 65 3.4 / 3.7, 16000 x 65
+// 4.1 / 3.9; fp32 1500 x 301 3.4 / 3.5, 600 x 1003 3.7 / 3.6.
 constexpr int64_t kFewElements = 1 << 19;
 
 template <typename T, typename IdxT, bool ADD>

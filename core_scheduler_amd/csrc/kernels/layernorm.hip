@@ -2218,12 +2218,13 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
   const auto clear_of = [&](const void *out, size_t bytes, const void *in, size_t in_bytes) {
     return out == nullptr || in == nullptr || !overlap(out, bytes, in, in_bytes);
   };
-  const bool dx_apart = clear_of(dx, n * sizeof(TDX), dy, n * sizeof(TDY)) && clear_of(dx, n * sizeof(TDX), x, n * sizeof(TX));
+  const size_t out = n * sizeof(TDX);
+  const bool dx_apart = clear_of(dx, out, dy, n * sizeof(TDY)) && clear_of(dx, out, x, n * sizeof(TX));
   bool apart = dx_apart;
   for (const void *sum : {(const void *)dgamma, (const void *)dbeta})
     apart = apart && clear_of(sum, params, dy, n * sizeof(TDY)) && clear_of(sum, params, x, n * sizeof(TX)) &&
-            clear_of(sum, params, mean, stat) && clear_of(sum, params, rstd, stat) && clear_of(sum, params, gamma, params) &&
-            clear_of(sum, params, dres, n * sizeof(TDX));
+            clear_of(sum, params, mean, stat) && clear_of(sum, params, rstd, stat) &&
+            clear_of(sum, params, gamma, params) && clear_of(sum, params, dres, out);
   BwdPlan plan = bwd_plan(rows, C, x_dtype, aligned, {dx != nullptr, want_dp, apart && phase == kBwdWhole});
   if (phase == kBwdRowsOnly && (plan.kind == kBwdNone || !plan.two_calls || std::is_same_v<TX, double>))
     return aligned ? CS_ERR_UNSUPPORTED : CS_ERR_MISALIGNED;

@@ -217,7 +217,8 @@ int cs_layernorm_forward(const void *x, const void *gamma, const void *beta,
 size_t cs_layernorm_backward_workspace_bytes(int64_t rows, int64_t C);
 /* Any of dx, dgamma, dbeta may be NULL (the reference's output masks
  * {1,0,0}, {0,1,1}, {0,1,0}); dgamma/dbeta are stored in param_dtype and,
- * when accumulate != 0, added to what is already there.  dy is stored as
+ * when accumulate != 0, added to what is already there.  dx may be dy or x,
+ * and dgamma or dbeta an input, at the price of a further launch.  dy is stored as
  * dy_dtype (x_dtype or CS_F32), dx as dx_dtype (same choice).  workspace
  * is needed whenever dgamma or dbeta is requested; its size never falls as
  * rows grows, so one buffer sized for the most rows serves every batch. */
@@ -289,10 +290,12 @@ int cs_layernorm_backward_finalize(const void *partials, int64_t partial_rows,
                                    void *stream);
 
 /* 1 where cs_layernorm_backward / _add, asked for dx and the parameter gradients
- * with every pointer on a 16-byte boundary, is a single launch: few enough rows
- * that the column sums are taken straight from them.  A sequence of such calls
- * gains nothing from the split above or the combined form below: the launch of
- * one with an earlier call's sums takes longer. */
+ * with every pointer on a 16-byte boundary and no output over an input, is a
+ * single launch although the rows have a split form (partial_rows > 0): few
+ * enough rows that the column sums are taken straight from them.  A sequence of
+ * such calls gains nothing from the split above or the combined form below: the
+ * launch of one with an earlier call's sums takes longer.  0 for rows without a
+ * split form, of which few are a single launch as well. */
 int cs_layernorm_backward_one_launch(int64_t rows, int64_t C, int x_dtype);
 
 /* cs_layernorm_backward_rows that also does an EARLIER call's

@@ -32,7 +32,8 @@
 //                   is short, of launch 1 where that has little to fill).
 // A list of at most 8192 entries skips 1 and 2: one launch ranks every key by
 // comparing it with all others (see emb_bwd_rank_kernel), and does the zero
-// fill next to that.
+// fill next to that.  A list of at most 1024 entries of whole aligned vectors
+// needs no sort: see emb_bwd_list_kernel.
 // The traffic that matters is the dense write of dweight (V*C elements), one
 // read of dout and a second write of the indexed rows.
 #include "common.hpp"
@@ -648,6 +649,10 @@ __global__ __launch_bounds__(kRankThreads) void emb_bwd_rank_kernel(
   }
 }
 
+__device__ __forceinline__ uint32_t lane_value(uint32_t v, int lane) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, lane);
+}
+
 // ------------------------------------------------------ backward: reduction
 constexpr int kOwn = 4;                         // sorted entries per wave
 constexpr int kRedWaves = kWindow / kOwn;       // 8
@@ -1102,6 +1107,272 @@ __global__ __launch_bounds__(kFinThreads, 5) void emb_bwd_finish_kernel(
   }
 }
 
+// -------------------------------------------- backward: a short list in one launch
+// Up to kListMost entries of whole aligned vectors: no sort.  Four waves own an entry and compare the list, which the
+// workgroup holds in its LDS, with the entry's id: they know how many ids are below it, so its place in the sorted
+// list, and where the others of its segment are.  If its run of the segment starts there, they add the run's rows: up
+// to kListWhole entries a run is the whole segment, in longer lists it is cut at the edges of the windows below and
+// emb_bwd_finish_kernel adds the partial rows, as it does for the longer lists.  Further workgroups of the launch sum
+// the position table, and others write zeros to the rows that no entry names.
+//
+// Bound by the launch and three trips to memory (the list, the rows, the stores), or by the zeros of a large table.
+// us per call, rank + reduce + finish launches before / now, Zipf ids: [1,123] x 768 bf16 into 50257 rows 21.1 / 14.8 (its
+// 77 MB of zeros alone 11.9), [9,19] x 128 into 5238 10.1 / 6.1, 16 x 64 into 1000 8.2 / 5.6, [16,41] x 640 into 32434
+// 14.4 / 11.7, [1,500] x 512 fp32 added to 4000 rows 12.9 / 8.8, [1,1024] x 768 into 1000 rows 12.3 / 10.8 and into 50257
+// 22.1 / 21.2.  Longer lists are left to the sort: the comparisons grow with the square, and a hot id's runs gather
+// where its tokens are (all of 8192 x 768 this way: 26 / 49).  One id in every entry, the longest runs there are: 128
+// entries 21.0 / 18.4, 1024 entries 12.3 / 12.9.
+constexpr int kListThreads = 512;
+constexpr int kListGroup = 4;  // waves that share an entry
+constexpr int kListEntries = kListThreads / kWave / kListGroup;
+constexpr int kListMost = 1024;
+constexpr int kListWhole = 192;  // (one id in every entry, x 768: 192 entries 21 us before and now, 256 would take 25)
+constexpr int kListVecs = 2;  // vectors a lane has of each row: a slice of the columns is 128 of them
+constexpr int64_t kListBlocks = 512;  // no more slices than make so many workgroups (1024 x 1600: 1024 41.7 us, 512 38.0)
+constexpr int64_t kListFillBytes = 64 << 10;  // zeros a workgroup writes (n = 123 x 768, 77 MB: 32 KB 14.4 us, 64 14.6, 256 16.0)
+constexpr int kListFillRows = 4096;  // most table rows a zero-filling workgroup looks after (a bit each in the LDS)
+
+template <typename IdxT>
+__device__ __forceinline__ uint32_t usable_id(IdxT raw, int64_t num_weights, int64_t padding_idx) {
+  const int64_t id = (int64_t)raw;
+  return id >= 0 && id < num_weights && id != padding_idx ? (uint32_t)id : kNoId;
+}
+
+// Launch layout, in block order:
+//   [0, entry_blocks)           kListEntries entries and a slice of the columns each
+//   + positions.blocks          position-table gradient
+//   + the rest                  zeros to the rows [blk * fill_rows, (blk + 1) * fill_rows) that no entry names
+template <typename T, typename IdxT>
+__global__ __launch_bounds__(kListThreads, 4) void emb_bwd_list_kernel(
+    const T *__restrict__ dout, const IdxT *__restrict__ ids, T *__restrict__ dweight, uint32_t *__restrict__ sorted_id,
+    float *__restrict__ partial, int n, int C, int64_t num_weights, int64_t padding_idx, int accumulate, int by_freq,
+    int entry_blocks, int slices, int fill_rows, Positions<T> positions) {
+  constexpr int VN = Vec16<T>::n;
+  constexpr int kWaves = kListThreads / kWave;
+  constexpr int kPerLane = kListMost / kListThreads;
+  constexpr int kChunks = kListMost / (4 * kWave);  // lane l looks at entries [4 l, 4 l + 4) of every chunk of 256
+  // the waves' sums (an f32x4 a lane and slot), or the position sums' slices, or a bit per row
+  constexpr int kPieces = VN / 4;
+  __shared__ f32x4 lds[kListThreads * kPosLdsBytesPerLane / sizeof(f32x4)];
+  static_assert(kPieces * kListThreads * sizeof(f32x4) <= sizeof(lds) && sizeof(lds) * 8 >= (size_t)kListFillRows, "they fit");
+  __shared__ u32x4 listed[kListMost / 4];
+  __shared__ uint16_t rows_of[kWaves][kListWhole];
+  __shared__ int long_run[kListEntries];
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = tid >> 6;
+  const int nvec = C / VN;
+  const int64_t blk = blockIdx.x;
+  if (blk >= entry_blocks && blk < entry_blocks + positions.blocks) {
+    positions_block<T, kListThreads>(positions.dout, positions.dwpe, blk - entry_blocks, positions.B, positions.TC,
+                                     positions.accumulate, positions.log2_slices, lds, tid);
+    return;
+  }
+
+  uint32_t id[kPerLane];
+  {
+    IdxT raw[kPerLane] = {};
+    if (n > 0) {
+#pragma unroll
+      for (int u = 0; u < kPerLane; ++u) {
+        const int i = u * kListThreads + tid;
+        raw[u] = ids[i < n ? i : n - 1];  // no load under a condition: they all go out at once
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kPerLane; ++u)
+      id[u] = u * kListThreads + tid < n ? usable_id(raw[u], num_weights, padding_idx) : kNoId;
+  }
+
+  if (blk >= entry_blocks) {  // ---- zeros
+    uint32_t *named = reinterpret_cast<uint32_t *>(lds);
+    const int64_t row0 = (blk - entry_blocks - positions.blocks) * fill_rows;
+    const int rows = num_weights - row0 < fill_rows ? (int)(num_weights - row0) : fill_rows;
+    for (int i = tid; i < (rows + 31) / 32; i += kListThreads) named[i] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kPerLane; ++u) {
+      const int64_t r = (int64_t)id[u] - row0;
+      if (id[u] != kNoId && r >= 0 && r < rows) atomicOr(&named[r >> 5], 1u << (r & 31));
+    }
+    __syncthreads();
+    T *base = dweight + row0 * C;
+    const u32x4 z = {0u, 0u, 0u, 0u};
+    const int total = rows * nvec;  // list_rows() bounds it
+    const int step_rows = kListThreads / nvec, step_vecs = kListThreads % nvec;
+    int row = tid / nvec, vec = tid - row * nvec;
+#pragma unroll 4
+    for (int f = tid; f < total; f += kListThreads) {
+      if (!((named[row >> 5] >> (row & 31)) & 1u)) store_stream(reinterpret_cast<u32x4 *>(base) + f, z);
+      row += step_rows;
+      vec += step_vecs;
+      if (vec >= nvec) {
+        vec -= nvec;
+        ++row;
+      }
+    }
+    return;
+  }
+
+  uint32_t *list = reinterpret_cast<uint32_t *>(listed);
+#pragma unroll
+  for (int u = 0; u < kPerLane; ++u) list[u * kListThreads + tid] = id[u];
+  __syncthreads();
+
+  // ---- the group's entry: its place among the sorted, and its segment
+  const int entry = wave / kListGroup, member = wave % kListGroup;
+  const int pair = (int)blk / slices, slice = (int)blk - pair * slices;
+  const int p = pair * kListEntries + entry;
+  const uint32_t my_id = p < n ? list[p] : kNoId;
+  uint32_t from[kChunks];  // the entries with this id, from this one on: a bit each
+  int below = 0, before = 0, after = 0;
+#pragma unroll
+  for (int c = 0; c < kChunks; ++c) {
+    const u32x4 v = listed[c * kWave + lane];
+    uint32_t m = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      m |= v[k] == my_id ? 1u << k : 0u;
+      below += v[k] < my_id ? 1 : 0;
+    }
+    const int at = p - (c * kWave + lane) * 4;  // this entry's bit, if it is one of the four
+    const uint32_t earlier = at >= 4 ? m : at <= 0 ? 0u : m & ((1u << at) - 1u);
+    from[c] = m & ~earlier;
+    before += __popc(earlier);
+    after += __popc(from[c]);
+  }
+  {  // a wave's counts are below 2^15: two to a register
+    const int two = wave_reduce(below | before << 16, SumOp{});
+    below = two & 0xFFFF;
+    before = two >> 16;
+    after = wave_reduce(after, SumOp{});
+  }
+  const int q = below + before;
+  const int w = q / kWindow;
+  const bool in_windows = n > kListWhole;
+  if (in_windows && p < n && slice == 0 && member == 0 && lane == 0) sorted_id[q] = my_id;
+  const bool leads = my_id != kNoId && (before == 0 || (in_windows && q % kWindow == 0));
+  const int edge = in_windows ? (w + 1) * kWindow : q + after;
+  const bool seg_ends = q + after <= edge;
+  const bool whole = before == 0 && seg_ends;
+  const int run = !leads ? 0 : seg_ends ? after : edge - q;
+  if (member == 0 && lane == 0) long_run[entry] = run > 1;
+  uint16_t *rows = rows_of[wave];  // every wave notes the run's rows for itself
+  if (run == 1) {
+    if (lane == 0) rows[0] = (uint16_t)p;
+  } else if (run > 1) {
+    int first = 0;
+#pragma unroll
+    for (int c = 0; c < kChunks; ++c) {
+      const uint64_t lanes_below = (1ull << lane) - 1ull;
+      int at = first;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint64_t b = __ballot((from[c] >> k) & 1u);
+        at += __popcll(b & lanes_below);
+        first += __popcll(b);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if ((from[c] >> k) & 1u) {
+          if (at < run) rows[at] = (uint16_t)((c * kWave + lane) * 4 + k);
+          ++at;
+        }
+      }
+    }
+  }
+  __syncthreads();
+
+  // ---- the rows
+  const float inv = by_freq ? 1.0f / (float)(before + after) : 1.0f;
+  T *dst = dweight + (int64_t)my_id * C;
+  float *dst_partial = partial + ((int64_t)w * 2 + (seg_ends ? 0 : 1)) * C;
+  auto finish = [&](int at, const float(&sum)[VN]) {
+    if (whole) {
+      Vec16<T> o;
+      if (accumulate) {
+        const Vec16<T> old = load16(dst + (int64_t)at * VN);
+#pragma unroll
+        for (int k = 0; k < VN; ++k) o.e[k] = from_acc<T>(to_acc(old.e[k]) + sum[k] * inv);
+      } else {
+#pragma unroll
+        for (int k = 0; k < VN; ++k) o.e[k] = from_acc<T>(sum[k] * inv);
+      }
+      store16_stream(dst + (int64_t)at * VN, o);
+    } else {
+#pragma unroll
+      for (int h = 0; h < kPieces; ++h)
+        *reinterpret_cast<f32x4 *>(dst_partial + (int64_t)at * VN + 4 * h) =
+            f32x4{sum[4 * h], sum[4 * h + 1], sum[4 * h + 2], sum[4 * h + 3]};
+    }
+  };
+  if (run == 1) {  // the waves share the columns
+    const T *src = dout + (int64_t)p * C;
+    for (int at = (slice * kListGroup + member) * kWave + lane; at < nvec; at += slices * kListGroup * kWave) {
+      const Vec16<T> v = load16_stream(src + (int64_t)at * VN);
+      float sum[VN];
+#pragma unroll
+      for (int k = 0; k < VN; ++k) sum[k] = 0.f + to_acc(v.e[k]);
+      finish(at, sum);
+    }
+  }
+  bool any_long = false;
+#pragma unroll
+  for (int e = 0; e < kListEntries; ++e) any_long |= long_run[e] != 0;
+  if (!any_long) return;
+  // the waves share the rows: eight of two vectors a lane in flight (a row past the run re-reads the last one, a vector
+  // past the row the row's last one, and neither is added); a step's rows are added in pairs, the waves' sums in order
+  constexpr int kRows = 8, kVecs = kListVecs;
+  for (int cb = slice * kWave * kVecs; cb < nvec; cb += slices * kWave * kVecs) {
+    float acc[kVecs][VN] = {};
+    for (int e0 = member; run > 1 && e0 < run; e0 += kListGroup * kRows) {
+      const int mine = e0 + (lane & (kRows - 1)) * kListGroup;
+      const uint32_t pos = rows[mine < run ? mine : run - 1];
+      Vec16<T> v[kRows][kVecs];
+#pragma unroll
+      for (int r = 0; r < kRows; ++r) {
+        const T *src = dout + (int64_t)lane_value(pos, r) * C;
+#pragma unroll
+        for (int j = 0; j < kVecs; ++j) {
+          const int at = cb + j * kWave + lane;
+          v[r][j] = load16_stream(src + (int64_t)(at < nvec ? at : nvec - 1) * VN);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < kVecs; ++j)
+#pragma unroll
+        for (int k = 0; k < VN; ++k) {
+          float x[kRows];
+#pragma unroll
+          for (int r = 0; r < kRows; ++r) x[r] = e0 + r * kListGroup < run ? to_acc(v[r][j].e[k]) : 0.f;
+          acc[j][k] += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < kVecs; ++j) {
+      if (cb + j * kWave >= nvec) break;  // workgroup-uniform
+#pragma unroll
+      for (int h = 0; h < kPieces; ++h)
+        lds[h * kListThreads + tid] = f32x4{acc[j][4 * h], acc[j][4 * h + 1], acc[j][4 * h + 2], acc[j][4 * h + 3]};
+      __syncthreads();
+      const int at = cb + j * kWave + lane;
+      if (run > 1 && member == 0 && at < nvec) {
+        float sum[VN];
+#pragma unroll
+        for (int h = 0; h < kPieces; ++h) {
+          f32x4 t = lds[h * kListThreads + tid];
+#pragma unroll
+          for (int g = 1; g < kListGroup; ++g) t += lds[h * kListThreads + tid + g * kWave];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) sum[4 * h + k] = t[k];
+        }
+        finish(at, sum);
+      }
+      __syncthreads();
+    }
+  }
+}
+
 // Standalone position-table gradient.  The vector form is positions_block on its own (the fused call runs it inside
 // one of its launches: see kPosEarlyWindows and kPosFewFill); the scalar form takes any C and any alignment.
 template <typename T>
@@ -1164,10 +1435,6 @@ __global__ __launch_bounds__(kThreads) void emb_bwd_positions_kernel(const T *__
 constexpr int kRagWindow = kWave;
 constexpr int kRagThreads = 256;
 constexpr int kRagInFlight = 16;
-
-__device__ __forceinline__ uint32_t lane_value(uint32_t v, int lane) {
-  return (uint32_t)__builtin_amdgcn_readlane((int)v, lane);
-}
 
 // Partial rows as emb_bwd_reduce_kernel leaves them: slot 0 entered over the window's left edge, slot 1 left over the
 // right.  The first window has no slot 0 and the last no slot 1, so they start one row earlier.
@@ -1555,6 +1822,50 @@ int allow_reduce_lds(size_t bytes) {
   return allow_dynamic_lds_once(reinterpret_cast<const void *>(&emb_bwd_reduce_kernel<T>), bytes, done);
 }
 
+// `pos_blocks` workgroups of position sums ahead of those that finish `windows` windows.
+template <typename T>
+int finish_launch(const void *dout, const uint32_t *sorted_id, const float *partial, void *dweight, void *dwpe, int64_t n,
+                  int64_t C, int accumulate, int by_freq, int64_t windows, int64_t pos_blocks, int64_t B, int64_t TC,
+                  int pos_log2_slices, hipStream_t s) {
+  const bool wide = C > kFinWideRow && windows * ceil_div(C, (int64_t)kFinThreads) > kFinMostAtOnce;
+  const int64_t slices = ceil_div(C, (int64_t)kFinThreads * (wide ? 2 : 1));
+  const int64_t fin_blocks = windows * slices, blocks = fin_blocks + pos_blocks;
+  if (blocks > 0x7fffffffLL) return CS_ERR_TOO_LARGE;
+  if (blocks == 0) return CS_OK;
+  const auto finish = wide ? emb_bwd_finish_kernel<T, 2> : emb_bwd_finish_kernel<T, 1>;
+  finish<<<dim3((unsigned)blocks), dim3(kFinThreads), 0, s>>>(sorted_id, partial, (T *)dweight, n, C, accumulate, by_freq,
+                                                              fin_blocks, (int)slices, (const T *)dout, (T *)dwpe, B, TC,
+                                                              pos_log2_slices);
+  return launch_status();
+}
+
+// Lists that emb_bwd_list_kernel takes: short, and of rows whose zero-filling workgroups count their vectors in 32 bits.
+bool list_rows(int64_t n, int64_t C) { return n <= kListMost && C <= 0x7fffffffLL / kListFillRows; }
+
+template <typename T, typename IdxT>
+int list_launch(const void *dout, const void *ids, void *dweight, char *ws, const BwdLayout &L, int64_t n, int64_t C,
+                int64_t num_weights, int64_t padding_idx, int accumulate, int by_freq, const Positions<T> &positions,
+                hipStream_t s) {
+  uint32_t *sorted_id = reinterpret_cast<uint32_t *>(ws + L.off_sorted_id);
+  float *partial = reinterpret_cast<float *>(ws + L.off_partial);
+  const int64_t pairs = ceil_div(n, (int64_t)kListEntries);
+  int64_t slices = ceil_div(C / Vec16<T>::n, (int64_t)kListVecs * kWave);
+  if (pairs * slices > kListBlocks) slices = pairs < kListBlocks ? kListBlocks / pairs : 1;
+  const int64_t entry_blocks = pairs * slices;
+  int64_t fill_rows = ceil_div(kListFillBytes, C * (int64_t)sizeof(T));
+  if (fill_rows > kListFillRows) fill_rows = kListFillRows;
+  const int64_t fill_blocks = accumulate ? 0 : ceil_div(num_weights, fill_rows);
+  const int64_t blocks = entry_blocks + positions.blocks + fill_blocks;
+  if (blocks > 0x7fffffffLL) return CS_ERR_TOO_LARGE;
+  if (blocks == 0) return CS_OK;
+  emb_bwd_list_kernel<T, IdxT><<<dim3((unsigned)blocks), dim3(kListThreads), 0, s>>>(
+      (const T *)dout, (const IdxT *)ids, (T *)dweight, sorted_id, partial, (int)n, (int)C, num_weights, padding_idx,
+      accumulate, by_freq, (int)entry_blocks, (int)slices, (int)fill_rows, positions);
+  const int st = launch_status();
+  if (st != CS_OK || n <= kListWhole) return st;
+  return finish_launch<T>(dout, sorted_id, partial, dweight, nullptr, n, C, accumulate, by_freq, L.n_windows, 0, 0, 1, 0, s);
+}
+
 template <typename T>
 int bwd_typed(const void *dout, const void *ids, void *dweight, void *dwpe, char *ws,
               const BwdLayout &L, int64_t n, int64_t C, int64_t num_weights, int64_t padding_idx,
@@ -1582,6 +1893,13 @@ int bwd_typed(const void *dout, const void *ids, void *dweight, void *dwpe, char
   using P = std::conditional_t<std::is_same_v<T, double>, float, T>;  // (fp64 rows are summed by column)
   const int log2_s = position_slices(B);
   auto pos_blocks = [&](int threads) { return dwpe ? ceil_div(TC / VN, (int64_t)(threads >> log2_s)) : 0; };
+  if constexpr (!std::is_same_v<T, double>) {
+    if (vec_ok && list_rows(n, C)) {
+      const Positions<T> positions{(const T *)dout, (T *)dwpe, B, TC, accumulate, log2_s, pos_blocks(kListThreads)};
+      const auto launch = idx_dtype == CS_I64 ? list_launch<T, int64_t> : list_launch<T, int32_t>;
+      return launch(dout, ids, dweight, ws, L, n, C, num_weights, padding_idx, accumulate, by_freq, positions, s);
+    }
+  }
   const bool pos_first = vec_ok && fill_vecs <= kPosFewFill && !(L.key64 ? ranked<uint64_t>(n) : ranked<uint32_t>(n));
   const Positions<P> positions{(const P *)dout, (P *)dwpe, B, TC, accumulate, log2_s, pos_first ? pos_blocks(kTile) : 0};
   int st;
@@ -1621,15 +1939,11 @@ int bwd_typed(const void *dout, const void *ids, void *dweight, void *dwpe, char
   if constexpr (!std::is_same_v<T, double>) {
     float *partial = reinterpret_cast<float *>(ws + L.off_partial);
     const int64_t windows = n > 0 ? L.n_windows : 0;
-    const bool wide = C > kFinWideRow && windows * ceil_div(C, (int64_t)kFinThreads) > kFinMostAtOnce;
-    const int64_t slices = ceil_div(C, (int64_t)kFinThreads * (wide ? 2 : 1));
-    const int64_t fin_blocks = windows * slices;
     // The position sums go where the chip is idle: next to the finish workgroups, or next to the reducing ones of a
     // list too short to occupy the chip with those.
     const bool pos_early = windows > 0 && windows <= kPosEarlyWindows;
     const int64_t red_blocks = windows + (pos_early && !pos_first ? pos_blocks(kRedThreads) : 0);
-    const int64_t last_blocks = fin_blocks + (pos_early || pos_first ? 0 : pos_blocks(kFinThreads));
-    if (red_blocks > 0x7fffffffLL || last_blocks > 0x7fffffffLL) return CS_ERR_TOO_LARGE;
+    if (red_blocks > 0x7fffffffLL) return CS_ERR_TOO_LARGE;
     if (windows > 0) {
       const size_t lds = (size_t)kRedWaves * 2 * kWave * kVpl * VN * sizeof(float);
       static_assert(kRedThreads * kPosLdsBytesPerLane <= (size_t)kRedWaves * 2 * kWave * kVpl * VN * sizeof(float),
@@ -1642,12 +1956,8 @@ int bwd_typed(const void *dout, const void *ids, void *dweight, void *dwpe, char
       st = launch_status();
       if (st != CS_OK) return st;
     }
-    if (last_blocks == 0) return CS_OK;
-    const auto finish = wide ? emb_bwd_finish_kernel<T, 2> : emb_bwd_finish_kernel<T, 1>;
-    finish<<<dim3((unsigned)last_blocks), dim3(kFinThreads), 0, s>>>(
-        sorted_id, partial, (T *)dweight, n, C, accumulate, by_freq, fin_blocks, (int)slices, (const T *)dout,
-        (T *)dwpe, B, TC, log2_s);
-    return launch_status();
+    return finish_launch<T>(dout, sorted_id, partial, dweight, dwpe, n, C, accumulate, by_freq, windows,
+                            pos_early || pos_first ? 0 : pos_blocks(kFinThreads), B, TC, log2_s, s);
   }
   return CS_ERR_UNSUPPORTED;
 }

@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "cs_hip_kernels.h"
 
 namespace cs_hip {
@@ -130,6 +132,25 @@ __device__ __forceinline__ void store16_unaligned_stream(T *p, const Vec16<T> &v
   __builtin_nontemporal_store(raw, reinterpret_cast<u32x4_at2 *>(p));
 }
 
+// One row, or none of it, behind a buffer descriptor: an access past `bytes` reads zeros or writes nothing, by the
+// hardware's own bounds check.  A lane without a vector passes kOutside instead of sitting out under a condition: behind
+// a branch the compiler no longer knows how many accesses are under way and waits for younger ones too, at worst for
+// the row just requested.  The row has to be the same for the whole wave.
+typedef __amdgpu_buffer_rsrc_t RowBuffer;
+constexpr int kOutside = 0x7fffff00;
+__device__ __forceinline__ RowBuffer row_buffer(const void *row, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(row), 0, bytes, 0x00020000);  // untyped, raw
+}
+constexpr int kBufferStream = 2;  // nt
+template <typename T>
+__device__ __forceinline__ Vec16<T> load16_stream(RowBuffer row, int offset) {
+  return __builtin_bit_cast(Vec16<T>, __builtin_amdgcn_raw_buffer_load_b128(row, offset, 0, kBufferStream));
+}
+template <typename T>
+__device__ __forceinline__ void store16_stream(RowBuffer row, int offset, const Vec16<T> &v) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), row, offset, 0, kBufferStream);
+}
+
 __host__ __device__ __forceinline__ bool is_aligned16(const void *p) {
   return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
 }
@@ -203,6 +224,30 @@ __device__ __forceinline__ int wave_reduce(int v, Op op) {
 template <typename Op>
 __device__ __forceinline__ double wave_reduce(double v, Op op) {
   return wave_reduce_generic(v, op);
+}
+
+// The same sum, in the same order, in lane 63 alone: the rows are folded by two more DPP steps.
+__device__ __forceinline__ float wave_sum_in_last_lane(float v) {
+  v += dpp_f32<kDppQuadXor1>(v);
+  v += dpp_f32<kDppQuadXor2>(v);
+  v += dpp_f32<kDppHalfMirror>(v);
+  v += dpp_f32<kDppRowMirror>(v);
+  const auto from_row = [](float x, auto ctrl, auto rows) {  // zero in the other rows
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value, decltype(rows)::value, 0xf, false));
+  };
+  v += from_row(v, std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});  // row_bcast15: rows 1 and 3
+  v += from_row(v, std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});  // row_bcast31: rows 2 and 3
+  return v;
+}
+// wave_reduce of a sum whose terms stand in lanes 0 to 15 of each row of 16 alike (the other rows of wave_reduce's would
+// be zeros).
+__device__ __forceinline__ float row16_sum(float v) {
+  v += dpp_f32<kDppQuadXor1>(v);
+  v += dpp_f32<kDppQuadXor2>(v);
+  v += dpp_f32<kDppHalfMirror>(v);
+  v += dpp_f32<kDppRowMirror>(v);
+  return v;
 }
 
 // Workgroup reduction through LDS.  `scratch` holds one A per wavefront.

@@ -1008,10 +1008,14 @@ __global__ __launch_bounds__(THREADS, WPE) void ln_bwd_kernel(
 //
 // Bound by HBM; what it took to get near was the number of loads in flight.  A wave-sized row slice
 // per wave and 8 elements per lane leave registers for two rows (the next one requested as soon as
-// the one before the current is done), gamma, beta or the column sums.  [4096,5120] bf16 with the
-// residual: forward 31.9 us (5.3 TB/s; one workgroup per row behind a separate add 64 us), backward
-// 42.1 us and 5.1 for the sums (4.0 TB/s without the partial rows' 42 MB; 40.7 and 4.6 with partial rows in fp32;
-// 382 with the plain kernels, whose column sums ran on 80 workgroups).  [12000,1003] fp32: 38.9 + 40.1 us against 58.5 + 1121.
+// the one before the current is done), gamma, beta or the column sums.  Whole vectors are accessed through a RowBuffer,
+// so that nothing in a step depends on a lane or on whether there is such a row: as long as it did, the compiler could not
+// tell how many accesses were under way and waited, at the head of every row, for the row just requested as well.
+// [4096,5120] bf16 with the residual, before / now: forward 32.4 / 29.9 us (5.6 TB/s; one workgroup per row behind a
+// separate add 64 us), backward 42.5 / 35.4 and 4.6 for the sums (4.7 TB/s without the partial rows' 42 MB; 382 with the
+// plain kernels, whose column sums ran on 80 workgroups).  [5824,7040] fp16 forward 66.9 / 56.2, [544,7616] fp32 21.6 / 15.6.
+// The backward is as close to its arithmetic as to the memory: 200 operations a row and lane, two of them fp64 adds, ten
+// waves on four SIMDs.  [12000,1003] fp32 37.6 + 41 us against 58.5 + 1121.
 template <typename T, int N, bool UA>
 __device__ __forceinline__ Raw<T, N> load_piece(const T *p) {
   Raw<T, N> r;
@@ -1040,6 +1044,17 @@ __device__ __forceinline__ void store_piece(T *p, const float (&in)[N]) {
     }
   }
 }
+template <typename T, int N>
+__device__ __forceinline__ void store_piece(RowBuffer row, int offset, const float (&in)[N]) {
+  constexpr int VN = Vec16<T>::n;
+#pragma unroll
+  for (int q = 0; q < N / VN; ++q) {
+    Vec16<T> v;
+#pragma unroll
+    for (int k = 0; k < VN; ++k) v.e[k] = from_acc<T>(in[q * VN + k]);
+    store16_stream(row, offset + q * 16, v);
+  }
+}
 // One lane's share of a row: VPT vectors and, with UA, one single element.
 template <typename T, int VN, int VPT, bool UA>
 struct Share {
@@ -1051,6 +1066,10 @@ template <int VN, int VPT, bool UA>
 struct Lanes {
   int at[VPT];   // first column of each vector (a lane without a vector re-reads the row's last one)
   bool has[VPT];
+  template <typename T>
+  __device__ __forceinline__ int offset(int j) const {  // in a RowBuffer
+    return has[j] ? at[j] * (int)sizeof(T) : kOutside;
+  }
   int ecol;      // the single element's column
   bool ehas;
   __device__ __forceinline__ Lanes(int C, int gw, int lane_in_group) {
@@ -1078,6 +1097,17 @@ __device__ __forceinline__ void load_share(Share<T, VN, VPT, UA> &s, const T *ro
   if constexpr (UA) s.e = row[l.ecol];
 }
 
+// the same of row `r` of whole aligned vectors: zeros where the lane has no vector, and past the last row
+template <typename T, int VN, int VPT>
+__device__ __forceinline__ void load_share(Share<T, VN, VPT, false> &s, const T *base, int64_t r, int64_t rows, int C,
+                                           const Lanes<VN, VPT, false> &l) {
+  const RowBuffer row = row_buffer(base + (r < rows ? r : 0) * C, r < rows ? C * (int)sizeof(T) : 0);
+#pragma unroll
+  for (int j = 0; j < VPT; ++j)
+#pragma unroll
+    for (int q = 0; q < VN / Vec16<T>::n; ++q) s.v[j].v[q] = load16_stream<T>(row, l.template offset<T>(j) + q * 16);
+}
+
 constexpr int kLnBlockMaxWaves = 16;
 
 // Sum over a group's row; v[j] belongs to the lane's vector j.  Rows of 257 to 512 vectors (BY_LANE) have three
@@ -1102,12 +1132,13 @@ __device__ __forceinline__ float row_sum(const float (&v)[VPT], int gw, int wave
   float t = v[0];
 #pragma unroll
   for (int j = 1; j < VPT; ++j) t += v[j];
-  t = wave_reduce(t, SumOp{});
-  if (gw == 1) return t;  // workgroup-uniform
-  if (lane == 0) red[wave] = t;
+  if (gw == 1) return wave_reduce(t, SumOp{});  // workgroup-uniform
+  t = wave_sum_in_last_lane(t);
+  if (lane == kWave - 1) red[wave] = t;
   lds_barrier();
-  const float r = red[group * gw + (lane < gw ? lane : 0)];
-  return wave_reduce(lane < gw ? r : 0.f, SumOp{});
+  const int w = lane % kLnBlockMaxWaves;
+  const float r = red[group * gw + (w < gw ? w : 0)];
+  return row16_sum(w < gw ? r : 0.f);
 }
 
 template <typename TX, typename TY, typename TP, int VPT, bool HAS_RES, bool UA, bool BY_LANE>
@@ -1117,7 +1148,7 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
     const TX *res, TX *sum_out, int gw, int groups) {
   constexpr int VN = Vec16<TX>::n;
   __shared__ float red[2][kLnBlockMaxWaves * (BY_LANE ? VPT * kWave : 1)];
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int group = wave / gw, lig = threadIdx.x - group * gw * kWave;
   const bool any_vec = C >= VN;
   const Lanes<VN, VPT, UA> own(C, gw, lig);
@@ -1132,13 +1163,15 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
     Share<TX, VN, VPT, UA> x, res;
   };
   auto fetch = [&](Row &d, int64_t r) {
-    const int64_t at = (r < rows ? r : rows - 1) * C;
-    load_share(d.x, x + at, own, any_vec);
-    if constexpr (HAS_RES) load_share(d.res, res + at, own, any_vec);
+    if constexpr (UA) {
+      const int64_t at = (r < rows ? r : rows - 1) * C;
+      load_share(d.x, x + at, own, any_vec);
+      if constexpr (HAS_RES) load_share(d.res, res + at, own, any_vec);
+    } else {
+      load_share(d.x, x, r, rows, C, own);
+      if constexpr (HAS_RES) load_share(d.res, res, r, rows, C, own);
+    }
   };
-  Row even, odd;
-  fetch(even, row);
-  if (steps > 1) fetch(odd, row + stride);
   float g[VPT][VN], b[VPT][VN], ge = 0.f, be = 0.f;
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
@@ -1161,10 +1194,14 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
     ge = to_acc(gamma[own.ecol]);
     if (beta) be = to_acc(beta[own.ecol]);
   }
+  Row even, odd;
+  fetch(even, row);
+  if (!UA || steps > 1) fetch(odd, row + stride);
   auto work = [&](Row &in, int64_t row) {
     Share<TX, VN, VPT, UA> &cur = in.x, &rcur = in.res;
     const bool row_ok = row < rows;
-    const int64_t at = row * C;
+    const int64_t at = (row_ok ? row : 0) * C;
+    const int y_bytes = row_ok ? C * (int)sizeof(TY) : 0;
     if constexpr (HAS_RES) {
       // cur = x + residual, one fp32 add and one rounding per element, as an add launch would give
 #pragma unroll
@@ -1174,12 +1211,10 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
         for (int k = 0; k < VN; ++k)
           sum.e[k] = from_acc<TX>(raw_get<TX, VN>(cur.v[j], k) + raw_get<TX, VN>(rcur.v[j], k));
         cur.v[j].v[0] = sum;
-        if (own.has[j] && row_ok) {
-          if constexpr (UA) {
-            store16_unaligned_stream(sum_out + at + own.at[j], sum);
-          } else {
-            store16_stream(sum_out + at + own.at[j], sum);
-          }
+        if constexpr (UA) {
+          if (own.has[j] && row_ok) store16_unaligned_stream(sum_out + at + own.at[j], sum);
+        } else {
+          store16_stream(row_buffer(sum_out + at, row_ok ? C * (int)sizeof(TX) : 0), own.template offset<TX>(j), sum);
         }
       }
       if constexpr (UA) {
@@ -1212,7 +1247,19 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
       q[0] += own.ehas ? d * d : 0.f;
     }
     const float rs = 1.0f / sqrtf(over_columns(row_sum<BY_LANE>(q, gw, wave, group, lane, red[1]), fc, inv_c) + eps);
-    if (row_ok) {
+    if constexpr (!UA) {
+      const int64_t r = row_ok ? row : 0;
+      const int first = lig == 0 ? 0 : kOutside, bytes = row_ok ? (int)sizeof(float) : 0;
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(mu), row_buffer(mean + r, bytes), first, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(rs), row_buffer(rstd + r, bytes), first, 0, 0);
+#pragma unroll
+      for (int j = 0; j < VPT; ++j) {
+        float o[VN];
+#pragma unroll
+        for (int k = 0; k < VN; ++k) o[k] = (raw_get<TX, VN>(cur.v[j], k) - mu) * rs * g[j][k] + b[j][k];
+        store_piece<TY, VN>(row_buffer(y + at, y_bytes), own.template offset<TY>(j), o);
+      }
+    } else if (row_ok) {
       if (lig == 0) {
         mean[row] = mu;
         rstd[row] = rs;
@@ -1231,14 +1278,37 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
       }
     }
   };
-  for (int64_t it = 0; it < steps; it += 2, row += 2 * stride) {
-    work(even, row);
-    if (it + 2 < steps) fetch(even, row + 2 * stride);
-    if (it + 1 < steps) {
-      work(odd, row + stride);
-      if (it + 3 < steps) fetch(odd, row + 3 * stride);
+  if constexpr (UA) {
+    for (int64_t it = 0; it < steps; it += 2, row += 2 * stride) {
+      work(even, row);
+      if (it + 2 < steps) fetch(even, row + 2 * stride);
+      if (it + 1 < steps) {
+        work(odd, row + stride);
+        if (it + 3 < steps) fetch(odd, row + 3 * stride);
+      }
     }
+    return;
   }
+  // Every step requests its two rows, there or not, and the first stands before the loop: what is under way at the
+  // loop's head is then the same whichever way it was reached, and the compiler waits for exactly the row it needs.
+  // Every step requests two rows, there or not, and the first step stands before the loop: what is under way at the
+  // loop's head is then the same whichever way it was reached, and the compiler waits for exactly the row it needs.
+  const auto step = [&] {
+    work(even, row);
+    __builtin_amdgcn_sched_barrier(0);  // neither row's work moves into the other's
+    fetch(even, row + 2 * stride);
+    __builtin_amdgcn_sched_barrier(0);
+    work(odd, row + stride);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(odd, row + 3 * stride);
+    __builtin_amdgcn_sched_barrier(0);
+    row += 2 * stride;
+  };
+  if (steps > 1) {
+    step();
+    for (int64_t it = 3; it < steps; it += 2) step();
+  }
+  if (steps & 1) work(even, row);
 }
 
 // Backward of the same rows.  The column sums of a lane's own columns stay in registers over all the
@@ -1278,7 +1348,7 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_bwd_block_kernel(
     bid -= side.blocks;
     nblocks -= side.blocks;
   }
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int group = wave / gw, lig = threadIdx.x - group * gw * kWave;
   const bool any_vec = C >= VN;
   const Lanes<VN, VPT, UA> own(C, gw, lig);
@@ -1295,15 +1365,18 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_bwd_block_kernel(
   };
   auto fetch = [&](Row &d, int64_t r) {
     const int64_t rr = r < rows ? r : rows - 1;
-    load_share(d.dy, dy + rr * C, own, any_vec);
-    load_share(d.x, x + rr * C, own, any_vec);
-    if constexpr (HAS_DRES) load_share(d.res, dres + rr * C, own, any_vec);
+    if constexpr (UA) {
+      load_share(d.dy, dy + rr * C, own, any_vec);
+      load_share(d.x, x + rr * C, own, any_vec);
+      if constexpr (HAS_DRES) load_share(d.res, dres + rr * C, own, any_vec);
+    } else {
+      load_share(d.dy, dy, r, rows, C, own);
+      load_share(d.x, x, r, rows, C, own);
+      if constexpr (HAS_DRES) load_share(d.res, dres, r, rows, C, own);
+    }
     d.mu = mean[rr];
     d.rs = rstd[rr];
   };
-  Row even, odd;  // as in the forward kernel, where both fit
-  fetch(even, row);
-  if (PF && steps > 1) fetch(odd, row + stride);
   double acc_g[VPT][VN], acc_b[VPT][VN], eacc_g = 0., eacc_b = 0.;
   float g[VPT][VN], ge = 0.f;
 #pragma unroll
@@ -1324,6 +1397,9 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_bwd_block_kernel(
     }
   }
   if constexpr (UA && HAS_DX) ge = to_acc(gamma[own.ecol]);
+  Row even, odd;  // as in the forward kernel, where both fit
+  fetch(even, row);
+  if (PF && (!UA || steps > 1)) fetch(odd, row + stride);
 
   int parity = 0;
   auto work = [&](Row &in, int64_t row) {
@@ -1336,11 +1412,18 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_bwd_block_kernel(
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
       const bool live = own.has[j] && row_ok;
+      const float live_mu = live ? mu : 0.f, live_rs = live ? rs : 0.f;
 #pragma unroll
       for (int k = 0; k < VN; ++k) {
-        // both masked: 0 * inf would leave a NaN in the sums
-        const float xh = live ? (raw_get<TX, VN>(xcur.v[j], k) - mu) * rs : 0.f;
-        const float dv = live ? raw_get<TDY, VN>(dcur.v[j], k) : 0.f;
+        // zero both where there is no row or vector: 0 * inf would leave a NaN in the sums.  (A RowBuffer reads zeros there.)
+        float xh, dv;
+        if constexpr (UA) {
+          xh = live ? (raw_get<TX, VN>(xcur.v[j], k) - mu) * rs : 0.f;
+          dv = live ? raw_get<TDY, VN>(dcur.v[j], k) : 0.f;
+        } else {
+          xh = (raw_get<TX, VN>(xcur.v[j], k) - live_mu) * live_rs;
+          dv = raw_get<TDY, VN>(dcur.v[j], k);
+        }
         if constexpr (HAS_DP) {
           acc_g[j][k] += (double)(dv * xh);
           acc_b[j][k] += (double)dv;
@@ -1368,26 +1451,30 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_bwd_block_kernel(
       }
     }
     if constexpr (HAS_DX) {
-      s1 = wave_reduce(s1, SumOp{});
-      s2 = wave_reduce(s2, SumOp{});
       if (gw > 1) {  // workgroup-uniform
-        if (lane == 0) {
+        s1 = wave_sum_in_last_lane(s1);
+        s2 = wave_sum_in_last_lane(s2);
+        if (lane == kWave - 1) {
           red[parity][0][wave] = s1;
           red[parity][1][wave] = s2;
         }
         lds_barrier();
-        const int from = group * gw + (lane < gw ? lane : 0);
+        const int w = lane % kLnBlockMaxWaves, from = group * gw + (w < gw ? w : 0);
         const float a = red[parity][0][from], c = red[parity][1][from];
-        s1 = wave_reduce(lane < gw ? a : 0.f, SumOp{});
-        s2 = wave_reduce(lane < gw ? c : 0.f, SumOp{});
+        s1 = row16_sum(w < gw ? a : 0.f);
+        s2 = row16_sum(w < gw ? c : 0.f);
         parity ^= 1;  // the other pair next time: one barrier per row is enough
+      } else {
+        s1 = wave_reduce(s1, SumOp{});
+        s2 = wave_reduce(s2, SumOp{});
       }
       s1 *= inv_c;
       s2 *= inv_c;
-      if (row_ok) {
+      if (!UA || row_ok) {
+        const RowBuffer out = row_buffer(dx + (row_ok ? row : 0) * C, row_ok ? C * (int)sizeof(TDX) : 0);
 #pragma unroll
         for (int j = 0; j < VPT; ++j) {
-          if (own.has[j]) {
+          if (!UA || own.has[j]) {
             float o[VN];
 #pragma unroll
             for (int k = 0; k < VN; ++k) {
@@ -1396,7 +1483,11 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_bwd_block_kernel(
               o[k] = rs * __builtin_fmaf(-xh, s2, __builtin_fmaf(dv, g[j][k], -s1));
               if constexpr (HAS_DRES) o[k] = round_through<TDX>(o[k]) + raw_get<TDX, VN>(rcur.v[j], k);
             }
-            store_piece<TDX, VN, UA>(dx + row * C + own.at[j], o);
+            if constexpr (UA) {
+              store_piece<TDX, VN, UA>(dx + row * C + own.at[j], o);
+            } else {
+              store_piece<TDX, VN>(out, own.template offset<TDX>(j), o);
+            }
           }
         }
         if constexpr (UA) {
@@ -1409,7 +1500,7 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_bwd_block_kernel(
       }
     }
   };
-  if constexpr (PF) {
+  if constexpr (UA && PF) {
     for (int64_t it = 0; it < steps; it += 2, row += 2 * stride) {
       work(even, row);
       if (it + 2 < steps) fetch(even, row + 2 * stride);
@@ -1418,6 +1509,23 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_bwd_block_kernel(
         if (it + 3 < steps) fetch(odd, row + 3 * stride);
       }
     }
+  } else if constexpr (PF) {
+    const auto step = [&] {  // as in the forward kernel
+      work(even, row);
+      __builtin_amdgcn_sched_barrier(0);  // neither row's work moves into the other's
+      fetch(even, row + 2 * stride);
+      __builtin_amdgcn_sched_barrier(0);
+      work(odd, row + stride);
+      __builtin_amdgcn_sched_barrier(0);
+      fetch(odd, row + 3 * stride);
+      __builtin_amdgcn_sched_barrier(0);
+      row += 2 * stride;
+    };
+    if (steps > 1) {
+      step();
+      for (int64_t it = 3; it < steps; it += 2) step();
+    }
+    if (steps & 1) work(even, row);
   } else {
     for (int64_t it = 0; it < steps; ++it, row += stride) {
       work(even, row);
@@ -1692,7 +1800,7 @@ struct BlockPlan {
 };
 // the fold of the widest row: 16 elements per lane and a tail of fewer than 8
 constexpr size_t kLnBlockFoldLds = ((size_t)16 * kLnBlockMaxWaves * kWave + 7) * sizeof(double);
-BlockPlan block_plan(int64_t rows, int64_t C, int x_dtype, bool backward, bool residual) {
+BlockPlan block_plan(int64_t rows, int64_t C, int x_dtype, bool backward, bool residual, bool whole_vectors = false) {
   BlockPlan p;
   if (x_dtype == CS_F64 || C <= 0) return p;
   const int vn = 16 / (int)dtype_size(x_dtype);
@@ -1706,17 +1814,22 @@ BlockPlan block_plan(int64_t rows, int64_t C, int x_dtype, bool backward, bool r
   if (vpt * vn > 16) return p;
   p.vpt = vpt;
   p.gw = (int)ceil_div(nvec, (int64_t)kWave * vpt);
+  // Forward with the residual, whole vectors: one workgroup of up to 12 waves per CU, whose loads are never waited for
+  // ahead of time (see ln_fwd_block_kernel); 512 workgroups of 8 waves put more under way than the memory likes
+  // ([4096,5120] bf16 30.9 us against 29.9, [16384,2304] 57.0 / 52.5, [16384,3584] 85.5 / 78.3).  Not where those make one
+  // step: [300,2304] 4.2 against 4.8.
+  const bool even_flow = !backward && residual && whole_vectors && (rows > 512 || p.gw > kLnBlockMaxWaves / 2);
   // Backward: as many rows side by side as 16 waves hold, so that one workgroup per CU, hence 256
   // partial rows, keeps the CU busy ([12000,1003] fp32 40.3 us against 43.3 with 8 waves; 512
   // workgroups 41.2, and [4096,5120] bf16 49.9 against 41.9).  Forward: 8 waves and two workgroups
   // per CU ([4096,1001] bf16 9.7 us against 11.4 with 16 waves, [4096,5120] 32.3 against 37.5 with 1024
   // workgroups).
-  int groups = (backward ? kLnBlockMaxWaves : kLnBlockMaxWaves / 2) / p.gw;
+  int groups = (backward ? kLnBlockMaxWaves : even_flow ? 12 : kLnBlockMaxWaves / 2) / p.gw;
   // Fewer side by side where there are not rows enough for every CU: [300,1003] bf16 backward 8.3 us against 8.5,
   // [64,1003] 6.8 against 8.7; up to three stay ([300,4099] 16.2 against 17.6, [300,2056] 9.9 / 11.8).  Rounded down in
   // the backward, so that the number of partial rows grows with the rows: a buffer for a long batch holds a short one's.
   if (!backward) {
-    const int64_t per_cu = ceil_div(rows, (int64_t)256);
+    const int64_t per_cu = even_flow ? rows / 256 : ceil_div(rows, (int64_t)256);
     if (groups > per_cu) groups = (int)per_cu;
   } else if (groups > 3 && groups > rows / 256) {
     groups = (int)(rows / 256);
@@ -1724,7 +1837,7 @@ BlockPlan block_plan(int64_t rows, int64_t C, int x_dtype, bool backward, bool r
   if (groups < 1) groups = 1;
   while (backward && groups > 1 && (size_t)groups * C * sizeof(double) > kLnBlockFoldLds) --groups;
   p.groups = groups;
-  const int cap = backward ? 256 : 512;
+  const int cap = backward || even_flow ? 256 : 512;
   const int64_t b = ceil_div(rows, (int64_t)p.groups);
   p.blocks = (int)(b < cap ? b : cap);
   return p;
@@ -1856,9 +1969,9 @@ int fwd_typed(const void *x, const void *gamma, const void *beta, void *y, void 
       }
       return launch_status();
     }
-    const BlockPlan b = block_plan(rows, C, x_dtype, false, res != nullptr);
+    const bool ua = !aligned || C % Vec16<TX>::n != 0;
+    const BlockPlan b = block_plan(rows, C, x_dtype, false, res != nullptr, !ua);
     if (b.vpt != 0) {
-      const bool ua = !aligned || C % Vec16<TX>::n != 0;
       const dim3 grid((unsigned)b.blocks), block((unsigned)(b.gw * b.groups * kWave));
       // rows of 257 to 512 vectors: see row_sum
       const bool by_lane = C / Vec16<TX>::n > 4 * kWave && C / Vec16<TX>::n <= 8 * kWave;

@@ -12,7 +12,7 @@
 // A row is read from HBM once and its gradient written once: 2 accesses per
 // element.  Which kernel does that depends on the row's width:
 //   up to 2048 vectors of 16 bytes   ce_rows_kernel: one workgroup per row, the row in
-//                                    registers, exact two-step max and sum (wave64
+//   (4096 of many rows)              registers, exact two-step max and sum (wave64
 //                                    butterfly, then LDS across the waves)
 //   up to 7168 (8192 at fp32)        ce_rows_stream_kernel: one persistent workgroup per
 //                                    CU that loads the next row while it works on the
@@ -22,8 +22,8 @@
 //   the loss alone of many rows      ce_loss_rows_kernel: one workgroup per row, nothing kept
 //   up to 16384 fp32 vectors of the  ce_rows_kernel with 1024 lanes (the loss alone, and the gradient
 //   few rows the last two leave      of a few rows more than there are CUs)
-//   wider, the loss alone, or narrow ce_rows_wide_kernel: two sweeps over the row, the
-//   rows that start off 16 bytes     second one served by the cache
+//   wider, or the loss alone of a    ce_rows_wide_kernel: two sweeps over the row, the
+//   few rows                         second one served by the cache
 //   fp64, unaligned base pointers    ce_rows_general_kernel
 // Probabilities are 2^(x*log2e - max*log2e) / sum with one fma and one hardware exp2 per
 // element; the row loss is ln(sum) - (x_t - max).
@@ -179,6 +179,7 @@ __global__ __launch_bounds__(1024) void ce_reduce_kernel(const float *__restrict
   }
 }
 
+constexpr int kNarrowMostThreads = 1024;
 template <typename T>
 __device__ __forceinline__ float vec_get(const Vec16<T> &v, int k) {
   return to_acc(v.e[k]);
@@ -206,118 +207,6 @@ __device__ __forceinline__ void store_own(TD *p, const float (&o)[N_ELEMS], int 
     if (c0 + k >= 0 && c0 + k < stride) p[k] = from_acc<TD>(o[k]);
 }
 
-template <typename T, typename TD, int BLOCK, int VPT>
-__global__ __launch_bounds__(BLOCK) void ce_rows_kernel(
-    const T *__restrict__ logits, TD *__restrict__ dlogits, const int64_t *__restrict__ targets,
-    float *__restrict__ row_loss, const int *__restrict__ ws_count, int64_t V, int64_t row_stride,
-    int64_t ignore_index, int reduction, float dloss) {
-  constexpr int VN = Vec16<T>::n;
-  __shared__ float scratch[(BLOCK + kWave - 1) / kWave];
-  const int64_t row = blockIdx.x;
-  const int tid = threadIdx.x;
-  const int nvec = (int)(row_stride / VN);  // whole row incl. padding, in vectors
-  const int iV = (int)V;
-  const T *x = logits + row * row_stride;
-  const int64_t target = targets[row];
-  const bool counts = target_counts(target, V, ignore_index);  // block-uniform
-
-  if (!counts) {
-    if (tid == 0 && row_loss) row_loss[row] = 0.f;
-    if (dlogits) {
-      float z[VN];
-#pragma unroll
-      for (int k = 0; k < VN; ++k) z[k] = 0.f;
-      for (int idx = tid; idx < nvec; idx += BLOCK)
-        store_out<T, TD, VN>(dlogits + row * row_stride + (int64_t)idx * VN, z);
-    }
-    return;
-  }
-
-  const int n_count =
-      reduction == CS_REDUCTION_MEAN ? rows_that_count(ws_count, targets, gridDim.x, V, ignore_index) : 0;
-  Vec16<T> xr[VPT];
-#pragma unroll
-  for (int j = 0; j < VPT; ++j) {
-    const int idx = tid + BLOCK * j;
-    // every lane loads (lanes past the row read its last vector, which nothing below uses): a
-    // load under the lane's own condition makes the compiler wait for it before the next one
-    xr[j] = load16_stream(x + (int64_t)(idx < nvec ? idx : nvec - 1) * VN);
-  }
-  const float x_t = tid == 0 ? to_acc(x[target]) : 0.f;
-
-  // ---- row maximum
-  float m = -INFINITY;
-#pragma unroll
-  for (int j = 0; j < VPT; ++j) {
-    const int c0 = (tid + BLOCK * j) * VN;
-    if (c0 + VN <= iV) {
-#pragma unroll
-      for (int k = 0; k < VN; ++k) m = fmaxf(m, vec_get(xr[j], k));
-    } else if (c0 < iV) {
-#pragma unroll
-      for (int k = 0; k < VN; ++k)
-        if (c0 + k < iV) m = fmaxf(m, vec_get(xr[j], k));
-    }
-  }
-  m = block_reduce(m, MaxOp{}, -INFINITY, scratch);
-  const float m2 = m * kLog2e;
-
-  // ---- sum of exponentials
-  float s = 0.f;
-#pragma unroll
-  for (int j = 0; j < VPT; ++j) {
-    const int c0 = (tid + BLOCK * j) * VN;
-    if (c0 + VN <= iV) {
-#pragma unroll
-      for (int k = 0; k < VN; ++k) s += __builtin_amdgcn_exp2f(__builtin_fmaf(vec_get(xr[j], k), kLog2e, -m2));
-    } else if (c0 < iV) {
-#pragma unroll
-      for (int k = 0; k < VN; ++k)
-        if (c0 + k < iV) s += __builtin_amdgcn_exp2f(__builtin_fmaf(vec_get(xr[j], k), kLog2e, -m2));
-    }
-  }
-  s = block_reduce(s, SumOp{}, 0.f, scratch);
-
-  const float log2_s = __builtin_amdgcn_logf(s);  // v_log_f32 is log2
-  // loss = ln(sum exp(x - max)) - (x_t - max): the difference to the maximum is formed with one
-  // fused multiply-add against the same rounded m2 the sum used, so a loss near 0 keeps its digits
-  if (tid == 0 && row_loss) row_loss[row] = (log2_s - __builtin_fmaf(x_t, kLog2e, -m2)) * kLn2;
-  if (dlogits == nullptr) return;
-
-  // ---- dlogits = (p - onehot) * scale with p = 2^(x*log2e - m2) / s.  The exponent is taken
-  // relative to the row maximum with one fused multiply-add, the same expression the sum above
-  // used, so the rounding of m2 cancels between numerator and denominator and p keeps fp32
-  // accuracy; folding log2(s) and log2(scale) into the exponent instead costs ~1e-6 relative,
-  // which the subtraction at the target column amplifies when p is close to 1.
-  float scale = dloss;
-  if (reduction == CS_REDUCTION_MEAN) scale = dloss / (float)n_count;
-  const float factor = scale / s;  // s >= 1: the maximum contributes 2^0
-  const int t_vec = (int)(target / VN), t_sub = (int)(target % VN);
-  TD *d = dlogits + row * row_stride;
-#pragma unroll
-  for (int j = 0; j < VPT; ++j) {
-    const int idx = tid + BLOCK * j;
-    if (idx < nvec) {
-      const int c0 = idx * VN;
-      float o[VN];
-#pragma unroll
-      for (int k = 0; k < VN; ++k)
-        o[k] = __builtin_amdgcn_exp2f(__builtin_fmaf(vec_get(xr[j], k), kLog2e, -m2)) * factor;
-      if (c0 + VN > iV) {  // last class vector and the padding
-#pragma unroll
-        for (int k = 0; k < VN; ++k)
-          if (c0 + k >= iV) o[k] = 0.f;
-      }
-      if (idx == t_vec) {
-#pragma unroll
-        for (int k = 0; k < VN; ++k)
-          if (k == t_sub) o[k] -= scale;
-      }
-      store_out<T, TD, VN>(d + (int64_t)c0, o);
-    }
-  }
-}
-
 // elements of T in a 128-byte line
 template <typename T>
 constexpr int kLineElems = 128 / (int)sizeof(T);
@@ -340,6 +229,157 @@ __device__ __forceinline__ VecE<T, EPV> load_e_stream(const T *p) {
   } else {
     const u32x2 raw = __builtin_nontemporal_load(reinterpret_cast<const u32x2 *>(p));
     return __builtin_bit_cast(VecE<T, EPV>, raw);
+  }
+}
+
+// Narrow rows: a workgroup per row, the whole row in registers, VPT accesses of EPV elements a lane, all under way before
+// the first is used; as many waves as the row has such shares.  RAGGED: lanes own aligned vectors of the whole array, as in
+// the streaming kernel below.  What is no class column is overwritten with -inf in the packed registers, so that no pass
+// masks element by element; a lane past the row's end loads its last vector again.
+template <typename T, typename TD, int VPT, int EPV, bool RAGGED, int MOST_THREADS = kNarrowMostThreads>
+__global__ __launch_bounds__(MOST_THREADS) void ce_rows_kernel(
+    const T *logits, TD *dlogits, const int64_t *__restrict__ targets, float *__restrict__ row_loss,
+    const int *__restrict__ ws_count, int64_t N, int64_t V, int64_t row_stride, int64_t ignore_index, int reduction,
+    float dloss, const float *__restrict__ class_weight) {
+  constexpr int VN = EPV;
+  __shared__ float scratch[MOST_THREADS / kWave];
+  const int64_t row = blockIdx.x;
+  const int tid = threadIdx.x, block = blockDim.x;
+  const int iV = (int)V, stride = (int)row_stride;
+  const int off = RAGGED ? (int)((row * row_stride) & (kLineElems<T> - 1)) : 0;
+  const int nvec = RAGGED ? (off + stride + VN - 1) / VN : stride / VN;
+  const T *x = logits + row * row_stride - off;
+  TD *d = dlogits + row * row_stride - off;
+  const int64_t target = targets[row];
+  const bool counts = target_counts(target, V, ignore_index);  // block-uniform
+  // a vector the row does not own all of
+  auto shared_vector = [&](int c0) { return RAGGED && (c0 < 0 || c0 + VN > stride); };
+
+  if (!counts) {
+    if (tid == 0 && row_loss) row_loss[row] = 0.f;
+    if (dlogits) {
+      float z[VN];
+#pragma unroll
+      for (int k = 0; k < VN; ++k) z[k] = 0.f;
+      for (int idx = tid; idx < nvec; idx += block) {
+        const int c0 = idx * VN - off;
+        if (shared_vector(c0)) {
+          store_own<TD, VN>(d + (int64_t)idx * VN, z, c0, stride);
+        } else {
+          store_out<T, TD, VN>(d + (int64_t)idx * VN, z);
+        }
+      }
+    }
+    return;
+  }
+
+  float scale = dloss;
+  if (reduction == CS_REDUCTION_MEAN)
+    scale = dloss / (class_weight ? reinterpret_cast<const float *>(ws_count)[1]
+                                  : (float)rows_that_count(ws_count, targets, N, V, ignore_index));
+  const float wt = class_weight ? class_weight[target] : 1.f;
+  scale *= wt;
+  // The array's last vector may not lie whole inside it: that of the last row, and of rows shorter than a vector ahead of
+  // it.  Where such a row has no other, nothing is loaded in one piece.
+  const int whole = nvec - (RAGGED && row * row_stride - off + (int64_t)nvec * VN > N * row_stride ? 1 : 0);
+  VecE<T, EPV> xr[VPT] = {};
+  if (!RAGGED || whole > 0) {  // block-uniform
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+      const int idx = tid + block * j;
+      xr[j] = load_e_stream<T, EPV>(x + (int64_t)(idx < whole ? idx : whole - 1) * VN);
+    }
+  }
+  const float x_t = tid == 0 ? to_acc(x[off + target]) : 0.f;
+  if (RAGGED && whole < nvec) {  // block-uniform
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+      if (tid + block * j == nvec - 1) {
+#pragma unroll
+        for (int k = 0; k < VN; ++k) {
+          const int c = (nvec - 1) * VN - off + k;
+          xr[j].e[k] = x[off + (c < stride ? c : 0)];
+        }
+      }
+    }
+  }
+
+  // ---- row maximum
+  float m = -INFINITY;
+#pragma unroll
+  for (int j = 0; j < VPT; ++j) {
+    const int c0 = (tid + block * j) * VN - off;
+    if (c0 + VN > iV || (RAGGED && j == 0 && c0 < 0)) {
+#pragma unroll
+      for (int k = 0; k < VN; ++k)
+        if (c0 + k >= iV || (RAGGED && j == 0 && c0 + k < 0)) xr[j].e[k] = from_acc<T>(-INFINITY);
+    }
+#pragma unroll
+    for (int k = 0; k < VN; ++k) m = fmaxf(m, to_acc(xr[j].e[k]));
+  }
+  m = block_reduce(m, MaxOp{}, -INFINITY, scratch);
+  const float m2 = m * kLog2e;
+
+  // ---- sum of exponentials: a tree over the lane's elements, then the lanes
+  float part[VPT];
+#pragma unroll
+  for (int j = 0; j < VPT; ++j) {
+    float e[VN];
+#pragma unroll
+    for (int k = 0; k < VN; ++k) e[k] = __builtin_amdgcn_exp2f(__builtin_fmaf(to_acc(xr[j].e[k]), kLog2e, -m2));
+#pragma unroll
+    for (int w = VN / 2; w > 0; w /= 2)
+#pragma unroll
+      for (int k = 0; k < w; ++k) e[k] += e[k + w];
+    part[j] = e[0];
+  }
+#pragma unroll
+  for (int w = VPT / 2; w > 0; w /= 2)
+#pragma unroll
+    for (int j = 0; j < w; ++j) part[j] += part[j + w];
+  const float s = block_reduce(part[0], SumOp{}, 0.f, scratch);
+
+  const float log2_s = __builtin_amdgcn_logf(s);  // v_log_f32 is log2
+  // loss = ln(sum exp(x - max)) - (x_t - max): the difference to the maximum is formed with one
+  // fused multiply-add against the same rounded m2 the sum used, so a loss near 0 keeps its digits
+  if (tid == 0 && row_loss) {
+    const float l = (log2_s - __builtin_fmaf(x_t, kLog2e, -m2)) * kLn2;
+    row_loss[row] = class_weight ? l * wt : l;
+  }
+  if (dlogits == nullptr) return;
+
+  // ---- dlogits = (p - onehot) * scale with p = 2^(x*log2e - m2) / s.  The exponent is taken
+  // relative to the row maximum with one fused multiply-add, the same expression the sum above
+  // used, so the rounding of m2 cancels between numerator and denominator and p keeps fp32
+  // accuracy; folding log2(s) and log2(scale) into the exponent instead costs ~1e-6 relative,
+  // which the subtraction at the target column amplifies when p is close to 1.
+  const float factor = scale / s;  // s >= 1: the maximum contributes 2^0
+  const int t_at = (int)target + off, t_vec = t_at / VN, t_sub = t_at % VN;
+#pragma unroll
+  for (int j = 0; j < VPT; ++j) {
+    const int idx = tid + block * j;
+    if (idx < nvec) {
+      const int c0 = idx * VN - off;
+      float o[VN];
+#pragma unroll
+      for (int k = 0; k < VN; ++k)
+        o[k] = __builtin_amdgcn_exp2f(__builtin_fmaf(to_acc(xr[j].e[k]), kLog2e, -m2)) * factor;
+      if (c0 + VN > iV) {  // last class vector and the padding: 0 also where the sum is not finite
+#pragma unroll
+        for (int k = 0; k < VN; ++k)
+          if (c0 + k >= iV) o[k] = 0.f;
+      }
+      if (idx == t_vec) {
+#pragma unroll
+        for (int k = 0; k < VN; ++k)
+          if (k == t_sub) o[k] -= scale;
+      }
+      if (shared_vector(c0)) {
+        store_own<TD, VN>(d + (int64_t)idx * VN, o, c0, stride);
+      } else {
+        store_out<T, TD, VN>(d + (int64_t)idx * VN, o);
+      }
+    }
   }
 }
 
@@ -1034,8 +1074,8 @@ __global__ __launch_bounds__(BLOCK, 6) void ce_loss_rows_kernel(
 }
 
 // Rows too wide for registers, rows too wide for the streaming kernel where only the loss is wanted or the
-// row-holding kernel would run a second round of few rows, and rows whose stride is not a multiple of the vector
-// width (a vocabulary used unpadded) where they are narrow.  Persistent workgroups walk rows.  A row is split into a head of
+// row-holding kernel would run a second round of few rows, and few unpadded rows with fp32 gradients that would leave
+// the streaming kernel's lanes half empty.  Persistent workgroups walk rows.  A row is split into a head of
 // single elements up to the first 16-byte boundary, a body of whole vectors and a tail; the
 // base pointers are 16-byte aligned, so gradient rows split at the same columns.  The body is
 // read twice in chunks of kWideU vectors per lane: the first sweep keeps a running (max, sum)
@@ -1395,25 +1435,16 @@ int64_t compute_units() {
   return n;
 }
 
-// Two-sweep kernel: workgroups of 1024 lanes, two per CU, for wide rows; of 256 lanes, eight
-// per CU, where a row has too few vectors to occupy 1024.
+// Two-sweep kernel: two workgroups of 1024 lanes per CU.
 template <typename T, typename TD>
 void launch_wide(const void *logits, void *dlogits, const int64_t *targets, float *row_loss,
                  const int *ws_count, int64_t N, int64_t V, int64_t row_stride, int64_t ignore_index,
                  int reduction, float dloss, const float *class_weight, hipStream_t s) {
   const int64_t cus = compute_units();
-  const int64_t nvec = row_stride / Vec16<T>::n;
-  if (nvec > 256 * kWideU * 2) {
-    const dim3 grid((unsigned)(N < 2 * cus ? N : 2 * cus));
-    ce_rows_wide_kernel<T, TD, 1024><<<grid, dim3(1024), 0, s>>>(
-        (const T *)logits, (TD *)dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index,
-        reduction, dloss, class_weight);
-  } else {
-    const dim3 grid((unsigned)(N < 8 * cus ? N : 8 * cus));
-    ce_rows_wide_kernel<T, TD, 256><<<grid, dim3(256), 0, s>>>(
-        (const T *)logits, (TD *)dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index,
-        reduction, dloss, class_weight);
-  }
+  const dim3 grid((unsigned)(N < 2 * cus ? N : 2 * cus));
+  ce_rows_wide_kernel<T, TD, 1024><<<grid, dim3(1024), 0, s>>>(
+      (const T *)logits, (TD *)dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index,
+      reduction, dloss, class_weight);
 }
 
 // Accesses (of 16 bytes; 8 where 16-bit logits give fp32 gradients) a row may take for the streaming
@@ -1460,6 +1491,32 @@ void launch_stream(const void *logits, void *dlogits, const int64_t *targets, fl
 #undef CS_CE_STREAM
 }
 
+// Rows of up to 2048 vectors of 16 bytes, four accesses a lane (eight of 8 bytes for fp32 gradients of 16-bit logits) and as
+// many waves as that takes: false where the row is too wide.  Twice as wide where there are more than two rows per CU; of
+// unpadded rows, whose edges take more instructions, one and a half times.  (Before, one wave of eight accesses up to 512
+// vectors and four waves beyond; unpadded and weighted rows in two sweeps; wider ones by the streaming kernel.)
+// us per call, before / now, bf16 unless said: padded [8192,4096] 29.8 / 28.6, [7501,7808] 46.1 / 42.7, [8192,16384]
+// 94.7 / 92.6; unpadded [16384,1001] 48.1 / 24.9, [13786,3378] 55.0 / 39.6, [6000,10001] 82.7 / 46.9, [2099,15215] 36.3 /
+// 29.4, fp32 [4096,7999] 62.1 / 49.6; fp32 gradients [15248,4553] fp16 109.4 / 77.5, [11936,9472] 156 / 119, [4096,16000]
+// 110 / 73; weighted [2000,12000] 32.6 / 24.8; few rows [16,4160] 7.8 / 6.6, [277,3448] 8.8 / 7.9.  The wider ones:
+// [2099,20215] 50.0 / 39.4, [1000,20215] 25.5 / 23.6, [6000,20215] fp16 weighted 119 / 88, [4096,32000] 97 / 89,
+// [4096,20000] with fp32 gradients 114 / 92; but unpadded [4096,32001] 106 / 113, [300,30000] 14.1 / 15.4, fp32
+// [338,15424] 13.6 / 14.6.
+template <typename T, typename TD, bool RAGGED>
+bool launch_narrow(const void *logits, void *dlogits, const int64_t *targets, float *row_loss, const int *ws_count,
+                   int64_t N, int64_t V, int64_t row_stride, int64_t ignore_index, int reduction, float dloss,
+                   const float *class_weight, hipStream_t s) {
+  constexpr int EPV = StreamPlan<T, TD>::kEpv, U = EPV * sizeof(T) == 8 ? 8 : 4;
+  const int64_t nvec = (row_stride + (RAGGED ? kLineElems<T> - 1 : 0) + EPV - 1) / EPV;
+  const int threads = N <= 2 * compute_units() ? 512 : RAGGED ? 768 : kNarrowMostThreads;
+  if (nvec > threads * U) return false;
+  ce_rows_kernel<T, TD, U, EPV, RAGGED>
+      <<<dim3((unsigned)N), dim3((unsigned)(ceil_div(nvec, (int64_t)(kWave * U)) * kWave)), 0, s>>>(
+          (const T *)logits, (TD *)dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index, reduction, dloss,
+          class_weight);
+  return true;
+}
+
 // Vectors per lane of the row-holding kernel: three, four or five units.
 template <typename T, typename TD>
 struct HoldPlan {
@@ -1500,9 +1557,7 @@ int launch_rows(const void *logits, void *dlogits, const int64_t *targets, float
   const bool vec_ok = base_ok && row_stride % VN == 0;
   const dim3 grid((unsigned)N);
   if constexpr (!std::is_same_v<T, double>) {
-    // per-class weights: the streaming kernel, the two-sweep kernel (any aligned row) and the
-    // general one take them; the small row-in-registers kernels do not (no caller of the reference
-    // sets weights), so weighted calls on narrow rows go to the two-sweep kernel
+    // per-class weights: every kernel but the fp32 one of 1024 lanes and 16 vectors takes them
     const int64_t nvec_all = row_stride / VN;
     const bool streams = nvec_all > 256 * 8 &&
                          row_stride <= (int64_t)StreamPlan<T, TD>::kEpv * StreamPlan<T, TD>::kMostVecs;
@@ -1531,30 +1586,29 @@ int launch_rows(const void *logits, void *dlogits, const int64_t *targets, float
                                 : sizeof(TD) == sizeof(T) && row_stride < 80000 ? 2 * N > 3 * cus
                                                                                 : 4 * N > 5 * cus;
     const bool holds = dlogits != nullptr && nvec_all > 256 * 8 && (N <= cus || past_one_round);
+    if (base_ok && nvec_all <= kNarrowMostThreads * 4 &&
+        (vec_ok ? launch_narrow<T, TD, false>(logits, dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index,
+                                              reduction, dloss, class_weight, s)
+                : launch_narrow<T, TD, true>(logits, dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index,
+                                             reduction, dloss, class_weight, s)))
+      return launch_status();
     if (vec_ok && (class_weight == nullptr || streams)) {
-      const int64_t nvec = row_stride / VN;
-#define CS_CE(BLOCK, VPT)                                                                   \
-  ce_rows_kernel<T, TD, BLOCK, VPT><<<grid, dim3(BLOCK), 0, s>>>(                           \
-      (const T *)logits, (TD *)dlogits, targets, row_loss, ws_count, V, row_stride,         \
-      ignore_index, reduction, dloss)
-      if (nvec <= 64 * 8) {
-        CS_CE(64, 8);
-      } else if (nvec <= 256 * 8) {
-        CS_CE(256, 8);
-      } else if (row_stride <= (int64_t)StreamPlan<T, TD>::kEpv * StreamPlan<T, TD>::kMostVecs) {
+      if (row_stride <= (int64_t)StreamPlan<T, TD>::kEpv * StreamPlan<T, TD>::kMostVecs) {
         launch_stream<T, TD, false>(logits, dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index,
                                     reduction, dloss, class_weight, s);
       } else if (holds && row_stride <= (int64_t)HoldPlan<T, TD>::kEpv * HoldPlan<T, TD>::kMostVecs) {
         launch_hold<T, TD, false>(logits, dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index,
                                   reduction, dloss, class_weight, s);
-      } else if (sizeof(T) == 4 && nvec <= 1024 * 16) {
+      } else if (sizeof(T) == 4 && nvec_all <= 1024 * 16) {
         // fp32 rows up to 65536 columns still fit in registers (at 16 bit this plan spills)
-        if constexpr (sizeof(T) == 4) CS_CE(1024, 16);
+        if constexpr (sizeof(T) == 4)
+          ce_rows_kernel<T, TD, 16, VN, false, 1024><<<grid, dim3(1024), 0, s>>>(
+              (const T *)logits, (TD *)dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index, reduction,
+              dloss, nullptr);
       } else {
         launch_wide<T, TD>(logits, dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index,
                            reduction, dloss, class_weight, s);
       }
-#undef CS_CE
       return launch_status();
     }
     // Unpadded rows that fill little of the streaming plan take two sweeps: with fp32 gradients of 16-bit logits rows

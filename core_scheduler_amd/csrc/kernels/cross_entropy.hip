@@ -52,44 +52,83 @@ __device__ __forceinline__ bool target_counts(int64_t t, int64_t V, int64_t igno
 // at a time a quarter of a million rows took 75 us each.
 constexpr int kSmallInFlight = 8;
 
-// Number of rows that count, and what the mean divides by: that number, or the sum of the class weights
-// of those rows.  One workgroup of 1024; valid in thread 0 (and every other).
-__device__ __forceinline__ void count_rows(const int64_t *__restrict__ targets, int64_t N, int64_t V,
-                                           int64_t ignore_index, const float *__restrict__ class_weight,
-                                           int *count, float *total) {
-  __shared__ int scratch[16];
-  __shared__ float wscratch[16];
-  const int tid = threadIdx.x;
-  int c = 0;
-  float wsum[kSmallInFlight];  // per-class weights of the rows that count: interleaved sums, fixed order
+// What one lane, and then the workgroup, knows of the rows: a loss, how many count, and the sum of their class weights.
+struct RowSums {
+  float loss;
+  int count;
+  float weight;
+};
+// Lane t's rows t, t + 1024, ...: `load` a step's, each its own before the first is used (a row past the end re-reads the
+// last one), then `use` them.  One row a lane where there are no more: eight loads for one cost 0.3 us.
+template <int ROWS, typename Load, typename Use>
+__device__ __forceinline__ void rows_of_lane_by(int64_t N, Load &&load, Use &&use) {
+  for (int64_t i0 = threadIdx.x; i0 < N; i0 += (int64_t)1024 * ROWS) {
+#pragma unroll
+    for (int u = 0; u < ROWS; ++u) {
+      const int64_t i = i0 + (int64_t)u * 1024;
+      load(u, i < N ? i : N - 1);
+    }
+#pragma unroll
+    for (int u = 0; u < ROWS; ++u) use(u, i0 + (int64_t)u * 1024 < N);
+  }
+}
+template <typename Load, typename Use>
+__device__ __forceinline__ void rows_of_lane(int64_t N, Load &&load, Use &&use) {
+  if (N <= 1024) {  // kernel-uniform
+    rows_of_lane_by<1>(N, load, use);
+  } else {
+    rows_of_lane_by<kSmallInFlight>(N, load, use);
+  }
+}
+// Lane t's share of the count and the weights, these in kSmallInFlight interleaved sums.
+__device__ __forceinline__ void count_rows(RowSums &sums, const int64_t *__restrict__ targets, int64_t N, int64_t V,
+                                           int64_t ignore_index, const float *__restrict__ class_weight) {
+  int64_t t[kSmallInFlight];
+  if (class_weight == nullptr) {  // kernel-uniform
+    rows_of_lane(
+        N, [&](int u, int64_t i) { t[u] = targets[i]; },
+        [&](int u, bool there) { sums.count += there && target_counts(t[u], V, ignore_index); });
+    return;
+  }
+  float w[kSmallInFlight], wsum[kSmallInFlight];
 #pragma unroll
   for (int u = 0; u < kSmallInFlight; ++u) wsum[u] = 0.f;
-  for (int64_t i0 = tid; i0 < N; i0 += (int64_t)1024 * kSmallInFlight) {
-    int64_t t[kSmallInFlight];
+  rows_of_lane(
+      N,
+      [&](int u, int64_t i) {
+        t[u] = targets[i];
+        w[u] = class_weight[target_counts(t[u], V, ignore_index) ? t[u] : 0];
+      },
+      [&](int u, bool there) {
+        const bool counts = there && target_counts(t[u], V, ignore_index);
+        sums.count += counts;
+        wsum[u] += counts ? w[u] : 0.f;
+      });
 #pragma unroll
-    for (int u = 0; u < kSmallInFlight; ++u) {
-      const int64_t i = i0 + (int64_t)u * 1024;
-      t[u] = i < N ? targets[i] : ignore_index;
-    }
-#pragma unroll
-    for (int u = 0; u < kSmallInFlight; ++u) c += target_counts(t[u], V, ignore_index);
-    if (class_weight != nullptr) {  // block-uniform
-      float w[kSmallInFlight];
-#pragma unroll
-      for (int u = 0; u < kSmallInFlight; ++u) w[u] = class_weight[target_counts(t[u], V, ignore_index) ? t[u] : 0];
-#pragma unroll
-      for (int u = 0; u < kSmallInFlight; ++u) wsum[u] += target_counts(t[u], V, ignore_index) ? w[u] : 0.f;
-    }
+  for (int u = 0; u < kSmallInFlight; ++u) sums.weight += wsum[u];
+}
+// The workgroup's sums, for its first wave, with one exchange: each in the order of block_reduce.  (The weights only where
+// there are any.)
+template <bool LOSS>
+__device__ __forceinline__ RowSums block_sums(RowSums s, bool weighted) {
+  __shared__ float loss_of[16], weight_of[16];
+  __shared__ int count_of[16];
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+  if constexpr (LOSS) s.loss = wave_reduce(s.loss, SumOp{});
+  s.count = wave_reduce(s.count, SumOp{});
+  if (weighted) s.weight = wave_reduce(s.weight, SumOp{});  // workgroup-uniform
+  if (lane == 0) {
+    if constexpr (LOSS) loss_of[wave] = s.loss;
+    count_of[wave] = s.count;
+    if (weighted) weight_of[wave] = s.weight;
   }
-  c = block_reduce(c, SumOp{}, 0, scratch);
-  *count = c;
-  *total = (float)c;  // without class weights every row that counts weighs 1
-  if (class_weight != nullptr) {
-    float ws_ = 0.f;
-#pragma unroll
-    for (int u = 0; u < kSmallInFlight; ++u) ws_ += wsum[u];
-    *total = block_reduce(ws_, SumOp{}, 0.f, wscratch);
-  }
+  __syncthreads();
+  if (wave != 0) return s;
+  const bool mine = lane < 16;
+  if constexpr (LOSS) s.loss = wave_reduce(mine ? loss_of[lane & 15] : 0.f, SumOp{});
+  s.count = wave_reduce(mine ? count_of[lane & 15] : 0, SumOp{});
+  if (weighted) s.weight = wave_reduce(mine ? weight_of[lane & 15] : 0.f, SumOp{});
+  return s;
 }
 
 // The same number for a row kernel of few rows, by every wave for itself: eight targets a lane, all requested at once,
@@ -118,12 +157,13 @@ __global__ __launch_bounds__(1024) void ce_count_kernel(const int64_t *__restric
                                                         int *__restrict__ ws_count,
                                                         float *__restrict__ ws_weight,
                                                         const float *__restrict__ class_weight) {
-  int c;
-  float total;
-  count_rows(targets, N, V, ignore_index, class_weight, &c, &total);
+  RowSums sums{0.f, 0, 0.f};
+  count_rows(sums, targets, N, V, ignore_index, class_weight);
+  sums = block_sums<false>(sums, class_weight != nullptr);
   if (threadIdx.x == 0) {
-    *ws_count = c;
-    *ws_weight = total;
+    *ws_count = sums.count;
+    // without class weights every row that counts weighs 1
+    *ws_weight = class_weight != nullptr ? sums.weight : (float)sums.count;
   }
 }
 
@@ -142,39 +182,28 @@ __global__ __launch_bounds__(1024) void ce_reduce_kernel(const float *__restrict
                                                          const int64_t *__restrict__ targets, int64_t V,
                                                          int64_t ignore_index,
                                                          const float *__restrict__ class_weight) {
-  __shared__ float scratch[16];
   const int tid = threadIdx.x;
-  float part[kSmallInFlight];
+  float v[kSmallInFlight], part[kSmallInFlight];
 #pragma unroll
   for (int u = 0; u < kSmallInFlight; ++u) part[u] = 0.f;
-  for (int64_t i0 = tid; i0 < N; i0 += (int64_t)1024 * kSmallInFlight) {
-    float v[kSmallInFlight];
+  rows_of_lane(
+      N, [&](int u, int64_t i) { v[u] = row_loss[i]; }, [&](int u, bool there) { part[u] += there ? v[u] : 0.f; });
+  RowSums sums{0.f, 0, 0.f};
 #pragma unroll
-    for (int u = 0; u < kSmallInFlight; ++u) {
-      const int64_t i = i0 + (int64_t)u * 1024;
-      v[u] = i < N ? row_loss[i] : 0.f;
-    }
-#pragma unroll
-    for (int u = 0; u < kSmallInFlight; ++u) part[u] += v[u];
-  }
-  float s = 0.f;
-#pragma unroll
-  for (int u = 0; u < kSmallInFlight; ++u) s += part[u];
-  int c = 0;
-  float total;
-  if constexpr (COUNT) {
-    count_rows(targets, N, V, ignore_index, class_weight, &c, &total);
-  } else {
-    // the float next to the count: the number of rows that count, or the sum of their class weights
-    total = reinterpret_cast<const float *>(ws_count)[1];
-  }
-  s = block_reduce(s, SumOp{}, 0.f, scratch);
+  for (int u = 0; u < kSmallInFlight; ++u) sums.loss += part[u];
+  if constexpr (COUNT) count_rows(sums, targets, N, V, ignore_index, class_weight);
+  sums = block_sums<true>(sums, COUNT && class_weight != nullptr);
   if (tid == 0) {
+    // the float next to the count: the number of rows that count, or the sum of their class weights
+    float total;
     if constexpr (COUNT) {
-      *ws_count = c;
+      total = class_weight != nullptr ? sums.weight : (float)sums.count;
+      *ws_count = sums.count;
       reinterpret_cast<float *>(ws_count)[1] = total;
+    } else {
+      total = reinterpret_cast<const float *>(ws_count)[1];
     }
-    if (loss) *loss = reduction == CS_REDUCTION_MEAN ? s / total : s;
+    if (loss) *loss = reduction == CS_REDUCTION_MEAN ? sums.loss / total : sums.loss;
     if (total_weight) *total_weight = total;
   }
 }
@@ -1385,7 +1414,6 @@ __global__ __launch_bounds__(1024) void ce_loss_combine_kernel(
     float *__restrict__ row_loss, int64_t N, int *__restrict__ ws_count, int reduction, float *__restrict__ loss,
     float *__restrict__ total_weight, const int64_t *__restrict__ targets, int64_t V, int64_t ignore_index,
     const float *__restrict__ class_weight) {
-  __shared__ float scratch[16];
   const int tid = threadIdx.x;
   const int row = tid < (int)N ? tid : (int)N - 1;
   const int64_t tgt = targets[row];
@@ -1408,14 +1436,12 @@ __global__ __launch_bounds__(1024) void ce_loss_combine_kernel(
   const float wt = counts && class_weight != nullptr ? class_weight[tgt] : 1.f;
   const float l = counts ? (__builtin_amdgcn_logf(s) - __builtin_fmaf(x_t, kLog2e, -m2)) * kLn2 * wt : 0.f;
   if (tid < (int)N) row_loss[row] = l;
-  int c = 0;
-  float total;
-  count_rows(targets, N, V, ignore_index, class_weight, &c, &total);
-  const float sum = block_reduce(l, SumOp{}, 0.f, scratch);
+  const RowSums sums = block_sums<true>(RowSums{l, counts, counts ? wt : 0.f}, class_weight != nullptr);
   if (tid == 0) {
-    *ws_count = c;
+    const float total = class_weight != nullptr ? sums.weight : (float)sums.count;
+    *ws_count = sums.count;
     reinterpret_cast<float *>(ws_count)[1] = total;
-    if (loss) *loss = reduction == CS_REDUCTION_MEAN ? sum / total : sum;
+    if (loss) *loss = reduction == CS_REDUCTION_MEAN ? sums.loss / total : sums.loss;
     if (total_weight) *total_weight = total;
   }
 }
@@ -1491,8 +1517,8 @@ void launch_stream(const void *logits, void *dlogits, const int64_t *targets, fl
 #undef CS_CE_STREAM
 }
 
-// Rows of up to 2048 vectors of 16 bytes, four accesses a lane (eight of 8 bytes for fp32 gradients of 16-bit logits) and as
-// many waves as that takes: false where the row is too wide.  Twice as wide where there are more than two rows per CU; of
+// Rows of up to 2048 vectors of 16 bytes, four accesses a lane (eight of 8 bytes for fp32 gradients of 16-bit logits; half or
+// a quarter of that where one wave then has the row) and as many waves as that takes: false where the row is too wide.  Twice as wide where there are more than two rows per CU; of
 // unpadded rows, whose edges take more instructions, one and a half times.  (Before, one wave of eight accesses up to 512
 // vectors and four waves beyond; unpadded and weighted rows in two sweeps; wider ones by the streaming kernel.)
 // us per call, before / now, bf16 unless said: padded [8192,4096] 29.8 / 28.6, [7501,7808] 46.1 / 42.7, [8192,16384]
@@ -1510,10 +1536,19 @@ bool launch_narrow(const void *logits, void *dlogits, const int64_t *targets, fl
   const int64_t nvec = (row_stride + (RAGGED ? kLineElems<T> - 1 : 0) + EPV - 1) / EPV;
   const int threads = N <= 2 * compute_units() ? 512 : RAGGED ? 768 : kNarrowMostThreads;
   if (nvec > threads * U) return false;
-  ce_rows_kernel<T, TD, U, EPV, RAGGED>
-      <<<dim3((unsigned)N), dim3((unsigned)(ceil_div(nvec, (int64_t)(kWave * U)) * kWave)), 0, s>>>(
-          (const T *)logits, (TD *)dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index, reduction, dloss,
-          class_weight);
+#define CS_CE_NARROW(VPT)                                                                                          \
+  ce_rows_kernel<T, TD, VPT, EPV, RAGGED>                                                                          \
+      <<<dim3((unsigned)N), dim3((unsigned)(ceil_div(nvec, (int64_t)(kWave * VPT)) * kWave)), 0, s>>>(             \
+          (const T *)logits, (TD *)dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index, reduction, \
+          dloss, class_weight)
+  if (nvec <= kWave * U / 4) {
+    CS_CE_NARROW(U / 4);
+  } else if (nvec <= kWave * U / 2) {
+    CS_CE_NARROW(U / 2);
+  } else {
+    CS_CE_NARROW(U);
+  }
+#undef CS_CE_NARROW
   return true;
 }
 

@@ -73,3 +73,23 @@ def test_rows_that_are_not_finite(stride, bad):
     clean = ops.fused_classifier(torch.where(torch.isfinite(x), x, torch.zeros_like(x)), t, 499)
     assert torch.isnan(rows[1]) and torch.isnan(d[1, :499]).all() and not d[:, 499:].any()
     assert torch.equal(rows[0], clean[1][0]) and torch.equal(d[0], clean[2][0]) and torch.equal(d[2], clean[2][2])
+
+
+@pytest.mark.parametrize("N", [1023, 1024, 1025, 8193])  # one row a lane of the last launch, and eight under way
+@pytest.mark.parametrize("weighted", [False, True])
+def test_sums_over_the_rows(N, weighted):
+    from core_scheduler_amd import ops
+
+    V = 40
+    x, t = randn((N, V), 64, dtype=F32).cuda(), randint(-1, V + 1, (N,), 65).cuda()  # some rows out of range
+    w = (torch.rand(V, generator=gen(66)) + 0.5).cuda() if weighted else None
+    keep = (t >= 0) & (t < V)
+    at = t.clamp(0, V - 1)
+    wt = (w.double()[at] if weighted else torch.ones(N, dtype=torch.float64, device="cuda")) * keep
+    want = (-x.double().log_softmax(1).gather(1, at[:, None])[:, 0] * wt).sum()
+    for reduction, by in (("sum", 1.0), ("mean", wt.sum())):
+        for gradient in (True, False):
+            loss, _, _, total = ops.fused_classifier(x, t, V, reduction=reduction, class_weight=w, want_dlogits=gradient)
+            # sums of positive terms, 2^-24 a level of a tree of at most 20
+            assert abs(loss.item() - (want / by).item()) <= 20 * 2.0 ** -24 * (want / by).item()
+            assert abs(total.item() - wt.sum().item()) <= 20 * 2.0 ** -24 * wt.sum().item()

@@ -685,31 +685,37 @@ constexpr int kVpl = CS_EMB_VPL;                // 16-byte column vectors per la
 // which leaves most of the chip idle then: kernels of a call, us, finish / sort: 16384 x 1600 bf16 accumulating 56.8 /
 // 51.9 (Zipf) and 63.1 / 58.4 (uniform), tables of 3 MB 45.1 / 41.5, 32 MB 49.1 / 47.2, 64 MB 51.2 / 51.4, 161 MB 55.7 /
 // 57.4; 32768 x 768 46 MB 54.5 / 53.8, 77 MB 55.1 / 57.1; 16384 x 512 fp32 8 MB 34.7 / 30.9, 103 MB 37.0 / 39.6.
+// Lists of up to this many windows have a slice of 64 vectors of the columns to a workgroup, so that more than half of the
+// CUs have one: kernels of a call, us, whole rows / slices: 4000 x 512 fp32 14.2 / 13.5, added to the table 16.7 / 14.1,
+// [3,400] x 1600 fp32 26.3 / 18.4, [4,1024] x 1600 into 1000 rows 20.4 / 19.1, [8,543] x 768 17.3 / 16.8, [3,349] x 1024
+// 14.9 / 14.0; but [8,1024] x 768 25.6 / 26.3, 16384 x 1600 56.2 / 58.9.
+constexpr int64_t kSlicedWindows = 192;
 constexpr int64_t kPosFewFill = (int64_t)3 << 20;
 constexpr int64_t kPosEarlyWindows = 256;
 
 // Workgroup w reduces sorted entries [kWindow w, kWindow (w + 1)).  partial rows live at
 // partial[(w*2 + slot) * C]: slot 0 for a run that came in over the window's
 // left edge and ends inside, slot 1 for a run that leaves over its right edge.
-template <typename T>
+template <typename T, int VPL>
 __global__ __launch_bounds__(kRedThreads, 2048 / kRedThreads) void emb_bwd_reduce_kernel(
     const T *__restrict__ dout, const uint32_t *__restrict__ sorted_id,
     const uint32_t *__restrict__ sorted_pos, T *__restrict__ dweight, float *__restrict__ partial,
-    int64_t n, int64_t C, int accumulate, int by_freq, int64_t windows, T *__restrict__ dwpe, int64_t B, int64_t TC,
-    int pos_log2_slices) {
+    int64_t n, int64_t C, int accumulate, int by_freq, int64_t windows, int slices, T *__restrict__ dwpe, int64_t B,
+    int64_t TC, int pos_log2_slices) {
   constexpr int VN = Vec16<T>::n;
-  constexpr int kChunkCols = kWave * kVpl * VN;
+  constexpr int kChunkCols = kWave * VPL * VN;
   extern __shared__ float lds[];  // [kRedWaves][2 slots][kChunkCols]
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = tid >> 6;
   const int nvec = (int)(C / VN);
-  const int64_t w = blockIdx.x;
-  if (w >= windows) {
-    positions_block<T, kRedThreads>(dout, dwpe, w - windows, B, TC, accumulate, pos_log2_slices,
+  if (blockIdx.x >= windows * slices) {
+    positions_block<T, kRedThreads>(dout, dwpe, blockIdx.x - windows * slices, B, TC, accumulate, pos_log2_slices,
                                     reinterpret_cast<f32x4 *>(lds), tid);
     return;
   }
+  const int64_t w = slices == 1 ? blockIdx.x : blockIdx.x / (unsigned)slices;
+  const int slice = (int)(blockIdx.x - w * slices);
   const int64_t p0 = w * kWindow;
 
   // ---- ids of the window (lane l <-> entry p0 + l), the entry before and the entry after
@@ -749,22 +755,22 @@ __global__ __launch_bounds__(kRedThreads, 2048 / kRedThreads) void emb_bwd_reduc
     return b < n_valid ? b : n_valid;
   };
 
-  for (int cb = 0; cb < nvec; cb += kWave * kVpl) {
+  for (int cb = slice * kWave * VPL; cb < nvec; cb += slices * kWave * VPL) {
     // ---- level 1: this wave's four entries
     const int e0 = wave * kOwn;
-    // all kOwn * kVpl row loads are in flight before the first is used: an entry past the valid
+    // all kOwn * VPL row loads are in flight before the first is used: an entry past the valid
     // ones reads row 0, a vector past the row re-reads the row's last one; neither is added
-    Vec16<T> r[kOwn][kVpl];
+    Vec16<T> r[kOwn][VPL];
 #pragma unroll
     for (int e = 0; e < kOwn; ++e) {
       const int64_t pos = e0 + e < n_valid ? (int64_t)__shfl(lane_pos, e, kWave) : 0;
 #pragma unroll
-      for (int j = 0; j < kVpl; ++j) {
+      for (int j = 0; j < VPL; ++j) {
         const int idx = cb + lane + kWave * j;
         r[e][j] = load16_stream(dout + pos * C + (int64_t)(idx < nvec ? idx : nvec - 1) * VN);
       }
     }
-    float acc[kVpl][VN];
+    float acc[VPL][VN];
     int piece_start = e0;
 #pragma unroll
     for (int e = 0; e < kOwn; ++e) {
@@ -774,12 +780,12 @@ __global__ __launch_bounds__(kRedThreads, 2048 / kRedThreads) void emb_bwd_reduc
       if (e == 0 || starts_here) {
         piece_start = q;
 #pragma unroll
-        for (int j = 0; j < kVpl; ++j)
+        for (int j = 0; j < VPL; ++j)
 #pragma unroll
           for (int k = 0; k < VN; ++k) acc[j][k] = 0.f;
       }
 #pragma unroll
-      for (int j = 0; j < kVpl; ++j) {
+      for (int j = 0; j < VPL; ++j) {
         if (cb + lane + kWave * j < nvec) {
 #pragma unroll
           for (int k = 0; k < VN; ++k) acc[j][k] += to_acc(r[e][j].e[k]);
@@ -800,7 +806,7 @@ __global__ __launch_bounds__(kRedThreads, 2048 / kRedThreads) void emb_bwd_reduc
           // scale_grad_by_freq: the sum over the id's entries divided by their number
           const float inv = by_freq ? 1.0f / (float)(q - piece_start + 1) : 1.0f;
 #pragma unroll
-          for (int j = 0; j < kVpl; ++j) {
+          for (int j = 0; j < VPL; ++j) {
             const int idx = cb + lane + kWave * j;
             if (idx < nvec) {
               Vec16<T> o;
@@ -818,7 +824,7 @@ __global__ __launch_bounds__(kRedThreads, 2048 / kRedThreads) void emb_bwd_reduc
         } else {
           float *dst = partial + (w * 2 + (seg_ends ? 0 : 1)) * C;
 #pragma unroll
-          for (int j = 0; j < kVpl; ++j) {
+          for (int j = 0; j < VPL; ++j) {
             const int idx = cb + lane + kWave * j;
             if (idx < nvec) {
 #pragma unroll
@@ -834,7 +840,7 @@ __global__ __launch_bounds__(kRedThreads, 2048 / kRedThreads) void emb_bwd_reduc
                 constexpr int H = VN / 4;
         f32x4 *dst = reinterpret_cast<f32x4 *>(lds) + (wave * 2 + slot) * (kChunkCols / 4);
 #pragma unroll
-        for (int j = 0; j < kVpl; ++j)
+        for (int j = 0; j < VPL; ++j)
 #pragma unroll
           for (int h = 0; h < H; ++h)
             dst[(j * H + h) * kWave + lane] =
@@ -864,7 +870,7 @@ __global__ __launch_bounds__(kRedThreads, 2048 / kRedThreads) void emb_bwd_reduc
         float *prow = partial + (w * 2 + (seg_ends ? 0 : 1)) * C;
         typedef float f32x4 __attribute__((ext_vector_type(4)));
         const f32x4 *lds4 = reinterpret_cast<const f32x4 *>(lds);
-        constexpr int kSlices = kChunkCols / 4 / kWave;  // groups of four columns per lane (kVpl * VN / 4)
+        constexpr int kSlices = kChunkCols / 4 / kWave;  // groups of four columns per lane (VPL * VN / 4)
         f32x4 t[kSlices];
 #pragma unroll
         for (int v = 0; v < kSlices; ++v) t[v] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1816,10 +1822,22 @@ int sort_launch(const void *ids, char *ws, const BwdLayout &L, int64_t n, int64_
   return launch_status();
 }
 
-template <typename T>
-int allow_reduce_lds(size_t bytes) {
+template <typename T, int VPL>
+int reduce_launch(const void *dout, const uint32_t *sorted_id, const uint32_t *sorted_pos, void *dweight, float *partial,
+                  int64_t n, int64_t C, int accumulate, int by_freq, int64_t windows, int slices, int64_t pos_blocks,
+                  void *dwpe, int64_t B, int64_t TC, int pos_log2_slices, hipStream_t s) {
+  constexpr int VN = Vec16<T>::n;
+  constexpr size_t kFold = (size_t)kRedWaves * 2 * kWave * VPL * VN * sizeof(float), kPos = kRedThreads * kPosLdsBytesPerLane;
+  constexpr size_t lds = kFold > kPos ? kFold : kPos;
+  const int64_t blocks = windows * slices + pos_blocks;
+  if (blocks > 0x7fffffffLL) return CS_ERR_TOO_LARGE;
   static std::atomic<bool> done[64];
-  return allow_dynamic_lds_once(reinterpret_cast<const void *>(&emb_bwd_reduce_kernel<T>), bytes, done);
+  const int st = allow_dynamic_lds_once(reinterpret_cast<const void *>(&emb_bwd_reduce_kernel<T, VPL>), lds, done);
+  if (st != CS_OK) return st;
+  emb_bwd_reduce_kernel<T, VPL><<<dim3((unsigned)blocks), dim3(kRedThreads), lds, s>>>(
+      (const T *)dout, sorted_id, sorted_pos, (T *)dweight, partial, n, C, accumulate, by_freq, windows, slices, (T *)dwpe, B,
+      TC, pos_log2_slices);
+  return launch_status();
 }
 
 // `pos_blocks` workgroups of position sums ahead of those that finish `windows` windows.
@@ -1942,18 +1960,16 @@ int bwd_typed(const void *dout, const void *ids, void *dweight, void *dwpe, char
     // The position sums go where the chip is idle: next to the finish workgroups, or next to the reducing ones of a
     // list too short to occupy the chip with those.
     const bool pos_early = windows > 0 && windows <= kPosEarlyWindows;
-    const int64_t red_blocks = windows + (pos_early && !pos_first ? pos_blocks(kRedThreads) : 0);
-    if (red_blocks > 0x7fffffffLL) return CS_ERR_TOO_LARGE;
     if (windows > 0) {
-      const size_t lds = (size_t)kRedWaves * 2 * kWave * kVpl * VN * sizeof(float);
-      static_assert(kRedThreads * kPosLdsBytesPerLane <= (size_t)kRedWaves * 2 * kWave * kVpl * VN * sizeof(float),
-                    "the slice sums of the positions fit");
-      st = allow_reduce_lds<T>(lds);
-      if (st != CS_OK) return st;
-      emb_bwd_reduce_kernel<T><<<dim3((unsigned)red_blocks), dim3(kRedThreads), lds, s>>>(
-          (const T *)dout, sorted_id, sorted_pos, (T *)dweight, partial, n, C, accumulate, by_freq, windows, (T *)dwpe,
-          B, TC, log2_s);
-      st = launch_status();
+      const int64_t pos = pos_early && !pos_first ? pos_blocks(kRedThreads) : 0;
+      const int64_t nvec = C / VN;
+      if (windows <= kSlicedWindows && nvec > kWave) {
+        st = reduce_launch<T, 1>(dout, sorted_id, sorted_pos, dweight, partial, n, C, accumulate, by_freq, windows,
+                                 (int)ceil_div(nvec, (int64_t)kWave), pos, dwpe, B, TC, log2_s, s);
+      } else {
+        st = reduce_launch<T, kVpl>(dout, sorted_id, sorted_pos, dweight, partial, n, C, accumulate, by_freq, windows, 1, pos,
+                                    dwpe, B, TC, log2_s, s);
+      }
       if (st != CS_OK) return st;
     }
     return finish_launch<T>(dout, sorted_id, partial, dweight, dwpe, n, C, accumulate, by_freq, windows,

@@ -71,3 +71,19 @@ def test_nothing_outside_the_table_is_written(n):
     want = torch.full_like(buf, 7.0).cpu()
     want[edge:edge + V * C] = torch.zeros(V, C).index_add_(0, ids[:n], dout[:n]).view(-1)
     assert torch.equal(buf.cpu(), want)
+
+
+@pytest.mark.parametrize("n", [6144, 6145])  # windows whose columns are dealt out to workgroups, and whole ones
+@pytest.mark.parametrize("C", [256, 260, 516, 1100])  # fp32: a slice of 64 vectors, one more, three, five
+def test_windows_in_slices(n, C):
+    from core_scheduler_amd import ops
+
+    V = 900
+    ids = zipf_ids(n, V, 26)
+    dout = torch.randint(-8, 9, (n, C), generator=gen(27)).float()  # whole numbers: every order gives the same sums
+    want = torch.zeros(V, C).index_add_(0, ids, dout)
+    got = ops.embedding_backward(dout.cuda(), ids.cuda(), V)
+    assert torch.equal(got.cpu(), want)
+    assert torch.equal(ops.embedding_backward(dout.cuda(), ids.cuda(), V, dweight=got).cpu(), 2 * want)
+    dwte, dwpe = ops.embedding_backward_fused(dout.view(1, n, C).cuda(), ids.view(1, n).cuda(), V)
+    assert torch.equal(dwte.cpu(), want) and torch.equal(dwpe.cpu(), dout)

@@ -132,11 +132,8 @@ __device__ __forceinline__ float row_lanes_sum(float v, bool upper) {
 #ifndef CS_LN_ADD_ROWS_VPL1
 #define CS_LN_ADD_ROWS_VPL1 4
 #endif
-#ifndef CS_LN_ADD_ROWS_VPL2
-#define CS_LN_ADD_ROWS_VPL2 4
-#endif
 #ifndef CS_LN_ADD_ROWS_VPL4
-#define CS_LN_ADD_ROWS_VPL4 2
+#define CS_LN_ADD_ROWS_VPL4 1
 #endif
 // two rows per wave (rows of up to 32, and of 65-96, vectors): row pairs a wave normalises per step
 #ifndef CS_LN_FWD_HALF
@@ -1779,10 +1776,19 @@ FastPlan fast_plan(int64_t C, int x_dtype) {
 // Grid caps: beyond these the waves loop over rows (with prefetch) instead of
 // the grid growing, which keeps the parameters in registers for many rows
 // and bounds the number of partial rows the backward pass leaves behind.
+// Forward: 512 workgroups of 4 waves, the two waves per SIMD that most of these kernels' registers allow: of twice as
+// many the second half starts when the first has ended, asks for its parameters again and ends with a part-filled
+// step.  1024 / 512 workgroups, us per call: bf16 [16384,768] with the residual 18.9 / 17.5, [16384,512] 14.1 / 12.3,
+// fp16 [16384,640] 21.5 / 17.1; without it [8192,1600] 13.6 / 11.4, [16384,1024] 15.4 / 13.8, [5000,3072] 14.5 / 13.0.
+// Rows of up to 32 vectors need few registers and keep 1024 (plain [50000,256] 11.3 / 12.9, [50000,64] 9.6 / 10.6).
 #ifndef CS_LN_FWD_MAX_BLOCKS
-#define CS_LN_FWD_MAX_BLOCKS 1024
+#define CS_LN_FWD_MAX_BLOCKS 512
+#endif
+#ifndef CS_LN_FWD_MAX_BLOCKS_H1
+#define CS_LN_FWD_MAX_BLOCKS_H1 1024
 #endif
 constexpr int kLnFwdMaxBlocks = CS_LN_FWD_MAX_BLOCKS;
+constexpr int kLnFwdMaxBlocksNarrow = CS_LN_FWD_MAX_BLOCKS_H1;
 constexpr int kLnBwdMaxBlocks = CS_LN_BWD_MAX_BLOCKS;
 constexpr int kLnBwdMaxBlocksNarrow = CS_LN_BWD_MAX_BLOCKS_VPL2;
 
@@ -1790,6 +1796,19 @@ int ln_blocks(int64_t rows, int rows_per_wave, int cap, int threads = kLnThreads
   const int64_t rows_per_block = (int64_t)(threads / kWave) * rows_per_wave;
   const int64_t b = ceil_div(rows, rows_per_block);
   return (int)(b < cap ? b : cap);
+}
+
+// Two vectors per lane and the residual: rows a wave normalises per step.  Two, so that the last step of the 512
+// workgroups is seldom nearly empty ([5000,1024] bf16 10.9 us with four, 9.4 with two; [10000,1024] 16.1 / 15.4);
+// four where one workgroup per CU then holds them all ([2500,512] fp32 6.0 us with two, 5.4 with four) or where their
+// steps are more than three quarters full ([8192,1024] bf16 11.9 / 11.5, [16384,1024] 24.5 / 22.9).  fp16 takes its sums
+// through more registers: with four rows 262 of them, one wave per SIMD ([8192,1024] 13.4 us with two, 22.5 with four).
+// Four vectors per lane: one row (bf16 [3000,1600] 10.2 us with two, 8.7 with one, [16384,2048] 48.0 / 46.3, fp16
+// [8192,1536] 34.6 / 19.8).
+int add_rows_vpl2(int64_t rows, bool fp16) {
+  const int64_t one_each = 256 * (kLnThreads / kWave) * 4, step = 2 * one_each;
+  if (fp16) return 2;
+  return rows <= one_each || rows * 4 > ceil_div(rows, step) * step * 3 ? 4 : 2;
 }
 
 // Rows on several waves (ln_fwd_block_kernel, ln_bwd_block_kernel): everything the row-per-wave plans
@@ -1909,7 +1928,8 @@ int fwd_typed(const void *x, const void *gamma, const void *beta, void *y, void 
       if (half_vpl != 0) {
         const int groups = res ? (half_vpl == 1 ? CS_LN_ADD_ROWS_H1 : CS_LN_ADD_ROWS_H3)
                                : (half_vpl == 1 ? CS_LN_FWD_ROWS_H1 : CS_LN_FWD_ROWS_H3);
-        const dim3 grid((unsigned)ln_blocks(rows, 2 * groups, kLnFwdMaxBlocks)), block(kLnThreads);
+        const dim3 grid((unsigned)ln_blocks(rows, 2 * groups, half_vpl == 1 ? kLnFwdMaxBlocksNarrow : kLnFwdMaxBlocks)),
+            block(kLnThreads);
 #define CS_LN_FWD_H(VPL, R, HAS_RES)                                                                 \
   ln_fwd_rows_kernel<TX, TY, TP, VPL, R, CS_LN_FWD_PF, HAS_RES, kHalf><<<grid, block, 0, s>>>(       \
       (const TX *)x, (const TP *)gamma, (const TP *)beta, (TY *)y, (float *)mean, (float *)rstd, rows, \
@@ -1926,9 +1946,10 @@ int fwd_typed(const void *x, const void *gamma, const void *beta, void *y, void 
 #undef CS_LN_FWD_H
         return launch_status();
       }
-      // with the residual stream a wave holds two inputs per row: half the rows per step
+      // with the residual stream a wave holds two inputs per row: fewer rows per step
+      constexpr bool kFp16 = std::is_same_v<TX, f16_t>;
       const int r_rows = res ? (p.vpl == 1   ? CS_LN_ADD_ROWS_VPL1
-                                : p.vpl == 2 ? CS_LN_ADD_ROWS_VPL2
+                                : p.vpl == 2 ? add_rows_vpl2(rows, kFp16)
                                              : CS_LN_ADD_ROWS_VPL4)
                              : p.fwd_rows;
       const dim3 grid((unsigned)ln_blocks(rows, r_rows, kLnFwdMaxBlocks)), block(kLnThreads);
@@ -1939,8 +1960,10 @@ int fwd_typed(const void *x, const void *gamma, const void *beta, void *y, void 
       if (res) {
         if (p.vpl == 1) {
           CS_LN_FWD(1, CS_LN_ADD_ROWS_VPL1, true);
+        } else if (p.vpl == 2 && r_rows == 2) {
+          CS_LN_FWD(2, 2, true);
         } else if (p.vpl == 2) {
-          CS_LN_FWD(2, CS_LN_ADD_ROWS_VPL2, true);
+          if constexpr (!kFp16) CS_LN_FWD(2, 4, true);
         } else {
           CS_LN_FWD(4, CS_LN_ADD_ROWS_VPL4, true);
         }

@@ -159,13 +159,8 @@ constexpr int kLnThreads = CS_LN_THREADS;  // 4 waves
 #ifndef CS_LN_BWD_THREADS
 #define CS_LN_BWD_THREADS 512
 #endif
-// grid caps of the backward row kernel, by 16-byte vectors per lane (the partial rows the
-// launch leaves behind are one per workgroup): 512 workgroups of 8 waves, four waves per SIMD,
-// for rows of up to 128 vectors; 256, two per SIMD, beyond (their accumulators take twice the
-// registers)
-#ifndef CS_LN_BWD_MAX_BLOCKS_VPL2
-#define CS_LN_BWD_MAX_BLOCKS_VPL2 512
-#endif
+// grid cap of the backward row kernels (the partial rows the launch leaves behind are one per workgroup): 256 workgroups
+// of 8 waves, two waves per SIMD, one workgroup per CU
 #ifndef CS_LN_BWD_MAX_BLOCKS
 #define CS_LN_BWD_MAX_BLOCKS 256
 #endif
@@ -672,12 +667,12 @@ __device__ __forceinline__ void ln_columns_wide(const TDY *__restrict__ dy, cons
 }
 
 // ----------------------------------------------------------- fast backward
-// One wave per row, the row (dy and x) in registers, gamma and the per-column partial sums in
+// Rows of 4 vectors per lane.  One wave per row, the row (dy and x) in registers, gamma and the per-column partial sums in
 // registers for all rows a wave visits (rows gw, gw + n_waves, ...).  No software prefetch:
 // WPE waves per SIMD are resident (the launch bound asks the compiler for that), so while one
 // wave waits for its row the others compute; measured on MI355X this beats two rows per wave
-// with the next step's rows prefetched ([8192,768] bf16: 12.3 -> 9.8 us, [16384,1600]: 32.8 ->
-// 30.3 us) because twice as many waves are in flight with half the registers each.
+// with the next step's rows prefetched ([16384,1600] bf16: 32.8 -> 30.3 us) because twice as many
+// waves are in flight with half the registers each.
 // The arithmetic uses explicit fused multiply-adds (contraction is off in this file, so every
 // variant of the kernel rounds alike): 17 VALU operations per element instead of 27, which
 // matters because at 16-bit storage this kernel is as close to its VALU limit as to HBM's.
@@ -728,14 +723,14 @@ __global__ __launch_bounds__(kLnBwdThreads, WPE) void ln_bwd_rows_kernel(
     if constexpr (HAS_DRES) {
       // three inputs: with loads under the lane's own condition the compiler waits for each
       // piece of the third before it issues the next (two extra round trips per row at
-      // [8192,768]: 21.0 -> 19.7 us, 53.1 -> 46.4 us at [16384,1600]); every lane loads instead
+      // [16384,1600]: 53.1 -> 46.4 us); every lane loads instead
       load_row_all_lanes<TDY, VN, VPL>(dcur, dy, row, C, nvec, lane);
       load_row_all_lanes<TX, VN, VPL>(xcur, x, row, C, nvec, lane);
       load_row_all_lanes<TDX, VN, VPL>(rcur, dres, row, C, nvec, lane);
       zero_past_row<TDY, VN, VPL>(dcur, nvec, lane);  // so that lanes past the row add nothing below
     } else {
       // two inputs: the conditional form has no such waits and needs half the registers
-      // (13.9 against 14.8 us, 34.0 against 36.4 us)
+      // (34.0 against 36.4 us)
       load_rows<TDY, VN, VPL, 1>(dcur, dy, row, rows, C, nvec, lane);
       load_rows<TX, VN, VPL, 1>(xcur, x, row, rows, C, nvec, lane);
     }
@@ -1790,7 +1785,6 @@ FastPlan fast_plan(int64_t C, int x_dtype) {
 constexpr int kLnFwdMaxBlocks = CS_LN_FWD_MAX_BLOCKS;
 constexpr int kLnFwdMaxBlocksNarrow = CS_LN_FWD_MAX_BLOCKS_H1;
 constexpr int kLnBwdMaxBlocks = CS_LN_BWD_MAX_BLOCKS;
-constexpr int kLnBwdMaxBlocksNarrow = CS_LN_BWD_MAX_BLOCKS_VPL2;
 
 int ln_blocks(int64_t rows, int rows_per_wave, int cap, int threads = kLnThreads) {
   const int64_t rows_per_block = (int64_t)(threads / kWave) * rows_per_wave;
@@ -2094,7 +2088,8 @@ enum BwdKind {
   kBwdHalf1,     // ln_bwd_kernel, two rows per wave, 1 vector per lane (rows of up to 32 vectors)
   kBwdHalf3,     // ln_bwd_kernel, two rows per wave, 3 vectors per lane (65 to 96 vectors: C = 768 at 16 bit)
   kBwdWave4,     // ln_bwd_kernel, a wave per row, 4 vectors per lane
-  kBwdRows,      // ln_bwd_rows_kernel, 1 / 2 / 4 vectors per lane
+  kBwdWave,      // ln_bwd_kernel, a wave per row, 1 or 2 vectors per lane
+  kBwdRows,      // ln_bwd_rows_kernel, 4 vectors per lane
   kBwdBlock,     // ln_bwd_block_kernel, several waves per row
 };
 struct BwdPlan {
@@ -2109,8 +2104,7 @@ struct BwdPlan {
   BlockPlan block;
 };
 constexpr int kLnMaxPartialRows = 512;
-static_assert(kLnBwdMaxBlocksNarrow <= kLnMaxPartialRows && kLnBwdMaxBlocks <= kLnMaxPartialRows &&
-                  CS_LN_PAIR_MAX_BLOCKS <= kLnMaxPartialRows,
+static_assert(kLnBwdMaxBlocks <= kLnMaxPartialRows && CS_LN_PAIR_MAX_BLOCKS <= kLnMaxPartialRows,
               "every plan's grid cap fits the finalize step's row limit");
 
 // Widths of the several-waves kernel whose backward pass can be split into a row pass and a later
@@ -2196,8 +2190,14 @@ BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, const BwdWa
     b.blocks = ln_blocks(rows, 1, kLnBwdMaxBlocks, b.threads);
     b.fold_lds = (size_t)(b.threads / kWave) * C * sizeof(float);
   } else {
-    b.kind = kBwdRows;
-    b.blocks = ln_blocks(rows, 1, p.vpl <= 2 ? kLnBwdMaxBlocksNarrow : kLnBwdMaxBlocks, kLnBwdThreads);
+    // Up to two vectors per lane, the next row requested while this one is worked on and x-hat kept across the row sums
+    // fit two waves per SIMD.  ln_bwd_rows_kernel with three or four took 512 workgroups for them, of which with
+    // dresidual a CU held one at a time, and left twice the partial rows.  us per call with dresidual, those / these: bf16
+    // [1500,1024] 8.5 / 8.2, [4096,1024] 15.9 / 11.6, [8192,1024] 21.8 / 18.0, [16384,1024] 33.2 / 27.7, [4096,512] 9.2 /
+    // 8.2, fp16 [8192,896] 20.8 / 16.5, fp32 [8192,512] 16.8 / 15.9; without it bf16 [4096,1024] 11.9 / 10.0; an earlier
+    // call's sums in the launch [8192,1024] 20.1 / 16.6, [1500,512] 4.5 / 4.3.  Level at plain [16384,512] (14.9).
+    b.kind = p.vpl <= 2 ? kBwdWave : kBwdRows;
+    b.blocks = ln_blocks(rows, 1, kLnBwdMaxBlocks, kLnBwdThreads);
     b.fold_lds = (size_t)(kLnBwdThreads / kWave) * C * sizeof(float);
   }
   return b;
@@ -2210,7 +2210,7 @@ BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, const BwdWa
 // 11.3 / 7.3, [1024,1024] 9.1 / 12.0; fp32 [512,384] 8.8 / 6.2, [1024,384] 9.0 / 9.8.
 constexpr int64_t kDirectRows = 512;
 bool direct_sums(const BwdPlan &p, int64_t rows) {
-  return (p.kind == kBwdHalf1 || p.kind == kBwdHalf3 || p.kind == kBwdRows) && rows <= kDirectRows;
+  return (p.kind == kBwdHalf1 || p.kind == kBwdHalf3 || p.kind == kBwdWave || p.kind == kBwdRows) && rows <= kDirectRows;
 }
 
 bool overlap(const void *a, size_t a_bytes, const void *b, size_t b_bytes) {
@@ -2405,31 +2405,31 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
         const size_t lds = (size_t)2 * kLnFinRows * kLnFinCols * sizeof(float);
         const dim3 grid((unsigned)(blocks + side.blocks)), block((unsigned)plan.threads);
         int st = CS_OK;
-#define CS_LN_DIRECT(HALF_VPL, VPL, HAS_DRES)                                                                           \
-  if (HALF_VPL != 0) {                                                                                                  \
-    st = launch_bwd_kernel<TDY, TX, TDX, TP, kLnBwdThreads, 32, HALF_VPL ? HALF_VPL : 1, 2, false, CS_LN_PAIR_KEEP, true, \
-                           false, HAS_DRES, true>(dy, x, mean, rstd, gamma, dx, workspace, rows, C, dres, side, blocks, \
-                                                  lds, s);                                                              \
-  } else {                                                                                                              \
-    ln_bwd_rows_kernel<TDY, TX, TDX, TP, VPL, 2, true, false, HAS_DRES, true><<<grid, block, lds, s>>>(                 \
-        (const TDY *)dy, (const TX *)x, (const float *)mean, (const float *)rstd, (const TP *)gamma, (TDX *)dx,         \
-        (float *)workspace, rows, (int)C, (const TDX *)dres, side);                                                     \
-    st = launch_status();                                                                                               \
+#define CS_LN_DIRECT(LPR, VPL, HAS_DRES)                                                                               \
+  if (LPR != 0) {                                                                                                      \
+    st = launch_bwd_kernel<TDY, TX, TDX, TP, kLnBwdThreads, LPR ? LPR : 64, LPR ? VPL : 1, 2, false, CS_LN_PAIR_KEEP,  \
+                           true, false, HAS_DRES, true>(dy, x, mean, rstd, gamma, dx, workspace, rows, C, dres, side,  \
+                                                        blocks, lds, s);                                               \
+  } else {                                                                                                             \
+    ln_bwd_rows_kernel<TDY, TX, TDX, TP, 4, 2, true, false, HAS_DRES, true><<<grid, block, lds, s>>>(                  \
+        (const TDY *)dy, (const TX *)x, (const float *)mean, (const float *)rstd, (const TP *)gamma, (TDX *)dx,        \
+        (float *)workspace, rows, (int)C, (const TDX *)dres, side);                                                    \
+    st = launch_status();                                                                                              \
   }
-#define CS_LN_DIRECT2(HALF_VPL, VPL)      \
+#define CS_LN_DIRECT2(LPR, VPL)           \
   if (dres) {                             \
-    CS_LN_DIRECT(HALF_VPL, VPL, true)     \
+    CS_LN_DIRECT(LPR, VPL, true)          \
   } else {                                \
-    CS_LN_DIRECT(HALF_VPL, VPL, false)    \
+    CS_LN_DIRECT(LPR, VPL, false)         \
   }
         if (plan.kind == kBwdHalf1) {
-          CS_LN_DIRECT2(1, 1)
+          CS_LN_DIRECT2(32, 1)
         } else if (plan.kind == kBwdHalf3) {
-          CS_LN_DIRECT2(3, 1)
-        } else if (plan.vpl == 1) {
-          CS_LN_DIRECT2(0, 1)
-        } else if (plan.vpl == 2) {
-          CS_LN_DIRECT2(0, 2)
+          CS_LN_DIRECT2(32, 3)
+        } else if (plan.kind == kBwdWave && plan.vpl == 1) {
+          CS_LN_DIRECT2(64, 1)
+        } else if (plan.kind == kBwdWave) {
+          CS_LN_DIRECT2(64, 2)
         } else {
           CS_LN_DIRECT2(0, 4)
         }
@@ -2458,6 +2458,9 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
   st = launch_bwd_kernel<TDY, TX, TDX, TP, CS_LN_W4_THREADS, 64, VPL, WPE, CS_LN_W4_PF, CS_LN_W4_KEEP, HAS_DX,  \
                          HAS_DP, HAS_DRES>(dy, x, mean, rstd, gamma, dx, workspace, rows, C, dres, pend, blocks, \
                                            lds, s)
+#define CS_LN_K64PF(VPL, WPE, HAS_DX, HAS_DP, HAS_DRES)                                                        \
+  st = launch_bwd_kernel<TDY, TX, TDX, TP, kLnBwdThreads, 64, VPL, WPE, true, true, HAS_DX, HAS_DP, HAS_DRES>(   \
+      dy, x, mean, rstd, gamma, dx, workspace, rows, C, dres, pend, blocks, lds, s)
 #define CS_LN_BWD_MASK(K, VPL, WPE)             \
   if (dx && want_dp && dres) {                  \
     K(VPL, WPE, true, true, true);              \
@@ -2515,12 +2518,10 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
         }
 #undef CS_LN_BWD_BLOCK
 #undef CS_LN_BWD_B
-      } else if (plan.vpl == 1) {
-        CS_LN_BWD_MASK(CS_LN_BWD, 1, 4)
-      } else if (plan.vpl == 2 && dres && want_dp) {
-        CS_LN_BWD(2, 3, true, true, true);  // four per SIMD would spill
-      } else if (plan.vpl == 2) {
-        CS_LN_BWD_MASK(CS_LN_BWD, 2, 4)
+      } else if (plan.kind == kBwdWave && plan.vpl == 1) {
+        CS_LN_BWD_MASK(CS_LN_K64PF, 1, 2)
+      } else if (plan.kind == kBwdWave) {
+        CS_LN_BWD_MASK(CS_LN_K64PF, 2, 2)
       } else {
         CS_LN_BWD_MASK(CS_LN_BWD, 4, 2)
       }
@@ -2528,6 +2529,7 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
 #undef CS_LN_K32
 #undef CS_LN_K32PF
 #undef CS_LN_K64
+#undef CS_LN_K64PF
 #undef CS_LN_BWD
       if (st == CS_OK) st = launch_status();
       if (st == CS_OK && want_dp && phase == kBwdWhole)

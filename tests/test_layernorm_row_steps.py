@@ -28,3 +28,31 @@ def test_row_steps(C, dtype, rows):
     want = (t - mu) * rs * gamma.double() + beta.double()
     ok = (y.double() - want).abs() <= 2e-5
     assert (ok if dtype == F32 else ok | (ulp_distance(y.cpu(), want.to(dtype).cpu()) <= 1).cuda()).all()
+
+
+@pytest.mark.parametrize("C,dtype", [(264, F16), (512, BF16), (520, BF16), (640, F16), (1024, BF16), (132, F32), (260, F32), (512, F32)])
+@pytest.mark.parametrize("rows", [1, 9, 512, 513, 2047, 2049, 4097])
+def test_backward_a_wave_per_row(C, dtype, rows):
+    """256 workgroups of eight waves, a row a wave and step: row counts on either side of a workgroup and of a step."""
+    from core_scheduler_amd import ops
+
+    x, dy, dres = (randn((rows, C), 70 + i, dtype=dtype).cuda() for i in range(3))
+    gamma = randn(C, 73, 0.2, 1.0).cuda()
+    _, mean, rstd = ops.layernorm_forward(x, gamma, gamma)
+    mu, rs = mean.double()[:, None], rstd.double()[:, None]
+    xh, d64 = (x.double() - mu) * rs, dy.double()
+    g = d64 * gamma.double()
+    want = rs * (g - g.mean(1, keepdim=True) - xh * (g * xh).mean(1, keepdim=True))
+    dx, dgamma, dbeta = ops.layernorm_backward(dy, x, mean, rstd, gamma)
+    # some ten fp32 roundings of terms of up to 40: 2^-24 * 10 * 40
+    ok = (dx.double() - want).abs() <= 2.4e-5
+    assert (ok if dtype == F32 else ok | (ulp_distance(dx.cpu(), want.to(dtype).cpu()) <= 1).cuda()).all()
+    for got, terms in ((dgamma, d64 * xh), (dbeta, d64)):
+        # x-hat in fp32 (2^-22 with its inputs' roundings), chains of up to 17 + 16 + 16 fp32 additions
+        assert ((got.double() - terms.sum(0)).abs() <= 2.0 ** -18 * terms.abs().sum(0) + 1e-6).all()
+    apart = ops.layernorm_backward(dy, x, mean, rstd, gamma, dresidual=dres)
+    assert torch.equal(apart[0], dx + dres) and torch.equal(apart[1], dgamma) and torch.equal(apart[2], dbeta)
+    chain = ops.LayerNormBackwardChain()
+    one, two = (chain.backward(dy, x, mean, rstd, gamma, dresidual=dres) for _ in range(2))
+    chain.flush()
+    assert all(torch.equal(a, b) and torch.equal(a, c) for a, b, c in zip(apart, one, two))

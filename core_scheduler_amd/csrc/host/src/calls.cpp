@@ -3,8 +3,9 @@
 //
 // A step's small ops cost more host than device time, and most of that was Python's: 1.3 us for an allocation,
 // 3-4 us of argument checks and ctypes conversions for a call, against 2.8 us for a launch, which stays.  One norm of
-// 77 rows, forward and backward: 30.7 -> 16.7 us (12 since its backward is one launch); the 25 calls of two short blocks
-// 237 -> 115; embedding forward and backward of 4000 tokens 23 -> 17.7 (device time again).
+// 77 rows, forward and backward: 30.7 -> 16.7 us (11.4 since its backward is one launch and its outputs are made
+// directly); the 25 calls of two short blocks 237 -> 115 (91-99 with fewer launches and cheaper outputs); embedding forward
+// and backward of 4000 tokens 23 -> 17.7 (device time again).
 //
 // Every function takes the arguments of its counterpart in ops.py by position and returns NotImplemented for
 // anything but the plain case: exact torch tensors, contiguous, on the current device, of exactly matching shapes and
@@ -115,7 +116,7 @@ static_assert(CS_REDUCTION_NONE == 0 && CS_REDUCTION_MEAN == 1 && CS_REDUCTION_S
 // ---------------------------------------------------------------- one call
 // An output costs more host time than it should: of 0.70 us, torch's allocator takes 0.22 and the tensor object 0.1; the
 // rest is the way there through the dispatcher, its device guard and its factory's options.  Where nothing listens on
-// that way the tensor is made directly (0.34 us; a norm, forward and backward, 12.0 -> 10.1).  The device is the current
+// that way the tensor is made directly (0.34 us; a norm, forward and backward, 13.2 -> 11.4).  The device is the current
 // one (Args::tensor).
 bool nothing_listens() {
   const auto expected = c10::default_included_set | c10::autocast_dispatch_keyset;

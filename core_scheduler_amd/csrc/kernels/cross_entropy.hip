@@ -1517,9 +1517,10 @@ void launch_stream(const void *logits, void *dlogits, const int64_t *targets, fl
 #undef CS_CE_STREAM
 }
 
-// Rows of up to 2048 vectors of 16 bytes, four accesses a lane (eight of 8 bytes for fp32 gradients of 16-bit logits; half or
-// a quarter of that where one wave then has the row) and as many waves as that takes: false where the row is too wide.  Twice as wide where there are more than two rows per CU; of
-// unpadded rows, whose edges take more instructions, one and a half times.  (Before, one wave of eight accesses up to 512
+// Rows of up to 2048 vectors of 16 bytes, four accesses a lane (eight of 8 bytes for fp32 gradients of 16-bit logits; half
+// or a quarter of that where one wave then has the row) and as many waves as that takes: false where the row is too wide.
+// Twice as wide where there are more than two rows per CU; of unpadded rows, whose edges take more instructions, one and a
+// half times.  (Before, one wave of eight accesses up to 512
 // vectors and four waves beyond; unpadded and weighted rows in two sweeps; wider ones by the streaming kernel.)
 // us per call, before / now, bf16 unless said: padded [8192,4096] 29.8 / 28.6, [7501,7808] 46.1 / 42.7, [8192,16384]
 // 94.7 / 92.6; unpadded [16384,1001] 48.1 / 24.9, [13786,3378] 55.0 / 39.6, [6000,10001] 82.7 / 46.9, [2099,15215] 36.3 /

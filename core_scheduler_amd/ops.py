@@ -93,7 +93,7 @@ def _workspace(nbytes, dev):
 def _native(name):
     """The native form of a call below.  It takes the plain case (checked there) and returns NotImplemented for
     everything else, which then goes through the Python body.  Host time: one norm, forward and backward, 30.7 us from
-    Python, 16.7 natively (12 since its backward is one launch); the 25 calls of two short blocks 237 and 115."""
+    Python, 16.7 natively (11.4 since its backward is one launch); the 25 calls of two short blocks 237 and 99."""
     return getattr(_calls, name, None) or (lambda *args: NotImplemented)
 
 

@@ -687,9 +687,12 @@ constexpr int kVpl = CS_EMB_VPL;                // 16-byte column vectors per la
 // 57.4; 32768 x 768 46 MB 54.5 / 53.8, 77 MB 55.1 / 57.1; 16384 x 512 fp32 8 MB 34.7 / 30.9, 103 MB 37.0 / 39.6.
 // Lists of up to this many windows have a slice of 64 vectors of the columns to a workgroup, so that more than half of the
 // CUs have one: kernels of a call, us, whole rows / slices: 4000 x 512 fp32 14.2 / 13.5, added to the table 16.7 / 14.1,
-// [3,400] x 1600 fp32 26.3 / 18.4, [4,1024] x 1600 into 1000 rows 20.4 / 19.1, [8,543] x 768 17.3 / 16.8, [3,349] x 1024
-// 14.9 / 14.0; but [8,1024] x 768 25.6 / 26.3, 16384 x 1600 56.2 / 58.9.
+// [3,400] x 1600 fp32 26.3 / 18.4, [4,1024] x 1600 into 1000 rows 20.4 / 19.1, [3,349] x 1024
+// 14.9 / 14.0; but [8,1024] x 768 25.6 / 26.3, 16384 x 1600 56.2 / 58.9.  Rows of two slices only while every workgroup has
+// a CU: 2048 x 640 bf16 13.2 / 12.7, but [14,309] x 640 15.7 / 16.3, into 1000 rows 14.7 / 15.7, [14,309] x 1024 20.9 /
+// 21.2 (three slices, fp32 x 640: 18.5 / 17.6).
 constexpr int64_t kSlicedWindows = 192;
+constexpr int64_t kSlicedWindowsTwo = 128;
 constexpr int64_t kPosFewFill = (int64_t)3 << 20;
 constexpr int64_t kPosEarlyWindows = 256;
 
@@ -1963,7 +1966,7 @@ int bwd_typed(const void *dout, const void *ids, void *dweight, void *dwpe, char
     if (windows > 0) {
       const int64_t pos = pos_early && !pos_first ? pos_blocks(kRedThreads) : 0;
       const int64_t nvec = C / VN;
-      if (windows <= kSlicedWindows && nvec > kWave) {
+      if (nvec > kWave && windows <= (nvec > 2 * kWave ? kSlicedWindows : kSlicedWindowsTwo)) {
         st = reduce_launch<T, 1>(dout, sorted_id, sorted_pos, dweight, partial, n, C, accumulate, by_freq, windows,
                                  (int)ceil_div(nvec, (int64_t)kWave), pos, dwpe, B, TC, log2_s, s);
       } else {

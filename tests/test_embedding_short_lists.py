@@ -73,7 +73,7 @@ def test_nothing_outside_the_table_is_written(n):
     assert torch.equal(buf.cpu(), want)
 
 
-@pytest.mark.parametrize("n", [6144, 6145])  # windows whose columns are dealt out to workgroups, and whole ones
+@pytest.mark.parametrize("n", [4096, 4097, 6144, 6145])  # either side of the lines for two slices, and for three or more
 @pytest.mark.parametrize("C", [256, 260, 516, 1100])  # fp32: a slice of 64 vectors, one more, three, five
 def test_windows_in_slices(n, C):
     from core_scheduler_amd import ops

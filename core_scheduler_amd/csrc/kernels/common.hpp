@@ -151,6 +151,16 @@ __device__ __forceinline__ void store16_stream(RowBuffer row, int offset, const 
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), row, offset, 0, kBufferStream);
 }
 
+// A workgroup per row.  A launch counts its work-items in 32 bits in each dimension, and one of more starts what the
+// remainder holds and reports no error (2^26 + 5 rows on a wave each: five of them), so many rows fill the second dimension
+// too.  Its last line may have no such row.
+constexpr int kLog2GridRows = 21;  // of up to 1024 lanes
+inline dim3 row_grid(int64_t rows) {
+  const int64_t line = (int64_t)1 << kLog2GridRows;
+  return rows <= line ? dim3((unsigned)rows) : dim3((unsigned)line, (unsigned)((rows + line - 1) >> kLog2GridRows));
+}
+__device__ __forceinline__ int64_t row_of_grid() { return blockIdx.x + ((int64_t)blockIdx.y << kLog2GridRows); }
+
 __host__ __device__ __forceinline__ bool is_aligned16(const void *p) {
   return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
 }

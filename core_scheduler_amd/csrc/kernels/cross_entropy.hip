@@ -272,7 +272,8 @@ __global__ __launch_bounds__(MOST_THREADS) void ce_rows_kernel(
     float dloss, const float *__restrict__ class_weight) {
   constexpr int VN = EPV;
   __shared__ float scratch[MOST_THREADS / kWave];
-  const int64_t row = blockIdx.x;
+  const int64_t row = row_of_grid();
+  if (row >= N) return;
   const int tid = threadIdx.x, block = blockDim.x;
   const int iV = (int)V, stride = (int)row_stride;
   const int off = RAGGED ? (int)((row * row_stride) & (kLineElems<T> - 1)) : 0;
@@ -1539,7 +1540,7 @@ bool launch_narrow(const void *logits, void *dlogits, const int64_t *targets, fl
   if (nvec > threads * U) return false;
 #define CS_CE_NARROW(VPT)                                                                                          \
   ce_rows_kernel<T, TD, VPT, EPV, RAGGED>                                                                          \
-      <<<dim3((unsigned)N), dim3((unsigned)(ceil_div(nvec, (int64_t)(kWave * VPT)) * kWave)), 0, s>>>(             \
+      <<<row_grid(N), dim3((unsigned)(ceil_div(nvec, (int64_t)(kWave * VPT)) * kWave)), 0, s>>>(                   \
           (const T *)logits, (TD *)dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index, reduction, \
           dloss, class_weight)
   if (nvec <= kWave * U / 4) {
@@ -1638,7 +1639,7 @@ int launch_rows(const void *logits, void *dlogits, const int64_t *targets, float
       } else if (sizeof(T) == 4 && nvec_all <= 1024 * 16) {
         // fp32 rows up to 65536 columns still fit in registers (at 16 bit this plan spills)
         if constexpr (sizeof(T) == 4)
-          ce_rows_kernel<T, TD, 16, VN, false, 1024><<<grid, dim3(1024), 0, s>>>(
+          ce_rows_kernel<T, TD, 16, VN, false, 1024><<<row_grid(N), dim3(1024), 0, s>>>(
               (const T *)logits, (TD *)dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index, reduction,
               dloss, nullptr);
       } else {

@@ -1279,11 +1279,12 @@ __global__ __launch_bounds__(BLOCK, 8) void ce_rows_wide_kernel(
 template <typename T, typename TD>
 __global__ __launch_bounds__(256) void ce_rows_general_kernel(
     const T *__restrict__ logits, TD *__restrict__ dlogits, const int64_t *__restrict__ targets,
-    float *__restrict__ row_loss, const int *__restrict__ ws_count, int64_t V, int64_t row_stride,
+    float *__restrict__ row_loss, const int *__restrict__ ws_count, int64_t N, int64_t V, int64_t row_stride,
     int64_t ignore_index, int reduction, float dloss, const float *__restrict__ class_weight) {
   using U = typename Acc<T>::type;
   __shared__ U scratch[4];
-  const int64_t row = blockIdx.x;
+  const int64_t row = row_of_grid();
+  if (row >= N) return;
   const T *x = logits + row * row_stride;
   const int64_t target = targets[row];
   const bool counts = target_counts(target, V, ignore_index);
@@ -1310,7 +1311,7 @@ __global__ __launch_bounds__(256) void ce_rows_general_kernel(
   U scale = (U)dloss;
   if (reduction == CS_REDUCTION_MEAN)
     scale = (U)dloss / (class_weight ? (U) reinterpret_cast<const float *>(ws_count)[1]
-                                     : (U)rows_that_count(ws_count, targets, gridDim.x, V, ignore_index));
+                                     : (U)rows_that_count(ws_count, targets, N, V, ignore_index));
   scale *= wt;
   for (int64_t c = threadIdx.x; c < row_stride; c += 256) {
     U o = 0;
@@ -1675,10 +1676,9 @@ int launch_rows(const void *logits, void *dlogits, const int64_t *targets, float
       return launch_status();
     }
   }
-  ce_rows_general_kernel<T, TD><<<grid, dim3(256), 0, s>>>((const T *)logits, (TD *)dlogits,
-                                                            targets, row_loss, ws_count, V,
-                                                            row_stride, ignore_index, reduction,
-                                                            dloss, class_weight);
+  ce_rows_general_kernel<T, TD><<<row_grid(N), dim3(256), 0, s>>>((const T *)logits, (TD *)dlogits, targets, row_loss,
+                                                                  ws_count, N, V, row_stride, ignore_index,
+                                                                  reduction, dloss, class_weight);
   return launch_status();
 }
 

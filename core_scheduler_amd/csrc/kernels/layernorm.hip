@@ -1647,10 +1647,11 @@ template <typename TX, typename TY, typename TP>
 __global__ __launch_bounds__(kLnThreads) void ln_fwd_general_kernel(
     const TX *__restrict__ x, const TP *__restrict__ gamma, const TP *__restrict__ beta,
     TY *__restrict__ y, typename Acc<TX>::type *__restrict__ mean,
-    typename Acc<TX>::type *__restrict__ rstd, int64_t C, typename Acc<TX>::type eps) {
+    typename Acc<TX>::type *__restrict__ rstd, int64_t rows, int64_t C, typename Acc<TX>::type eps) {
   using U = typename Acc<TX>::type;
   __shared__ U scratch[kLnThreads / kWave];
-  const int64_t row = blockIdx.x;
+  const int64_t row = row_of_grid();
+  if (row >= rows) return;
   const TX *xr = x + row * C;
   U s = 0;
   for (int64_t c = threadIdx.x; c < C; c += kLnThreads) s += to_acc(xr[c]);
@@ -1677,10 +1678,11 @@ __global__ __launch_bounds__(kLnThreads) void ln_bwd_dx_general_kernel(
     const TDY *__restrict__ dy, const TX *__restrict__ x,
     const typename Acc<TX>::type *__restrict__ mean,
     const typename Acc<TX>::type *__restrict__ rstd, const TP *__restrict__ gamma,
-    TDX *__restrict__ dx, int64_t C, const TDX *__restrict__ dres) {
+    TDX *__restrict__ dx, int64_t rows, int64_t C, const TDX *__restrict__ dres) {
   using U = typename Acc<TX>::type;
   __shared__ U scratch[kLnThreads / kWave];
-  const int64_t row = blockIdx.x;
+  const int64_t row = row_of_grid();
+  if (row >= rows) return;
   const U mu = mean[row], rs = rstd[row];
   U s1 = 0, s2 = 0;
   for (int64_t c = threadIdx.x; c < C; c += kLnThreads) {
@@ -2036,8 +2038,8 @@ int fwd_typed(const void *x, const void *gamma, const void *beta, void *y, void 
     if (st != CS_OK) return st;
     x = sum_out;
   }
-  ln_fwd_general_kernel<TX, TY, TP><<<dim3((unsigned)rows), dim3(kLnThreads), 0, s>>>(
-      (const TX *)x, (const TP *)gamma, (const TP *)beta, (TY *)y, (U *)mean, (U *)rstd, C,
+  ln_fwd_general_kernel<TX, TY, TP><<<row_grid(rows), dim3(kLnThreads), 0, s>>>(
+      (const TX *)x, (const TP *)gamma, (const TP *)beta, (TY *)y, (U *)mean, (U *)rstd, rows, C,
       (U)eps);
   return launch_status();
 }
@@ -2554,9 +2556,9 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
     if (st != CS_OK) return st;
   }
   if (dx) {
-    ln_bwd_dx_general_kernel<TDY, TX, TDX, TP><<<dim3((unsigned)rows), dim3(kLnThreads), 0, s>>>(
+    ln_bwd_dx_general_kernel<TDY, TX, TDX, TP><<<row_grid(rows), dim3(kLnThreads), 0, s>>>(
         (const TDY *)dy, (const TX *)x, (const U *)mean, (const U *)rstd, (const TP *)gamma,
-        (TDX *)dx, C, (const TDX *)dres);
+        (TDX *)dx, rows, C, (const TDX *)dres);
     const int st = launch_status();
     if (st != CS_OK) return st;
   }

@@ -56,3 +56,53 @@ def test_backward_a_wave_per_row(C, dtype, rows):
     one, two = (chain.backward(dy, x, mean, rstd, gamma, dresidual=dres) for _ in range(2))
     chain.flush()
     assert all(torch.equal(a, b) and torch.equal(a, c) for a, b, c in zip(apart, one, two))
+
+
+def _dx_in_fp32(dy, x, mean, rstd, gamma):
+    """dx in fp32 as a wave forms it: 64 lanes of four columns, chains over a lane's columns, a tree over the lanes, the
+    products dy * gamma unrounded in the last line.  (A fused multiply-add: the product of two floats is exact in 64 bits.)"""
+    def fma(a, b, c):
+        return (a.double() * b.double() + c.double()).float()
+
+    def tree(t):
+        while t.shape[1] > 1:
+            t = t[:, 0::2] + t[:, 1::2]
+        return t
+
+    rows, C = x.shape
+    xh = (x - mean[:, None]) * rstd[:, None]
+    s1, s2 = (torch.zeros(rows, 64, device=x.device) for _ in range(2))
+    for j in range(0, C, 256):
+        for k in range(4):
+            at = torch.arange(j + k, min(j + 256, C), 4)
+            n = len(at)
+            t = dy[:, at] * gamma[at]
+            s1[:, :n] += t
+            s2[:, :n] = fma(t, xh[:, at], s2[:, :n])
+    s1, s2 = (tree(s) * torch.tensor(1.0 / C, dtype=torch.float32, device=x.device) for s in (s1, s2))
+    return rstd[:, None] * fma(-xh, s2, fma(dy, gamma, -s1))
+
+
+@pytest.mark.parametrize("C", [132, 200, 256, 396, 512])  # 33 to 64 vectors, and 97 to 128
+@pytest.mark.parametrize("rows", [400, 2049])  # one launch with the sums, and two
+@pytest.mark.parametrize("along", [0.0, 0.9, 0.999])
+def test_dx_is_as_exact_as_its_formula(C, rows, along):
+    """dy that lies along x-hat leaves little of dx, and what was rounded ahead of the subtraction shows."""
+    from core_scheduler_amd import ops
+
+    x, noise = (randn((rows, C), 75 + i).cuda() for i in range(2))
+    gamma = randn(C, 77, 0.2, 1.0).cuda()
+    _, mean, rstd = ops.layernorm_forward(x, gamma, gamma)
+    rs = rstd.double()[:, None]
+    xh = (x.double() - mean.double()[:, None]) * rs
+    dy = (along * xh + (1 - along ** 2) ** 0.5 * noise.double()).float()
+    g = dy.double() * gamma.double()
+    want = rs * (g - g.mean(1, keepdim=True) - xh * (g * xh).mean(1, keepdim=True))
+    dx = ops.layernorm_backward(dy, x, mean, rstd, gamma)[0]
+    formula = _dx_in_fp32(dy, x, mean, rstd, gamma)
+
+    def error(t):
+        return (t.double() - want).pow(2).mean().sqrt().item()
+
+    # (the product rounded, and rstd multiplied into the terms: 8 to 18% more where along is 0.9 or more)
+    assert error(dx) <= 1.02 * error(formula)

@@ -2113,6 +2113,7 @@ struct BwdPlan {
   size_t partial_elem = sizeof(float);  // bytes of a partial row's element
   bool two_calls = true;  // the partial rows may be added up by a later call (kBwdBlock: see block_two_calls)
   bool direct = false;    // kBwdBlock: the launch of dx takes the column sums (direct_wide_rows)
+  bool more_waves = false;  // kBwdWave: four waves per SIMD that load a row at a time (dx_alone_more_waves)
   BlockPlan block;
 };
 constexpr int kLnMaxPartialRows = 512;
@@ -2168,6 +2169,17 @@ bool general_rows(const BwdWants &w, const BlockPlan &b, int64_t rows, int64_t C
   return rows <= 64 && C / vn <= 8 * kWave;
 }
 
+// dx alone of a wave per row has no column sums in its registers: four waves per SIMD on 512 workgroups, without the next
+// row's prefetch, instead of two with it.  us per call, two waves / four: bf16 [3000,512] 3.95 / 3.76, [8192,512] 6.5 / 5.8,
+// [30000,512] 18.8 / 16.8, fp32 [8192,256] 6.1 / 5.4; of two vectors per lane fp16 [8192,896] 9.7 / 8.8, [12289,896] 13.3 /
+// 12.6, bf16 [5000,1024] 7.4 / 7.0, [16384,1024] 17.8 / 17.7.  Two waves where those rows make two steps or fewer of them
+// (bf16 [4096,1024] 5.3 / 5.9, fp32 [4096,400] 4.5 / 4.9), or so many that their rows in flight are the better use of the
+// memory ([30000,1024] 31.5 / 32.7, fp16 [30000,896] 27.6 / 28.5).
+bool dx_alone_more_waves(int64_t rows, int vpl) {
+  const int64_t step = (int64_t)kLnBwdMaxBlocks * (kLnBwdThreads / kWave);
+  return vpl == 1 || (rows > 2 * step && rows <= 10 * step);
+}
+
 BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, const BwdWants &w = BwdWants{}) {
   BwdPlan b;
   const FastPlan p = aligned ? fast_plan(C, x_dtype) : FastPlan{};
@@ -2209,7 +2221,8 @@ BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, const BwdWa
     // 8.2, fp16 [8192,896] 20.8 / 16.5, fp32 [8192,512] 16.8 / 15.9; without it bf16 [4096,1024] 11.9 / 10.0; an earlier
     // call's sums in the launch [8192,1024] 20.1 / 16.6, [1500,512] 4.5 / 4.3.  Level at plain [16384,512] (14.9).
     b.kind = p.vpl <= 2 ? kBwdWave : kBwdRows;
-    b.blocks = ln_blocks(rows, 1, kLnBwdMaxBlocks, kLnBwdThreads);
+    b.more_waves = b.kind == kBwdWave && !w.sums && dx_alone_more_waves(rows, p.vpl);
+    b.blocks = ln_blocks(rows, 1, b.more_waves ? 512 : kLnBwdMaxBlocks, kLnBwdThreads);
     b.fold_lds = (size_t)(kLnBwdThreads / kWave) * C * sizeof(float);
   }
   return b;
@@ -2471,8 +2484,9 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
                          HAS_DP, HAS_DRES>(dy, x, mean, rstd, gamma, dx, workspace, rows, C, dres, pend, blocks, \
                                            lds, s)
 #define CS_LN_K64PF(VPL, WPE, HAS_DX, HAS_DP, HAS_DRES)                                                        \
-  st = launch_bwd_kernel<TDY, TX, TDX, TP, kLnBwdThreads, 64, VPL, WPE, true, true, HAS_DX, HAS_DP, HAS_DRES>(   \
+  st = launch_bwd_kernel<TDY, TX, TDX, TP, kLnBwdThreads, 64, VPL, WPE, WPE == 2, true, HAS_DX, HAS_DP, HAS_DRES>( \
       dy, x, mean, rstd, gamma, dx, workspace, rows, C, dres, pend, blocks, lds, s)
+#define CS_LN_K64PF1(VPL, WPE, HAS_DX, HAS_DP, HAS_DRES) CS_LN_K64PF(VPL, (HAS_DP ? WPE : 4), HAS_DX, HAS_DP, HAS_DRES)
 #define CS_LN_BWD_MASK(K, VPL, WPE)             \
   if (dx && want_dp && dres) {                  \
     K(VPL, WPE, true, true, true);              \
@@ -2531,7 +2545,13 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
 #undef CS_LN_BWD_BLOCK
 #undef CS_LN_BWD_B
       } else if (plan.kind == kBwdWave && plan.vpl == 1) {
-        CS_LN_BWD_MASK(CS_LN_K64PF, 1, 2)
+        CS_LN_BWD_MASK(CS_LN_K64PF1, 1, 2)
+      } else if (plan.kind == kBwdWave && plan.more_waves) {
+        if (dres) {
+          CS_LN_K64PF(2, 4, true, false, true);
+        } else {
+          CS_LN_K64PF(2, 4, true, false, false);
+        }
       } else if (plan.kind == kBwdWave) {
         CS_LN_BWD_MASK(CS_LN_K64PF, 2, 2)
       } else {
@@ -2542,6 +2562,7 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
 #undef CS_LN_K32PF
 #undef CS_LN_K64
 #undef CS_LN_K64PF
+#undef CS_LN_K64PF1
 #undef CS_LN_BWD
       if (st == CS_OK) st = launch_status();
       if (st == CS_OK && want_dp && phase == kBwdWhole)

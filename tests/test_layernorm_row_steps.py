@@ -106,3 +106,17 @@ def test_dx_is_as_exact_as_its_formula(C, rows, along):
 
     # (the product rounded, and rstd multiplied into the terms: 8 to 18% more where along is 0.9 or more)
     assert error(dx) <= 1.02 * error(formula)
+
+
+@pytest.mark.parametrize("C,dtype", [(512, BF16), (1024, BF16), (520, F16), (132, F32), (400, F32)])
+@pytest.mark.parametrize("rows", [1, 513, 4095, 4096, 4097, 8193, 20480, 20481])  # where the launch of dx alone changes
+def test_dx_alone_has_the_bits_of_the_full_call(C, dtype, rows):
+    from core_scheduler_amd import ops
+
+    x, dy, dres = (torch.randn(rows, C, device="cuda", generator=torch.Generator("cuda").manual_seed(78 + i)).to(dtype) for i in range(3))
+    gamma = randn(C, 81, 0.2, 1.0).cuda()
+    args = (dy, x, *ops.layernorm_forward(x, gamma)[1:], gamma)
+    for more in ({}, {"dresidual": dres}):
+        alone = ops.layernorm_backward(*args, need_dgamma=False, need_dbeta=False, **more)
+        assert alone[1] is None and alone[2] is None
+        assert torch.equal(alone[0], ops.layernorm_backward(*args, **more)[0])

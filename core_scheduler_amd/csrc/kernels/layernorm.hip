@@ -2113,11 +2113,11 @@ struct BwdPlan {
   size_t partial_elem = sizeof(float);  // bytes of a partial row's element
   bool two_calls = true;  // the partial rows may be added up by a later call (kBwdBlock: see block_two_calls)
   bool direct = false;    // kBwdBlock: the launch of dx takes the column sums (direct_wide_rows)
-  bool more_waves = false;  // kBwdWave: four waves per SIMD that load a row at a time (dx_alone_more_waves)
+  bool four_waves = false;  // kBwdWave: four waves per SIMD that load a row at a time (see there)
   BlockPlan block;
 };
 constexpr int kLnMaxPartialRows = 512;
-static_assert(kLnBwdMaxBlocks <= kLnMaxPartialRows && CS_LN_PAIR_MAX_BLOCKS <= kLnMaxPartialRows,
+static_assert(2 * kLnBwdMaxBlocks <= kLnMaxPartialRows && CS_LN_PAIR_MAX_BLOCKS <= kLnMaxPartialRows,
               "every plan's grid cap fits the finalize step's row limit");
 
 // Widths of the several-waves kernel whose backward pass can be split into a row pass and a later
@@ -2169,15 +2169,24 @@ bool general_rows(const BwdWants &w, const BlockPlan &b, int64_t rows, int64_t C
   return rows <= 64 && C / vn <= 8 * kWave;
 }
 
-// dx alone of a wave per row has no column sums in its registers: four waves per SIMD on 512 workgroups, without the next
-// row's prefetch, instead of two with it.  us per call, two waves / four: bf16 [3000,512] 3.95 / 3.76, [8192,512] 6.5 / 5.8,
-// [30000,512] 18.8 / 16.8, fp32 [8192,256] 6.1 / 5.4; of two vectors per lane fp16 [8192,896] 9.7 / 8.8, [12289,896] 13.3 /
-// 12.6, bf16 [5000,1024] 7.4 / 7.0, [16384,1024] 17.8 / 17.7.  Two waves where those rows make two steps or fewer of them
-// (bf16 [4096,1024] 5.3 / 5.9, fp32 [4096,400] 4.5 / 4.9), or so many that their rows in flight are the better use of the
-// memory ([30000,1024] 31.5 / 32.7, fp16 [30000,896] 27.6 / 28.5).
-bool dx_alone_more_waves(int64_t rows, int vpl) {
+// A wave per row: four waves per SIMD on 512 workgroups, a row at a time, instead of two that request the next row as well.
+// us per call, two waves / four.
+// One vector per lane, dx alone: there are no column sums in the registers.  bf16 [3000,512] 3.95 / 3.76, [8192,512] 6.5 /
+// 5.8, [30000,512] 18.8 / 16.8, fp32 [8192,256] 6.1 / 5.4.  With the sums, many rows of up to 56 vectors, which leave lanes
+// idle; plain / with dresidual / the sums alone: fp16 [8192,384] 9.4 / 9.7, 10.1 / 10.5, 8.0 / 8.2, [14000,384] 12.6 / 11.5,
+// 13.5 / 13.0, 10.3 / 9.4, bf16 [60000,264] 34.2 / 24.6, 37.2 / 29.5, 26.2 / 18.3, fp32 [14000,192] 11.7 / 10.7, 12.4 / 12.0, 9.6 / 8.7.
+// Of 57 to 64 vectors dy, x and dresidual fill the memory by themselves, while plain rows and the sums alone do not: bf16
+// [14000,512] 13.2 / 13.2, 14.8 / 15.0, 10.4 / 10.3, [60000,512] 38.5 / 36.1, 44.2 / 46.9, 28.4 / 23.9, fp32 [60000,256] 36.4 /
+// 35.0, 43.1 / 46.2, 26.7 / 23.0.  All forms of a call have to leave the same partial rows (the split form, which is asked
+// for them without knowing of a dx or dresidual, gives the bits of the single call), and dresidual is what training has.
+// Two vectors per lane, dx alone: fp16 [8192,896] 9.7 / 8.8, [12289,896] 13.3 / 12.6, bf16 [5000,1024] 7.4 / 7.0, [16384,1024]
+// 17.8 / 17.7; not where those rows make two steps or fewer of the two waves (bf16 [4096,1024] 5.3 / 5.9, fp32 [4096,400]
+// 4.5 / 4.9), or so many that their rows in flight are the better use of the memory ([30000,1024] 31.5 / 32.7, fp16
+// [30000,896] 27.6 / 28.5).
+bool four_waves(int64_t rows, int64_t nvec, bool sums) {
   const int64_t step = (int64_t)kLnBwdMaxBlocks * (kLnBwdThreads / kWave);
-  return vpl == 1 || (rows > 2 * step && rows <= 10 * step);
+  if (nvec > kWave) return !sums && rows > 2 * step && rows <= 10 * step;
+  return !sums || (rows > 5 * step && nvec <= 56);
 }
 
 BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, const BwdWants &w = BwdWants{}) {
@@ -2221,8 +2230,8 @@ BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, const BwdWa
     // 8.2, fp16 [8192,896] 20.8 / 16.5, fp32 [8192,512] 16.8 / 15.9; without it bf16 [4096,1024] 11.9 / 10.0; an earlier
     // call's sums in the launch [8192,1024] 20.1 / 16.6, [1500,512] 4.5 / 4.3.  Level at plain [16384,512] (14.9).
     b.kind = p.vpl <= 2 ? kBwdWave : kBwdRows;
-    b.more_waves = b.kind == kBwdWave && !w.sums && dx_alone_more_waves(rows, p.vpl);
-    b.blocks = ln_blocks(rows, 1, b.more_waves ? 512 : kLnBwdMaxBlocks, kLnBwdThreads);
+    b.four_waves = b.kind == kBwdWave && four_waves(rows, nvec, w.sums);
+    b.blocks = ln_blocks(rows, 1, b.four_waves ? 2 * kLnBwdMaxBlocks : kLnBwdMaxBlocks, kLnBwdThreads);
     b.fold_lds = (size_t)(kLnBwdThreads / kWave) * C * sizeof(float);
   }
   return b;
@@ -2545,8 +2554,12 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
 #undef CS_LN_BWD_BLOCK
 #undef CS_LN_BWD_B
       } else if (plan.kind == kBwdWave && plan.vpl == 1) {
-        CS_LN_BWD_MASK(CS_LN_K64PF1, 1, 2)
-      } else if (plan.kind == kBwdWave && plan.more_waves) {
+        if (plan.four_waves) {
+          CS_LN_BWD_MASK(CS_LN_K64PF1, 1, 4)
+        } else {
+          CS_LN_BWD_MASK(CS_LN_K64PF1, 1, 2)
+        }
+      } else if (plan.kind == kBwdWave && plan.four_waves) {
         if (dres) {
           CS_LN_K64PF(2, 4, true, false, true);
         } else {

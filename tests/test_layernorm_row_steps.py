@@ -31,9 +31,10 @@ def test_row_steps(C, dtype, rows):
 
 
 @pytest.mark.parametrize("C,dtype", [(264, F16), (512, BF16), (520, BF16), (640, F16), (1024, BF16), (132, F32), (260, F32), (512, F32)])
-@pytest.mark.parametrize("rows", [1, 9, 512, 513, 2047, 2049, 4097])
+@pytest.mark.parametrize("rows", [1, 9, 512, 513, 2047, 2049, 4097, 10241, 24577])
 def test_backward_a_wave_per_row(C, dtype, rows):
-    """256 workgroups of eight waves, a row a wave and step: row counts on either side of a workgroup and of a step."""
+    """256 or, of many narrow rows, 512 workgroups of eight waves, a row a wave and step: row counts on either side of a
+    workgroup, of a step and of the lines between the two."""
     from core_scheduler_amd import ops
 
     x, dy, dres = (randn((rows, C), 70 + i, dtype=dtype).cuda() for i in range(3))

@@ -868,7 +868,11 @@ __global__ __launch_bounds__(THREADS, WPE) void ln_bwd_kernel(
       acc_g[j][k] = 0.f;
       acc_b[j][k] = 0.f;
     }
-    if constexpr (HAS_DX) load_n<TP, VN>(gamma + (idx < nvec ? idx : nvec - 1) * VN, g[j]);
+    if constexpr (HAS_DX) {
+      load_n<TP, VN>(gamma + (idx < nvec ? idx : nvec - 1) * VN, g[j]);
+#pragma unroll
+      for (int k = 0; k < VN; ++k) g[j][k] = idx < nvec ? g[j][k] : 0.f;  // not the last vector's: 0 * inf is NaN
+    }
   }
 
   Strip<TDY, VN, VPL> dcur, dnxt;
@@ -1398,7 +1402,10 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_bwd_block_kernel(
       }
     }
   }
-  if constexpr (UA && HAS_DX) ge = to_acc(gamma[own.ecol]);
+  if constexpr (UA && HAS_DX) {
+    ge = to_acc(gamma[own.ecol]);
+    ge = own.ehas ? ge : 0.f;
+  }
   Row even, odd;  // as in the forward kernel, where both fit
   fetch(even, row);
   if (PF && (!UA || steps > 1)) fetch(odd, row + stride);

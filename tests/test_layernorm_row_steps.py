@@ -121,3 +121,26 @@ def test_dx_alone_has_the_bits_of_the_full_call(C, dtype, rows):
         alone = ops.layernorm_backward(*args, need_dgamma=False, need_dbeta=False, **more)
         assert alone[1] is None and alone[2] is None
         assert torch.equal(alone[0], ops.layernorm_backward(*args, **more)[0])
+
+
+@pytest.mark.parametrize("C,dtype", [(8, BF16), (72, F16), (132, F32), (264, BF16), (640, BF16), (1000, F16), (400, F32), (1600, BF16),
+                                     (2056, BF16), (1003, BF16), (3, F32)])
+@pytest.mark.parametrize("rows", [3, 700])  # one launch with the sums, and two
+def test_infinite_gamma_of_the_last_column(C, dtype, rows):
+    """An infinity in gamma makes a row's sums infinite, and its dx where the two infinities do not meet; lanes that have no
+    part of the row add nothing to them."""
+    from core_scheduler_amd import ops
+
+    x = randn((rows, C), 82).to(dtype).cuda()
+    dy = (randn((rows, C), 83).abs() + 0.5).to(dtype).cuda()
+    gamma = torch.ones(C, device="cuda")
+    _, mean, rstd = ops.layernorm_forward(x, gamma)
+    gamma[-1] = float("inf")
+    xh = (x.double() - mean.double()[:, None]) * rstd.double()[:, None]
+    g = dy.double() * gamma.double()
+    want = rstd.double()[:, None] * (g - g.mean(1, keepdim=True) - xh * (g * xh).mean(1, keepdim=True))
+    assert torch.isinf(want).any()
+    for sums in (True, False):
+        dx = ops.layernorm_backward(dy, x, mean, rstd, gamma, need_dgamma=sums, need_dbeta=sums)[0].double()
+        assert torch.equal(dx.isnan(), want.isnan()) and torch.equal(dx.isinf(), want.isinf())
+        assert torch.equal(dx[dx.isinf()], want[want.isinf()])

@@ -18,6 +18,7 @@
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/ops/empty.h>
 #include <ATen/ops/empty_like.h>
+#include <ATen/record_function.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
@@ -115,17 +116,19 @@ static_assert(CS_REDUCTION_NONE == 0 && CS_REDUCTION_MEAN == 1 && CS_REDUCTION_S
 
 // ---------------------------------------------------------------- one call
 // An output costs more host time than it should: of 0.70 us, torch's allocator takes 0.22 and the tensor object 0.1; the
-// rest is the way there through the dispatcher, its device guard and its factory's options.  Where nothing listens on
-// that way the tensor is made directly (0.34 us; a norm, forward and backward, 13.2 -> 11.4).  The device is the current
-// one (Args::tensor).
+// rest is the way there through the dispatcher, its device guard and its factory's options.  Where no dispatch key, no
+// deterministic fill and no profiler has a part in that way the tensor is made directly (0.34 us; a norm, forward and
+// backward, 13.2 -> 11.4).  The device is the current one (Args::tensor).
 bool nothing_listens() {
   const auto expected = c10::default_included_set | c10::autocast_dispatch_keyset;
   return (c10::impl::tls_local_dispatch_key_set().included_ - expected).empty() &&
-         !at::globalContext().deterministicAlgorithms();  // which fills new tensors
+         !at::globalContext().deterministicAlgorithms() &&  // which fills new tensors
+         !at::hasCallbacks();                               // that see every call of the dispatcher
 }
+thread_local bool direct_outputs;  // of the call under way (unlocked): asked once, the callbacks take a lock of 25 ns
 at::Tensor empty(at::IntArrayRef sizes, at::ScalarType t, const at::Tensor &like) {
   c10::Allocator *const device_memory = c10::hip::HIPCachingAllocatorMasqueradingAsCUDA::get();
-  if (!nothing_listens()) return at::empty(sizes, at::TensorOptions().dtype(t).device(like.device()));
+  if (!direct_outputs) return at::empty(sizes, at::TensorOptions().dtype(t).device(like.device()));
   return at::detail::empty_generic(sizes, device_memory, c10::DispatchKeySet(c10::DispatchKey::CUDA), t, std::nullopt);
 }
 // (a dimension of one element may have any stride, which empty_like keeps)
@@ -176,6 +179,7 @@ void raise_for(const char *name, int code) {
 template <typename Body>
 int unlocked(int device, Body &&body) {
   pybind11::gil_scoped_release release;
+  direct_outputs = nothing_listens();
   return body(static_cast<void *>(c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream()));
 }
 

@@ -33,3 +33,14 @@ def test_outputs_are_ordinary_tensors(inside):
             assert _kind(empty) == _kind(torch.empty_like(x[:0]))
     finally:
         torch.use_deterministic_algorithms(False)
+
+
+def test_a_profiler_sees_the_outputs():
+    from core_scheduler_amd import ops
+
+    x, g = torch.randn(5, 768, device="cuda"), torch.ones(768, device="cuda")
+    _, mean, rstd = ops.layernorm_forward(x, g)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as trace:
+        ops.layernorm_backward(x, x, mean, rstd, g)
+    made = [e for e in trace.key_averages() if e.key == "aten::empty"]
+    assert made and made[0].count >= 3  # dx, dgamma, dbeta

@@ -54,8 +54,10 @@ def test_rows_in_registers(N, V, stride, dtype, gdt, weighted):
     if gdt != F32:
         ok |= (ulp_distance(d.cpu(), want.to(gdt).cpu()) <= 1).cuda()
     assert ok.all() and not d[:, V:].any() and torch.equal(logits, x)
-    if N <= 512:  # the loss alone goes the same way
-        assert torch.equal(ops.fused_classifier(x, t, V, class_weight=w, want_dlogits=False)[1], rows) or gdt != dtype
+    alone = ops.fused_classifier(x, t, V, class_weight=w, want_dlogits=False)[1]
+    assert ((alone.double() - want_rows).abs() <= 2.0 ** -19 * (want_rows.abs() + 8)).all()
+    if N <= 512 and gdt == dtype:  # the loss alone goes the same way
+        assert torch.equal(alone, rows)
     if gdt == dtype and not weighted:  # the gradient over the logits
         _, rows2, d2, _ = ops.fused_classifier(logits, t, V, inplace=True)
         assert torch.equal(d2, d) and torch.equal(rows2, rows) and d2.data_ptr() == logits.data_ptr()

@@ -375,6 +375,28 @@ __global__ __launch_bounds__(kLnThreads) void ln_fwd_rows_kernel(
   }
 }
 
+// Vector `idx` of a parameter row, zeros where the row has no such one: the last vector's again would do for anything that
+// is masked later, but a lane's zero of dy times an infinite gamma is NaN.
+template <typename T, int N>
+__device__ __forceinline__ void load_n_or_zeros(RowBuffer row, bool there, int idx, float (&out)[N]) {
+  constexpr int kBytes = N * (int)sizeof(T);
+  const int at = there ? idx * kBytes : kOutside;
+  if constexpr (kBytes == 8) {
+    struct alignas(8) Half {
+      T e[N];
+    } v = __builtin_bit_cast(Half, __builtin_amdgcn_raw_buffer_load_b64(row, at, 0, 0));
+#pragma unroll
+    for (int k = 0; k < N; ++k) out[k] = to_acc(v.e[k]);
+  } else {
+    constexpr int VN = Vec16<T>::n;
+#pragma unroll
+    for (int q = 0; q < N / VN; ++q) {
+      const auto v = __builtin_bit_cast(Vec16<T>, __builtin_amdgcn_raw_buffer_load_b128(row, at + q * 16, 0, 0));
+#pragma unroll
+      for (int k = 0; k < VN; ++k) out[q * VN + k] = to_acc(v.e[k]);
+    }
+  }
+}
 template <typename T, int VN, int VPL>
 struct Strip {
   Raw<T, VN> v[VPL];
@@ -859,6 +881,7 @@ __global__ __launch_bounds__(THREADS, WPE) void ln_bwd_kernel(
   const int nvec = C / VN;
   const float inv_c = 1.0f / (float)C;
 
+  const RowBuffer gamma_row = row_buffer(gamma, C * (int)sizeof(TP));
   float acc_g[VPL][VN], acc_b[VPL][VN], g[VPL][VN];
 #pragma unroll
   for (int j = 0; j < VPL; ++j) {
@@ -868,11 +891,7 @@ __global__ __launch_bounds__(THREADS, WPE) void ln_bwd_kernel(
       acc_g[j][k] = 0.f;
       acc_b[j][k] = 0.f;
     }
-    if constexpr (HAS_DX) {
-      load_n<TP, VN>(gamma + (idx < nvec ? idx : nvec - 1) * VN, g[j]);
-#pragma unroll
-      for (int k = 0; k < VN; ++k) g[j][k] = idx < nvec ? g[j][k] : 0.f;  // not the last vector's: 0 * inf is NaN
-    }
+    if constexpr (HAS_DX) load_n_or_zeros<TP, VN>(gamma_row, idx < nvec, idx, g[j]);
   }
 
   Strip<TDY, VN, VPL> dcur, dnxt;

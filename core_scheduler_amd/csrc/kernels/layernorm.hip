@@ -2215,6 +2215,11 @@ bool four_waves(int64_t rows, int64_t nvec, bool sums) {
   return !sums || (rows > 5 * step && nvec <= 56);
 }
 
+// A wave per row: more rows than these have 512 workgroups, so that a wave's fp32 chain of column sums is no longer than
+// with four waves per SIMD.  Error of dgamma and dbeta on 256, of that on 512: 1.08 at 131072 rows, 1.2 at 262144, 1.34 at a million.
+// (No slower: fp32 [262144,256] 142 / 142 us with ln_bwd_rows_kernel / now, bf16 [80000,1024] 90.5 / 89.1.)
+constexpr int64_t kOneWorkgroupRows = 65536;
+
 BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, const BwdWants &w = BwdWants{}) {
   BwdPlan b;
   const FastPlan p = aligned ? fast_plan(C, x_dtype) : FastPlan{};
@@ -2257,7 +2262,8 @@ BwdPlan bwd_plan(int64_t rows, int64_t C, int x_dtype, bool aligned, const BwdWa
     // call's sums in the launch [8192,1024] 20.1 / 16.6, [1500,512] 4.5 / 4.3.  Level at plain [16384,512] (14.9).
     b.kind = p.vpl <= 2 ? kBwdWave : kBwdRows;
     b.four_waves = b.kind == kBwdWave && four_waves(rows, nvec, w.sums);
-    b.blocks = ln_blocks(rows, 1, b.four_waves ? 2 * kLnBwdMaxBlocks : kLnBwdMaxBlocks, kLnBwdThreads);
+    const bool many_rows = b.kind == kBwdWave && rows > kOneWorkgroupRows;
+    b.blocks = ln_blocks(rows, 1, b.four_waves || many_rows ? 2 * kLnBwdMaxBlocks : kLnBwdMaxBlocks, kLnBwdThreads);
     b.fold_lds = (size_t)(kLnBwdThreads / kWave) * C * sizeof(float);
   }
   return b;

@@ -1889,8 +1889,10 @@ BlockPlan block_plan(int64_t rows, int64_t C, int x_dtype, bool backward, bool r
   // Forward with the residual, whole vectors: one workgroup of up to 12 waves per CU, whose loads are never waited for
   // ahead of time (see ln_fwd_block_kernel); 512 workgroups of 8 waves put more under way than the memory likes
   // ([4096,5120] bf16 30.9 us against 29.9, [16384,2304] 57.0 / 52.5, [16384,3584] 85.5 / 78.3).  Not where those make one
-  // step: [300,2304] 4.2 against 4.8.
-  const bool even_flow = !backward && residual && whole_vectors && (rows > 512 || p.gw > kLnBlockMaxWaves / 2);
+  // step: [300,2304] 4.2 against 4.8.  Nor fp16 of up to 8 waves, whose conversions want more of them: [4096,3584] 22.5 us
+  // on 512, 27.7 on 256, [8192,4096] 49.1 / 54.1.
+  const bool even_flow = !backward && residual && whole_vectors &&
+                         (p.gw > kLnBlockMaxWaves / 2 || (rows > 512 && x_dtype != CS_F16));
   // Backward: as many rows side by side as 16 waves hold, so that one workgroup per CU, hence 256
   // partial rows, keeps the CU busy ([12000,1003] fp32 40.3 us against 43.3 with 8 waves; 512
   // workgroups 41.2, and [4096,5120] bf16 49.9 against 41.9).  Forward: 8 waves and two workgroups

@@ -1830,25 +1830,43 @@ FastPlan fast_plan(int64_t C, int x_dtype) {
 // Grid caps: beyond these the waves loop over rows (with prefetch) instead of
 // the grid growing, which keeps the parameters in registers for many rows
 // and bounds the number of partial rows the backward pass leaves behind.
-// Forward: 512 workgroups of 4 waves, the two waves per SIMD that most of these kernels' registers allow: of twice as
-// many the second half starts when the first has ended, asks for its parameters again and ends with a part-filled
-// step.  1024 / 512 workgroups, us per call: bf16 [16384,768] with the residual 18.9 / 17.5, [16384,512] 14.1 / 12.3,
-// fp16 [16384,640] 21.5 / 17.1; without it [8192,1600] 13.6 / 11.4, [16384,1024] 15.4 / 13.8, [5000,3072] 14.5 / 13.0.
-// Rows of up to 32 vectors need few registers and keep 1024 (plain [50000,256] 11.3 / 12.9, [50000,64] 9.6 / 10.6).
 #ifndef CS_LN_FWD_MAX_BLOCKS
 #define CS_LN_FWD_MAX_BLOCKS 512
 #endif
-#ifndef CS_LN_FWD_MAX_BLOCKS_H1
-#define CS_LN_FWD_MAX_BLOCKS_H1 1024
-#endif
 constexpr int kLnFwdMaxBlocks = CS_LN_FWD_MAX_BLOCKS;
-constexpr int kLnFwdMaxBlocksNarrow = CS_LN_FWD_MAX_BLOCKS_H1;
 constexpr int kLnBwdMaxBlocks = CS_LN_BWD_MAX_BLOCKS;
 
 int ln_blocks(int64_t rows, int rows_per_wave, int cap, int threads = kLnThreads) {
   const int64_t rows_per_block = (int64_t)(threads / kWave) * rows_per_wave;
   const int64_t b = ceil_div(rows, rows_per_block);
   return (int)(b < cap ? b : cap);
+}
+
+// Forward: 512 workgroups of 4 waves, the two waves per SIMD that most of these kernels' registers allow: of twice as
+// many the second half starts when the first has ended, asks for its parameters again and ends with a part-filled
+// step.  us per call, 1024 / 512 workgroups: bf16 [16384,768] with the residual 18.9 / 17.5, [16384,512] 14.1 / 12.3,
+// fp16 [16384,640] 21.5 / 17.1; without it [8192,1600] 13.6 / 11.4, [16384,1024] 15.4 / 13.8, [5000,3072] 14.5 / 13.0.
+// 1024 still, us with them / with 512,
+// * without the residual: up to 64 vectors, whose registers let more waves in (bf16 [40000,320] 13.5 / 16.3, fp32 [20000,160]
+//   6.9 / 7.7, [50000,256] 11.3 / 12.9), fp32 up to 96 ([20000,320] 8.4 / 10.4, [20000,384] 9.4 / 11.2), and where 512 would make a second
+//   step less than half full of fp32 rows ([5000,1024] 7.6 / 8.2, [9000,448] 6.9 / 7.5, [2100,1280] 5.5 / 5.9) or of 65 to 96
+//   vectors (bf16 [9000,768] 7.0 / 7.5; from a step and a half on 512 are 10% the quicker);
+// * with it: up to 64 vectors of fp32 ([20000,160] 9.3 / 10.5) and of 16 bits up to 14336 rows ([9000,512] bf16 8.9 / 9.8, fp16
+//   10.8 / 11.8; but [16384,512] 13.6 / 11.9, 15.1 / 13.2), up to 128 (fp16 64) from 20481 to 32768 rows, where three or four steps
+//   of 512 are more than two of 1024 (by 2-13%), and fp32 rows of more than 384 from 10241 rows on ([14600,2048] 77 / 85).
+int fwd_blocks(int64_t rows, int rows_per_wave, int64_t nvec, bool residual, int x_dtype) {
+  const int64_t step = (int64_t)kLnFwdMaxBlocks * (kLnThreads / kWave) * rows_per_wave;
+  const bool fp32 = x_dtype == CS_F32;
+  bool twice = nvec <= kHalf;
+  if (!residual) {
+    const bool halves = nvec > kWave && nvec <= 3 * kHalf;
+    twice |= nvec <= kWave || (fp32 && halves) || ((fp32 || halves) && rows * 2 <= step * 3);
+  } else {
+    twice |= nvec <= kWave && (fp32 || rows <= 14336);
+    twice |= nvec <= (x_dtype == CS_F16 ? 1 : 2) * kWave && rows > 20480 && rows <= 32768;
+    twice |= fp32 && nvec > 6 * kWave && rows > 10240;
+  }
+  return ln_blocks(rows, rows_per_wave, twice ? 2 * kLnFwdMaxBlocks : kLnFwdMaxBlocks);
 }
 
 // Two vectors per lane and the residual: rows a wave normalises per step.  Two, so that the last step of the 512
@@ -1983,7 +2001,7 @@ int fwd_typed(const void *x, const void *gamma, const void *beta, void *y, void 
       if (half_vpl != 0) {
         const int groups = res ? (half_vpl == 1 ? CS_LN_ADD_ROWS_H1 : CS_LN_ADD_ROWS_H3)
                                : (half_vpl == 1 ? CS_LN_FWD_ROWS_H1 : CS_LN_FWD_ROWS_H3);
-        const dim3 grid((unsigned)ln_blocks(rows, 2 * groups, half_vpl == 1 ? kLnFwdMaxBlocksNarrow : kLnFwdMaxBlocks)),
+        const dim3 grid((unsigned)fwd_blocks(rows, 2 * groups, nvec, res != nullptr, x_dtype)),
             block(kLnThreads);
 #define CS_LN_FWD_H(VPL, R, HAS_RES)                                                                 \
   ln_fwd_rows_kernel<TX, TY, TP, VPL, R, CS_LN_FWD_PF, HAS_RES, kHalf><<<grid, block, 0, s>>>(       \
@@ -2007,7 +2025,7 @@ int fwd_typed(const void *x, const void *gamma, const void *beta, void *y, void 
                                 : p.vpl == 2 ? add_rows_vpl2(rows, kFp16)
                                              : CS_LN_ADD_ROWS_VPL4)
                              : p.fwd_rows;
-      const dim3 grid((unsigned)ln_blocks(rows, r_rows, kLnFwdMaxBlocks)), block(kLnThreads);
+      const dim3 grid((unsigned)fwd_blocks(rows, r_rows, nvec, res != nullptr, x_dtype)), block(kLnThreads);
 #define CS_LN_FWD(VPL, R, HAS_RES)                                                          \
   ln_fwd_rows_kernel<TX, TY, TP, VPL, R, CS_LN_FWD_PF, HAS_RES><<<grid, block, 0, s>>>(     \
       (const TX *)x, (const TP *)gamma, (const TP *)beta, (TY *)y, (float *)mean,           \
@@ -2035,7 +2053,7 @@ int fwd_typed(const void *x, const void *gamma, const void *beta, void *y, void 
   }
   if constexpr (!std::is_same_v<TX, double>) {
     if (aligned && wave_per_row8(rows, C, x_dtype, res != nullptr)) {
-      const dim3 grid((unsigned)ln_blocks(rows, 1, kLnFwdMaxBlocks)), block(kLnThreads);
+      const dim3 grid((unsigned)fwd_blocks(rows, 1, C / Vec16<TX>::n, res != nullptr, x_dtype)), block(kLnThreads);
       if (res) {
         ln_fwd_rows_kernel<TX, TY, TP, 8, 1, CS_LN_FWD_PF, true><<<grid, block, 0, s>>>(
             (const TX *)x, (const TP *)gamma, (const TP *)beta, (TY *)y, (float *)mean, (float *)rstd, rows, (int)C,

@@ -1,5 +1,5 @@
-"""Forward LayerNorm, a wave per row: 512 workgroups walk the rows in steps of one, two or four rows a wave, so what counts
-is row counts on either side of a full step, and of the line where the rows per step change."""
+"""Forward LayerNorm, a wave per row: 512 or 1024 workgroups walk the rows in steps of one, two or four rows a wave, so what counts
+is row counts on either side of a full step, and of the lines where the rows per step and the workgroups change."""
 import pytest
 import torch
 
@@ -10,7 +10,7 @@ BF16, F16, F32 = torch.bfloat16, torch.float16, torch.float32
 
 
 @pytest.mark.parametrize("C,dtype", [(1024, BF16), (520, F16), (260, F32), (1600, BF16), (1032, F16), (1024, F32), (768, BF16), (512, BF16), (2056, BF16)])
-@pytest.mark.parametrize("rows", [2049, 4096, 4097, 6145, 8191, 8193, 16385])
+@pytest.mark.parametrize("rows", [2049, 4096, 4097, 6145, 8191, 8193, 10241, 12289, 14337, 16385, 20481, 32769])
 def test_row_steps(C, dtype, rows):
     from core_scheduler_amd import ops
 

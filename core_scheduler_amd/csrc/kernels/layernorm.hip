@@ -1187,6 +1187,14 @@ __device__ __forceinline__ float row_sum(const float (&v)[VPT], int gw, int wave
   return row16_sum(w < gw ? r : 0.f);
 }
 
+// A wave's number, where UNIFORM known to be the same for all of its lanes: rows then have scalar addresses and descriptors,
+// and the statistics come by scalar loads.  Ragged rows without column sums, and fp32 ones, are the quicker without.
+template <bool UNIFORM>
+__device__ __forceinline__ int block_wave() {
+  const int wave = threadIdx.x >> 6;
+  return UNIFORM ? __builtin_amdgcn_readfirstlane(wave) : wave;
+}
+
 template <typename TX, typename TY, typename TP, int VPT, bool HAS_RES, bool UA, bool BY_LANE>
 __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
     const TX *x /* sum_out may be x: not restrict */, const TP *__restrict__ gamma, const TP *__restrict__ beta,
@@ -1194,7 +1202,7 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
     const TX *res, TX *sum_out, int gw, int groups) {
   constexpr int VN = Vec16<TX>::n;
   __shared__ float red[2][kLnBlockMaxWaves * (BY_LANE ? VPT * kWave : 1)];
-  const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & (kWave - 1), wave = block_wave<!UA>();
   const int group = wave / gw, lig = threadIdx.x - group * gw * kWave;
   const bool any_vec = C >= VN;
   const Lanes<VN, VPT, UA> own(C, gw, lig);
@@ -1394,7 +1402,7 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_bwd_block_kernel(
     bid -= side.blocks;
     nblocks -= side.blocks;
   }
-  const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & (kWave - 1), wave = block_wave<!UA || (HAS_DP && sizeof(TX) == 2)>();
   const int group = wave / gw, lig = threadIdx.x - group * gw * kWave;
   const bool any_vec = C >= VN;
   const Lanes<VN, VPT, UA> own(C, gw, lig);

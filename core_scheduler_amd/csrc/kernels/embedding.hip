@@ -1135,8 +1135,13 @@ constexpr int kListThreads = 512;
 constexpr int kListGroup = 4;  // waves that share an entry
 constexpr int kListEntries = kListThreads / kWave / kListGroup;
 constexpr int kListMost = 1024;
-constexpr int kListWhole = 192;  // (one id in every entry, x 768: 192 entries 21 us before and now, 256 would take 25)
-constexpr int kListVecs = 2;  // vectors a lane has of each row: a slice of the columns is 128 of them
+constexpr int kListWhole = 192;
+// Vectors a lane has of each row: a slice of the columns is 128 of them, and a run at most kWindow rows, one step of eight
+// for each of the four waves.  Runs of a whole list are up to kListWhole rows: 16-bit rows then have 16 in flight, of one
+// vector a lane, where the slices of 64 are not too many workgroups (one id in 192 entries x 768 into 1000 rows 11.8 / 7.5 us;
+// fp32 needs too many registers for that: 99 instead of 80, and 64 columns 4.8 / 5.2).
+constexpr int kListVecs = 2;
+constexpr int kListInFlight = 16;
 constexpr int64_t kListBlocks = 512;  // no more slices than make so many workgroups (1024 x 1600: 1024 41.7 us, 512 38.0)
 constexpr int64_t kListFillBytes = 64 << 10;  // zeros a workgroup writes (n = 123 x 768, 77 MB: 32 KB 14.4 us, 64 14.6, 256 16.0)
 constexpr int kListFillRows = 4096;  // most table rows a zero-filling workgroup looks after (a bit each in the LDS)
@@ -1151,7 +1156,7 @@ __device__ __forceinline__ uint32_t usable_id(IdxT raw, int64_t num_weights, int
 //   [0, entry_blocks)           kListEntries entries and a slice of the columns each
 //   + positions.blocks          position-table gradient
 //   + the rest                  zeros to the rows [blk * fill_rows, (blk + 1) * fill_rows) that no entry names
-template <typename T, typename IdxT>
+template <typename T, typename IdxT, int VECS>
 __global__ __launch_bounds__(kListThreads, 4) void emb_bwd_list_kernel(
     const T *__restrict__ dout, const IdxT *__restrict__ ids, T *__restrict__ dweight, uint32_t *__restrict__ sorted_id,
     float *__restrict__ partial, int n, int C, int64_t num_weights, int64_t padding_idx, int accumulate, int by_freq,
@@ -1329,9 +1334,9 @@ __global__ __launch_bounds__(kListThreads, 4) void emb_bwd_list_kernel(
 #pragma unroll
   for (int e = 0; e < kListEntries; ++e) any_long |= long_run[e] != 0;
   if (!any_long) return;
-  // the waves share the rows: eight of two vectors a lane in flight (a row past the run re-reads the last one, a vector
+  // the waves share the rows: kListInFlight vectors a lane in flight (a row past the run re-reads the last one, a vector
   // past the row the row's last one, and neither is added); a step's rows are added in pairs, the waves' sums in order
-  constexpr int kRows = 8, kVecs = kListVecs;
+  constexpr int kRows = kListInFlight / VECS, kVecs = VECS;
   for (int cb = slice * kWave * kVecs; cb < nvec; cb += slices * kWave * kVecs) {
     float acc[kVecs][VN] = {};
     for (int e0 = member; run > 1 && e0 < run; e0 += kListGroup * kRows) {
@@ -1354,7 +1359,11 @@ __global__ __launch_bounds__(kListThreads, 4) void emb_bwd_list_kernel(
           float x[kRows];
 #pragma unroll
           for (int r = 0; r < kRows; ++r) x[r] = e0 + r * kListGroup < run ? to_acc(v[r][j].e[k]) : 0.f;
-          acc[j][k] += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+#pragma unroll
+          for (int w = 1; w < kRows; w *= 2)
+#pragma unroll
+            for (int r = 0; r < kRows; r += 2 * w) x[r] += x[r + w];
+          acc[j][k] += x[0];
         }
     }
 #pragma unroll
@@ -1870,7 +1879,10 @@ int list_launch(const void *dout, const void *ids, void *dweight, char *ws, cons
   uint32_t *sorted_id = reinterpret_cast<uint32_t *>(ws + L.off_sorted_id);
   float *partial = reinterpret_cast<float *>(ws + L.off_partial);
   const int64_t pairs = ceil_div(n, (int64_t)kListEntries);
-  int64_t slices = ceil_div(C / Vec16<T>::n, (int64_t)kListVecs * kWave);
+  const bool in_windows = n > kListWhole;
+  const int64_t nvec = C / Vec16<T>::n;
+  const bool narrow = sizeof(T) == 2 && !in_windows && pairs * ceil_div(nvec, (int64_t)kWave) <= kListBlocks;
+  int64_t slices = ceil_div(nvec, (int64_t)(narrow ? 1 : kListVecs) * kWave);
   if (pairs * slices > kListBlocks) slices = pairs < kListBlocks ? kListBlocks / pairs : 1;
   const int64_t entry_blocks = pairs * slices;
   int64_t fill_rows = ceil_div(kListFillBytes, C * (int64_t)sizeof(T));
@@ -1879,11 +1891,15 @@ int list_launch(const void *dout, const void *ids, void *dweight, char *ws, cons
   const int64_t blocks = entry_blocks + positions.blocks + fill_blocks;
   if (blocks > 0x7fffffffLL) return CS_ERR_TOO_LARGE;
   if (blocks == 0) return CS_OK;
-  emb_bwd_list_kernel<T, IdxT><<<dim3((unsigned)blocks), dim3(kListThreads), 0, s>>>(
+  auto kernel = emb_bwd_list_kernel<T, IdxT, kListVecs>;
+  if constexpr (sizeof(T) == 2) {
+    if (narrow) kernel = emb_bwd_list_kernel<T, IdxT, 1>;
+  }
+  kernel<<<dim3((unsigned)blocks), dim3(kListThreads), 0, s>>>(
       (const T *)dout, (const IdxT *)ids, (T *)dweight, sorted_id, partial, (int)n, (int)C, num_weights, padding_idx,
       accumulate, by_freq, (int)entry_blocks, (int)slices, (int)fill_rows, positions);
   const int st = launch_status();
-  if (st != CS_OK || n <= kListWhole) return st;
+  if (st != CS_OK || !in_windows) return st;
   return finish_launch<T>(dout, sorted_id, partial, dweight, nullptr, n, C, accumulate, by_freq, L.n_windows, 0, 0, 1, 0, s);
 }
 

@@ -87,3 +87,18 @@ def test_windows_in_slices(n, C):
     assert torch.equal(ops.embedding_backward(dout.cuda(), ids.cuda(), V, dweight=got).cpu(), 2 * want)
     dwte, dwpe = ops.embedding_backward_fused(dout.view(1, n, C).cuda(), ids.view(1, n).cuda(), V)
     assert torch.equal(dwte.cpu(), want) and torch.equal(dwpe.cpu(), dout)
+
+
+@pytest.mark.parametrize("kind", ["one", "zipf", "any"])
+@pytest.mark.parametrize("n", [5, 64, 65, 129, 192])  # a run of a step of 16 rows for each of four waves, and more
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_whole_runs_of_16_bits(n, kind, dtype):
+    from core_scheduler_amd import ops
+
+    for C, V in ((8, 5000), (520, 40), (1032, 300), (3080, 60)):  # up to one slice of 64 vectors, two, three, and 128 to a lane's two
+        ids = _ids(kind, n, V)
+        dout = torch.randint(-8, 9, (n, C), generator=gen(28)).float()  # whole numbers: every order gives the same sums
+        keep = (ids >= 0) & (ids < V)
+        want = torch.zeros(V, C).index_add_(0, ids[keep], dout[keep])
+        got = ops.embedding_backward(dout.to(dtype).cuda(), ids.cuda(), V)
+        assert torch.equal(got.cpu(), want.to(dtype)), C

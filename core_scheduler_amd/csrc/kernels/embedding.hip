@@ -1129,8 +1129,8 @@ __global__ __launch_bounds__(kFinThreads, 5) void emb_bwd_finish_kernel(
 // 77 MB of zeros alone 11.9), [9,19] x 128 into 5238 10.1 / 6.1, 16 x 64 into 1000 8.2 / 5.6, [16,41] x 640 into 32434
 // 14.4 / 11.7, [1,500] x 512 fp32 added to 4000 rows 12.9 / 8.8, [1,1024] x 768 into 1000 rows 12.3 / 10.8 and into 50257
 // 22.1 / 21.2.  Longer lists are left to the sort: the comparisons grow with the square, and a hot id's runs gather
-// where its tokens are (all of 8192 x 768 this way: 26 / 49).  One id in every entry, the longest runs there are: 128
-// entries 21.0 / 18.4, 1024 entries 12.3 / 12.9.
+// where its tokens are (all of 8192 x 768 this way: 26 / 49).  One id in every entry, the longest runs there are: x 768
+// into 50257 rows 192 entries 21.5 / 19.1, 193 20.5 / 17.9, 1024 21.6 / 20.7.
 constexpr int kListThreads = 512;
 constexpr int kListGroup = 4;  // waves that share an entry
 constexpr int kListEntries = kListThreads / kWave / kListGroup;
@@ -1150,6 +1150,16 @@ template <typename IdxT>
 __device__ __forceinline__ uint32_t usable_id(IdxT raw, int64_t num_weights, int64_t padding_idx) {
   const int64_t id = (int64_t)raw;
   return id >= 0 && id < num_weights && id != padding_idx ? (uint32_t)id : kNoId;
+}
+
+// The pair of entries of the workgroup whose turn it is: of every window's the next comes first.  Runs of one id over the
+// whole list start at the first entry of each window, and workgroups go to the eight XCDs in turn: in the list's own order
+// all of them were on one (1024 entries x 768 into 50257 rows, not in any cache: 23.3 us, so 20.7).  Two slices use two XCDs,
+// which will do (512 x 1600 into 1000 rows 11.7 / 10.4, but with different ids 9.8 / 10.9).
+constexpr int kPairsAWindow = kWindow / kListEntries;
+__device__ __forceinline__ int list_pair(int turn, int pairs) {
+  const int window = turn / kPairsAWindow, first = window * kPairsAWindow;
+  return first + kPairsAWindow <= pairs ? first + (turn + window) % kPairsAWindow : turn;
 }
 
 // Launch layout, in block order:
@@ -1235,7 +1245,8 @@ __global__ __launch_bounds__(kListThreads, 4) void emb_bwd_list_kernel(
 
   // ---- the group's entry: its place among the sorted, and its segment
   const int entry = wave / kListGroup, member = wave % kListGroup;
-  const int pair = (int)blk / slices, slice = (int)blk - pair * slices;
+  const int turn = (int)blk / slices, slice = (int)blk - turn * slices;
+  const int pair = slices == 1 ? list_pair(turn, (n + kListEntries - 1) / kListEntries) : turn;
   const int p = pair * kListEntries + entry;
   const uint32_t my_id = p < n ? list[p] : kNoId;
   uint32_t from[kChunks];  // the entries with this id, from this one on: a bit each

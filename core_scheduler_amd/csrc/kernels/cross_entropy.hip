@@ -261,12 +261,15 @@ __device__ __forceinline__ VecE<T, EPV> load_e_stream(const T *p) {
   }
 }
 
+// Waves per SIMD that a narrow row's registers have to allow: workgroups are short, and rows that make a little more than
+// one round of the resident ones take two (fp16 [3000,3001] with fp32 gradients, 82 registers: 20.1 us, 16.3 with 80).
+constexpr int narrow_waves(int bytes, int access) { return bytes > 64 ? 4 : access == 16 ? 8 : 6; }
 // Narrow rows: a workgroup per row, the whole row in registers, VPT accesses of EPV elements a lane, all under way before
 // the first is used; as many waves as the row has such shares.  RAGGED: lanes own aligned vectors of the whole array, as in
 // the streaming kernel below.  What is no class column is overwritten with -inf in the packed registers, so that no pass
 // masks element by element; a lane past the row's end loads its last vector again.
 template <typename T, typename TD, int VPT, int EPV, bool RAGGED, int MOST_THREADS = kNarrowMostThreads>
-__global__ __launch_bounds__(MOST_THREADS) void ce_rows_kernel(
+__global__ __launch_bounds__(MOST_THREADS, narrow_waves(VPT *EPV * (int)sizeof(T), EPV * (int)sizeof(T))) void ce_rows_kernel(
     const T *logits, TD *dlogits, const int64_t *__restrict__ targets, float *__restrict__ row_loss,
     const int *__restrict__ ws_count, int64_t N, int64_t V, int64_t row_stride, int64_t ignore_index, int reduction,
     float dloss, const float *__restrict__ class_weight) {
@@ -364,9 +367,9 @@ __global__ __launch_bounds__(MOST_THREADS) void ce_rows_kernel(
     part[j] = e[0];
   }
 #pragma unroll
-  for (int w = VPT / 2; w > 0; w /= 2)
+  for (int w = VPT; w > 1; w = (w + 1) / 2)
 #pragma unroll
-    for (int j = 0; j < w; ++j) part[j] += part[j + w];
+    for (int j = 0; j < w / 2; ++j) part[j] += part[j + (w + 1) / 2];
   const float s = block_reduce(part[0], SumOp{}, 0.f, scratch);
 
   const float log2_s = __builtin_amdgcn_logf(s);  // v_log_f32 is log2
@@ -1520,7 +1523,8 @@ void launch_stream(const void *logits, void *dlogits, const int64_t *targets, fl
 }
 
 // Rows of up to 2048 vectors of 16 bytes, four accesses a lane (eight of 8 bytes for fp32 gradients of 16-bit logits; half
-// or a quarter of that where one wave then has the row) and as many waves as that takes: false where the row is too wide.
+// or a quarter of that where one wave then has the row, three quarters where those take no more waves) and as many waves as
+// that takes: false where the row is too wide.
 // Twice as wide where there are more than two rows per CU; of unpadded rows, whose edges take more instructions, one and a
 // half times.  (Before, one wave of eight accesses up to 512
 // vectors and four waves beyond; unpadded and weighted rows in two sweeps; wider ones by the streaming kernel.)
@@ -1531,6 +1535,8 @@ void launch_stream(const void *logits, void *dlogits, const int64_t *targets, fl
 // [2099,20215] 50.0 / 39.4, [1000,20215] 25.5 / 23.6, [6000,20215] fp16 weighted 119 / 88, [4096,32000] 97 / 89,
 // [4096,20000] with fp32 gradients 114 / 92; but unpadded [4096,32001] 106 / 113, [300,30000] 14.1 / 15.4, fp32
 // [338,15424] 13.6 / 14.6.
+// Three quarters, four accesses a lane (or eight) / three: unpadded fp16 [3000,4097] 19.4 / 18.2, [3000,2001] with fp32 gradients
+// 15.9 / 14.9, the loss alone of padded bf16 [30000,2624] 39 / 34.8, fp16 [9000,3008] 17.1 / 15.7.
 template <typename T, typename TD, bool RAGGED>
 bool launch_narrow(const void *logits, void *dlogits, const int64_t *targets, float *row_loss, const int *ws_count,
                    int64_t N, int64_t V, int64_t row_stride, int64_t ignore_index, int reduction, float dloss,
@@ -1548,6 +1554,8 @@ bool launch_narrow(const void *logits, void *dlogits, const int64_t *targets, fl
     CS_CE_NARROW(U / 4);
   } else if (nvec <= kWave * U / 2) {
     CS_CE_NARROW(U / 2);
+  } else if (ceil_div(nvec, (int64_t)(kWave * U * 3 / 4)) == ceil_div(nvec, (int64_t)(kWave * U))) {
+    CS_CE_NARROW(U * 3 / 4);
   } else {
     CS_CE_NARROW(U);
   }

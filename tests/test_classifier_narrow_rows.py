@@ -19,6 +19,10 @@ BF16, F16, F32 = torch.bfloat16, torch.float16, torch.float32
     (2, 16384, 16384, BF16, BF16), (2, 16377, 16392, BF16, BF16),
     (2, 8161, 8161, F32, F32), (2, 8192, 8192, F32, F32),
     (2, 16321, 16321, F16, F32), (2, 16384, 16384, BF16, F32),
+    # three accesses a lane of two waves, and of three: the widest rows, and the next ones
+    (3, 3072, 3072, BF16, BF16), (3, 3073, 3080, F16, F16), (3, 4545, 4545, F16, F16), (3, 4546, 4546, BF16, BF16),
+    (3, 1536, 1536, F32, F32), (3, 1540, 1540, F32, F32), (3, 2257, 2257, F32, F32), (3, 3009, 3009, F16, F32),
+    (3, 3010, 3010, BF16, F32), (3, 4608, 4608, BF16, F32),
     (513, 24513, 24513, BF16, BF16), (513, 24514, 24514, BF16, BF16), (513, 32767, 32768, F16, F16),
     (513, 12257, 12257, F32, F32), (513, 24512, 24513, BF16, F32), (513, 32760, 32768, BF16, F32),
 ])

@@ -1119,12 +1119,13 @@ __global__ __launch_bounds__(BLOCK, 6) void ce_loss_rows_kernel(
 constexpr int kWideU = 2;  // 16-byte vectors per lane and chunk
 static_assert(kWideU == 2, "the chunk sum below adds two vector sums");
 
-template <typename T, typename TD, int BLOCK>
-__global__ __launch_bounds__(BLOCK, 8) void ce_rows_wide_kernel(
+template <typename T, typename TD>
+__global__ __launch_bounds__(1024, 8) void ce_rows_wide_kernel(
     const T *logits, TD *dlogits, const int64_t *__restrict__ targets, float *__restrict__ row_loss,
     const int *__restrict__ ws_count, int64_t N, int64_t V, int64_t row_stride,
     int64_t ignore_index, int reduction, float dloss, const float *__restrict__ class_weight) {
   constexpr int VN = Vec16<T>::n;
+  constexpr int BLOCK = 1024;
   constexpr int kWaves = BLOCK / kWave;
   constexpr int kTailLane = 32;  // lanes [0, VN) own head elements, [32, 32 + VN) tail elements
   static_assert(VN <= kTailLane, "head and tail lanes overlap");
@@ -1473,7 +1474,7 @@ void launch_wide(const void *logits, void *dlogits, const int64_t *targets, floa
                  int reduction, float dloss, const float *class_weight, hipStream_t s) {
   const int64_t cus = compute_units();
   const dim3 grid((unsigned)(N < 2 * cus ? N : 2 * cus));
-  ce_rows_wide_kernel<T, TD, 1024><<<grid, dim3(1024), 0, s>>>(
+  ce_rows_wide_kernel<T, TD><<<grid, dim3(1024), 0, s>>>(
       (const T *)logits, (TD *)dlogits, targets, row_loss, ws_count, N, V, row_stride, ignore_index,
       reduction, dloss, class_weight);
 }
@@ -1657,11 +1658,13 @@ int launch_rows(const void *logits, void *dlogits, const int64_t *targets, float
       }
       return launch_status();
     }
-    // Unpadded rows that fill little of the streaming plan take two sweeps: with fp32 gradients of 16-bit logits rows
-    // of up to six of its 13 accesses ([1030,18001] bf16 39.6 us streamed, 35.0 in two sweeps, [257,22001] 19.1 / 17.1,
-    // [3100,22001] 100 / 103; [3100,26001] 108 / 116), and the loss alone of more than two rows per CU of four to six
-    // of its seven ([600,38001] 21.4 / 19.5, [860,46001] 27.8 / 27.0; but [600,50257] 22.3 / 23.5).  So few rows come here
-    // for the loss alone only in separate phases, or with a workspace that has no room for their splits (loss_splits).
+    // Unpadded rows that fill little of the streaming plan take two sweeps: with fp32 gradients of 16-bit logits the few rows
+    // of up to 24576 columns that launch_narrow leaves (two per CU; us streamed / in two sweeps, bf16 [64,18001] 10.7 / 10.5,
+    // [257,18001] 16.8 / 15.6, [257,22001] 17.7 / 17.5, weighted rows and fp16 10-20% in favour of the two sweeps from 257 to 400
+    // rows; but [512,22001] 19.8 / 21.3, [512,24001] 20.3 / 22.7; wider ones, [3100,26001] 108 / 116), and the loss alone of more than
+    // two rows per CU of four to six of its seven accesses ([600,38001] 21.4 / 19.5, [860,46001] 27.8 / 27.0; but [600,50257]
+    // 22.3 / 23.5).  So few rows come here for the loss alone only in separate phases, or with a workspace that has no room
+    // for their splits (loss_splits).
     const bool sparse = sizeof(TD) > sizeof(T) ? row_stride <= 24 * 1024
                                                : sizeof(T) == 2 && dlogits == nullptr && N > 2 * cus &&
                                                      row_stride > 32 * 1024 && row_stride <= 48 * 1024;

@@ -691,7 +691,7 @@ __device__ __forceinline__ void ln_columns_wide(const TDY *__restrict__ dy, cons
 // ----------------------------------------------------------- fast backward
 // Rows of 4 vectors per lane.  One wave per row, the row (dy and x) in registers, gamma and the per-column partial sums in
 // registers for all rows a wave visits (rows gw, gw + n_waves, ...).  No software prefetch:
-// WPE waves per SIMD are resident (the launch bound asks the compiler for that), so while one
+// two waves per SIMD are resident (the launch bound asks the compiler for that), so while one
 // wave waits for its row the others compute; measured on MI355X this beats two rows per wave
 // with the next step's rows prefetched ([16384,1600] bf16: 32.8 -> 30.3 us) because twice as many
 // waves are in flight with half the registers each.
@@ -701,14 +701,13 @@ __device__ __forceinline__ void ln_columns_wide(const TDY *__restrict__ dy, cons
 // HAS_DRES: dx_out = dx + dresidual, the gradient add that follows LayerNorm::backward on the
 // residual stream; dx is rounded to its type first, then the sum, as two kernels would.
 // DIRECT: the launch's first workgroups take the column sums of this very call from its rows (ln_columns_direct).
-template <typename TDY, typename TX, typename TDX, typename TP, int VPL, int WPE, bool HAS_DX,
-          bool HAS_DP, bool HAS_DRES, bool DIRECT = false>
-__global__ __launch_bounds__(kLnBwdThreads, WPE) void ln_bwd_rows_kernel(
+template <typename TDY, typename TX, typename TDX, typename TP, bool HAS_DX, bool HAS_DP, bool HAS_DRES, bool DIRECT = false>
+__global__ __launch_bounds__(kLnBwdThreads, 2) void ln_bwd_rows_kernel(
     const TDY *__restrict__ dy, const TX *__restrict__ x, const float *__restrict__ mean,
     const float *__restrict__ rstd, const TP *__restrict__ gamma, TDX *dx,
     float *__restrict__ partial, int64_t rows, int C, const TDX *dres /* dx may be dres */,
     const LnPending pend) {
-  constexpr int VN = Vec16<TX>::n;
+  constexpr int VN = Vec16<TX>::n, VPL = 4;
   extern __shared__ float lds[];  // [waves per block][C], at least 16 x 32 floats with pending sums
   if ((int)blockIdx.x < pend.blocks) {
     if constexpr (DIRECT) {
@@ -1343,8 +1342,6 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
     }
     return;
   }
-  // Every step requests its two rows, there or not, and the first stands before the loop: what is under way at the
-  // loop's head is then the same whichever way it was reached, and the compiler waits for exactly the row it needs.
   // Every step requests two rows, there or not, and the first step stands before the loop: what is under way at the
   // loop's head is then the same whichever way it was reached, and the compiler waits for exactly the row it needs.
   const auto step = [&] {
@@ -2248,12 +2245,12 @@ bool general_rows(const BwdWants &w, const BlockPlan &b, int64_t rows, int64_t C
 // us per call, two waves / four.
 // One vector per lane, dx alone: there are no column sums in the registers.  bf16 [3000,512] 3.95 / 3.76, [8192,512] 6.5 /
 // 5.8, [30000,512] 18.8 / 16.8, fp32 [8192,256] 6.1 / 5.4.  With the sums, many rows of up to 56 vectors, which leave lanes
-// idle; plain / with dresidual / the sums alone: fp16 [8192,384] 9.4 / 9.7, 10.1 / 10.5, 8.0 / 8.2, [14000,384] 12.6 / 11.5,
-// 13.5 / 13.0, 10.3 / 9.4, bf16 [60000,264] 34.2 / 24.6, 37.2 / 29.5, 26.2 / 18.3, fp32 [14000,192] 11.7 / 10.7, 12.4 / 12.0, 9.6 / 8.7.
-// Of 57 to 64 vectors dy, x and dresidual fill the memory by themselves, while plain rows and the sums alone do not: bf16
-// [14000,512] 13.2 / 13.2, 14.8 / 15.0, 10.4 / 10.3, [60000,512] 38.5 / 36.1, 44.2 / 46.9, 28.4 / 23.9, fp32 [60000,256] 36.4 /
-// 35.0, 43.1 / 46.2, 26.7 / 23.0.  All forms of a call have to leave the same partial rows (the split form, which is asked
-// for them without knowing of a dx or dresidual, gives the bits of the single call), and dresidual is what training has.
+// idle; plain / with dresidual / the sums alone: bf16 [14000,264] 11.8 / 11.1, 12.3 / 12.2, 9.0 / 9.0, [60000,264] 30.8 / 25.7, 33.7 /
+// 30.8, 20.5 / 19.4, fp32 [14000,160] 11.3 / 10.1, 11.7 / 10.6, 8.0 / 8.4, [60000,160] 30.3 / 24.1, 31.9 / 29.4, 18.4 / 18.2 (but fp32
+// [14000,132] 11.6 / 11.6, 11.7 / 11.9, 8.6 / 10.2).  Of 57 to 64 vectors rows with dresidual fill the memory with the two: bf16
+// [60000,512] 37.8 / 36.1, 45.2 / 46.9, 23.6 / 23.9.  All forms of a call have to leave the same partial rows (the split form,
+// which is asked for them without knowing of a dx or dresidual, gives the bits of the single call), and dresidual is what
+// training has.
 // Two vectors per lane, dx alone: fp16 [8192,896] 9.7 / 8.8, [12289,896] 13.3 / 12.6, bf16 [5000,1024] 7.4 / 7.0, [16384,1024]
 // 17.8 / 17.7; not where those rows make two steps or fewer of the two waves (bf16 [4096,1024] 5.3 / 5.9, fp32 [4096,400]
 // 4.5 / 4.9), or so many that their rows in flight are the better use of the memory ([30000,1024] 31.5 / 32.7, fp16
@@ -2526,7 +2523,7 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
                            true, false, HAS_DRES, true>(dy, x, mean, rstd, gamma, dx, workspace, rows, C, dres, side,  \
                                                         blocks, lds, s);                                               \
   } else {                                                                                                             \
-    ln_bwd_rows_kernel<TDY, TX, TDX, TP, 4, 2, true, false, HAS_DRES, true><<<grid, block, lds, s>>>(                  \
+    ln_bwd_rows_kernel<TDY, TX, TDX, TP, true, false, HAS_DRES, true><<<grid, block, lds, s>>>(                        \
         (const TDY *)dy, (const TX *)x, (const float *)mean, (const float *)rstd, (const TP *)gamma, (TDX *)dx,        \
         (float *)workspace, rows, (int)C, (const TDX *)dres, side);                                                    \
     st = launch_status();                                                                                              \
@@ -2557,8 +2554,9 @@ int bwd_typed(const void *dy, const void *x, const void *mean, const void *rstd,
       if (pend.blocks != 0 && lds < pend_lds) lds = pend_lds;
       const dim3 grid((unsigned)(blocks + pend.blocks)), block((unsigned)plan.threads);
       int st = CS_OK;
-#define CS_LN_BWD(VPL, WPE, HAS_DX, HAS_DP, HAS_DRES)                                       \
-  ln_bwd_rows_kernel<TDY, TX, TDX, TP, VPL, WPE, HAS_DX, HAS_DP, HAS_DRES>                  \
+// (the first two arguments are CS_LN_BWD_MASK's and have no use here)
+#define CS_LN_BWD(UNUSED, UNUSED_TOO, HAS_DX, HAS_DP, HAS_DRES)                             \
+  ln_bwd_rows_kernel<TDY, TX, TDX, TP, HAS_DX, HAS_DP, HAS_DRES>                            \
       <<<grid, block, lds, s>>>((const TDY *)dy, (const TX *)x, (const float *)mean,        \
                                 (const float *)rstd, (const TP *)gamma, (TDX *)dx,          \
                                 (float *)workspace, rows, (int)C, (const TDX *)dres, pend)

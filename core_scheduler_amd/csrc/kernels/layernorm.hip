@@ -1187,7 +1187,10 @@ __device__ __forceinline__ float row_sum(const float (&v)[VPT], int gw, int wave
 }
 
 // A wave's number, where UNIFORM known to be the same for all of its lanes: rows then have scalar addresses and descriptors,
-// and the statistics come by scalar loads.  Ragged rows without column sums, and fp32 ones, are the quicker without.
+// and the statistics come by scalar loads.  Ragged rows of one fp32 vector a lane, and dx alone of one vector a lane, are the quicker
+// without (fp32 [40000,65] with dresidual 22.6 us uniform, 18.9 by lane, forward [10000,300] 6.6 / 6.1, dx alone [6144,3] 4.35 /
+// 3.8); the others not, as it takes a dozen registers (bf16 forward [4096,7001] 28.7 / 35.1, with the residual [4096,5001]
+// 39.1 / 45.7).
 template <bool UNIFORM>
 __device__ __forceinline__ int block_wave() {
   const int wave = threadIdx.x >> 6;
@@ -1201,7 +1204,7 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_fwd_block_kernel(
     const TX *res, TX *sum_out, int gw, int groups) {
   constexpr int VN = Vec16<TX>::n;
   __shared__ float red[2][kLnBlockMaxWaves * (BY_LANE ? VPT * kWave : 1)];
-  const int lane = threadIdx.x & (kWave - 1), wave = block_wave<!UA>();
+  const int lane = threadIdx.x & (kWave - 1), wave = block_wave<(!UA || VPT > 1 || sizeof(TX) == 2)>();
   const int group = wave / gw, lig = threadIdx.x - group * gw * kWave;
   const bool any_vec = C >= VN;
   const Lanes<VN, VPT, UA> own(C, gw, lig);
@@ -1399,7 +1402,7 @@ __global__ __launch_bounds__(kLnBlockMaxWaves *kWave) void ln_bwd_block_kernel(
     bid -= side.blocks;
     nblocks -= side.blocks;
   }
-  const int lane = threadIdx.x & (kWave - 1), wave = block_wave<!UA || (HAS_DP && sizeof(TX) == 2)>();
+  const int lane = threadIdx.x & (kWave - 1), wave = block_wave<(!UA || VPT > 1 || (HAS_DP && sizeof(TX) == 2))>();
   const int group = wave / gw, lig = threadIdx.x - group * gw * kWave;
   const bool any_vec = C >= VN;
   const Lanes<VN, VPT, UA> own(C, gw, lig);
